@@ -95,14 +95,13 @@ typedef struct {
                              push per colour class) as one captured hipGraph
                              (default); 0 = launch them one by one.  profile = 1
                              always launches them one by one. */
-  int tile_order;         /* tile distance field that orders the relabel
-                             passes of graphs of more than 2048 tiles: 0 =
-                             separable taxicab distance transform (default, D
-                             launches), 1 = jump flooding
-                             (graphcut_bfs_block.cl:43-63, 2 ceil(log2) + 2
-                             launches); the distances are identical.  Cut
-                             and tag passes, and every pass of a smaller
-                             graph, take the tiles in colour order */
+  int tile_order;         /* method of the tile distance field
+                             (jfc_debug_tile_order): 0 = separable taxicab
+                             distance transform (default), 1 = jump flooding
+                             (graphcut_bfs_block.cl:43-63); the distances are
+                             identical.  Solves take their tiles in colour
+                             order and their relabels run on regions of 4096
+                             nodes, neither of which the field orders */
   int method;             /* JFC_METHOD_JFCUT (0): tile push-relabel in LDS;
                              JFC_METHOD_FASTCUT (1): the widget's Fast-Cut
                              comparator (radioButtonCutMethodJFCut unchecked,
@@ -132,8 +131,6 @@ typedef struct {
 #define JFC_TILE_64x4 2
 #define JFC_TILE_16x16 3
 #define JFC_TILE_8x8x4 4
-/* 32x4x2 push tiles (whole 128-byte rows) run their global relabels on
- * 8x8x4 tiles, whose relabel fronts cross half as many tiles in y and z. */
 #define JFC_TILE_32x4x2 5
 
 typedef struct {
@@ -141,12 +138,12 @@ typedef struct {
   int converged;            /* 1 if every instance reached the certificate */
   int sweeps;               /* push-relabel sweeps run */
   int global_relabels;      /* exact global relabels run */
-  int relabel_passes;       /* tile passes inside the global relabels */
+  int relabel_passes;       /* region passes inside the global relabels */
   int cut_passes;           /* tile passes of the canonical-cut search */
   int certificate_failures; /* cut searches that still found an augmenting path */
   int64_t push_tiles;       /* tile visits of the push-relabel kernel */
   int64_t push_launches;    /* push-relabel kernel launches */
-  int64_t relabel_tiles;    /* tile visits of the relabel kernel */
+  int64_t relabel_tiles;    /* region visits of the relabel kernel */
   int64_t cut_tiles;        /* tile visits of the cut kernel */
   int64_t push_bytes;       /* algorithmic HBM bytes of the push-relabel visits */
   double ms_total;          /* device time of the solve (HIP events) */

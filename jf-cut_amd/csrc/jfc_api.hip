@@ -107,11 +107,11 @@ std::map<std::string, Tuned> g_tune;
 
 int log2_round(double v) { return v <= 1.0 ? 0 : (int)std::lround(std::log2(v)); }
 
-// Device counters (int64): [0] push tile visits, [1] relabel tile visits,
-// [2] cut tile visits, [4] tag tile visits, [kIterSlots, +64) local
-// iterations of the push kernel (workgroup b adds to slot b % 64, so no
-// single address takes one atomic per workgroup).
-constexpr int kIterSlots = 5, kTotals = kIterSlots + 64;
+// Device counters (int64): [0] push tile visits, [2] cut tile visits, [4] tag
+// tile visits, [kIterSlots, +64) local iterations of the push kernel,
+// [kRegionSlots, +64) region visits of the relabel passes (workgroup b adds
+// to slot b % 64, so no single address takes one atomic per workgroup).
+constexpr int kIterSlots = 5, kRegionSlots = kIterSlots + 64, kTotals = kRegionSlots + 64;
 // Graphs of at most this many tiles: a search pass gives every tile a
 // workgroup of its own or nearly (a device of 256 compute units keeps
 // several tile visits per unit resident), so its passes skip the distance
@@ -167,31 +167,23 @@ struct jfc_graph {
   int *d_ctr = nullptr;
   unsigned char *d_flag = nullptr, *d_dirty = nullptr, *d_seed = nullptr;
   unsigned char *d_dirty2 = nullptr;  // second dirty buffer of small-graph searches
-  unsigned char *d_defi = nullptr;  // tiles that may hold a deficit node
-  int gr_tag = 1;                   // tag of the last global relabel's heights
   unsigned char *d_mat = nullptr;  // per tile: residual planes written this solve
   unsigned char *d_hmat = nullptr; // per tile: heights stored this solve
   unsigned char *d_touched = nullptr;  // per tile: planes or masks written by a flush
-  int *d_jf0 = nullptr, *d_jf1 = nullptr, *d_tdist = nullptr, *d_hist = nullptr,
-      *d_order = nullptr;
-  // The tiling of the 3D global relabel when it is not the push tiling:
-  // 32x4x2 push tiles read whole 128-byte rows (an 8x8x4 tile's rows are 32
-  // bytes), but a relabel front crosses about one tile per pass, and 32x4x2
-  // tiles are half as deep in y and z, so their relabels run on 8x8x4 tiles
-  // (the 2560x1440x50 video volume: push 1.48 ms on 32x4x2 tiles against
-  // 2.81 on 8x8x4, relabel 2.95 ms on 8x8x4 against 4.56 on 32x4x2).  shape 0: the relabel runs on
-  // the push tiling.  The relabel writes the push tiling's active flags.
-  struct RelabelTiles {
-    int shape = 0;
+  // The regions of the global relabel (jfc_region.hip), the same for every
+  // push tile shape: descriptors and tables like the push tiling's, the marks
+  // of two passes, the packed bit planes and the borders' distances.
+  struct Regions {
     std::vector<InstDesc> inst;
     InstDesc *d_inst = nullptr;
     int *d_tile_inst = nullptr;
-    int ntiles = 0, max_tile_dim = 1, nbins = 2;
-    unsigned char *d_dirty = nullptr, *d_defi = nullptr;
-    int *d_jf0 = nullptr, *d_jf1 = nullptr, *d_tdist = nullptr, *d_hist = nullptr,
-        *d_order = nullptr, *d_lines = nullptr;
-    int lines_total[3] = {0, 0, 0};
-  } rt;
+    int n = 0;
+    unsigned char *d_dirty[2] = {nullptr, nullptr};
+    int *d_any = nullptr;  // 4 words: a mark is set for pass p (slot p % 4)
+    RegionBuf buf{nullptr, nullptr, nullptr, 0};
+    int tag = 1;           // of the last relabel
+    int seq = 0;           // passes run, the number their posted words carry
+  } rg;
   // One device block holds every word a solve reads back at its end (one
   // copy): the per-instance sums, the remaining deficits, the counters, the
   // sweep state and the flag words, in this order (res_words long longs).
@@ -201,8 +193,6 @@ struct jfc_graph {
   long long *d_def = nullptr;  // in d_res; per instance: remaining deficit after the cut
   long long *d_energy = nullptr;  // per instance: cut energy (jfc_get_energy)
   int *d_row_off = nullptr;    // per instance: first row; [count] = rows
-  int *d_lines = nullptr;      // per axis: prefix count of tile lines per instance
-  int lines_total[3] = {0, 0, 0};
   int nrows = 0;
   int *d_sweep = nullptr;
   int sweep_cap = 0;
@@ -241,8 +231,9 @@ struct jfc_graph {
   } *pin = nullptr;
   // Pinned copy of d_res (the solve's results).
   long long *pin_res = nullptr;
-  // Stop words the sweeps post (k_sweep_end), in fine-grained pinned memory
-  // the device writes through to; d_ring is its device address.
+  // Stop words the sweeps post (k_sweep_end), then the words of two groups
+  // of relabel passes, in fine-grained pinned memory the device writes
+  // through to; d_ring is its device address.
   int *ring = nullptr, *d_ring = nullptr;
   hipEvent_t cnt_ev[2] = {nullptr, nullptr};
   hipEvent_t stop_ev[kStopRing] = {};
@@ -261,7 +252,7 @@ struct jfc_graph {
     if (hipHostMalloc((void **)&pin, sizeof(HostPin), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void **)&pin_res, res_words * sizeof(long long), hipHostMallocDefault) !=
             hipSuccess ||
-        hipHostMalloc((void **)&ring, kStopRing * sizeof(int), hipHostMallocCoherent) !=
+        hipHostMalloc((void **)&ring, (kStopRing + 2) * sizeof(int), hipHostMallocCoherent) !=
             hipSuccess ||
         hipHostGetDevicePointer((void **)&d_ring, ring, 0) != hipSuccess) {
       (void)hipGetLastError();
@@ -298,16 +289,9 @@ struct jfc_graph {
   void release_tiles() {
     drop_graphs();
     dfree(d_tile_inst); dfree(d_color_tiles); dfree(d_list[0]); dfree(d_list[1]);
-    dfree(d_flag); dfree(d_dirty); dfree(d_dirty2); dfree(d_seed); dfree(d_defi); dfree(d_jf0);
-    dfree(d_jf1);
-    dfree(d_tdist); dfree(d_hist); dfree(d_order); dfree(d_inst); dfree(d_mat);
+    dfree(d_flag); dfree(d_dirty); dfree(d_dirty2); dfree(d_seed); dfree(d_inst); dfree(d_mat);
     dfree(d_hmat);
     dfree(d_touched);
-    dfree(d_lines);
-    dfree(rt.d_inst); dfree(rt.d_tile_inst); dfree(rt.d_dirty); dfree(rt.d_defi);
-    dfree(rt.d_jf0); dfree(rt.d_jf1); dfree(rt.d_tdist); dfree(rt.d_hist); dfree(rt.d_order);
-    dfree(rt.d_lines);
-    rt = RelabelTiles{};
   }
   void release_aux() {
     if (aux_fork) (void)hipEventDestroy(aux_fork);
@@ -321,6 +305,9 @@ struct jfc_graph {
   }
   void release() {
     release_tiles();
+    dfree(rg.d_inst); dfree(rg.d_tile_inst); dfree(rg.d_dirty[0]); dfree(rg.d_dirty[1]);
+    dfree(rg.d_any); dfree(rg.buf.packed); dfree(rg.buf.base); dfree(rg.buf.border);
+    rg = Regions{};
     dfree(cs); dfree(ct); dfree(c0); dfree(cap); dfree(e); dfree(h); dfree(lab); dfree(tag);
     dfree(d_ctr); dfree(d_res); dfree(d_sweep); dfree(d_energy); dfree(d_row_off);
     d_red = d_total = d_def = nullptr;
@@ -364,11 +351,6 @@ struct jfc_graph {
                  inst.empty() ? InstDesc{} : inst[0]};
   }
   Planes planes() const { return Planes{e, h, cap, c0, cs, ct, lab, Ntot, rmask}; }
-  TileLines lines() const {
-    const int n1 = (int)inst.size() + 1;
-    return TileLines{{d_lines, d_lines + n1, d_lines + 2 * n1},
-                     {lines_total[0], lines_total[1], lines_total[2]}};
-  }
   long long inst_nodes(int i) const {
     return (long long)inst[i].nx * inst[i].ny * inst[i].nz;
   }
@@ -421,20 +403,6 @@ struct jfc_graph {
             cls[c].push_back(t);
           }
     }
-    // tile lines along x, y, z per instance (separable distance transform)
-    const int n1 = (int)inst.size() + 1;
-    std::vector<int> lines(3 * n1, 0);
-    for (size_t i = 0; i < inst.size(); ++i) {
-      const InstDesc &I = inst[i];
-      const long long per[3] = {(long long)I.ty * I.tz, (long long)I.tx * I.tz,
-                                (long long)I.tx * I.ty};
-      for (int a = 0; a < 3; ++a) {
-        const long long nx = lines[a * n1 + i] + per[a];
-        if (nx >= (1LL << 31) / 4) return fail(JFC_ERR_INVALID, "too many tile lines");
-        lines[a * n1 + i + 1] = (int)nx;
-      }
-    }
-    for (int a = 0; a < 3; ++a) lines_total[a] = lines[a * n1 + n1 - 1];
     std::vector<int> flat;
     color_off.assign(ncolors + 1, 0);
     for (int c = 0; c < ncolors; ++c) {
@@ -446,56 +414,30 @@ struct jfc_graph {
     if ((rc = dalloc(&d_inst, inst.size(), "instances")) ||
         (rc = dalloc(&d_tile_inst, ntiles, "tile table")) ||
         (rc = dalloc(&d_color_tiles, ntiles, "colour classes")) ||
-        (rc = dalloc(&d_list[0], list_cap(sh), "tile list")) ||
-        (rc = dalloc(&d_list[1], list_cap(sh), "tile list")) ||
+        (rc = dalloc(&d_list[0], ntiles, "tile list")) ||
+        (rc = dalloc(&d_list[1], ntiles, "tile list")) ||
         (rc = dalloc(&d_flag, ntiles, "tile flags")) ||
         (rc = dalloc(&d_dirty, ntiles, "tile flags")) ||
         (rc = dalloc(&d_dirty2, ntiles, "tile flags")) ||
         (rc = dalloc(&d_seed, ntiles, "tile seeds")) ||
-        (rc = dalloc(&d_defi, ntiles, "tile seeds")) ||
-        (rc = dalloc(&d_jf0, ntiles, "jump flooding")) ||
-        (rc = dalloc(&d_jf1, ntiles, "jump flooding")) ||
-        (rc = dalloc(&d_tdist, ntiles, "tile distance")) ||
-        (rc = dalloc(&d_hist, nbins, "tile histogram")) ||
-        (rc = dalloc(&d_order, ntiles, "tile order")) ||
         (rc = dalloc(&d_mat, ntiles, "tile states")) ||
         (rc = dalloc(&d_hmat, ntiles, "tile states")) ||
-        (rc = dalloc(&d_touched, ntiles, "tile states")) ||
-        (rc = dalloc(&d_lines, 3 * n1, "tile lines")))
+        (rc = dalloc(&d_touched, ntiles, "tile states")))
       return rc;
-    JFC_HIP(hipMemcpy(d_lines, lines.data(), lines.size() * sizeof(int), hipMemcpyHostToDevice));
     JFC_HIP(hipMemcpy(d_inst, inst.data(), inst.size() * sizeof(InstDesc), hipMemcpyHostToDevice));
     JFC_HIP(hipMemcpy(d_tile_inst, tile_inst.data(), ntiles * sizeof(int), hipMemcpyHostToDevice));
     JFC_HIP(hipMemcpy(d_color_tiles, flat.data(), ntiles * sizeof(int), hipMemcpyHostToDevice));
-    return sh == SH_32x4x2 ? build_relabel_tiles(SH_8x8x4) : JFC_OK;
+    return JFC_OK;
   }
 
-  // Tile count of shape sh over the instances.
-  long long count_tiles(int sh) const {
+  // The relabel's region tables and buffers (once per graph).
+  int build_regions() {
+    const bool d3 = dim == 3;
     int tw, th, td;
-    shape_dims(sh, &tw, &th, &td);
-    long long n = 0;
-    for (const auto &I : inst)
-      n += (long long)((I.nx + tw - 1) / tw) * ((I.ny + th - 1) / th) * ((I.nz + td - 1) / td);
-    return n;
-  }
-  // Capacity of the compaction lists: the tiles of the push tiling, or of
-  // the relabel tiling where that is another.
-  long long list_cap(int sh) const {
-    return sh == SH_32x4x2 ? std::max(count_tiles(sh), count_tiles(SH_8x8x4)) : count_tiles(sh);
-  }
-
-  // The relabel tiling's tables (rt) for shape sh2 over the same instances:
-  // descriptors, tile -> instance table, tile lines and the search buffers.
-  int build_relabel_tiles(int sh2) {
-    rt.shape = sh2;
-    int tw, th, td;
-    shape_dims(sh2, &tw, &th, &td);
-    rt.inst = inst;
+    region_dims(d3, &tw, &th, &td);
+    rg.inst = inst;
     long long off = 0;
-    int maxsum = 0;
-    rt.max_tile_dim = 1;
-    for (auto &I : rt.inst) {
+    for (auto &I : rg.inst) {
       I.tx = (I.nx + tw - 1) / tw;
       I.ty = (I.ny + th - 1) / th;
       I.tz = (I.nz + td - 1) / td;
@@ -504,75 +446,39 @@ struct jfc_graph {
       I.tile_off = (int)off;
       I.ntiles = (int)nt;
       off += nt;
-      rt.max_tile_dim = std::max(rt.max_tile_dim, std::max(I.tx, std::max(I.ty, I.tz)));
-      maxsum = std::max(maxsum, I.tx + I.ty + I.tz);
     }
-    rt.ntiles = (int)off;
-    rt.nbins = std::min(maxsum + 2, 4096);
-    std::vector<int> tile_inst(rt.ntiles);
-    const int n1 = (int)rt.inst.size() + 1;
-    std::vector<int> lines(3 * n1, 0);
-    for (size_t i = 0; i < rt.inst.size(); ++i) {
-      const InstDesc &I = rt.inst[i];
+    rg.n = (int)off;
+    rg.buf.planes = Kg + region_state_planes();
+    std::vector<int> tile_inst(rg.n);
+    for (size_t i = 0; i < rg.inst.size(); ++i) {
+      const InstDesc &I = rg.inst[i];
       std::fill(tile_inst.begin() + I.tile_off, tile_inst.begin() + I.tile_off + I.ntiles, (int)i);
-      const long long per[3] = {(long long)I.ty * I.tz, (long long)I.tx * I.tz,
-                                (long long)I.tx * I.ty};
-      for (int a = 0; a < 3; ++a) {
-        const long long nx = lines[a * n1 + i] + per[a];
-        if (nx >= (1LL << 31) / 4) return fail(JFC_ERR_INVALID, "too many tile lines");
-        lines[a * n1 + i + 1] = (int)nx;
-      }
     }
-    for (int a = 0; a < 3; ++a) rt.lines_total[a] = lines[a * n1 + n1 - 1];
+    const size_t border = (size_t)rg.n * region_border_words(d3);
     int rc;
-    if ((rc = dalloc(&rt.d_inst, rt.inst.size(), "instances")) ||
-        (rc = dalloc(&rt.d_tile_inst, rt.ntiles, "tile table")) ||
-        (rc = dalloc(&rt.d_dirty, rt.ntiles, "tile flags")) ||
-        (rc = dalloc(&rt.d_defi, rt.ntiles, "tile seeds")) ||
-        (rc = dalloc(&rt.d_jf0, rt.ntiles, "jump flooding")) ||
-        (rc = dalloc(&rt.d_jf1, rt.ntiles, "jump flooding")) ||
-        (rc = dalloc(&rt.d_tdist, rt.ntiles, "tile distance")) ||
-        (rc = dalloc(&rt.d_hist, rt.nbins, "tile histogram")) ||
-        (rc = dalloc(&rt.d_order, rt.ntiles, "tile order")) ||
-        (rc = dalloc(&rt.d_lines, 3 * n1, "tile lines")))
+    if ((rc = dalloc(&rg.d_inst, rg.inst.size(), "regions")) ||
+        (rc = dalloc(&rg.d_tile_inst, rg.n, "regions")) ||
+        (rc = dalloc(&rg.d_dirty[0], rg.n, "region marks")) ||
+        (rc = dalloc(&rg.d_dirty[1], rg.n, "region marks")) ||
+        (rc = dalloc(&rg.d_any, 4, "region marks")) ||
+        (rc = dalloc(&rg.buf.packed, (size_t)rg.n * rg.buf.planes * 64, "region bit planes")) ||
+        (rc = dalloc(&rg.buf.base, rg.n, "region bases")) ||
+        (rc = dalloc(&rg.buf.border, border, "region borders")))
       return rc;
-    JFC_HIP(hipMemcpy(rt.d_lines, lines.data(), lines.size() * sizeof(int), hipMemcpyHostToDevice));
-    JFC_HIP(hipMemcpy(rt.d_inst, rt.inst.data(), rt.inst.size() * sizeof(InstDesc),
+    launch_fill_i32(rg.buf.border, (long long)border, 0, 0);
+    JFC_HIP(hipMemcpy(rg.d_inst, rg.inst.data(), rg.inst.size() * sizeof(InstDesc),
                       hipMemcpyHostToDevice));
-    JFC_HIP(hipMemcpy(rt.d_tile_inst, tile_inst.data(), rt.ntiles * sizeof(int),
+    JFC_HIP(hipMemcpy(rg.d_tile_inst, tile_inst.data(), rg.n * sizeof(int),
                       hipMemcpyHostToDevice));
     return JFC_OK;
   }
-
-  // The tiling a search runs on (the relabel tiling for relabels, else the
-  // push tiling).
-  struct SearchTiling {
-    int shape;
-    Tiles T;
-    int ntiles, nbins, max_tile_dim;
-    unsigned char *dirty, *defi;
-    int *jf0, *jf1, *tdist, *hist, *order;
-    TileLines lines;
-    const InstDesc *pinst;  // push tiling descriptors when the tiling is another
-    int pdims;              // push tile dimensions, log2 (x | y << 4 | z << 8)
-  };
-  SearchTiling search_tiling(bool relabel) const {
-    if (!relabel || !rt.shape)
-      return SearchTiling{shape, tiles(), ntiles, nbins, max_tile_dim, d_dirty, d_defi, d_jf0,
-                          d_jf1, d_tdist, d_hist, d_order, lines(), nullptr, 0};
+  Tiles region_tiles() const {
     Tiles T = tiles();
-    T.inst = rt.d_inst;
-    T.tile_inst = rt.d_tile_inst;
-    T.ntiles = rt.ntiles;
-    T.one = rt.inst.empty() ? InstDesc{} : rt.inst[0];
-    const int n1 = (int)rt.inst.size() + 1;
-    const TileLines L{{rt.d_lines, rt.d_lines + n1, rt.d_lines + 2 * n1},
-                      {rt.lines_total[0], rt.lines_total[1], rt.lines_total[2]}};
-    int tw, th, td;
-    shape_dims(shape, &tw, &th, &td);
-    const int pdims = __builtin_ctz(tw) | __builtin_ctz(th) << 4 | __builtin_ctz(td) << 8;
-    return SearchTiling{rt.shape, T, rt.ntiles, rt.nbins, rt.max_tile_dim, rt.d_dirty, rt.d_defi,
-                        rt.d_jf0, rt.d_jf1, rt.d_tdist, rt.d_hist, rt.d_order, L, d_inst, pdims};
+    T.inst = rg.d_inst;
+    T.tile_inst = rg.d_tile_inst;
+    T.ntiles = rg.n;
+    T.one = rg.inst.empty() ? InstDesc{} : rg.inst[0];
+    return T;
   }
 };
 
@@ -795,7 +701,10 @@ static int create_impl(jfc_graph **out, int count, const int32_t *shapes) {
       g->tuned_sp = it->second.sp;
     }
   }
-  if ((rc = g->set_shape(default_shape(g->dim)))) { delete g; return rc; }
+  if ((rc = g->set_shape(default_shape(g->dim))) || (rc = g->build_regions())) {
+    delete g;
+    return rc;
+  }
   if (hipDeviceSynchronize() != hipSuccess) {
     delete g;
     return fail(JFC_ERR_DEVICE, "device initialisation failed");
@@ -1126,84 +1035,54 @@ struct Solver {
   }
   void advance() { g->slot ^= 1; }
 
-  // relabel / cut passes issued between two host checks
+  // search passes issued between two host checks
   static constexpr int kPassGroup = 4;
 
-  enum SearchMode { kRelabel = 0, kCut = 1, kTag = 2 };
+  enum SearchMode { kCut = 0, kTag = 1 };
 
-  // Tile passes of a monotone search (relabel, cut or tag) until no tile is
-  // dirty.  The first pass visits every tile (relabel, in jump-flooding
-  // distance order) or the seed tiles (cut, tag); later passes visit the
-  // dirty tiles, alternating direction (back-and-forth,
-  // QGCWidget.cpp:2221-2240).  Tile visits are counted on the device
-  // (d_total) and read once per solve.
-  // cleared: the caller has zeroed the dirty flags and the distance
-  // histogram already (search_fills).
+  // Tile passes of a flood (cut or tag) until no tile is dirty.  The first
+  // pass visits the seed tiles; later passes visit the dirty tiles,
+  // alternating direction (back-and-forth, QGCWidget.cpp:2221-2240).  Tile
+  // visits are counted on the device (d_total) and read once per solve.
+  // cleared: the caller has zeroed the dirty flags already (search_fills).
   int search(int mode, int *passes, bool cleared = false) {
-    const jfc_graph::SearchTiling ST = g->search_tiling(mode == kRelabel);
-    const Tiles &T = ST.T;
+    const Tiles T = g->tiles();
     Planes P = g->planes();
     if (mode == kTag) P.lab = g->tag;
-    // Relabel passes take the tiles in distance order from the tiles holding
-    // a deficit node (d_defi, kept by the fold and the push visits): a relax
-    // visit reads its halo heights device-coherently, so a tile settled
-    // earlier in the same pass is seen and one pass carries the front across
-    // many tiles.  The cut and tag floods read their halo labels with plain
-    // loads and gain nothing from the order (the 15000x10000 8-connected
-    // cut's: 0.58 ms ordered, 0.50 ms not, the same 9 passes; the 2560x1440x50
-    // video volume's: 0.74 -> 0.61 ms), and a graph
-    // of at most kSmallTiles tiles gives every tile a workgroup of its own in
-    // a pass: those take the tiles in colour order and skip the five launches
-    // of the distance ordering.
-    // (A relabel tiling other than the push tiling has no colour lists: its
-    // relabels always take the distance order.)
-    int *order = ST.order;
-    if ((ST.ntiles <= kSmallTiles && !ST.pinst) || mode != kRelabel) {
-      order = g->d_color_tiles;
-    } else {
-      launch_tile_order(ST.shape, T, ST.defi, ST.jf0, ST.jf1, ST.tdist, ST.hist, ST.nbins,
-                        ST.order, ST.max_tile_dim, nullptr, ST.lines, o.tile_order, st, cleared);
-    }
+    int *order = g->d_color_tiles;
     // A small graph's passes after the first take their tiles straight from
     // the flags (Queue::pick over the colour lists, no compaction launch).
     // The flags are then double-buffered: pass p takes the tiles flagged in
     // D[p & 1] and flags the next pass's in D[(p + 1) & 1], so a flag set
     // during a pass is read only after the launch boundary that makes the
     // labels or heights behind it visible.
-    const bool direct = ST.ntiles <= kSmallTiles && !ST.pinst;
-    unsigned char *const D[2] = {direct ? g->d_dirty2 : ST.dirty, ST.dirty};
+    const bool direct = g->ntiles <= kSmallTiles;
+    unsigned char *const D[2] = {direct ? g->d_dirty2 : g->d_dirty, g->d_dirty};
     if (!cleared) {
-      launch_fill_u8(ST.dirty, ST.ntiles, 0, st);
-      if (direct) launch_fill_u8(g->d_dirty2, ST.ntiles, 0, st);
+      launch_fill_u8(g->d_dirty, g->ntiles, 0, st);
+      if (direct) launch_fill_u8(g->d_dirty2, g->ntiles, 0, st);
     }
-    const int nwg = std::min(g->nwg, ST.ntiles);
-    // totals: [1] relabel tiles, [2] cut tiles, [4] tag tiles
-    long long *total = g->d_total + (mode == kTag ? 4 : 1 + mode);
+    const int nwg = std::min(g->nwg, g->ntiles);
+    long long *total = g->d_total + (mode == kTag ? 4 : 2);
     if (int rc = g->ensure_pin()) return rc;
     // dirty: the flags this pass sets for the next
-    auto flood = [&](const Queue &q, bool full_pass, unsigned char *dirty) {
-      if (mode == kCut) launch_reach(ST.shape, nwg, T, P, q, dirty, g->d_flagword, st);
-      else if (mode == kTag) launch_tag(ST.shape, nwg, T, P, q, dirty, g->lab, st);
-      else launch_relax(ST.shape, nwg, T, P, q, dirty, g->d_flag, full_pass && g->dim != 3,
-                        g->gr_tag, st, ST.pinst, ST.pdims);
+    auto flood = [&](const Queue &q, unsigned char *dirty) {
+      if (mode == kCut) launch_reach(g->shape, nwg, T, P, q, dirty, g->d_flagword, st);
+      else launch_tag(g->shape, nwg, T, P, q, dirty, g->lab, st);
     };
-    if (mode != kRelabel) {
-      // tiles without a seed gain labels only through their halo, so the
-      // first pass visits the seed tiles (in distance order)
-      if (direct) {
-        Queue qd{order, g->d_ctr, g->slot, ST.ntiles};
-        qd.pick = g->d_seed;
-        qd.cnt = g->d_ctr + QSLOT * g->slot;
-        qd.total = total;
-        flood(qd, false, D[1]);
-      } else {
-        Queue q = queue_from_list();
-        launch_compact(order, ST.ntiles, 0, g->d_seed, nullptr, nullptr, q, nullptr, total,
-                       nullptr, st);
-        flood(q, false, D[1]);
-      }
+    // tiles without a seed gain labels only through their halo, so the
+    // first pass visits the seed tiles
+    if (direct) {
+      Queue qd{order, g->d_ctr, g->slot, g->ntiles};
+      qd.pick = g->d_seed;
+      qd.cnt = g->d_ctr + QSLOT * g->slot;
+      qd.total = total;
+      flood(qd, D[1]);
     } else {
-      flood(Queue{order, g->d_ctr, g->slot, ST.ntiles}, true, D[1]);
+      Queue q = queue_from_list();
+      launch_compact(order, g->ntiles, 0, g->d_seed, nullptr, nullptr, q, nullptr, total,
+                     nullptr, st);
+      flood(q, D[1]);
     }
     advance();
     *passes += 1;
@@ -1222,16 +1101,16 @@ struct Solver {
         if (direct) {
           // the pass's visit count goes to its slot's count word (zeroed by
           // the launch before, as a compaction's would be)
-          Queue qd{order, g->d_ctr, g->slot, ST.ntiles};
+          Queue qd{order, g->d_ctr, g->slot, g->ntiles};
           qd.pick = D[pass & 1];
           qd.cnt = g->d_ctr + QSLOT * g->slot;
           qd.total = total;
-          flood(qd, false, D[(pass + 1) & 1]);
+          flood(qd, D[(pass + 1) & 1]);
         } else {
           Queue qc = queue_from_list();
-          launch_compact(order, ST.ntiles, pass & 1, ST.dirty, nullptr, nullptr, qc, nullptr,
+          launch_compact(order, g->ntiles, pass & 1, g->d_dirty, nullptr, nullptr, qc, nullptr,
                          total, nullptr, st);
-          flood(qc, false, ST.dirty);
+          flood(qc, g->d_dirty);
         }
         advance();
         *passes += 1;
@@ -1261,41 +1140,81 @@ struct Solver {
     return search(kTag, passes);
   }
 
-  // Exact relabel (graphcut_init_global_relabel + graphcut_global_relabel,
-  // graphcut_global_relabel.cl:19-124).  In 2D there is no separate init pass
-  // over the nodes: the first tile pass starts every tile from e and marks
-  // the heights it writes with a fresh tag, so a neighbour's stale height is
-  // recognised and replaced by its start value (a relabel of the
-  // 15000x10000 8-connected cut 1.03 -> 0.94 ms).  3D relabels keep the pass, which also makes the tile seeds
-  // exact: 3D tiles have a halo as large as the tile, and without the pass
-  // (halo excess read in the first tile pass, seeds from the push visits'
-  // deficit flags) the 2560x1440x50 video volume took 14.7 ms instead of
-  // 13.4.
-  // The zeroing a search needs (dirty flags, distance histogram), to go into
-  // its caller's fill launch.
-  void search_fills(FillSet &f, bool relabel = false) const {
-    const jfc_graph::SearchTiling ST = g->search_tiling(relabel);
-    f.add(ST.hist, ST.nbins, 0, 4);
-    f.add(ST.dirty, ST.ntiles, 0, 1);
-    if (ST.ntiles <= kSmallTiles && !ST.pinst) f.add(g->d_dirty2, ST.ntiles, 0, 1);
+  // The zeroing a flood needs, to go into its caller's fill launch.
+  void search_fills(FillSet &f) const {
+    f.add(g->d_dirty, g->ntiles, 0, 1);
+    if (g->ntiles <= kSmallTiles) f.add(g->d_dirty2, g->ntiles, 0, 1);
   }
 
+  // Exact relabel (graphcut_init_global_relabel + graphcut_global_relabel,
+  // graphcut_global_relabel.cl:19-124) on the graph's regions
+  // (jfc_region.hip): every region once, then the marked ones until no mark
+  // is left, then every region again to write the heights.
   int global_relabel() {
     hipEvent_t a = tm.mark();
-    g->gr_tag = 3 - g->gr_tag;
-    const jfc_graph::SearchTiling ST = g->search_tiling(true);
+    if (int rc = g->ensure_pin()) return rc;
+    auto &rg = g->rg;
+    rg.tag = 3 - rg.tag;
     {
       FillSet f;
-      search_fills(f, true);
-      if (g->dim == 3) f.add(ST.defi, ST.ntiles, 0, 1);
-      // the relax passes set the push tiling's active flags, never clear them
-      if (ST.pinst) f.add(g->d_flag, g->ntiles, 0, 1);
+      f.add(rg.d_dirty[0], rg.n, 0, 1);
+      f.add(rg.d_dirty[1], rg.n, 0, 1);
+      f.add(rg.d_any, 4, 0, 4);
+      f.add(g->d_flag, g->ntiles, 0, 1);  // kFinal sets the active tiles' flags
       launch_fill_multi(f, st);
     }
-    if (g->dim == 3)
-      launch_gr_init(ST.shape, ST.T, g->planes(), g->gr_tag, ST.defi, st, true);
-    int rc = search(kRelabel, &s.relabel_passes, true);
-    if (rc) return rc;
+    const bool d3 = g->dim == 3;
+    const Tiles T = g->region_tiles();
+    const Planes P = g->planes();
+    int tw, th, td;
+    shape_dims(g->shape, &tw, &th, &td);
+    RegionPass A{};
+    A.tag = rg.tag;
+    A.visits = g->d_total + kRegionSlots;
+    A.active = g->d_flag;
+    A.pinst = g->d_inst;
+    A.pone = g->inst[0];
+    A.pdims = __builtin_ctz(tw) | __builtin_ctz(th) << 4 | __builtin_ctz(td) << 8;
+    int pass = 0;
+    auto issue = [&](int kind, int group) {
+      A.dirty_in = rg.d_dirty[pass & 1];
+      A.dirty_out = rg.d_dirty[(pass + 1) & 1];
+      A.any_in = rg.d_any + (pass & 3);
+      A.any_out = rg.d_any + ((pass + 1) & 3);
+      A.any_clear = rg.d_any + ((pass + 2) & 3);
+      A.post = g->d_ring + kStopRing + group;
+      A.seq = rg.seq = (rg.seq + 1) & 0xffffff;
+      launch_region(d3, T, P, rg.buf, A, kind, 2 * g->nwg, st);
+      ++pass;
+    };
+    issue(kPack, 0);
+    // Passes go out in groups, one group ahead of the host's check, so the
+    // device is not idle during it.  A pass with no mark returns at once and
+    // says so in its group's word.  The first groups are short, as most
+    // relabels of dense graphs settle within them; later ones grow, as each
+    // check costs a gap of about 6 us between two passes.
+    int want[2] = {0, 0};
+    auto issue_group = [&](int k) -> int {
+      const int size = k < 2 ? 2 : k < 4 ? 4 : 8;
+      for (int j = 0; j < size; ++j) issue(kBorders, k & 1);
+      want[k & 1] = A.seq;
+      JFC_HIP(hipEventRecord(g->cnt_ev[k & 1], st));
+      return JFC_OK;
+    };
+    if (int rc = issue_group(0)) return rc;
+    for (int k = 0;; ++k) {
+      if (int rc = issue_group(k + 1)) return rc;
+      JFC_HIP(hipEventSynchronize(g->cnt_ev[k & 1]));
+      const volatile int *word = g->ring + kStopRing + (k & 1);
+      int w = *word;
+      for (int spin = 0; (w >> 1) != want[k & 1] && spin < (1 << 20); ++spin) w = *word;
+      if ((w >> 1) != want[k & 1])
+        return fail(JFC_ERR_DEVICE, "a relabel pass's word did not reach the host");
+      if (!(w & 1)) break;
+      if (pass > 1000000) return fail(JFC_ERR_STATE, "search did not settle");
+    }
+    issue(kFinal, 0);
+    s.relabel_passes += pass;
     launch_fill_u8(g->d_hmat, g->ntiles, 1, st);  // every height is stored now
     gr_ev.push_back({a, tm.mark()});
     s.global_relabels++;
@@ -1362,7 +1281,7 @@ struct Solver {
       }
       hipEvent_t a = (timed && o.profile) ? tm.mark() : nullptr;
       launch_push(g->shape, std::min(g->nwg, std::max(1, n)), T, P, q, g->d_flag, g->d_mat,
-                  g->d_touched, g->d_defi, g->d_hmat, o.max_local_iters, o.sparse_local_iters,
+                  g->d_touched, g->d_hmat, o.max_local_iters, o.sparse_local_iters,
                   g->d_sweep_state, g->d_total + kIterSlots, s_);
       if (timed && o.profile) push_ev.push_back({a, tm.mark()});
       advance();
@@ -1378,7 +1297,7 @@ struct Solver {
                    g->d_sweep_state, g->d_total, g->d_sweep_state + 2, st);
     hipEvent_t a = o.profile ? tm.mark() : nullptr;
     launch_fc_sweep(g->shape, std::min(g->nwg, g->ntiles), g->tiles(), g->planes(), q,
-                    g->d_flag, g->d_defi, st);
+                    g->d_flag, st);
     if (o.profile) push_ev.push_back({a, tm.mark()});
     advance();
     launch_sweep_end(sweep_ctl(), st);
@@ -1449,7 +1368,6 @@ struct Solver {
       f.add(g->d_touched, g->ntiles, 0, 1);
       // the fold's tile flags
       if (!o.initial_relabel) f.add(g->d_flag, g->ntiles, 0, 1);
-      f.add(g->d_defi, g->ntiles, 0, 1);
       launch_fill_multi(f, st);
     }
     g->slot = 0;
@@ -1476,7 +1394,7 @@ struct Solver {
     }
     s.solve_bytes += nodes * (12 + (masks == 2 ? 4 * K + 8 : masks == 3 ? 4 * K + 4 : 8));
     if (int rc0 = g->ensure_pin()) return rc0;
-    launch_fold(g->shape, T, P, g->d_red, o.initial_relabel ? nullptr : g->d_flag, g->d_defi,
+    launch_fold(g->shape, T, P, g->d_red, o.initial_relabel ? nullptr : g->d_flag, nullptr,
                 o.method == JFC_METHOD_FASTCUT && !o.initial_relabel, g->mask0, masks, st, true);
     // Fast-Cut reads and writes the residual planes directly
     if (o.method == JFC_METHOD_FASTCUT) launch_fc_materialize(P, g->mask0, g->Kg, st);
@@ -1595,19 +1513,23 @@ struct Solver {
     s.local_iters = 0;
     for (int k = 0; k < 64; ++k) s.local_iters += totals[kIterSlots + k];
     g->last_sweeps = s.sweeps;
-    // a relabel's first pass visits every tile without a compaction
-    s.relabel_tiles = totals[1] + (long long)g->ntiles * s.global_relabels;
+    // region visits: every region in a relabel's first and last pass, the
+    // marked ones between
+    long long marked = 0;
+    for (int k = 0; k < 64; ++k) marked += totals[kRegionSlots + k];
+    s.relabel_tiles = marked + 2LL * g->rg.n * s.global_relabels;
     s.cut_tiles = totals[2];
     s.push_bytes = totals[0] * 256LL * push_bytes_per_node(g->Kg);
-    // relabels: a first pass over every tile (2D: read e and mask, write h;
-    // 3D: after a pass over the nodes that reads e and writes h), later
-    // passes read h, e and mask and write h; cut searches: one pass over the
-    // nodes (read e, write the label) and flood visits (read label, e and
-    // mask, write label)
-    const long long first = (long long)g->ntiles * s.global_relabels;
-    s.solve_bytes += s.push_bytes + first * 256LL * (g->dim == 3 ? 16 : 12) +
-                     totals[1] * 256LL * 16 + (g->dim == 3 ? 8LL * nodes * s.global_relabels : 0) +
-                     5LL * nodes * cuts + totals[2] * 256LL * 10;
+    // relabels: the first pass reads e and the mask and writes the bit planes
+    // and borders, the last reads the bit planes and writes h, a marked
+    // region reads its bit planes and borders; cut searches: one pass over
+    // the nodes (read e, write the label) and flood visits (read label, e
+    // and mask, write label)
+    const long long rplanes = 512LL * g->rg.buf.planes;  // bytes per region
+    const long long rborder = 4LL * region_border_words(g->dim == 3);
+    s.solve_bytes += s.push_bytes +
+                     (12LL * nodes + g->rg.n * (2 * rplanes + 2 * rborder)) * s.global_relabels +
+                     marked * (rplanes + 2 * rborder) + 5LL * nodes * cuts + totals[2] * 256LL * 10;
     s.ms_total = Timer::ms(t0, t1);
     for (auto &p : push_ev) s.ms_push += Timer::ms(p.first, p.second);
     for (auto &p : gr_ev) s.ms_relabel += Timer::ms(p.first, p.second);
@@ -1786,15 +1708,36 @@ extern "C" int jfc_debug_tile_order(jfc_graph *g, int method, const uint8_t *til
                                     int32_t *tile_dist, int32_t *order, int32_t *max_dist) {
   if (!g || !tile_seed) return fail(JFC_ERR_INVALID, "null argument");
   if (method != 0 && method != 1) return fail(JFC_ERR_INVALID, "method must be 0 or 1");
-  JFC_HIP(hipMemcpy(g->d_seed, tile_seed, g->ntiles, hipMemcpyHostToDevice));
-  launch_tile_order(g->shape, g->tiles(), g->d_seed, g->d_jf0, g->d_jf1, g->d_tdist,
-                    g->d_hist, g->nbins, g->d_order, g->max_tile_dim, g->d_flagword + 2,
-                    g->lines(), method, 0);
-  JFC_HIP(hipDeviceSynchronize());
-  if (tile_dist) JFC_HIP(hipMemcpy(tile_dist, g->d_tdist, g->ntiles * 4, hipMemcpyDeviceToHost));
-  if (order) JFC_HIP(hipMemcpy(order, g->d_order, g->ntiles * 4, hipMemcpyDeviceToHost));
-  if (max_dist) JFC_HIP(hipMemcpy(max_dist, g->d_flagword + 2, 4, hipMemcpyDeviceToHost));
-  return JFC_OK;
+  // tile lines along x, y, z per instance (separable distance transform)
+  const int n1 = (int)g->inst.size() + 1;
+  std::vector<int> lines(3 * n1, 0);
+  for (size_t i = 0; i < g->inst.size(); ++i) {
+    const InstDesc &I = g->inst[i];
+    const int per[3] = {I.ty * I.tz, I.tx * I.tz, I.tx * I.ty};
+    for (int a = 0; a < 3; ++a) lines[a * n1 + i + 1] = lines[a * n1 + i] + per[a];
+  }
+  // work space of the ordering: four words per tile, the bins and the lines
+  const size_t nt = g->ntiles;
+  int *w = nullptr;
+  if (int rc = dalloc(&w, 4 * nt + g->nbins + lines.size(), "tile ordering")) return rc;
+  int *jf0 = w, *jf1 = w + nt, *tdist = w + 2 * nt, *d_order = w + 3 * nt, *hist = w + 4 * nt,
+      *d_lines = hist + g->nbins;
+  auto run = [&]() -> int {
+    JFC_HIP(hipMemcpy(g->d_seed, tile_seed, nt, hipMemcpyHostToDevice));
+    JFC_HIP(hipMemcpy(d_lines, lines.data(), lines.size() * sizeof(int), hipMemcpyHostToDevice));
+    const TileLines L{{d_lines, d_lines + n1, d_lines + 2 * n1},
+                      {lines[n1 - 1], lines[2 * n1 - 1], lines[3 * n1 - 1]}};
+    launch_tile_order(g->shape, g->tiles(), g->d_seed, jf0, jf1, tdist, hist, g->nbins, d_order,
+                      g->max_tile_dim, g->d_flagword + 2, L, method, 0);
+    JFC_HIP(hipDeviceSynchronize());
+    if (tile_dist) JFC_HIP(hipMemcpy(tile_dist, tdist, nt * 4, hipMemcpyDeviceToHost));
+    if (order) JFC_HIP(hipMemcpy(order, d_order, nt * 4, hipMemcpyDeviceToHost));
+    if (max_dist) JFC_HIP(hipMemcpy(max_dist, g->d_flagword + 2, 4, hipMemcpyDeviceToHost));
+    return JFC_OK;
+  };
+  const int rc = run();
+  dfree(w);
+  return rc;
 }
 
 extern "C" int jfc_debug_tile_flags(jfc_graph *g, int which, uint8_t *flags) {
@@ -1802,8 +1745,8 @@ extern "C" int jfc_debug_tile_flags(jfc_graph *g, int which, uint8_t *flags) {
   const int nI = (int)g->inst.size();
   launch_fill_i32((int *)g->d_red, 2LL * nI * RED_SLOTS, 0, 0);
   launch_fold(g->shape, g->tiles(), g->planes(), g->d_red, which == 2 ? g->d_flag : nullptr,
-              g->d_defi, false, nullptr, 0, 0);
-  unsigned char *src = which == 0 ? g->d_defi : g->d_flag;
+              which == 0 ? g->d_seed : nullptr, false, nullptr, 0, 0);
+  unsigned char *src = which == 0 ? g->d_seed : g->d_flag;
   if (which == 1) {
     launch_cut_init(g->shape, g->tiles(), g->planes(), g->d_seed, g->d_def, 0);
     src = g->d_seed;

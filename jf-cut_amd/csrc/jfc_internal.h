@@ -10,19 +10,6 @@ namespace jfc {
 
 // Height of a node proven unable to reach any deficit node.
 constexpr int HINF = 0x3fffffff;
-// A height word holds the height in bits 0-29 and, in bits 30-31, the tag of
-// the global relabel that wrote it (1 or 2, alternating; 0 from the push
-// kernels and the zero start).  Every reader masks with HMASK.  A relabel's
-// first pass takes a neighbour's word as a distance bound only when it
-// carries the running relabel's tag; any other word is stale, and the
-// neighbour's start value (0 at a deficit, HINF elsewhere) is used instead.
-// The first pass rewrites every word with the tag, so a word left from the
-// relabel before last can never carry the running tag.
-constexpr int HMASK = 0x3fffffff;
-__host__ __device__ inline int tag_word(int h, int tag) {
-  return (int)((unsigned)h | ((unsigned)tag << 30));
-}
-
 // Per-instance reduction slots (int64): folded constant, initial deficit,
 // energy, initial supply.  (The final deficit has an array of its own.)
 constexpr int RED_CONST = 0, RED_DEF0 = 1, RED_ENERGY = 3, RED_SUP0 = 4,
@@ -56,7 +43,7 @@ struct GraphAux {
 
 struct Planes {
   int *e;            // excess (> 0) / deficit (< 0), folded terminal arcs
-  int *h;            // height word (HMASK bits); HINF = cannot reach a deficit
+  int *h;            // height; HINF = cannot reach a deficit
   int *cap;          // K residual planes, plane d at cap + d * stride
   const int *c0;     // input neighbour planes (same layout)
   const int *cs;     // input source capacities
@@ -142,8 +129,8 @@ struct FillSet {
 };
 void launch_fill_multi(const FillSet &f, hipStream_t st);
 
-// active (or null): tiles holding an excess node; defi: tiles holding a
-// deficit node (the relabel's jump-flooding seeds).  Both zeroed here.
+// active, defi (either may be null): tiles holding an excess / a deficit node.
+// Both zeroed here.
 // zero_h: also write h = 0 over all nodes (the Fast-Cut kernels read every
 // height; the push kernel instead treats the heights of tiles it has not
 // visited in the solve as 0, see launch_push).
@@ -175,12 +162,10 @@ struct TileLines {
   const int *prefix[3];
   int total[3];
 };
-// hist_cleared: the caller has zeroed hist (nbins ints) already.
 void launch_tile_order(int shape, const Tiles &T, const unsigned char *seed,
                        int *jf0, int *jf1, int *tdist, int *hist, int nbins,
                        int *order, int max_tile_dim, int *max_dist,
-                       const TileLines &lines, int jump_flooding, hipStream_t st,
-                       bool hist_cleared = false);
+                       const TileLines &lines, int jump_flooding, hipStream_t st);
 
 // Sweep bookkeeping on the device.  state (8 ints): [0] active tiles of the
 // running sweep, [1] sweep index, [2] stop word (0 sweep on, 1 no active
@@ -220,9 +205,7 @@ void launch_compact(const int *src, int n, int reverse, unsigned char *flag,
                     int *sweep_cnt, long long *total, const int *stop, hipStream_t st,
                     const unsigned char *hmat = nullptr);
 // mat: per tile, 1 once every residual plane of the tile was written in
-// this solve (cleared when a solve starts).  defi: a visit rewrites its
-// tile's deficit flag (pushes never create deficits, so unvisited tiles'
-// flags stay a superset).  hmat: per tile, 1 once its heights are stored in
+// this solve (cleared when a solve starts).  hmat: per tile, 1 once its heights are stored in
 // this solve (by a push visit, which then writes all of them, or by a global
 // relabel); heights of a tile with hmat 0 read as 0, the labelling a solve
 // starts from.  max_iters caps the local iterations of a visit, sparse_iters
@@ -234,30 +217,40 @@ void launch_compact(const int *src, int n, int reverse, unsigned char *flag,
 constexpr int kSparseAfter = 8;  // sweeps before the sparse cap applies
 void launch_push(int shape, int nwg, const Tiles &T, const Planes &P,
                  const Queue &q, unsigned char *flag, unsigned char *mat,
-                 unsigned char *touched, unsigned char *defi, unsigned char *hmat,
+                 unsigned char *touched, unsigned char *hmat,
                  int max_iters, int sparse_iters, const int *sweep_state,
                  long long *iter_total, hipStream_t st);
 // Fast-Cut comparator (jfc_fastcut.hip)
 void launch_fc_materialize(const Planes &P, const unsigned *mask0, int K, hipStream_t st);
 void launch_fc_sweep(int shape, int nwg, const Tiles &T, const Planes &P, const Queue &q,
-                     unsigned char *flag, unsigned char *defi, hipStream_t st);
-// Relabel start values written over all nodes with `tag`, and the exact
-// deficit flags of the tiles (3D relabels).
-void launch_gr_init(int shape, const Tiles &T, const Planes &P, int tag, unsigned char *defi,
-                    hipStream_t st, bool cleared = false);
-// One relabel pass.  The first pass (first_pass, every tile) starts each
-// tile from e (0 at deficits, HINF elsewhere) and writes every height word
-// with `tag`; later passes, and every pass after launch_gr_init, relax the
-// queued tiles from their stored heights.  `active` holds the tiles' active
-// flags; with `pinst` (3D shapes only: a relabel tiling other than the push tiling) it
-// is indexed by the push tiling instead -- pinst its instance descriptors,
-// pdims its tile dimensions as log2 (x | y << 4 | z << 8) -- and every
-// visit sets the flags of the push tiles holding active nodes (the caller
-// clears them before the relabel).
-void launch_relax(int shape, int nwg, const Tiles &T, const Planes &P,
-                  const Queue &q, unsigned char *dirty, unsigned char *active,
-                  bool first_pass, int tag, hipStream_t st, const InstDesc *pinst = nullptr,
-                  int pdims = 0);
+                     unsigned char *flag, hipStream_t st);
+// Global relabel on bit-parallel regions (jfc_region.hip): regions of 64 x 64
+// nodes in 2D, 64 x 8 x 8 in 3D.  T is the region tiling (descriptors with
+// the regions' counts and offsets).
+struct RegionBuf {
+  unsigned long long *packed;  // bit planes: (region * planes + plane) * 64 + row
+  int *border;                 // region_border_words() distances per region, zero at first
+  int *base;                   // per region: distance its counting planes start at
+  int planes;                  // directions stored + region_state_planes()
+};
+enum RegionPassKind { kPack = 0, kBorders = 1, kFinal = 2 };
+struct RegionPass {
+  int tag;                            // of this relabel, 1 or 2, alternating
+  unsigned char *dirty_in, *dirty_out;  // marks this pass takes / sets for the next
+  int *any_in, *any_out, *any_clear;  // whether a mark is set; the slot after next is cleared
+  int *post;                          // pinned word: seq * 2 + (any mark was set for this pass)
+  int seq;
+  long long *visits;                  // 64 counters of kBorders visits
+  unsigned char *active;              // push tiles' active flags, cleared by the caller
+  const InstDesc *pinst;              // push tiling
+  InstDesc pone;                      // its instance 0
+  int pdims;                          // push tile dimensions, log2 (x | y << 4 | z << 8)
+};
+int region_border_words(bool d3);
+int region_state_planes();
+void region_dims(bool d3, int *tw, int *th, int *td);
+void launch_region(bool d3, const Tiles &T, const Planes &P, const RegionBuf &R,
+                   const RegionPass &A, int pass, int nwg, hipStream_t st);
 void launch_reach(int shape, int nwg, const Tiles &T, const Planes &P,
                   const Queue &q, unsigned char *dirty, int *cert,
                   hipStream_t st);

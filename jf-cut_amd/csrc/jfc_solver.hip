@@ -2,8 +2,6 @@
 //
 // Reference counterparts (paths relative to src/QVisualizer/):
 //   k_push     graphcut_relabel_push   cl/GraphCut/graphcut_push_relabel.cl:25-203 (2D), :215-439 (3D)
-//   k_relax    graphcut_global_relabel cl/GraphCut/graphcut_global_relabel.cl:50-124, :128-249
-//   k_gr_init  graphcut_init_global_relabel  graphcut_global_relabel.cl:19-48
 //   k_reach    graphcut_compute_cut    cl/GraphCut/graphcut_compute_cut.cl:51-140, :182-282
 //   k_cut_init graphcut_init_cut       graphcut_compute_cut.cl:19-49
 //   k_compact  graphcut_count_node + clogs scan + graphcut_scatter_node
@@ -206,17 +204,6 @@ __device__ __forceinline__ int block_or_bits(int bits, int *s_w, int parity) {
 // The barrier also orders the workgroup's LDS accesses like __syncthreads.
 __device__ __forceinline__ int block_any(int pred, int *s_w, int &parity) {
   const int w = __ballot(pred) != 0;
-  int *buf = s_w + 4 * parity;
-  parity ^= 1;
-  if (lane_id() == 0) buf[threadIdx.x >> 6] = w;
-  __syncthreads();
-  return buf[0] | buf[1] | buf[2] | buf[3];
-}
-
-// block_any for two bits at once: bit b of the result is set when some lane
-// has bit b of `bits` set (one ballot per bit, one barrier).
-__device__ __forceinline__ int block_any2(int bits, int *s_w, int &parity) {
-  const int w = (__ballot(bits & 1) != 0 ? 1 : 0) | (__ballot(bits & 2) != 0 ? 2 : 0);
   int *buf = s_w + 4 * parity;
   parity ^= 1;
   if (lane_id() == 0) buf[threadIdx.x >> 6] = w;
@@ -460,11 +447,9 @@ static int row_grid(int nsteps) {
 // With `active` set it flags the tiles holding excess (`active` zeroed by the
 // launcher); with `zero_h` it starts the labelling at zero heights over all
 // nodes (the reference clears h, QGCWidget.cpp:2400; the push kernel reads
-// the heights of tiles it has not visited in the solve as 0 instead).  It
-// always flags the tiles holding a deficit node in `defi`, the seeds of a
-// global relabel's tile ordering (the seed flags of
-// graphcut_init_global_relabel, graphcut_global_relabel.cl:19-48, kept
-// current by the push visits instead of a pass over e).
+// the heights of tiles it has not visited in the solve as 0 instead); with
+// `defi` it flags the tiles holding a deficit node (the seed flags of
+// graphcut_init_global_relabel, graphcut_global_relabel.cl:19-48).
 //
 // The same pass starts the residual-arc masks of the solve (MASKS): 0 leaves
 // them alone, 1 copies mask0 to rmask, 2 builds mask0 from the input planes
@@ -537,7 +522,7 @@ __global__ __launch_bounds__(256) void k_fold(Tiles T, Planes P, long long *red,
           dbits |= (unsigned)(s < t) << i;
         }
         if (active) flag_group<S>(active, R[u].tile0, g[u], bits);
-        flag_group<S>(defi, R[u].tile0, g[u], dbits);
+        if (defi) flag_group<S>(defi, R[u].tile0, g[u], dbits);
       }
     }
   }
@@ -549,7 +534,7 @@ void launch_fold(int shape, const Tiles &T, const Planes &P, long long *red,
                  int masks, hipStream_t st, bool cleared) {
   if (!cleared) {
     if (active) launch_fill_u8(active, T.ntiles, 0, st);
-    launch_fill_u8(defi, T.ntiles, 0, st);
+    if (defi) launch_fill_u8(defi, T.ntiles, 0, st);
   }
   const int z = zero_h ? 1 : 0;
   const int n = (T.nrows + T.row_step - 1) / T.row_step;
@@ -626,52 +611,6 @@ void launch_cut_init(int shape, const Tiles &T, const Planes &P,
   JFC_DISPATCH(shape,
                (k_cut_init<S><<<row_grid<&k_cut_init<S>>((T.nrows + T.row_step - 1) / T.row_step),
                                 256, 0, st>>>(T, P, seed, def)));
-}
-
-// graphcut_init_global_relabel (graphcut_global_relabel.cl:19-48) as a pass
-// over the nodes: h = 0 at deficit nodes, HINF elsewhere, written with the
-// relabel's tag, and the exact deficit flags of the tiles (`defi`, zeroed by
-// the launcher).  Used before the first tile pass of a 3D relabel; in 2D the
-// first tile pass starts from e itself.
-template <class S>
-__global__ __launch_bounds__(256) void k_gr_init(Tiles T, Planes P, int tag,
-                                                 unsigned char *defi) {
-  const int zero = tag_word(0, tag), inf = tag_word(HINF, tag);
-  const int nsteps = row_steps(T);
-  for (int step = blockIdx.x; step < nsteps; step += gridDim.x) {
-    const RowStep<S> RS(T, step);
-    for (int k0 = threadIdx.x; k0 < RS.slots; k0 += RS_U * 256) {
-      Group g[RS_U];
-      RowRef<S> R[RS_U];
-      int4 e[RS_U];
-#pragma unroll
-      for (int u = 0; u < RS_U; ++u) {
-        const int k = k0 + u * 256;
-        if (k < RS.slots) RS.at(T, k, R[u], g[u]);
-        else { R[u] = RS.R0; g[u] = Group{0, 0}; }
-        e[u] = load4(P.e, R[u].v0 + g[u].x, g[u].n);
-      }
-#pragma unroll
-      for (int u = 0; u < RS_U; ++u) {
-        if (g[u].n == 0) continue;
-        int4 h;
-        h.x = e[u].x < 0 ? zero : inf; h.y = e[u].y < 0 ? zero : inf;
-        h.z = e[u].z < 0 ? zero : inf; h.w = e[u].w < 0 ? zero : inf;
-        store4(P.h, R[u].v0 + g[u].x, g[u].n, h);
-        unsigned bits = 0;
-        for (int i = 0; i < g[u].n; ++i) bits |= (unsigned)(comp(e[u], i) < 0) << i;
-        flag_group<S>(defi, R[u].tile0, g[u], bits);
-      }
-    }
-  }
-}
-
-void launch_gr_init(int shape, const Tiles &T, const Planes &P, int tag, unsigned char *defi,
-                    hipStream_t st, bool cleared) {
-  if (!cleared) launch_fill_u8(defi, T.ntiles, 0, st);
-  const int n = (T.nrows + T.row_step - 1) / T.row_step;
-  JFC_DISPATCH(shape,
-               (k_gr_init<S><<<row_grid<&k_gr_init<S>>(n), 256, 0, st>>>(T, P, tag, defi)));
 }
 
 // Cut energy on the input capacities (QGCWidget.cpp:2452-2520), summed per
@@ -1043,8 +982,7 @@ __global__ __launch_bounds__(256) void k_scatter_order(const int *tdist, int n, 
 void launch_tile_order(int shape, const Tiles &T, const unsigned char *seed,
                        int *jf0, int *jf1, int *tdist, int *hist, int nbins,
                        int *order, int max_tile_dim, int *max_dist,
-                       const TileLines &lines, int jump_flooding, hipStream_t st,
-                       bool hist_cleared) {
+                       const TileLines &lines, int jump_flooding, hipStream_t st) {
   const int n = T.ntiles;
   const int g = (n + 255) / 256;
   const int d3 = shape_is_3d(shape) ? 1 : 0;
@@ -1077,7 +1015,7 @@ void launch_tile_order(int shape, const Tiles &T, const unsigned char *seed,
     launch_fill_i32(max_dist, 1, 0, st);
     k_max_dist<<<g, 256, 0, st>>>(tdist, n, nbins - 1, max_dist);
   }
-  if (!hist_cleared) launch_fill_i32(hist, nbins, 0, st);
+  launch_fill_i32(hist, nbins, 0, st);
   const int gh = std::min(g, 512);
   k_hist<<<gh, 256, nbins * sizeof(int), st>>>(tdist, n, nbins, hist);
   k_scan_1wg<<<1, 1024, 0, st>>>(hist, nbins);
@@ -1472,7 +1410,7 @@ template <class S, bool ONE>
 // (32x4x2, slim flush) fit 96: 5 waves.
 __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
     Tiles T, Planes P, Queue q, unsigned char *flag, unsigned char *mat, unsigned char *touched,
-    unsigned char *defi, unsigned char *hmat, int max_iters, int sparse_iters,
+    unsigned char *hmat, int max_iters, int sparse_iters,
     const int *sweep_state, long long *iter_total) {
   __shared__ int s_h[S::PADN];
   __shared__ int s_e[S::PADN];
@@ -1547,7 +1485,7 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
         ht = tile_of<S>(I, r.ox + x, r.oy + y, r.oz + z);
       }
       const int hw = P.h[hc[c].g];
-      hh[c] = hmat[ht] ? hw & HMASK : 0;
+      hh[c] = hmat[ht] ? hw : 0;
       hm[c] = P.rmask[hc[c].g];
     }
     // heights not yet stored in this solve read as 0 (the start labelling);
@@ -1555,7 +1493,7 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
     // the entry, so no load stands between the entry and the plane loads.
     const bool h_stored = (ent & kEntryHeights) != 0;
     const int hw0 = P.h[gv];
-    int e0 = P.e[gv], h0 = h_stored ? hw0 & HMASK : 0;
+    int e0 = P.e[gv], h0 = h_stored ? hw0 : 0;
     unsigned rm = 0;
     int c0r[S::KMAX];
     if (!fresh_tile) {
@@ -1728,7 +1666,7 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
     }
 
     // ---- write back what changed (stores only)
-    int act = 0, dfc = 0;
+    int act = 0;
     if (valid) {
       const int e1 = s_e[L.me], h1 = s_h[L.me];
       if (e1 != e0) P.e[gv] = e1;
@@ -1746,7 +1684,6 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
         }
       if (m1 != (fresh_tile ? rm : m0)) P.rmask[gv] = m1;
       act = e1 > 0 && h1 < HINF;
-      dfc = e1 < 0;
     }
     // ---- flush flow that crossed into the halo: excess and the reverse
     // residual of each crossing arc (graphcut_push_relabel.cl:184-195).
@@ -1783,12 +1720,8 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
       const unsigned flip = fp[c] | (fr[c] << 8);
       if (flip) atomicXor(&P.rmask[g], flip);
     }
-    // the tile's active flag and deficit flag, one barrier for both
-    const int ad = block_any2(act | (dfc << 1), s_w, par);
-    if (tid == 0) {
-      if (ad & 1) flag[t] = 1;
-      defi[t] = (unsigned char)(ad >> 1);
-    }
+    act = block_any(act, s_w, par);
+    if (act && tid == 0) flag[t] = 1;
     if (fresh_tile && tid == 0) mat[t] = 1;
     if (!h_stored && tid == 0) hmat[t] = 1;
     Qc.advance();
@@ -1800,330 +1733,17 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
 
 void launch_push(int shape, int nwg, const Tiles &T, const Planes &P,
                  const Queue &q, unsigned char *flag, unsigned char *mat,
-                 unsigned char *touched, unsigned char *defi, unsigned char *hmat,
+                 unsigned char *touched, unsigned char *hmat,
                  int max_iters, int sparse_iters, const int *sweep_state,
                  long long *iter_total, hipStream_t st) {
   if (T.ninst == 1) {
     JFC_DISPATCH(shape, (k_push<S, true><<<resident_grid<&k_push<S, true>>(nwg), 256, 0, st>>>(
-                            T, P, q, flag, mat, touched, defi, hmat, max_iters, sparse_iters,
+                            T, P, q, flag, mat, touched, hmat, max_iters, sparse_iters,
                             sweep_state, iter_total)));
   } else {
     JFC_DISPATCH(shape, (k_push<S, false><<<resident_grid<&k_push<S, false>>(nwg), 256, 0, st>>>(
-                            T, P, q, flag, mat, touched, defi, hmat, max_iters, sparse_iters,
+                            T, P, q, flag, mat, touched, hmat, max_iters, sparse_iters,
                             sweep_state, iter_total)));
-  }
-}
-
-// ---- exact global relabel: tile-local Bellman-Ford to a fixpoint ------------------
-//
-// h(u) = min(h(u), min over arcs with residual > 0 of h(v) + 1), iterated in
-// LDS until the tile is stable; tiles whose halo changed are revisited.  The
-// fixpoint over all tiles is the exact breadth-first distance to the nearest
-// deficit node (graphcut_global_relabel.cl:50-124).
-template <class S, bool FIRST, bool ONE>
-__global__ __launch_bounds__(256) void k_relax(Tiles T, Planes P, Queue q,
-                                               unsigned char *dirty,
-                                               unsigned char *active, int tag,
-                                               const InstDesc *pinst, int pdims) {
-  constexpr bool first = FIRST;
-  __shared__ int s_h[S::PADN];
-  const int tid = threadIdx.x;
-  const Lane<S> L(tid);
-  __shared__ int s_next[3];
-  __shared__ int s_w[8];
-  int par = 0;
-  VisitCursor Qc(q, s_next);
-  while (Qc.idx >= 0) {
-    const int t = Qc.ent;
-    const TileRef r = ONE ? tile_ref_of<S>(T.one, t) : tile_ref<S>(T, t);
-    const InstDesc &I = r.I;
-    const int K = I.K;
-    const int gx = r.ox + L.lx, gy = r.oy + L.ly, gz = r.oz + L.lz;
-    const bool valid = gx < I.nx && gy < I.ny && gz < I.nz;
-    // every load of the visit is issued before any is used (dead lanes and
-    // halo cells read a valid dummy address)
-    const long long gv = valid ? node_index(I, gx, gy, gz) : 0;
-    // halo: the ring cells, split evenly over the four waves (as in k_push)
-    HaloCell hc[kRingPerLane<S>];
-    int hp[kRingPerLane<S>];
-    int hh[kRingPerLane<S>], he[kRingPerLane<S>];
-#pragma unroll
-    for (int c = 0; c < kRingPerLane<S>; ++c) {
-      const int j = c * 64 + (tid & 63);
-      const int k = (tid >> 6) * kRingQ<S> + j;
-      hp[c] = j < kRingQ<S> && k < Ring<S>::N ? Ring<S>::pos(k) : S::PADN;
-      hc[c] = halo_cell<S>(I, r.ox, r.oy, r.oz, hp[c], K);
-      // device-coherent read: a neighbour tile settled earlier in this same
-      // pass (possibly on another XCD) is seen at once, so one pass carries
-      // the distance front across many tiles in list order.  Any tagged
-      // value read is an upper bound of the distance, so stale is safe.
-      hh[c] = __hip_atomic_load(&P.h[hc[c].g], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      he[c] = first ? P.e[hc[c].g] : 0;
-    }
-    // the first pass starts from e (the relabel's initial labelling) and
-    // needs no stored height
-    int e0 = P.e[gv];
-    int h0 = first ? 0 : P.h[gv] & HMASK;
-    unsigned mask = P.rmask[gv] & ((1u << K) - 1u);
-    if (first) h0 = e0 < 0 ? 0 : HINF;
-    if (!valid) {
-      h0 = HINF;
-      e0 = 0;
-      mask = 0;
-    }
-    s_h[L.me] = h0;
-#pragma unroll
-    for (int c = 0; c < kRingPerLane<S>; ++c) {
-      if (!hc[c].halo) continue;
-      int v = HINF;
-      if (hc[c].live) {
-        // an untagged word is left from the pushes or the relabel before:
-        // the neighbour still holds its start value
-        v = ((unsigned)hh[c] >> 30) == (unsigned)tag ? hh[c] & HMASK : (he[c] < 0 ? 0 : HINF);
-      }
-      s_h[hp[c]] = v;
-    }
-    __syncthreads();
-    // the next entry loads while the tile iterates
-    if (tid == 0) Qc.prefetch();
-    int any;
-    do {
-      int ch = 0;
-      if (mask) {
-        // all neighbour words read before any is used (one LDS wait)
-        const int h = s_h[L.me];
-        int hv[S::KMAX];
-#pragma unroll
-        for (int d = 0; d < S::KMAX; ++d) hv[d] = s_h[L.me + lds_off<S>(d)];
-        int m = h;
-#pragma unroll
-        for (int d = 0; d < S::KMAX; ++d)
-          if (mask & (1u << d)) m = min(m, hv[d] + 1);
-        if (m < h) {
-          s_h[L.me] = m;
-          ch = 1;
-        }
-      }
-      any = block_any(ch, s_w, par);
-    } while (any);
-    if (valid) {
-      const int h1 = s_h[L.me];
-      // the first pass writes every word (with the tag); later passes the
-      // changed ones
-      if (first || h1 != h0)
-        __hip_atomic_store(&P.h[gv], tag_word(h1, tag), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-      if (h1 != h0) {
-#pragma unroll
-        for (int d = 0; d < S::KMAX; ++d) {
-          if (d >= K) break;
-          int dx, dy, dz;
-          dir_of<S::D3>(d, dx, dy, dz);
-          const int lx = L.lx + dx, ly = L.ly + dy, lz = L.lz + dz;
-          if (lx >= 0 && lx < S::TW && ly >= 0 && ly < S::TH && lz >= 0 && lz < S::TD) continue;
-          const int X = gx + dx, Y = gy + dy, Z = gz + dz;
-          if (X < 0 || X >= I.nx || Y < 0 || Y >= I.ny || Z < 0 || Z >= I.nz) continue;
-          dirty[tile_of<S>(I, X, Y, Z)] = 1;
-        }
-      }
-    }
-    // graphcut_count_node fused in: the tile's last visit leaves its
-    // active flag (a node with excess and a finite height)
-    if (tid == 0) Qc.publish();
-    const bool on = valid && e0 > 0 && s_h[L.me] < HINF;
-    const int act = block_any(on, s_w, par);
-    if (pinst) {
-      // flags of the push tiling: each active node sets its push tile's.
-      // During a relabel e is fixed and heights only fall, so a node once
-      // active stays active, and setting flags (never clearing) is exact.
-      if (on) {
-        const InstDesc &PI = pinst[ONE ? 0 : T.tile_inst[t]];
-        active[PI.tile_off + (gx >> (pdims & 15)) +
-               PI.tx * ((gy >> ((pdims >> 4) & 15)) + PI.ty * (gz >> (pdims >> 8)))] = 1;
-      }
-    } else if (tid == 0) {
-      active[t] = (unsigned char)act;
-    }
-    Qc.advance();
-  }
-}
-
-// One wavefront per tile.  A relax visit is bound by its load latency (the
-// local fixpoint is a few cheap LDS iterations), so the tiles in flight per
-// CU matter more than the lanes per tile: a 64-lane wave owning a tile keeps
-// up to four times as many tiles in flight as a 256-lane workgroup.  Lane l
-// holds the nodes l + 64 j; the iterations are ordered by program order in
-// the wave, and a lane's later nodes already see its earlier nodes' new
-// heights (Gauss-Seidel within the iteration, still monotone).
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-
-template <class S, bool FIRST, bool ONE>
-__global__ __launch_bounds__(64) void k_relax_w(Tiles T, Planes P, Queue q,
-                                                unsigned char *dirty, unsigned char *active,
-                                                int tag) {
-  constexpr bool first = FIRST;
-  constexpr int NJ = S::NT / 64;
-  constexpr int NR = (Ring<S>::N + 63) / 64;
-  __shared__ int s_h[S::PADN];
-  __shared__ int s_next[3];
-  const int lane = threadIdx.x;
-  VisitCursor Qc(q, s_next);
-  while (Qc.idx >= 0) {
-    const int t = Qc.ent;
-    const TileRef r = ONE ? tile_ref_of<S>(T.one, t) : tile_ref<S>(T, t);
-    const InstDesc &I = r.I;
-    const int K = I.K;
-    // loads: ring heights (device-coherent and tagged, as in k_relax) and
-    // the lane's nodes
-    int hh[NR], he[NR];
-    bool hlive[NR];
-    long long hg[NR];
-#pragma unroll
-    for (int i = 0; i < NR; ++i) {
-      const int k = lane + 64 * i;
-      const HaloCell hc =
-          halo_cell<S>(I, r.ox, r.oy, r.oz, k < Ring<S>::N ? Ring<S>::pos(k) : S::PADN, K);
-      hlive[i] = hc.live;
-      hg[i] = hc.g;
-      hh[i] = __hip_atomic_load(&P.h[hc.g], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      he[i] = 0;
-    }
-    int h0[NJ];
-    unsigned mk[NJ];
-    bool pos[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const Lane<S> L(lane + 64 * j);
-      const int gx = r.ox + L.lx, gy = r.oy + L.ly, gz = r.oz + L.lz;
-      const bool valid = gx < I.nx && gy < I.ny && gz < I.nz;
-      const long long gv = valid ? node_index(I, gx, gy, gz) : 0;
-      const int e0 = P.e[gv];
-      h0[j] = first ? 0 : P.h[gv] & HMASK;
-      mk[j] = P.rmask[gv] & ((1u << K) - 1u);
-      pos[j] = e0 > 0;
-      if (first) h0[j] = e0 < 0 ? 0 : HINF;
-      if (!valid) {
-        h0[j] = HINF;
-        mk[j] = 0;
-        pos[j] = false;
-      }
-    }
-    // first pass: the excess of a halo node is needed only where its height
-    // word is stale, so it is loaded after the word and only there (most of
-    // a 2D tile's halo loads are side-column cells, one 128-byte line each)
-    if (first) {
-#pragma unroll
-      for (int i = 0; i < NR; ++i)
-        if (hlive[i] && ((unsigned)hh[i] >> 30) != (unsigned)tag) he[i] = P.e[hg[i]];
-    }
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) s_h[Lane<S>(lane + 64 * j).me] = h0[j];
-#pragma unroll
-    for (int i = 0; i < NR; ++i) {
-      const int k = lane + 64 * i;
-      if (k >= Ring<S>::N) continue;
-      int v = HINF;
-      if (hlive[i])
-        v = ((unsigned)hh[i] >> 30) == (unsigned)tag ? hh[i] & HMASK : (he[i] < 0 ? 0 : HINF);
-      s_h[Ring<S>::pos(k)] = v;
-    }
-    wave_lds_sync();
-    // the next entry loads while the tile iterates
-    if (lane == 0) Qc.prefetch();
-    bool any;
-    do {
-      bool ch = false;
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        if (!mk[j]) continue;
-        const int me = Lane<S>(lane + 64 * j).me;
-        const int h = s_h[me];
-        int hv[S::KMAX];
-#pragma unroll
-        for (int d = 0; d < S::KMAX; ++d) hv[d] = s_h[me + lds_off<S>(d)];
-        int m = h;
-#pragma unroll
-        for (int d = 0; d < S::KMAX; ++d)
-          if (mk[j] & (1u << d)) m = min(m, hv[d] + 1);
-        if (m < h) {
-          s_h[me] = m;
-          ch = true;
-        }
-      }
-      any = __ballot(ch) != 0;
-      wave_lds_sync();
-    } while (any);
-    bool act = false;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const Lane<S> L(lane + 64 * j);
-      const int gx = r.ox + L.lx, gy = r.oy + L.ly, gz = r.oz + L.lz;
-      if (!(gx < I.nx && gy < I.ny && gz < I.nz)) continue;
-      const int h1 = s_h[L.me];
-      act |= pos[j] && h1 < HINF;
-      if (first || h1 != h0[j])
-        __hip_atomic_store(&P.h[node_index(I, gx, gy, gz)], tag_word(h1, tag), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-      if (h1 == h0[j]) continue;
-#pragma unroll
-      for (int d = 0; d < S::KMAX; ++d) {
-        if (d >= K) break;
-        int dx, dy, dz;
-        dir_of<S::D3>(d, dx, dy, dz);
-        const int lx = L.lx + dx, ly = L.ly + dy, lz = L.lz + dz;
-        if (lx >= 0 && lx < S::TW && ly >= 0 && ly < S::TH && lz >= 0 && lz < S::TD) continue;
-        const int X = gx + dx, Y = gy + dy, Z = gz + dz;
-        if (X < 0 || X >= I.nx || Y < 0 || Y >= I.ny || Z < 0 || Z >= I.nz) continue;
-        dirty[tile_of<S>(I, X, Y, Z)] = 1;
-      }
-    }
-    const bool a = __ballot(act) != 0;
-    if (lane == 0) {
-      active[t] = (unsigned char)a;
-      Qc.publish();
-    }
-    wave_lds_sync();
-    Qc.advance();
-  }
-}
-
-// 2D tiles: the wave-per-tile kernel (a relabel of the 15000x10000
-// 8-connected cut 1.67 -> 1.21 ms).
-// 3D tiles iterate more per visit (fronts cross 8x8x4 tiles in z as well)
-// and there the 256-lane visit's four parallel waves win (the 512^3
-// volume's relabels 19 -> 15 ms), so 3D keeps the workgroup kernel.
-template <bool FIRST, bool ONE>
-static void relax_launch(int shape, int nwg, const Tiles &T, const Planes &P, const Queue &q,
-                         unsigned char *dirty, unsigned char *active, int tag, hipStream_t st,
-                         const InstDesc *pinst, int pdims) {
-  if (shape_is_3d(shape)) {
-    JFC_DISPATCH(shape, (k_relax<S, FIRST, ONE><<<resident_grid<&k_relax<S, FIRST, ONE>>(nwg),
-                                                  256, 0, st>>>(T, P, q, dirty, active, tag,
-                                                                pinst, pdims)));
-  } else {
-    JFC_DISPATCH(shape,
-                 (k_relax_w<S, FIRST, ONE><<<resident_grid_b<&k_relax_w<S, FIRST, ONE>, 64>(
-                                                 4 * nwg),
-                                             64, 0, st>>>(T, P, q, dirty, active, tag)));
-  }
-}
-
-void launch_relax(int shape, int nwg, const Tiles &T, const Planes &P,
-                  const Queue &q, unsigned char *dirty, unsigned char *active,
-                  bool first_pass, int tag, hipStream_t st, const InstDesc *pinst, int pdims) {
-  if (first_pass) {
-    if (T.ninst == 1)
-      relax_launch<true, true>(shape, nwg, T, P, q, dirty, active, tag, st, pinst, pdims);
-    else relax_launch<true, false>(shape, nwg, T, P, q, dirty, active, tag, st, pinst, pdims);
-  } else {
-    if (T.ninst == 1)
-      relax_launch<false, true>(shape, nwg, T, P, q, dirty, active, tag, st, pinst, pdims);
-    else relax_launch<false, false>(shape, nwg, T, P, q, dirty, active, tag, st, pinst, pdims);
   }
 }
 
