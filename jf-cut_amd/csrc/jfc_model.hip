@@ -296,44 +296,48 @@ __device__ __forceinline__ void put_table(double *q, const long long *c, int K, 
   q[k * 4] = n2;
 }
 
-// Initial centroids per side (one workgroup of 256 lanes, blockIdx.x =
-// side): the distinct seeded keys in ascending order, the j-th centre taken
-// from key number j * (m - 1) / (K - 1), rounded to fixed point
-// (QGCWidget.cpp:2001-2039).
-__global__ __launch_bounds__(256) void k_km_init(Scratch s, int C, int nkeys, int Kf, int Kb) {
-  constexpr int KPL = NKEYS_MAX / 256;  // keys per lane
-  __shared__ int s_cnt[256];
-  __shared__ long long s_pick[KMAX_CLUSTERS];
-  __shared__ long long s_cent[KMAX_CLUSTERS * 3];
-  const int side = blockIdx.x, K = side ? Kb : Kf, tid = threadIdx.x;
+// Initial centroids of a side, by a whole workgroup of NT lanes: the distinct
+// seeded keys in ascending order, the j-th centre taken from key number
+// j * (m - 1) / (K - 1), rounded to fixed point (QGCWidget.cpp:2001-2039).
+// Returns them in s_cent (false: no seeds, reported by the host).  The key
+// counts are read once, coalesced, as one LDS flag per key: read by each lane
+// for its own keys, 16 dependent rounds of scattered loads, the step took 16
+// us at any size; it takes 8.
+template <int NT>
+__device__ bool km_init(const Scratch &s, int side, int C, int nkeys, int K, long long *s_cent) {
+  constexpr int KPL = NKEYS_MAX / NT;  // keys per lane
+  __shared__ unsigned char s_has[NKEYS_MAX];
+  __shared__ int s_cnt[NT];
+  const int tid = threadIdx.x;
   const long long *kc = s.kcnt + side * NKEYS_MAX;
   const long long *ks = s.ksum + side * NKEYS_MAX;
-  long long *cent = s.cent + side * KMAX_CLUSTERS * 3;
-  int mine = 0;
+#pragma unroll
   for (int q = 0; q < KPL; ++q) {
-    const int k = tid * KPL + q;
-    if (k < nkeys && kc[k]) ++mine;
+    const int k = tid + NT * q;
+    s_has[k] = k < nkeys && kc[min(k, nkeys - 1)] != 0;
   }
+  if (tid < KMAX_CLUSTERS * 3) s_cent[tid] = 0;
+  __syncthreads();
+  int mine = 0;
+#pragma unroll
+  for (int q = 0; q < KPL; ++q) mine += s_has[tid * KPL + q];
   s_cnt[tid] = mine;
   __syncthreads();
-  // inclusive scan over the 256 counts
-  for (int o = 1; o < 256; o <<= 1) {
+  // inclusive scan over the lanes' counts
+  for (int o = 1; o < NT; o <<= 1) {
     const int v = tid >= o ? s_cnt[tid - o] : 0;
     __syncthreads();
     s_cnt[tid] += v;
     __syncthreads();
   }
-  const int m = s_cnt[255];
-  if (tid < K) s_pick[tid] = K > 1 ? (long long)tid * (m - 1) / (K - 1) : 0;
-  if (tid < K * C) s_cent[tid] = 0;
-  __syncthreads();
-  if (m == 0) return;  // no seeds: reported by the host
+  const int m = s_cnt[NT - 1];
+  if (m == 0) return false;
   int r = s_cnt[tid] - mine;  // rank of this lane's first non-empty key
   for (int q = 0; q < KPL; ++q) {
     const int k = tid * KPL + q;
-    if (k >= nkeys || !kc[k]) continue;
+    if (!s_has[k]) continue;
     for (int j = 0; j < K; ++j)
-      if (s_pick[j] == r) {
+      if (r == (K > 1 ? (int)((long long)j * (m - 1) / (K - 1)) : 0)) {
         const long long nn = kc[k];
         for (int c = 0; c < C; ++c)
           s_cent[j * C + c] = (ks[k * C + c] * (1 << KM_FRAC) + nn / 2) / nn;
@@ -341,8 +345,16 @@ __global__ __launch_bounds__(256) void k_km_init(Scratch s, int C, int nkeys, in
     ++r;
   }
   __syncthreads();
+  return true;
+}
+
+// One workgroup of 256 lanes per side (blockIdx.x).
+__global__ __launch_bounds__(256) void k_km_init(Scratch s, int C, int nkeys, int Kf, int Kb) {
+  __shared__ long long s_cent[KMAX_CLUSTERS * 3];
+  const int side = blockIdx.x, K = side ? Kb : Kf, tid = threadIdx.x;
+  if (!km_init<256>(s, side, C, nkeys, K, s_cent)) return;
   if (tid < K * C) {
-    cent[tid] = s_cent[tid];
+    s.cent[side * KMAX_CLUSTERS * 3 + tid] = s_cent[tid];
     s.cbuf[side * KMAX_CLUSTERS * 3 + tid] = s_cent[tid];  // c_0 for the first iteration
   }
   put_table(s.q + side * KMAX_CLUSTERS * 4, s_cent, K, C);
@@ -412,6 +424,30 @@ __device__ __forceinline__ void near_d2(const double (*X)[C], const double *n2, 
   for (int p = 0; p < P; ++p) D[p] = n2[p] + m[p];
 }
 
+// The rounded mean of each non-empty cluster, else the old centre, into s_new
+// (which may be `old`), by a whole workgroup; returns whether any moved.
+__device__ bool km_means(const unsigned long long *s_sum, const long long *old, int K, int C,
+                         long long *s_new) {
+  const int j = threadIdx.x;
+  int changed = 0;
+  if (j < K * C) {
+    const int k = j / C, c = j % C;
+    const long long nk = (long long)s_sum[k * (C + 1) + C];
+    long long nc = old[j];
+    if (nk) {
+      // floor(a / nk) for 0 <= a < 2^53: the float64 quotient is off by one at most
+      const long long a = (long long)s_sum[k * (C + 1) + c] * (1 << KM_FRAC) + nk / 2;
+      long long v = (long long)((double)a / (double)nk);
+      const long long r = a - v * nk;
+      v += r < 0 ? -1 : r >= nk ? 1 : 0;
+      changed = v != nc;
+      nc = v;
+    }
+    s_new[j] = nc;
+  }
+  return __syncthreads_or(changed) != 0;
+}
+
 // The centre update (QGCWidget.cpp:2088-2101) from one iteration's partial
 // sums (nb workgroups' rows of `part`), by a whole workgroup: the rounded
 // mean of each non-empty cluster, else the old centre, into s_new.  Returns
@@ -426,19 +462,7 @@ __device__ bool km_update(const long long *part, int nb, const long long *old, i
     if (v) atomicAdd(&s_sum[i % E], v);
   }
   __syncthreads();
-  int changed = 0;
-  if (j < K * C) {
-    const int k = j / C, c = j % C;
-    const long long nk = (long long)s_sum[k * (C + 1) + C];
-    long long nc = old[j];
-    if (nk) {
-      const long long v = ((long long)s_sum[k * (C + 1) + c] * (1 << KM_FRAC) + nk / 2) / nk;
-      changed = v != nc;
-      nc = v;
-    }
-    s_new[j] = nc;
-  }
-  return __syncthreads_or(changed) != 0;
+  return km_means(s_sum, old, K, C, s_new);
 }
 
 // The final centres of a side: stored with their table, and the done flag
@@ -454,6 +478,63 @@ __device__ void km_finish(Scratch &s, int side, const long long *c, int K, int C
   }
 }
 
+// Cluster sums of the seeds a lane holds, added up in registers (KB >= K
+// clusters).
+template <int C, int KB>
+struct KmSums {
+  unsigned acc[KB][C + 1];
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int k = 0; k < KB; ++k)
+#pragma unroll
+      for (int c = 0; c <= C; ++c) acc[k][c] = 0;
+  }
+  // the assignment (graphcut_kmeans.cl:21-89): nearest centroid, lowest index
+  // on ties
+  template <int BPC>
+  __device__ __forceinline__ void add(unsigned packed, const double *q, int K) {
+    int x[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+      x[c] = BPC == 2 ? (int)packed : (int)((packed >> (8 * c)) & 255u);
+    double X[C], n2;
+    scaled_feature<C>(x, X, &n2);
+    int best;
+    near_part<C>(X, q, K, &best);
+#pragma unroll
+    for (int k = 0; k < KB; ++k) {
+      const bool hit = k == best;
+#pragma unroll
+      for (int c = 0; c < C; ++c) acc[k][c] += hit ? (unsigned)x[c] : 0u;
+      acc[k][C] += hit ? 1u : 0u;
+    }
+  }
+  // the wave's sums, each added to s_sum once: value e is summed by DPP adds
+  // (32 bits hold a wave's sum of kChunk seeds per lane) and lands in lane e
+  static constexpr int kChunk = 1020;
+  __device__ __forceinline__ void flush(unsigned long long *s_sum, int K) {
+    unsigned mine = 0;
+#pragma unroll
+    for (int k = 0; k < KB; ++k) {
+      if (k >= K) break;
+#pragma unroll
+      for (int c = 0; c <= C; ++c) {
+        unsigned t = acc[k][c];
+        t += __builtin_amdgcn_update_dpp(0u, t, 0x111, 0xf, 0xf, true);  // row_shr:1
+        t += __builtin_amdgcn_update_dpp(0u, t, 0x112, 0xf, 0xf, true);
+        t += __builtin_amdgcn_update_dpp(0u, t, 0x114, 0xf, 0xf, true);
+        t += __builtin_amdgcn_update_dpp(0u, t, 0x118, 0xf, 0xf, true);
+        t += __builtin_amdgcn_update_dpp(0u, t, 0x142, 0xa, 0xf, false);  // row_bcast:15
+        t += __builtin_amdgcn_update_dpp(0u, t, 0x143, 0xc, 0xf, false);  // row_bcast:31
+        t = __builtin_amdgcn_readlane(t, 63);
+        if (lane_id() == k * (C + 1) + c) mine = t;
+      }
+    }
+    if (lane_id() < K * (C + 1) && mine)
+      atomicAdd(&s_sum[lane_id()], (unsigned long long)mine);
+  }
+};
+
 // Lloyd iteration `it` of a side (blockIdx.y), one launch per iteration.
 // Each workgroup first forms the iteration's centres c_{it-1}: the initial
 // ones for it = 1, else the update of iteration it - 1 from its partial
@@ -462,10 +543,12 @@ __device__ void km_finish(Scratch &s, int side, const long long *c, int K, int C
 // converged after it - 1 iterations: workgroup 0 stores the final centres
 // and the done flag, and later launches return at once.  Then the
 // assignment (graphcut_kmeans.cl:21-89): nearest centroid, lowest index on
-// ties; each lane sums its seeds per cluster in registers (KB >= K
-// clusters), loading 4 list entries ahead; the sums meet in a wave
-// reduction, and the workgroup's are stored (no atomics) in its row of the
-// iteration's partial sums.
+// ties; each lane sums its seeds per cluster in registers, loading 4 list
+// entries ahead; the waves' sums meet in LDS, and the workgroup's are stored
+// (no atomics) in its row of the iteration's partial sums.  An iteration is a
+// chain of short steps, so their latency is what counts: with the waves'
+// sums added by 64-bit shuffles it took 10.6-11.2 us from 5,000 to 31,000
+// seeds a side.
 template <int BPC, int C, int KB>
 __global__ __launch_bounds__(256) void k_km_iter(Scratch s, int Kf, int Kb, int nb, int it) {
   const int side = blockIdx.y, K = side ? Kb : Kf;
@@ -489,14 +572,15 @@ __global__ __launch_bounds__(256) void k_km_iter(Scratch s, int Kf, int Kb, int 
     s.cbuf[((it & 1) * 2 + side) * KMAX_CLUSTERS * 3 + threadIdx.x] = s_c[threadIdx.x];
   put_table(s_q, s_c, K, C);
   __syncthreads();
-  unsigned acc[KB][C + 1];
-#pragma unroll
-  for (int k = 0; k < KB; ++k)
-#pragma unroll
-    for (int c = 0; c <= C; ++c) acc[k][c] = 0;
+  if ((int)threadIdx.x < KMAX_CLUSTERS * 4) s_sum[threadIdx.x] = 0;
+  __syncthreads();
+  KmSums<C, KB> sums;
+  sums.clear();
   const long long n = min((long long)s.ctl[side], s.cap);
   const long long stride = (long long)gridDim.x * blockDim.x;
-  for (long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x; i0 < n; i0 += 4 * stride) {
+  int held = 0;
+  for (long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+       __ballot(i0 < n); i0 += 4 * stride) {
     unsigned pk[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -506,45 +590,56 @@ __global__ __launch_bounds__(256) void k_km_iter(Scratch s, int Kf, int Kb, int 
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       if (i0 + u * stride >= n) break;
-      int x[C];
-#pragma unroll
-      for (int c = 0; c < C; ++c) x[c] = BPC == 2 ? (int)pk[u] : (int)((pk[u] >> (8 * c)) & 255u);
-      double X[C], n2;
-      scaled_feature<C>(x, X, &n2);
-      int best;
-      near_part<C>(X, (const double *)s_q, K, &best);
-#pragma unroll
-      for (int k = 0; k < KB; ++k) {
-        const bool hit = k == best;
-#pragma unroll
-        for (int c = 0; c < C; ++c) acc[k][c] += hit ? (unsigned)x[c] : 0u;
-        acc[k][C] += hit ? 1u : 0u;
-      }
+      sums.template add<BPC>(pk[u], s_q, K);
+    }
+    if ((held += 4) >= KmSums<C, KB>::kChunk) {
+      sums.flush(s_sum, K);
+      sums.clear();
+      held = 0;
     }
   }
-  // a lane holds at most n / (grid * 256) < 2^16 seeds, so its sums fit 32
-  // bits; the wave's and the workgroup's are summed in 64 bits
-  __shared__ unsigned long long s_red[4][KB * (C + 1)];
-  const int w = threadIdx.x >> 6;
-#pragma unroll
-  for (int k = 0; k < KB; ++k) {
-#pragma unroll
-    for (int c = 0; c <= C; ++c) {
-      if (k < K) {
-        unsigned long long t = acc[k][c];
-        for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o);
-        if (lane_id() == 0) s_red[w][k * (C + 1) + c] = t;
-      }
-    }
-  }
+  sums.flush(s_sum, K);
   __syncthreads();
-  const int E = K * (C + 1);
-  if ((int)threadIdx.x < E) {
-    const unsigned long long t = s_red[0][threadIdx.x] + s_red[1][threadIdx.x] +
-                                 s_red[2][threadIdx.x] + s_red[3][threadIdx.x];
+  if ((int)threadIdx.x < K * (C + 1))
     s.part[(long long)((it & 1) * 2 + side) * kPartSide + (long long)blockIdx.x * (KMAX_CLUSTERS * 4) +
-           threadIdx.x] = (long long)t;
+           threadIdx.x] = (long long)s_sum[threadIdx.x];
+}
+
+// The whole k-means of a side with up to kLoopSeeds seeds, one workgroup of
+// 1024 lanes per side (blockIdx.x): the initial centres, then Lloyd
+// iterations from seeds held in LDS until no centre moves or `iters`
+// are done.  A few thousand seeds are one or a few rounds of a workgroup, less
+// than the launches between iterations cost, and the loop ends with the
+// iteration that converges.
+constexpr int kLoopSeeds = 8192;
+
+template <int BPC, int C, int KB>
+__global__ __launch_bounds__(1024) void k_km_loop(Scratch s, int nkeys, int Kf, int Kb, int iters) {
+  __shared__ unsigned s_list[kLoopSeeds];
+  __shared__ long long s_c[KMAX_CLUSTERS * 3];
+  __shared__ double s_q[KMAX_CLUSTERS * 4];
+  __shared__ unsigned long long s_sum[KMAX_CLUSTERS * 4];
+  const int side = blockIdx.x, K = side ? Kb : Kf, tid = threadIdx.x;
+  const int n = (int)min((long long)s.ctl[side], s.cap);
+  if (!km_init<1024>(s, side, C, nkeys, K, s_c)) return;
+  // each lane reads back only the entries it wrote
+  for (int i = tid; i < n; i += 1024) s_list[i] = (unsigned)s.list[side ? s.cap - 1 - i : i];
+  bool moved = true;
+  int it = 0;
+  while (moved && it < iters) {
+    ++it;
+    put_table(s_q, s_c, K, C);
+    if (tid < KMAX_CLUSTERS * 4) s_sum[tid] = 0;
+    __syncthreads();
+    KmSums<C, KB> sums;
+    sums.clear();
+#pragma unroll 1
+    for (int i = tid; i < n; i += 1024) sums.template add<BPC>(s_list[i], s_q, K);
+    sums.flush(s_sum, K);
+    __syncthreads();
+    moved = km_means(s_sum, s_c, K, C, s_c);
   }
+  km_finish(s, side, s_c, K, C, !moved, it);
 }
 
 // The update of the last iteration, one workgroup of 256 lanes per side
@@ -1199,20 +1294,27 @@ int run_model(const InstDesc &I, const void *img, const unsigned char *seeds,
     MODEL_HIP(hipMemcpyAsync(slots, s.sums, NSUM * 2 * sizeof(long long), hipMemcpyDeviceToHost, sb));
     MODEL_HIP(hipEventRecord(S.ready, sb));
   }
-  // k-means on the device: iteration `it` assigns and updates; a side whose
-  // centres stop moving is done and its later launches return at once
-  k_km_init<<<2, 256, 0, st>>>(s, C, nkeys, prm->k_fg, prm->k_bg);
-  // up to KM_GRID workgroups per side, about 4 seeds per lane
+  // k-means on the device: in one launch for few seeds, else a launch per
+  // iteration (it assigns and updates; a side whose centres stop moving is
+  // done and its later launches return at once)
   const long long most = std::max(ctl[0], ctl[1]);
-  const int nb = (int)std::min<long long>(KM_GRID, std::max<long long>(1, (most + 1023) / 1024));
-  const dim3 ag(nb, 2);
-  const int kmax = std::max(prm->k_fg, prm->k_bg);
-  for (int it = 1; it <= iters; ++it) {
-    if (kmax <= 4) k_km_iter<BPC, C, 4><<<ag, 256, 0, st>>>(s, prm->k_fg, prm->k_bg, nb, it);
-    else if (kmax <= 8) k_km_iter<BPC, C, 8><<<ag, 256, 0, st>>>(s, prm->k_fg, prm->k_bg, nb, it);
-    else k_km_iter<BPC, C, 16><<<ag, 256, 0, st>>>(s, prm->k_fg, prm->k_bg, nb, it);
+  const int Kf = prm->k_fg, Kb = prm->k_bg, kmax = std::max(Kf, Kb);
+  if (most <= kLoopSeeds && iters > 0) {
+    if (kmax <= 4) k_km_loop<BPC, C, 4><<<2, 1024, 0, st>>>(s, nkeys, Kf, Kb, iters);
+    else if (kmax <= 8) k_km_loop<BPC, C, 8><<<2, 1024, 0, st>>>(s, nkeys, Kf, Kb, iters);
+    else k_km_loop<BPC, C, 16><<<2, 1024, 0, st>>>(s, nkeys, Kf, Kb, iters);
+  } else {
+    k_km_init<<<2, 256, 0, st>>>(s, C, nkeys, Kf, Kb);
+    // up to KM_GRID workgroups per side, about 4 seeds per lane
+    const int nb = (int)std::min<long long>(KM_GRID, std::max<long long>(1, (most + 1023) / 1024));
+    const dim3 ag(nb, 2);
+    for (int it = 1; it <= iters; ++it) {
+      if (kmax <= 4) k_km_iter<BPC, C, 4><<<ag, 256, 0, st>>>(s, Kf, Kb, nb, it);
+      else if (kmax <= 8) k_km_iter<BPC, C, 8><<<ag, 256, 0, st>>>(s, Kf, Kb, nb, it);
+      else k_km_iter<BPC, C, 16><<<ag, 256, 0, st>>>(s, Kf, Kb, nb, it);
+    }
+    if (iters > 0) k_km_final<<<2, 256, 0, st>>>(s, C, Kf, Kb, nb, iters);
   }
-  if (iters > 0) k_km_final<<<2, 256, 0, st>>>(s, C, prm->k_fg, prm->k_bg, nb, iters);
   // unary terms from the final centres, straight into the stored rows
   Unary u;
   u.den = prm->range * prm->range * (1LL << (2 * KM_FRAC));
