@@ -22,7 +22,9 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <numeric>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 using namespace jfc;
@@ -107,17 +109,18 @@ std::map<std::string, Tuned> g_tune;
 
 int log2_round(double v) { return v <= 1.0 ? 0 : (int)std::lround(std::log2(v)); }
 
-// Device counters (int64): [0] push tile visits, [2] cut tile visits, [4] tag
-// tile visits, [kIterSlots, +64) local iterations of the push kernel,
-// [kRegionSlots, +64) region visits of the relabel passes (workgroup b adds
-// to slot b % 64, so no single address takes one atomic per workgroup).
-constexpr int kIterSlots = 5, kRegionSlots = kIterSlots + 64, kTotals = kRegionSlots + 64;
-// Graphs of at most this many tiles: a search pass gives every tile a
+// Device counters (int64): [0] push tile visits, [kIterSlots, +64) local
+// iterations of the push kernel, [kRegionSlots, +64) / [kFloodSlots, +64) region
+// visits of the relabel / cut passes, [kDefSlots, +64) the remaining deficit of
+// a one-instance graph (workgroup b adds to slot b % 64, so no single address
+// takes one atomic per workgroup).
+constexpr int kIterSlots = 1, kRegionSlots = kIterSlots + 64, kFloodSlots = kRegionSlots + 64,
+              kDefSlots = kFloodSlots + 64, kTotals = kDefSlots + 64;
+// Colour classes of at most this many tiles: a push launch gives every tile a
 // workgroup of its own or nearly (a device of 256 compute units keeps
-// several tile visits per unit resident), so its passes skip the distance
-// ordering, and its launches take their tiles from the flags (no compaction
-// launches).  The reference's fixtures (1083-1200 tiles of 32x8 or 16x16)
-// solve 5-15% faster at 2048 than at 1024.
+// several tile visits per unit resident), so it takes its tiles from the
+// flags (no compaction launch).  The reference's fixtures (1083-1200 tiles of
+// 32x8 or 16x16) solve 5-15% faster at 2048 than at 1024.
 constexpr int kSmallTiles = 2048;
 // words of the results block besides the per-instance ones: the counters,
 // the sweep state (kSweepState ints) and 4 flag words
@@ -165,15 +168,16 @@ struct jfc_graph {
   int *d_tile_inst = nullptr, *d_color_tiles = nullptr;
   int *d_list[2] = {nullptr, nullptr};
   int *d_ctr = nullptr;
-  unsigned char *d_flag = nullptr, *d_dirty = nullptr, *d_seed = nullptr;
-  unsigned char *d_dirty2 = nullptr;  // second dirty buffer of small-graph searches
+  unsigned char *d_flag = nullptr, *d_seed = nullptr;
   unsigned char *d_mat = nullptr;  // per tile: residual planes written this solve
   unsigned char *d_hmat = nullptr; // per tile: heights stored this solve
   unsigned char *d_touched = nullptr;  // per tile: planes or masks written by a flush
-  // The regions of the global relabel (jfc_region.hip), the same for every
-  // push tile shape: descriptors and tables like the push tiling's, the marks
-  // of two passes, the packed bit planes and the borders' distances.
+  // The regions of the global relabel and of the cut and tag floods
+  // (jfc_region.hip, jfc_flood.hip), the same for every push tile shape:
+  // descriptors and tables like the push tiling's, the marks of two passes,
+  // the packed bit planes, the borders' distances and labels.
   struct Regions {
+    unsigned char *block = nullptr;  // holds every array below
     std::vector<InstDesc> inst;
     InstDesc *d_inst = nullptr;
     int *d_tile_inst = nullptr;
@@ -181,6 +185,8 @@ struct jfc_graph {
     unsigned char *d_dirty[2] = {nullptr, nullptr};
     int *d_any = nullptr;  // 4 words: a mark is set for pass p (slot p % 4)
     RegionBuf buf{nullptr, nullptr, nullptr, 0};
+    unsigned long long *d_out = nullptr;  // floods: labels sent across borders
+    unsigned char *d_open = nullptr;      // floods: regions with packed arcs
     int tag = 1;           // of the last relabel
     int seq = 0;           // passes run, the number their posted words carry
   } rg;
@@ -223,7 +229,6 @@ struct jfc_graph {
   // a wait on an event instead of a staged pageable copy).
   struct HostPin {
     long long total;  // tile visits so far (sweep checks)
-    int cnt[2];       // last list count of two pass groups (searches)
     int recent[3];    // active tiles of the latest sweeps
     int flag;         // certificate word of a cut search
     int bad;          // validation word of a setter
@@ -289,7 +294,7 @@ struct jfc_graph {
   void release_tiles() {
     drop_graphs();
     dfree(d_tile_inst); dfree(d_color_tiles); dfree(d_list[0]); dfree(d_list[1]);
-    dfree(d_flag); dfree(d_dirty); dfree(d_dirty2); dfree(d_seed); dfree(d_inst); dfree(d_mat);
+    dfree(d_flag); dfree(d_seed); dfree(d_inst); dfree(d_mat);
     dfree(d_hmat);
     dfree(d_touched);
   }
@@ -305,8 +310,7 @@ struct jfc_graph {
   }
   void release() {
     release_tiles();
-    dfree(rg.d_inst); dfree(rg.d_tile_inst); dfree(rg.d_dirty[0]); dfree(rg.d_dirty[1]);
-    dfree(rg.d_any); dfree(rg.buf.packed); dfree(rg.buf.base); dfree(rg.buf.border);
+    dfree(rg.block);
     rg = Regions{};
     dfree(cs); dfree(ct); dfree(c0); dfree(cap); dfree(e); dfree(h); dfree(lab); dfree(tag);
     dfree(d_ctr); dfree(d_res); dfree(d_sweep); dfree(d_energy); dfree(d_row_off);
@@ -417,8 +421,6 @@ struct jfc_graph {
         (rc = dalloc(&d_list[0], ntiles, "tile list")) ||
         (rc = dalloc(&d_list[1], ntiles, "tile list")) ||
         (rc = dalloc(&d_flag, ntiles, "tile flags")) ||
-        (rc = dalloc(&d_dirty, ntiles, "tile flags")) ||
-        (rc = dalloc(&d_dirty2, ntiles, "tile flags")) ||
         (rc = dalloc(&d_seed, ntiles, "tile seeds")) ||
         (rc = dalloc(&d_mat, ntiles, "tile states")) ||
         (rc = dalloc(&d_hmat, ntiles, "tile states")) ||
@@ -455,16 +457,30 @@ struct jfc_graph {
       std::fill(tile_inst.begin() + I.tile_off, tile_inst.begin() + I.tile_off + I.ntiles, (int)i);
     }
     const size_t border = (size_t)rg.n * region_border_words(d3);
-    int rc;
-    if ((rc = dalloc(&rg.d_inst, rg.inst.size(), "regions")) ||
-        (rc = dalloc(&rg.d_tile_inst, rg.n, "regions")) ||
-        (rc = dalloc(&rg.d_dirty[0], rg.n, "region marks")) ||
-        (rc = dalloc(&rg.d_dirty[1], rg.n, "region marks")) ||
-        (rc = dalloc(&rg.d_any, 4, "region marks")) ||
-        (rc = dalloc(&rg.buf.packed, (size_t)rg.n * rg.buf.planes * 64, "region bit planes")) ||
-        (rc = dalloc(&rg.buf.base, rg.n, "region bases")) ||
-        (rc = dalloc(&rg.buf.border, border, "region borders")))
-      return rc;
+    // one allocation, carved in 256-byte steps (the first walk sizes it)
+    const size_t n = rg.n;
+    unsigned char *base = nullptr;
+    for (size_t total = 0;;) {
+      size_t off2 = 0;
+      auto carve = [&](auto *&p, size_t count) {
+        p = (std::remove_reference_t<decltype(p)>)(base ? base + off2 : nullptr);
+        off2 += (count * sizeof(*p) + 255) / 256 * 256;
+      };
+      carve(rg.buf.packed, n * rg.buf.planes * 64);
+      carve(rg.buf.border, border);
+      carve(rg.d_out, n * flood_out_words(d3));
+      carve(rg.buf.base, n);
+      carve(rg.d_inst, rg.inst.size());
+      carve(rg.d_tile_inst, n);
+      carve(rg.d_any, 4);
+      carve(rg.d_dirty[0], n);
+      carve(rg.d_dirty[1], n);
+      carve(rg.d_open, n);
+      if (total) break;
+      total = off2;
+      if (int rc = dalloc(&rg.block, total, "regions")) return rc;
+      base = rg.block;
+    }
     launch_fill_i32(rg.buf.border, (long long)border, 0, 0);
     JFC_HIP(hipMemcpy(rg.d_inst, rg.inst.data(), rg.inst.size() * sizeof(InstDesc),
                       hipMemcpyHostToDevice));
@@ -1035,169 +1051,36 @@ struct Solver {
   }
   void advance() { g->slot ^= 1; }
 
-  // search passes issued between two host checks
-  static constexpr int kPassGroup = 4;
-
-  enum SearchMode { kCut = 0, kTag = 1 };
-
-  // Tile passes of a flood (cut or tag) until no tile is dirty.  The first
-  // pass visits the seed tiles; later passes visit the dirty tiles,
-  // alternating direction (back-and-forth, QGCWidget.cpp:2221-2240).  Tile
-  // visits are counted on the device (d_total) and read once per solve.
-  // cleared: the caller has zeroed the dirty flags already (search_fills).
-  int search(int mode, int *passes, bool cleared = false) {
-    const Tiles T = g->tiles();
-    Planes P = g->planes();
-    if (mode == kTag) P.lab = g->tag;
-    int *order = g->d_color_tiles;
-    // A small graph's passes after the first take their tiles straight from
-    // the flags (Queue::pick over the colour lists, no compaction launch).
-    // The flags are then double-buffered: pass p takes the tiles flagged in
-    // D[p & 1] and flags the next pass's in D[(p + 1) & 1], so a flag set
-    // during a pass is read only after the launch boundary that makes the
-    // labels or heights behind it visible.
-    const bool direct = g->ntiles <= kSmallTiles;
-    unsigned char *const D[2] = {direct ? g->d_dirty2 : g->d_dirty, g->d_dirty};
-    if (!cleared) {
-      launch_fill_u8(g->d_dirty, g->ntiles, 0, st);
-      if (direct) launch_fill_u8(g->d_dirty2, g->ntiles, 0, st);
-    }
-    const int nwg = std::min(g->nwg, g->ntiles);
-    long long *total = g->d_total + (mode == kTag ? 4 : 2);
-    if (int rc = g->ensure_pin()) return rc;
-    // dirty: the flags this pass sets for the next
-    auto flood = [&](const Queue &q, unsigned char *dirty) {
-      if (mode == kCut) launch_reach(g->shape, nwg, T, P, q, dirty, g->d_flagword, st);
-      else launch_tag(g->shape, nwg, T, P, q, dirty, g->lab, st);
-    };
-    // tiles without a seed gain labels only through their halo, so the
-    // first pass visits the seed tiles
-    if (direct) {
-      Queue qd{order, g->d_ctr, g->slot, g->ntiles};
-      qd.pick = g->d_seed;
-      qd.cnt = g->d_ctr + QSLOT * g->slot;
-      qd.total = total;
-      flood(qd, D[1]);
-    } else {
-      Queue q = queue_from_list();
-      launch_compact(order, g->ntiles, 0, g->d_seed, nullptr, nullptr, q, nullptr, total,
-                     nullptr, st);
-      flood(q, D[1]);
-    }
-    advance();
-    *passes += 1;
-    // later passes over the dirty tiles, alternating direction, in groups;
-    // an empty compaction ends the search.  Each group ends by copying its
-    // last list count to pinned memory, and groups are issued one ahead of
-    // the host check, so the device runs group k+1 while the host waits for
-    // group k's count instead of idling through every check.  A group issued
-    // after convergence compacts empty lists and changes nothing.
-    int pass = 1;
-    auto issue_group = [&](int k) -> int {
-      // the first group is short: a cut flood has done its work within a
-      // pass or two, and passes queued past the end each cost two launches
-      const int size = k == 0 ? 2 : kPassGroup;
-      for (int j = 0; j < size; ++j, ++pass) {
-        if (direct) {
-          // the pass's visit count goes to its slot's count word (zeroed by
-          // the launch before, as a compaction's would be)
-          Queue qd{order, g->d_ctr, g->slot, g->ntiles};
-          qd.pick = D[pass & 1];
-          qd.cnt = g->d_ctr + QSLOT * g->slot;
-          qd.total = total;
-          flood(qd, D[(pass + 1) & 1]);
-        } else {
-          Queue qc = queue_from_list();
-          launch_compact(order, g->ntiles, pass & 1, g->d_dirty, nullptr, nullptr, qc, nullptr,
-                         total, nullptr, st);
-          flood(qc, g->d_dirty);
-        }
-        advance();
-        *passes += 1;
-      }
-      // the last pass's slot is the one before the current
-      JFC_HIP(hipMemcpyAsync(&g->pin->cnt[k & 1], g->d_ctr + QSLOT * (g->slot ^ 1), sizeof(int),
-                             hipMemcpyDeviceToHost, st));
-      JFC_HIP(hipEventRecord(g->cnt_ev[k & 1], st));
-      return JFC_OK;
-    };
-    if (int rc = issue_group(0)) return rc;
-    for (int k = 0;; ++k) {
-      if (int rc = issue_group(k + 1)) return rc;
-      JFC_HIP(hipEventSynchronize(g->cnt_ev[k & 1]));
-      if (g->pin->cnt[k & 1] == 0) break;
-      if (pass > 1000000) return fail(JFC_ERR_STATE, "search did not settle");
-    }
-    return JFC_OK;
-  }
-
-  // Tag post-process over the current labels; g->tag holds the foreground
-  // seed bytes on entry.
-  int tag_pass(int *passes) {
-    launch_fill_i32(g->d_ctr, 2 * QSLOT, 0, st);
-    g->slot = 0;
-    launch_tag_init(g->shape, g->tiles(), g->tag, g->d_seed, st);
-    return search(kTag, passes);
-  }
-
-  // The zeroing a flood needs, to go into its caller's fill launch.
-  void search_fills(FillSet &f) const {
-    f.add(g->d_dirty, g->ntiles, 0, 1);
-    if (g->ntiles <= kSmallTiles) f.add(g->d_dirty2, g->ntiles, 0, 1);
-  }
-
-  // Exact relabel (graphcut_init_global_relabel + graphcut_global_relabel,
-  // graphcut_global_relabel.cl:19-124) on the graph's regions
-  // (jfc_region.hip): every region once, then the marked ones until no mark
-  // is left, then every region again to write the heights.
-  int global_relabel() {
-    hipEvent_t a = tm.mark();
+  // Passes over the regions until no region is marked: `issue(kind, ctl)`
+  // launches one.  Passes go out in groups, one group ahead of the host's
+  // check, so the device is not idle during it.  A pass with no mark returns at
+  // once and says so in its group's word.  The first groups are short, as
+  // most searches of dense graphs settle within them; later ones grow, as
+  // each check costs a gap of about 6 us between two passes.
+  template <class Issue>
+  int region_passes(int slots, int *passes, Issue issue) {
     if (int rc = g->ensure_pin()) return rc;
     auto &rg = g->rg;
-    rg.tag = 3 - rg.tag;
-    {
-      FillSet f;
-      f.add(rg.d_dirty[0], rg.n, 0, 1);
-      f.add(rg.d_dirty[1], rg.n, 0, 1);
-      f.add(rg.d_any, 4, 0, 4);
-      f.add(g->d_flag, g->ntiles, 0, 1);  // kFinal sets the active tiles' flags
-      launch_fill_multi(f, st);
-    }
-    const bool d3 = g->dim == 3;
-    const Tiles T = g->region_tiles();
-    const Planes P = g->planes();
-    int tw, th, td;
-    shape_dims(g->shape, &tw, &th, &td);
-    RegionPass A{};
-    A.tag = rg.tag;
-    A.visits = g->d_total + kRegionSlots;
-    A.active = g->d_flag;
-    A.pinst = g->d_inst;
-    A.pone = g->inst[0];
-    A.pdims = __builtin_ctz(tw) | __builtin_ctz(th) << 4 | __builtin_ctz(td) << 8;
     int pass = 0;
-    auto issue = [&](int kind, int group) {
-      A.dirty_in = rg.d_dirty[pass & 1];
-      A.dirty_out = rg.d_dirty[(pass + 1) & 1];
-      A.any_in = rg.d_any + (pass & 3);
-      A.any_out = rg.d_any + ((pass + 1) & 3);
-      A.any_clear = rg.d_any + ((pass + 2) & 3);
-      A.post = g->d_ring + kStopRing + group;
-      A.seq = rg.seq = (rg.seq + 1) & 0xffffff;
-      launch_region(d3, T, P, rg.buf, A, kind, 2 * g->nwg, st);
+    auto next = [&](int kind, int group) {
+      PassCtl c;
+      c.dirty_in = rg.d_dirty[pass & 1];
+      c.dirty_out = rg.d_dirty[(pass + 1) & 1];
+      c.any_in = rg.d_any + (pass & 3);
+      c.any_out = rg.d_any + ((pass + 1) & 3);
+      c.any_clear = rg.d_any + ((pass + 2) & 3);
+      c.post = g->d_ring + kStopRing + group;
+      c.seq = rg.seq = (rg.seq + 1) & 0xffffff;
+      c.visits = g->d_total + slots;
+      issue(kind, c);
       ++pass;
     };
-    issue(kPack, 0);
-    // Passes go out in groups, one group ahead of the host's check, so the
-    // device is not idle during it.  A pass with no mark returns at once and
-    // says so in its group's word.  The first groups are short, as most
-    // relabels of dense graphs settle within them; later ones grow, as each
-    // check costs a gap of about 6 us between two passes.
+    next(kPack, 0);
     int want[2] = {0, 0};
     auto issue_group = [&](int k) -> int {
       const int size = k < 2 ? 2 : k < 4 ? 4 : 8;
-      for (int j = 0; j < size; ++j) issue(kBorders, k & 1);
-      want[k & 1] = A.seq;
+      for (int j = 0; j < size; ++j) next(kBorders, k & 1);
+      want[k & 1] = rg.seq;
       JFC_HIP(hipEventRecord(g->cnt_ev[k & 1], st));
       return JFC_OK;
     };
@@ -1209,12 +1092,75 @@ struct Solver {
       int w = *word;
       for (int spin = 0; (w >> 1) != want[k & 1] && spin < (1 << 20); ++spin) w = *word;
       if ((w >> 1) != want[k & 1])
-        return fail(JFC_ERR_DEVICE, "a relabel pass's word did not reach the host");
+        return fail(JFC_ERR_DEVICE, "a search pass's word did not reach the host");
       if (!(w & 1)) break;
       if (pass > 1000000) return fail(JFC_ERR_STATE, "search did not settle");
     }
-    issue(kFinal, 0);
-    s.relabel_passes += pass;
+    next(kFinal, 0);
+    *passes += pass;
+    return JFC_OK;
+  }
+
+  // The zeroing region passes need, to go into their caller's fill launch.
+  void region_fills(FillSet &f) const {
+    f.add(g->rg.d_dirty[0], g->rg.n, 0, 1);
+    f.add(g->rg.d_dirty[1], g->rg.n, 0, 1);
+    f.add(g->rg.d_any, 4, 0, 4);
+  }
+
+  // A cut or tag flood over the regions (jfc_flood.hip).  fills: zeroing of the
+  // caller's, done in the same launch.
+  int flood(bool tag, bool stop, FillSet fills, int *passes) {
+    auto &rg = g->rg;
+    const bool d3 = g->dim == 3;
+    region_fills(fills);
+    fills.add(rg.d_out, 2LL * rg.n * flood_out_words(d3), 0, 4);
+    launch_fill_multi(fills, st);
+    const Tiles T = g->region_tiles();
+    Planes P = g->planes();
+    if (tag) P.lab = g->tag;
+    const FloodBuf R{rg.buf.packed, rg.d_out, rg.d_open, rg.buf.planes};
+    FloodPass A{};
+    A.cert = g->d_flagword;
+    A.stop = stop;
+    A.def = g->inst.size() == 1 ? g->d_total + kDefSlots : g->d_def;
+    A.object = g->lab;
+    return region_passes(kFloodSlots, passes, [&](int kind, const PassCtl &c) {
+      A.c = c;
+      launch_flood(d3, tag, T, P, R, A, kind, 2 * g->nwg, st);
+    });
+  }
+
+  // Exact relabel (graphcut_init_global_relabel + graphcut_global_relabel,
+  // graphcut_global_relabel.cl:19-124) on the graph's regions
+  // (jfc_region.hip): every region once, then the marked ones until no mark
+  // is left, then every region again to write the heights.
+  int global_relabel() {
+    hipEvent_t a = tm.mark();
+    auto &rg = g->rg;
+    rg.tag = 3 - rg.tag;
+    {
+      FillSet f;
+      region_fills(f);
+      f.add(g->d_flag, g->ntiles, 0, 1);  // kFinal sets the active tiles' flags
+      launch_fill_multi(f, st);
+    }
+    const bool d3 = g->dim == 3;
+    const Tiles T = g->region_tiles();
+    const Planes P = g->planes();
+    int tw, th, td;
+    shape_dims(g->shape, &tw, &th, &td);
+    RegionPass A{};
+    A.tag = rg.tag;
+    A.active = g->d_flag;
+    A.pinst = g->d_inst;
+    A.pone = g->inst[0];
+    A.pdims = __builtin_ctz(tw) | __builtin_ctz(th) << 4 | __builtin_ctz(td) << 8;
+    if (int rc = region_passes(kRegionSlots, &s.relabel_passes, [&](int kind, const PassCtl &c) {
+          A.c = c;
+          launch_region(d3, T, P, rg.buf, A, kind, 2 * g->nwg, st);
+        }))
+      return rc;
     launch_fill_u8(g->d_hmat, g->ntiles, 1, st);  // every height is stored now
     gr_ev.push_back({a, tm.mark()});
     s.global_relabels++;
@@ -1223,26 +1169,20 @@ struct Solver {
 
   int cuts = 0;  // canonical-cut searches run
 
-  // Returns 1 in *found when an augmenting path still exists.
   hipEvent_t last_cut_end = nullptr;
 
   // Returns 1 in *found when an augmenting path still exists.  The search is
   // the solve's last step when it finds none, so the certificate word comes
   // back with every result of the solve, in one copy of the results block.
-  int canonical_cut(int *found) {
+  // stop: a search that finds a path may end there, without labels.
+  int canonical_cut(int *found, bool stop) {
     hipEvent_t a = tm.mark();
     ++cuts;
-    {
-      FillSet f;
-      f.add(g->d_flagword, 1, 0, 4);
-      f.add(g->d_seed, g->ntiles, 0, 1);
-      f.add(g->d_def, 2LL * (long long)g->inst.size(), 0, 4);
-      search_fills(f);
-      launch_fill_multi(f, st);
-    }
-    launch_cut_init(g->shape, g->tiles(), g->planes(), g->d_seed, g->d_def, st, true);
-    int rc = search(kCut, &s.cut_passes, true);
-    if (rc) return rc;
+    FillSet f;
+    f.add(g->d_flagword, 1, 0, 4);
+    f.add(g->d_def, 2LL * (long long)g->inst.size(), 0, 4);
+    f.add(g->d_total + kDefSlots, 2 * 64, 0, 4);
+    if (int rc = flood(false, stop, f, &s.cut_passes)) return rc;
     last_cut_end = tm.mark();
     cut_ev.push_back({a, last_cut_end});
     JFC_HIP(hipMemcpyAsync(g->pin_res, g->d_res, g->res_words * sizeof(long long),
@@ -1463,7 +1403,7 @@ struct Solver {
         // the canonical-cut search proves that (and is the solve's last
         // step) at less cost than the relabel that would show it
         int found = 0;
-        if ((rc = canonical_cut(&found))) return rc;
+        if ((rc = canonical_cut(&found, true))) return rc;
         if (!found) {
           done = true;
           break;
@@ -1476,7 +1416,7 @@ struct Solver {
       }
       // no active tile: the canonical cut doubles as the certificate
       int found = 0;
-      if ((rc = canonical_cut(&found))) return rc;
+      if ((rc = canonical_cut(&found, true))) return rc;
       if (!found) {
         done = true;
         break;
@@ -1490,7 +1430,7 @@ struct Solver {
     if (!done) {
       // labels of the current preflow are still useful to callers
       int found = 0;
-      if ((rc = canonical_cut(&found))) return rc;
+      if ((rc = canonical_cut(&found, false))) return rc;
     }
     // the last cut search ran on the final excess, left the remaining deficit
     // of every instance in d_def and copied the results block back (the
@@ -1499,7 +1439,8 @@ struct Solver {
     const long long *pred = g->pin_res, *pdef = pred + red.size(), *totals = pdef + nI;
     s.sweeps = ((const int *)(totals + kTotals))[1];
     std::copy(pred, pred + red.size(), red.begin());
-    const std::vector<long long> def(pdef, pdef + nI);
+    std::vector<long long> def(pdef, pdef + nI);
+    if (nI == 1) def[0] = std::accumulate(totals + kDefSlots, totals + kDefSlots + 64, 0LL);
     for (int i = 0; i < nI; ++i)
       if (red[i * RED_SLOTS + RED_DEF0] == 0 && red[i * RED_SLOTS + RED_SUP0] == 0 &&
           red[i * RED_SLOTS + RED_CONST] == 0)
@@ -1518,18 +1459,22 @@ struct Solver {
     long long marked = 0;
     for (int k = 0; k < 64; ++k) marked += totals[kRegionSlots + k];
     s.relabel_tiles = marked + 2LL * g->rg.n * s.global_relabels;
-    s.cut_tiles = totals[2];
+    // cut floods: every region in the first and last pass, the marked between
+    long long sent_to = 0;
+    for (int k = 0; k < 64; ++k) sent_to += totals[kFloodSlots + k];
+    s.cut_tiles = sent_to + 2LL * g->rg.n * cuts;
     s.push_bytes = totals[0] * 256LL * push_bytes_per_node(g->Kg);
     // relabels: the first pass reads e and the mask and writes the bit planes
     // and borders, the last reads the bit planes and writes h, a marked
-    // region reads its bit planes and borders; cut searches: one pass over
-    // the nodes (read e, write the label) and flood visits (read label, e
-    // and mask, write label)
+    // region reads its bit planes and borders; cut searches: the first pass
+    // reads e, the last writes the labels, a visited region reads its mask or
+    // bit planes
     const long long rplanes = 512LL * g->rg.buf.planes;  // bytes per region
     const long long rborder = 4LL * region_border_words(g->dim == 3);
     s.solve_bytes += s.push_bytes +
                      (12LL * nodes + g->rg.n * (2 * rplanes + 2 * rborder)) * s.global_relabels +
-                     marked * (rplanes + 2 * rborder) + 5LL * nodes * cuts + totals[2] * 256LL * 10;
+                     marked * (rplanes + 2 * rborder) + 5LL * nodes * cuts +
+                     sent_to * 512LL * (g->Kg + 2);
     s.ms_total = Timer::ms(t0, t1);
     for (auto &p : push_ev) s.ms_push += Timer::ms(p.first, p.second);
     for (auto &p : gr_ev) s.ms_relabel += Timer::ms(p.first, p.second);
@@ -1646,7 +1591,7 @@ extern "C" int jfc_get_tags(jfc_graph *g, int inst, const uint8_t *fg, uint8_t *
   S.tm.pool = &g->ev_pool;
   S.tm.st = g->ustream;
   int passes = 0;
-  if ((rc = S.tag_pass(&passes))) return rc;
+  if ((rc = S.flood(true, false, FillSet{}, &passes))) return rc;
   if ((rc = get_rows(g, g->inst[inst], tags, g->tag + o, 1, on_device))) return rc;
   return sync_user(g);
 }
@@ -1744,13 +1689,9 @@ extern "C" int jfc_debug_tile_flags(jfc_graph *g, int which, uint8_t *flags) {
   if (!g || !flags || which < 0 || which > 2) return fail(JFC_ERR_INVALID, "bad argument");
   const int nI = (int)g->inst.size();
   launch_fill_i32((int *)g->d_red, 2LL * nI * RED_SLOTS, 0, 0);
-  launch_fold(g->shape, g->tiles(), g->planes(), g->d_red, which == 2 ? g->d_flag : nullptr,
+  launch_fold(g->shape, g->tiles(), g->planes(), g->d_red, which ? g->d_flag : nullptr,
               which == 0 ? g->d_seed : nullptr, false, nullptr, 0, 0);
   unsigned char *src = which == 0 ? g->d_seed : g->d_flag;
-  if (which == 1) {
-    launch_cut_init(g->shape, g->tiles(), g->planes(), g->d_seed, g->d_def, 0);
-    src = g->d_seed;
-  }
   JFC_HIP(hipDeviceSynchronize());
   JFC_HIP(hipMemcpy(flags, src, g->ntiles, hipMemcpyDeviceToHost));
   g->solved = false;

@@ -150,11 +150,6 @@ void launch_seeds(int *cs, int *ct, const unsigned char *fg, const unsigned char
 void launch_excess_split(const int *ef, int *cs, int *ct, long long n,
                          hipStream_t st);
 
-// Also sums the remaining deficit max(-e, 0) per instance into def[inst].
-// seed and def are zeroed here, unless the caller has (cleared).
-void launch_cut_init(int shape, const Tiles &T, const Planes &P,
-                     unsigned char *seed, long long *def, hipStream_t st, bool cleared = false);
-
 // Jump-flooding tile distance + counting sort of tiles by distance.
 // Lines of the tile grids along each axis: prefix[a][i] = lines along axis a
 // in the instances before i, total[a] = all of them.
@@ -234,33 +229,47 @@ struct RegionBuf {
   int planes;                  // directions stored + region_state_planes()
 };
 enum RegionPassKind { kPack = 0, kBorders = 1, kFinal = 2 };
-struct RegionPass {
-  int tag;                            // of this relabel, 1 or 2, alternating
+// What every pass over the regions (relabel, cut or tag) shares.
+struct PassCtl {
   unsigned char *dirty_in, *dirty_out;  // marks this pass takes / sets for the next
   int *any_in, *any_out, *any_clear;  // whether a mark is set; the slot after next is cleared
   int *post;                          // pinned word: seq * 2 + (any mark was set for this pass)
   int seq;
   long long *visits;                  // 64 counters of kBorders visits
+};
+struct RegionPass {
+  PassCtl c;
+  int tag;                            // of this relabel, 1 or 2, alternating
   unsigned char *active;              // push tiles' active flags, cleared by the caller
   const InstDesc *pinst;              // push tiling
   InstDesc pone;                      // its instance 0
   int pdims;                          // push tile dimensions, log2 (x | y << 4 | z << 8)
 };
+// Cut and tag floods on the same regions (jfc_flood.hip).
+struct FloodBuf {
+  unsigned long long *packed;  // the relabel's planes, free between relabels
+  unsigned long long *out;     // flood_out_words() per region: labels sent to the
+                               // neighbours; zeroed by the caller
+  unsigned char *open;         // per region: its direction planes are packed
+  int planes;
+};
+struct FloodPass {
+  PassCtl c;
+  int *cert;             // cut: set when a labelled node has a deficit
+  bool stop;             // cut: end the search once *cert is set
+  long long *def;        // cut: remaining deficit, per instance, or (one
+                         // instance) 64 partial sums; zeroed by the caller
+  const unsigned char *object;  // tag: the labels the flood stays in; P.lab then holds the
+                                // foreground seeds on entry, the tags at the end
+};
+int flood_out_words(bool d3);
+void launch_flood(bool d3, bool tag, const Tiles &T, const Planes &P, const FloodBuf &R,
+                  const FloodPass &A, int pass, int nwg, hipStream_t st);
 int region_border_words(bool d3);
 int region_state_planes();
 void region_dims(bool d3, int *tw, int *th, int *td);
 void launch_region(bool d3, const Tiles &T, const Planes &P, const RegionBuf &R,
                    const RegionPass &A, int pass, int nwg, hipStream_t st);
-void launch_reach(int shape, int nwg, const Tiles &T, const Planes &P,
-                  const Queue &q, unsigned char *dirty, int *cert,
-                  hipStream_t st);
-// Tag post-process: init (tag plane holds foreground bytes on entry) and one
-// flood pass over the queued tiles.
-void launch_tag_init(int shape, const Tiles &T, unsigned char *tag,
-                     unsigned char *seed, hipStream_t st);
-void launch_tag(int shape, int nwg, const Tiles &T, const Planes &P,
-                const Queue &q, unsigned char *dirty, const unsigned char *object,
-                hipStream_t st);
 // energy: one int64 per instance, zeroed by the caller.
 void launch_energy(int shape, const Tiles &T, const Planes &P, long long *energy,
                    hipStream_t st);

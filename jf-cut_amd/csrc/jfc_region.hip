@@ -46,48 +46,13 @@
 // 512^3 volume kPack takes 425 us (8 bytes per node read: 226 us at the rate
 // of a large copy), kFinal 156 us (134 us).  There a relabel goes from 1.8 to
 // 1.5 ms, on the 2560x1440x50 video volume from 2.9-3.0 to 2.5-2.7 ms.
-#include "jfc_device.h"
+#include "jfc_rows.h"
 
 #include <algorithm>
 
 namespace jfc {
 
-typedef unsigned long long u64;
-
-// v_writelane: `old` with lane `lane` replaced by the uniform `v`
-extern "C" __device__ int jfc_llvm_writelane(int v, int lane, int old) __asm(
-    "llvm.amdgcn.writelane.i32");
-
 namespace {
-
-template <bool D3>
-struct Reg {
-  static constexpr int TH = D3 ? 8 : 64, TD = D3 ? 8 : 1;
-  static constexpr int K = D3 ? 6 : 8;
-  // border rows along x: 2D rows 0 and 63; 3D the four faces in y and z, 8
-  // rows each (faces: 0 low y, 1 high y, 2 low z, 3 high z)
-  static constexpr int NV = D3 ? 32 : 2;
-  static __device__ __forceinline__ constexpr int row(int j) {
-    if (!D3) return j ? 63 : 0;
-    const int k = j & 7;
-    switch (j >> 3) {
-      case 0: return 8 * k;
-      case 1: return 8 * k + 7;
-      case 2: return k;
-      default: return 56 + k;
-    }
-  }
-  // the direction that leaves the region through border row j
-  static __device__ __forceinline__ constexpr int dir(int j) {
-    if (!D3) return j ? 2 : 3;
-    switch (j >> 3) {
-      case 0: return 3;
-      case 1: return 2;
-      case 2: return 5;
-      default: return 4;
-    }
-  }
-};
 
 // Border array of a region: columns x = 0 and x = 63 by row, then the border
 // rows by x.
@@ -107,43 +72,6 @@ constexpr int kStatePlanes = 3 + kCntBits;
 // the planes: its visits search from scratch)
 constexpr int kNoBase = -1;
 
-// one-bit shifts of a row's word as two full-rate 32-bit instructions
-__device__ __forceinline__ u64 shr1(u64 f) {
-  const unsigned lo = (unsigned)f, hi = (unsigned)(f >> 32);
-  return (u64)(hi >> 1) << 32 | __builtin_amdgcn_alignbit(hi, lo, 1);
-}
-__device__ __forceinline__ u64 shl1(u64 f) {
-  const unsigned lo = (unsigned)f, hi = (unsigned)(f >> 32);
-  return (u64)__builtin_amdgcn_alignbit(hi, lo, 31) << 32 | lo << 1;
-}
-__device__ __forceinline__ u64 from_next(u64 f) {  // lane r: lane r + 1's word, 0 in lane 63
-  const unsigned lo = __builtin_amdgcn_update_dpp(0u, (unsigned)f, 0x130, 0xf, 0xf, true);
-  const unsigned hi = __builtin_amdgcn_update_dpp(0u, (unsigned)(f >> 32), 0x130, 0xf, 0xf, true);
-  return (u64)hi << 32 | lo;
-}
-__device__ __forceinline__ u64 from_prev(u64 f) {  // lane r: lane r - 1's word, 0 in lane 0
-  const unsigned lo = __builtin_amdgcn_update_dpp(0u, (unsigned)f, 0x138, 0xf, 0xf, true);
-  const unsigned hi = __builtin_amdgcn_update_dpp(0u, (unsigned)(f >> 32), 0x138, 0xf, 0xf, true);
-  return (u64)hi << 32 | lo;
-}
-__device__ __forceinline__ u64 from_lane(u64 f, int addr) {  // lane addr / 4's word
-  const unsigned lo = __builtin_amdgcn_ds_bpermute(addr, (int)(unsigned)f);
-  const unsigned hi = __builtin_amdgcn_ds_bpermute(addr, (int)(unsigned)(f >> 32));
-  return (u64)hi << 32 | lo;
-}
-// row r's word as a uniform value
-__device__ __forceinline__ u64 row_word(u64 w, int r) {
-  const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)w, r);
-  const unsigned hi = __builtin_amdgcn_readlane((int)(unsigned)(w >> 32), r);
-  return (u64)hi << 32 | lo;
-}
-__device__ __forceinline__ void set_row(int &lo, int &hi, int r, u64 w) {
-  lo = jfc_llvm_writelane((int)(unsigned)w, r, lo);
-  hi = jfc_llvm_writelane((int)(unsigned)(w >> 32), r, hi);
-}
-__device__ __forceinline__ bool bit_of_lane(u64 uniform) {
-  return __builtin_amdgcn_inverse_ballot_w64(uniform);
-}
 __device__ __forceinline__ unsigned wave_or(unsigned v) {
   v |= __builtin_amdgcn_update_dpp(0u, v, 0x111, 0xf, 0xf, false);  // row_shr:1
   v |= __builtin_amdgcn_update_dpp(0u, v, 0x112, 0xf, 0xf, false);
@@ -203,14 +131,10 @@ __device__ __forceinline__ void region_visit(const Tiles &T, const Planes &P,
   const int wv0 = W > 1 ? 64 / W * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;  // first row
   const InstDesc &I = ONE ? T.one : T.inst[T.tile_inst[t]];
   const int K = I.K;
-  const int lt = t - I.tile_off;
-  const int ltx = lt % I.tx, lq = lt / I.tx;
-  const int lty = lq % I.ty, ltz = lq / I.ty;
-  const int ox = ltx * 64, oy = lty * G::TH, oz = ltz * G::TD;
-  const int wx = min(64, I.nx - ox);
+  const RegionRef r = region_ref<D3>(I, t, lane);
+  const int ox = r.ox, oy = r.oy, oz = r.oz, wx = r.wx;
   const int ly = D3 ? lane & 7 : lane, lz = D3 ? lane >> 3 : 0;
-  const u64 xmask = wx == 64 ? ~0ull : (1ull << wx) - 1;
-  const u64 valid = oy + ly < I.ny && oz + lz < I.nz ? xmask : 0;
+  const u64 valid = r.valid;
 
   // ---- bit planes: open arcs per direction, deficits, excess
   u64 M[KM], D = 0, X = 0;
@@ -356,11 +280,10 @@ __device__ __forceinline__ void region_visit(const Tiles &T, const Planes &P,
   }
 
   // ---- distances of the border nodes through the neighbours' borders
-  const bool hasl = ltx > 0, hasr = ltx + 1 < I.tx;
-  const bool hasd = lty > 0, hasu = lty + 1 < I.ty;
+  const bool hasl = r.hasl, hasr = r.hasr, hasd = r.hasd, hasu = r.hasu;
   const bool diag = !D3 && K == 8;
   const long long b0 = (long long)t * BN;
-  const long long by = (long long)I.tx * BN, bz = by * I.ty;
+  const long long by = (long long)r.sy * BN, bz = (long long)r.sz * BN;
   // every word is loaded before any is used; a missing neighbour's is the
   // region's own, and discarded
   auto word = [&](bool have, long long off, int idx) {
@@ -379,7 +302,7 @@ __device__ __forceinline__ void region_visit(const Tiles &T, const Planes &P,
       wc[2] = word(hc[2], BN - by, kLeft + 63);
       wc[3] = word(hc[3], BN + by, kLeft);
     }
-    const bool has[4] = {hasd, hasu, ltz > 0, ltz + 1 < I.tz};
+    const bool has[4] = {hasd, hasu, r.hasf, r.hasb};
     const long long off[4] = {-by, by, -bz, bz};
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
@@ -491,7 +414,7 @@ __device__ __forceinline__ void region_visit(const Tiles &T, const Planes &P,
   // smallest border distance that improves a border node, with the nodes
   // nearer than the block settled and those at the level before it as the
   // frontier.
-  int L;  // first level of the block
+  int L = 0;  // first level of the block
   u64 nw = 0;
   bool scratch = true;
   if (PASS == kBorders) {
@@ -582,12 +505,12 @@ __device__ __forceinline__ void region_visit(const Tiles &T, const Planes &P,
         if (!D3 || (j & 7) == 0) face[f] = c;
         else face[f] |= c;
       }
-      const int sy = I.tx, sz = I.tx * I.ty;
+      const int sy = r.sy, sz = r.sz;
       bool any = false;
       auto mark = [&](bool have, u64 changed, int nb) {
         if (have && changed) {
           any = true;
-          if (lane == 0) A.dirty_out[nb] = 1;
+          if (lane == 0) A.c.dirty_out[nb] = 1;
         }
       };
       mark(hasl, cl, t - 1);
@@ -595,8 +518,8 @@ __device__ __forceinline__ void region_visit(const Tiles &T, const Planes &P,
       mark(hasd, face[0], t - sy);
       mark(hasu, face[1], t + sy);
       if constexpr (D3) {
-        mark(ltz > 0, face[2], t - sz);
-        mark(ltz + 1 < I.tz, face[3], t + sz);
+        mark(r.hasf, face[2], t - sz);
+        mark(r.hasb, face[3], t + sz);
       } else if (diag) {
         mark(hasl && hasd, cl & 1, t - 1 - sy);
         mark(hasl && hasu, cl >> 63, t - 1 + sy);
@@ -680,10 +603,10 @@ __global__ __launch_bounds__(64 * W) void k_region(Tiles T, Planes P, RegionBuf 
   bool marked = false;
   if (PASS == kBorders) {
     // some region was marked for this pass; the host learns it from here
-    const int work = *A.any_in;
+    const int work = *A.c.any_in;
     if (blockIdx.x == 0 && lane == 0) {
-      *A.any_clear = 0;
-      __hip_atomic_store(A.post, A.seq * 2 + (work != 0), __ATOMIC_RELAXED,
+      *A.c.any_clear = 0;
+      __hip_atomic_store(A.c.post, A.c.seq * 2 + (work != 0), __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_SYSTEM);
     }
     if (!work) return;
@@ -701,8 +624,8 @@ __global__ __launch_bounds__(64 * W) void k_region(Tiles T, Planes P, RegionBuf 
     const int G = gridDim.x;
     for (int base = blockIdx.x; base < T.ntiles; base += 64 * G) {
       const long long mine = base + (long long)lane * G;
-      const bool f = mine < T.ntiles && A.dirty_in[mine];
-      if (f) A.dirty_in[mine] = 0;
+      const bool f = mine < T.ntiles && A.c.dirty_in[mine];
+      if (f) A.c.dirty_in[mine] = 0;
       u64 m = __ballot(f);
       visits += __popcll(m);
       while (m) {
@@ -712,16 +635,10 @@ __global__ __launch_bounds__(64 * W) void k_region(Tiles T, Planes P, RegionBuf 
       }
     }
     if (visits && lane == 0)
-      atomicAdd((u64 *)&A.visits[blockIdx.x & 63], (u64)visits);
+      atomicAdd((u64 *)&A.c.visits[blockIdx.x & 63], (u64)visits);
   }
-  if (PASS != kFinal && marked && lane == 0) *A.any_out = 1;
+  if (PASS != kFinal && marked && lane == 0) *A.c.any_out = 1;
 }
-
-// Graphs of up to this many regions leave most of the device's 1024 SIMDs with
-// one wave or none in a pass over every region: there four waves share the
-// rows of a region.  Above it a wave per region fills the device and the
-// exchange through LDS would only add to its work.
-constexpr int kSharedRegions = 512;
 
 template <bool D3, bool ONE>
 void launch(const Tiles &T, const Planes &P, const RegionBuf &R, const RegionPass &A, int pass,

@@ -1,0 +1,125 @@
+// jfc_rows.h -- regions of 4096 nodes as 64-bit row words, shared by the global
+// relabel (jfc_region.hip) and the cut and tag floods (jfc_flood.hip).
+//
+// One wavefront owns a region: 64 x 64 nodes in 2D, 64 x 8 x 8 in 3D.  Lane r
+// holds row r (2D: y = r; 3D: y = r & 7, z = r >> 3), bit x = column x.
+#pragma once
+
+#include "jfc_device.h"
+
+namespace jfc {
+
+typedef unsigned long long u64;
+
+// v_writelane: `old` with lane `lane` replaced by the uniform `v`
+extern "C" __device__ int jfc_llvm_writelane(int v, int lane, int old) __asm(
+    "llvm.amdgcn.writelane.i32");
+
+template <bool D3>
+struct Reg {
+  static constexpr int TH = D3 ? 8 : 64, TD = D3 ? 8 : 1;
+  static constexpr int K = D3 ? 6 : 8;
+  // border rows along x: 2D rows 0 and 63; 3D the four faces in y and z, 8
+  // rows each (faces: 0 low y, 1 high y, 2 low z, 3 high z)
+  static constexpr int NV = D3 ? 32 : 2;
+  static __device__ __forceinline__ constexpr int row(int j) {
+    if (!D3) return j ? 63 : 0;
+    const int k = j & 7;
+    switch (j >> 3) {
+      case 0: return 8 * k;
+      case 1: return 8 * k + 7;
+      case 2: return k;
+      default: return 56 + k;
+    }
+  }
+  // the direction that leaves the region through border row j
+  static __device__ __forceinline__ constexpr int dir(int j) {
+    if (!D3) return j ? 2 : 3;
+    switch (j >> 3) {
+      case 0: return 3;
+      case 1: return 2;
+      case 2: return 5;
+      default: return 4;
+    }
+  }
+};
+
+// one-bit shifts of a row's word as two full-rate 32-bit instructions
+__device__ __forceinline__ u64 shr1(u64 f) {
+  const unsigned lo = (unsigned)f, hi = (unsigned)(f >> 32);
+  return (u64)(hi >> 1) << 32 | __builtin_amdgcn_alignbit(hi, lo, 1);
+}
+__device__ __forceinline__ u64 shl1(u64 f) {
+  const unsigned lo = (unsigned)f, hi = (unsigned)(f >> 32);
+  return (u64)__builtin_amdgcn_alignbit(hi, lo, 31) << 32 | lo << 1;
+}
+__device__ __forceinline__ u64 from_next(u64 f) {  // lane r: lane r + 1's word, 0 in lane 63
+  const unsigned lo = __builtin_amdgcn_update_dpp(0u, (unsigned)f, 0x130, 0xf, 0xf, true);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0u, (unsigned)(f >> 32), 0x130, 0xf, 0xf, true);
+  return (u64)hi << 32 | lo;
+}
+__device__ __forceinline__ u64 from_prev(u64 f) {  // lane r: lane r - 1's word, 0 in lane 0
+  const unsigned lo = __builtin_amdgcn_update_dpp(0u, (unsigned)f, 0x138, 0xf, 0xf, true);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0u, (unsigned)(f >> 32), 0x138, 0xf, 0xf, true);
+  return (u64)hi << 32 | lo;
+}
+__device__ __forceinline__ u64 from_lane(u64 f, int addr) {  // lane addr / 4's word
+  const unsigned lo = __builtin_amdgcn_ds_bpermute(addr, (int)(unsigned)f);
+  const unsigned hi = __builtin_amdgcn_ds_bpermute(addr, (int)(unsigned)(f >> 32));
+  return (u64)hi << 32 | lo;
+}
+// row r's word as a uniform value
+__device__ __forceinline__ u64 row_word(u64 w, int r) {
+  const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)w, r);
+  const unsigned hi = __builtin_amdgcn_readlane((int)(unsigned)(w >> 32), r);
+  return (u64)hi << 32 | lo;
+}
+__device__ __forceinline__ void set_row(int &lo, int &hi, int r, u64 w) {
+  lo = jfc_llvm_writelane((int)(unsigned)w, r, lo);
+  hi = jfc_llvm_writelane((int)(unsigned)(w >> 32), r, hi);
+}
+__device__ __forceinline__ bool bit_of_lane(u64 uniform) {
+  return __builtin_amdgcn_inverse_ballot_w64(uniform);
+}
+
+// Graphs of up to this many regions leave most of the device's 1024 SIMDs with
+// one wave or none in a pass over every region: there four waves share the
+// rows of a region.  Above it a wave per region fills the device and the
+// exchange through LDS would only add to its work.
+constexpr int kSharedRegions = 512;
+
+// A region's place in its instance.
+struct RegionRef {
+  int ox, oy, oz, wx;       // origin; columns inside the grid
+  bool hasl, hasr;          // neighbours at x - 1, x + 1
+  bool hasd, hasu;          // at y - 1, y + 1
+  bool hasf, hasb;          // at z - 1, z + 1
+  int sy, sz;               // region index steps in y and z
+  u64 valid;                // the lane's row inside the grid
+};
+
+template <bool D3>
+__device__ __forceinline__ RegionRef region_ref(const InstDesc &I, int t, int lane) {
+  using G = Reg<D3>;
+  RegionRef r;
+  const int lt = t - I.tile_off;
+  const int ltx = lt % I.tx, lq = lt / I.tx;
+  const int lty = lq % I.ty, ltz = lq / I.ty;
+  r.ox = ltx * 64;
+  r.oy = lty * G::TH;
+  r.oz = ltz * G::TD;
+  r.wx = min(64, I.nx - r.ox);
+  r.hasl = ltx > 0;
+  r.hasr = ltx + 1 < I.tx;
+  r.hasd = lty > 0;
+  r.hasu = lty + 1 < I.ty;
+  r.hasf = ltz > 0;
+  r.hasb = ltz + 1 < I.tz;
+  r.sy = I.tx;
+  r.sz = I.tx * I.ty;
+  const int y = r.oy + (D3 ? lane & 7 : lane), z = r.oz + (D3 ? lane >> 3 : 0);
+  r.valid = y < I.ny && z < I.nz ? (r.wx == 64 ? ~0ull : (1ull << r.wx) - 1) : 0;
+  return r;
+}
+
+}  // namespace jfc

@@ -2,13 +2,10 @@
 //
 // Reference counterparts (paths relative to src/QVisualizer/):
 //   k_push     graphcut_relabel_push   cl/GraphCut/graphcut_push_relabel.cl:25-203 (2D), :215-439 (3D)
-//   k_reach    graphcut_compute_cut    cl/GraphCut/graphcut_compute_cut.cl:51-140, :182-282
-//   k_cut_init graphcut_init_cut       graphcut_compute_cut.cl:19-49
 //   k_compact  graphcut_count_node + clogs scan + graphcut_scatter_node
 //                               cl/GraphCut/graphcut_count_block.cl:19-65
 //   k_jf_*     graphcut_bfs_jump_flooding / _histogram / _mapping
 //              cl/GraphCut/graphcut_bfs_block.cl:43-91 (+ reduce_histogram, INF reduce.cl:56-141)
-//   k_cut_init also reduce_flow  bin/x64/cl/Infrastructures/reduce.cl:17-42 (int64 here)
 //
 // Layout: every graph stores int32 planes (e, h, K residual planes) in
 // structure-of-arrays order over all instances.  Kernels work on tiles of
@@ -177,30 +174,9 @@ struct Chunk {
 
 static int tile_grid(int ntiles) { return ntiles < 4096 ? (ntiles > 0 ? ntiles : 1) : 4096; }
 
-// Streaming tile kernels keep TU tiles in flight per lane (their loads are
-// issued before any use) so that enough bytes are outstanding to cover HBM
-// latency with one 256-lane group per tile.
-constexpr int TU = 4;
-
-// Bitwise OR of TU per-tile bits over the 256-lane workgroup (4 waves):
-// one ballot per bit, one LDS word per wave.  The buffer half alternates with
-// `parity`, so the words read in one group are never overwritten before
-// every lane has passed the next group's barrier.  (__syncthreads_or only
-// tells whether any lane is non-zero.)
-__device__ __forceinline__ int block_or_bits(int bits, int *s_w, int parity) {
-  int m = 0;
-#pragma unroll
-  for (int u = 0; u < TU; ++u)
-    if (__ballot((bits >> u) & 1)) m |= 1 << u;
-  int *buf = s_w + 4 * parity;
-  if (lane_id() == 0) buf[threadIdx.x >> 6] = m;
-  __syncthreads();
-  return buf[0] | buf[1] | buf[2] | buf[3];
-}
-
 // Any lane of the 256-lane workgroup with pred set: one ballot per wave, one
-// LDS word per wave, one barrier.  The buffer half alternates with `parity`
-// (as in block_or_bits), so a second barrier is not needed before reuse.
+// LDS word per wave, one barrier.  The buffer half alternates with `parity`,
+// so a second barrier is not needed before reuse.
 // The barrier also orders the workgroup's LDS accesses like __syncthreads.
 __device__ __forceinline__ int block_any(int pred, int *s_w, int &parity) {
   const int w = __ballot(pred) != 0;
@@ -209,26 +185,6 @@ __device__ __forceinline__ int block_any(int pred, int *s_w, int &parity) {
   if (lane_id() == 0) buf[threadIdx.x >> 6] = w;
   __syncthreads();
   return buf[0] | buf[1] | buf[2] | buf[3];
-}
-
-// Node of lane L in tile t; inst = -1 past the end of the chunk.
-struct TileNode {
-  int inst;
-  bool valid;
-  long long v;
-};
-
-template <class S>
-__device__ __forceinline__ TileNode tile_node(const Tiles &T, int t, int t_end,
-                                              const Lane<S> &L) {
-  TileNode n{-1, false, 0};
-  if (t >= t_end) return n;
-  const TileRef r = tile_ref<S>(T, t);
-  n.inst = T.tile_inst[t];
-  const int gx = r.ox + L.lx, gy = r.oy + L.ly, gz = r.oz + L.lz;
-  n.valid = gx < r.I.nx && gy < r.I.ny && gz < r.I.nz;
-  n.v = node_index(r.I, gx, gy, gz);
-  return n;
 }
 
 // ---- row-streaming passes ----------------------------------------------------
@@ -336,15 +292,6 @@ __device__ __forceinline__ void store4(int *p, long long v, int n, int4 a) {
   if (n > 1) p[v + 1] = a.y;
   if (n > 2) p[v + 2] = a.z;
   if (n > 3) p[v + 3] = a.w;
-}
-
-__device__ __forceinline__ void store4_u8(unsigned char *p, long long v, int n, unsigned bits) {
-  if (n == 4 && (((size_t)(p + v)) & 3) == 0) {
-    *(unsigned *)(p + v) = (bits & 1u) | ((bits >> 1) & 1u) << 8 | ((bits >> 2) & 1u) << 16 |
-                           ((bits >> 3) & 1u) << 24;
-    return;
-  }
-  for (int i = 0; i < n; ++i) p[v + i] = (unsigned char)((bits >> i) & 1u);
 }
 
 __device__ __forceinline__ int comp(const int4 &a, int i) {
@@ -553,66 +500,6 @@ void launch_fold(int shape, const Tiles &T, const Planes &P, long long *red,
   }
 }
 
-// graphcut_init_cut (graphcut_compute_cut.cl:19-49): label = 1 where
-// excess > 0, tiles holding such a node seed the jump flooding (`seed`
-// zeroed by the launcher).  The same pass sums the remaining deficit
-// max(-e, 0) per instance into def[inst] (reduce_flow, reduce.cl:17-42, in
-// int64): the cut search is the last step of a solve and reads the final
-// excess.
-template <class S>
-__global__ __launch_bounds__(256) void k_cut_init(Tiles T, Planes P, unsigned char *seed,
-                                                  long long *def) {
-  __shared__ long long buf[4];
-  long long *dst[1] = {def};
-  const int stride[1] = {1};
-  InstSums<1> sums;
-  sums.reset();
-  // two groups in flight per lane: 67 registers, 7 waves per SIMD (four: 95,
-  // 5 waves, 0.013 ms slower on the 15000x10000 8-connected cut)
-  constexpr int U = 2;
-  const int nsteps = row_steps(T);
-  for (int step = blockIdx.x; step < nsteps; step += gridDim.x) {
-    const RowStep<S> RS(T, step);
-    sums.enter(RS.R0.inst, dst, stride, buf);
-    for (int k0 = threadIdx.x; k0 < RS.slots; k0 += U * 256) {
-      Group g[U];
-      RowRef<S> R[U];
-      int4 e[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int k = k0 + u * 256;
-        if (k < RS.slots) RS.at(T, k, R[u], g[u]);
-        else { R[u] = RS.R0; g[u] = Group{0, 0}; }
-        e[u] = load4(P.e, R[u].v0 + g[u].x, g[u].n);
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (g[u].n == 0) continue;
-        unsigned bits = 0;
-        for (int i = 0; i < g[u].n; ++i) {
-          const int x = comp(e[u], i);
-          sums.a[0] += max(-x, 0);
-          bits |= (unsigned)(x > 0) << i;
-        }
-        store4_u8(P.lab, R[u].v0 + g[u].x, g[u].n, bits);
-        flag_group<S>(seed, R[u].tile0, g[u], bits);
-      }
-    }
-  }
-  sums.flush(dst, stride, buf);
-}
-
-void launch_cut_init(int shape, const Tiles &T, const Planes &P,
-                     unsigned char *seed, long long *def, hipStream_t st, bool cleared) {
-  if (!cleared) {
-    launch_fill_u8(seed, T.ntiles, 0, st);
-    launch_fill_i32((int *)def, 2LL * T.ninst, 0, st);
-  }
-  JFC_DISPATCH(shape,
-               (k_cut_init<S><<<row_grid<&k_cut_init<S>>((T.nrows + T.row_step - 1) / T.row_step),
-                                256, 0, st>>>(T, P, seed, def)));
-}
-
 // Cut energy on the input capacities (QGCWidget.cpp:2452-2520), summed per
 // instance into energy[inst] (zeroed by the caller).
 template <class S>
@@ -714,43 +601,6 @@ void launch_backward_all(int shape, const Tiles &T, const Planes &P, float *dcs,
                          float *dct, float *dnb, long long user_total, hipStream_t st) {
   JFC_DISPATCH(shape, (k_backward<S><<<tile_grid(T.ntiles), 256, 0, st>>>(
                           T, P, 0, T.ntiles, dcs, dct, dnb, user_total)));
-}
-
-// ---- initialisation of relabel / cut searches --------------------------------
-
-// graphcut_init_tag (graphcut_compute_tag.cl:19-49): the tag plane arrives
-// holding the foreground seed bytes; it leaves as 0/1, and tiles with a seed
-// seed the jump flooding.
-template <class S>
-__global__ __launch_bounds__(256) void k_tag_init(Tiles T, unsigned char *tag,
-                                                  unsigned char *seed) {
-  const Lane<S> L(threadIdx.x);
-  const Chunk C(T.ntiles);
-  __shared__ int s_w[8];
-  int par = 0;
-  for (int t = C.t0; t < C.t1; t += TU) {
-    TileNode nd[TU];
-    unsigned char f[TU];
-#pragma unroll
-    for (int u = 0; u < TU; ++u) nd[u] = tile_node<S>(T, t + u, C.t1, L);
-#pragma unroll
-    for (int u = 0; u < TU; ++u) f[u] = nd[u].valid ? tag[nd[u].v] : 0;
-    int bits = 0;
-#pragma unroll
-    for (int u = 0; u < TU; ++u)
-      if (nd[u].valid) {
-        tag[nd[u].v] = (unsigned char)(f[u] != 0);
-        bits |= (f[u] != 0) << u;
-      }
-    bits = block_or_bits(bits, s_w, par ^= 1);
-    if (threadIdx.x < TU && t + (int)threadIdx.x < C.t1)
-      seed[t + threadIdx.x] = (unsigned char)((bits >> threadIdx.x) & 1);
-  }
-}
-
-void launch_tag_init(int shape, const Tiles &T, unsigned char *tag, unsigned char *seed,
-                     hipStream_t st) {
-  JFC_DISPATCH(shape, (k_tag_init<S><<<tile_grid(T.ntiles), 256, 0, st>>>(T, tag, seed)));
 }
 
 // ---- jump flooding over the tile grid + counting sort --------------------------
@@ -1745,143 +1595,6 @@ void launch_push(int shape, int nwg, const Tiles &T, const Planes &P,
                             T, P, q, flag, mat, touched, hmat, max_iters, sparse_iters,
                             sweep_state, iter_total)));
   }
-}
-
-// ---- canonical cut: residual reachability from excess nodes -------------------------
-//
-// A labelled node labels every neighbour it has residual capacity toward
-// (graphcut_compute_cut.cl:95-113, here from the tail of the arc so only the
-// node's own planes are read).  Labels entering the halo are written to HBM
-// and mark the neighbour tile for the next pass.  A labelled node with a
-// deficit means an augmenting path still exists: *cert is set
-// (graphcut_compute_cut.cl:135-139).
-//
-// TAG: the same flood for the tag post-process (graphcut_compute_tag.cl:51-140,
-// :142-242): P.lab is the tag plane, a tagged node tags its axis neighbours
-// (4 in 2D, 6 in 3D) that are on the source side of the cut (`object`).
-// LDS codes: 0 open, 1 labelled on entry, 2 labelled here, 4 closed.
-template <class S, bool TAG, bool ONE>
-__global__ __launch_bounds__(256) void k_reach(Tiles T, Planes P, Queue q,
-                                               unsigned char *dirty, int *cert,
-                                               const unsigned char *object) {
-  __shared__ unsigned char s_l[S::PADN];
-  const int tid = threadIdx.x;
-  const Lane<S> L(tid);
-  __shared__ int s_next[3];
-  __shared__ int s_w[8];
-  int par = 0;
-  VisitCursor Qc(q, s_next);
-  constexpr unsigned kAxis = S::D3 ? 0x3fu : 0xfu;
-  while (Qc.idx >= 0) {
-    const int t = Qc.ent;
-    const TileRef r = ONE ? tile_ref_of<S>(T.one, t) : tile_ref<S>(T, t);
-    const InstDesc &I = r.I;
-    const int K = TAG ? (S::D3 ? 6 : 4) : I.K;
-    const int gx = r.ox + L.lx, gy = r.oy + L.ly, gz = r.oz + L.lz;
-    const bool valid = gx < I.nx && gy < I.ny && gz < I.nz;
-    // every load of the visit is issued before any is used (dead lanes and
-    // halo cells read a valid dummy address)
-    const long long gv = valid ? node_index(I, gx, gy, gz) : 0;
-    // halo: the ring cells, split evenly over the four waves (as in k_push)
-    HaloCell hc[kRingPerLane<S>];
-    int hp[kRingPerLane<S>];
-    unsigned char hl[kRingPerLane<S>], ho[kRingPerLane<S>];
-#pragma unroll
-    for (int c = 0; c < kRingPerLane<S>; ++c) {
-      const int j = c * 64 + (tid & 63);
-      const int k = (tid >> 6) * kRingQ<S> + j;
-      hp[c] = j < kRingQ<S> && k < Ring<S>::N ? Ring<S>::pos(k) : S::PADN;
-      hc[c] = halo_cell<S>(I, r.ox, r.oy, r.oz, hp[c], K);
-      hl[c] = P.lab[hc[c].g];
-      if (TAG) ho[c] = object[hc[c].g];
-    }
-    unsigned char l0 = P.lab[gv];
-    unsigned mask;
-    bool deficit = false;
-    if (TAG) {
-      l0 = l0 ? 1 : object[gv] ? 0 : 4;
-      mask = kAxis;
-    } else {
-      deficit = P.e[gv] < 0;
-      mask = P.rmask[gv] & ((1u << K) - 1u);
-    }
-    if (!valid) {
-      l0 = TAG ? 4 : 0;
-      mask = 0;
-      deficit = false;
-    }
-    if (!TAG && l0 && deficit) *cert = 1;
-    s_l[L.me] = l0;
-#pragma unroll
-    for (int c = 0; c < kRingPerLane<S>; ++c) {
-      if (!hc[c].halo) continue;
-      unsigned char lv = 1;
-      if (hc[c].live) lv = TAG ? (hl[c] ? 1 : ho[c] ? 0 : 4) : hl[c];
-      s_l[hp[c]] = lv;
-    }
-    __syncthreads();
-    // the next entry loads while the tile iterates
-    if (tid == 0) Qc.prefetch();
-    int any;
-    do {
-      int ch = 0;
-      const unsigned me = s_l[L.me];
-      if (mask && (me == 1u || me == 2u)) {
-        // neighbour labels read up front (one LDS wait); another lane may
-        // label the same neighbour meanwhile, and both then write the same 2
-        unsigned char lv[S::KMAX];
-#pragma unroll
-        for (int d = 0; d < S::KMAX; ++d) lv[d] = s_l[L.me + lds_off<S>(d)];
-#pragma unroll
-        for (int d = 0; d < S::KMAX; ++d)
-          if ((mask & (1u << d)) && lv[d] == 0) {
-            s_l[L.me + lds_off<S>(d)] = 2;
-            ch = 1;
-          }
-      }
-      any = block_any(ch, s_w, par);
-    } while (any);
-    if (valid && s_l[L.me] == 2) {
-      P.lab[gv] = 1;
-      if (!TAG && deficit) *cert = 1;
-    }
-    // halo cells labelled by this visit (only live ring cells can be)
-#pragma unroll
-    for (int c = 0; c < kRingPerLane<S>; ++c) {
-      if (!hc[c].live || s_l[hp[c]] != 2) continue;
-      int x, y, z, nout;
-      bool inter;
-      pad_coords<S>(hp[c], x, y, z, inter, nout);
-      const int X = r.ox + x, Y = r.oy + y, Z = r.oz + z;
-      P.lab[hc[c].g] = 1;
-      dirty[tile_of<S>(I, X, Y, Z)] = 1;
-    }
-    if (tid == 0) Qc.publish();
-    __syncthreads();
-    Qc.advance();
-  }
-}
-
-template <bool TAG, bool ONE>
-static void reach_launch(int shape, int nwg, const Tiles &T, const Planes &P, const Queue &q,
-                         unsigned char *dirty, int *cert, const unsigned char *object,
-                         hipStream_t st) {
-  JFC_DISPATCH(shape, (k_reach<S, TAG, ONE><<<resident_grid<&k_reach<S, TAG, ONE>>(nwg), 256, 0,
-                                              st>>>(T, P, q, dirty, cert, object)));
-}
-
-void launch_reach(int shape, int nwg, const Tiles &T, const Planes &P,
-                  const Queue &q, unsigned char *dirty, int *cert,
-                  hipStream_t st) {
-  if (T.ninst == 1) reach_launch<false, true>(shape, nwg, T, P, q, dirty, cert, nullptr, st);
-  else reach_launch<false, false>(shape, nwg, T, P, q, dirty, cert, nullptr, st);
-}
-
-void launch_tag(int shape, int nwg, const Tiles &T, const Planes &P,
-                const Queue &q, unsigned char *dirty, const unsigned char *object,
-                hipStream_t st) {
-  if (T.ninst == 1) reach_launch<true, true>(shape, nwg, T, P, q, dirty, nullptr, object, st);
-  else reach_launch<true, false>(shape, nwg, T, P, q, dirty, nullptr, object, st);
 }
 
 }  // namespace jfc

@@ -54,3 +54,23 @@ def test_long_corridor_gpu(gpu, shape):
     assert g.flow() == f
     assert np.array_equal(g.labels(), l)
     g.close()
+
+
+@pytest.mark.parametrize("shape", [s + (1,) for s in SHAPES_2D] + SHAPES_3D)
+def test_region_edges_tag_gpu(gpu, shape):
+    """The tag flood over the regions: seeds on and off the source side, at the
+    corners and inside, on a cut of dense terminals (many small components)."""
+    nx, ny, nz = shape
+    conn = 6 if nz > 1 else 8
+    rng = np.random.default_rng(31 * nx + 7 * ny + nz)
+    cs, ct, caps = random_grid(rng, nx, ny, nz, conn, cap_max=8)
+    cs[0], ct[-1] = 500, 700
+    say("case region edges tag", shape)
+    g, st = solve_grid(gpu, nx, ny, nz, conn, cs, ct, caps)
+    assert st.converged == 1
+    lab = g.labels()
+    for frac in (0.0, 0.02, 0.3):
+        fg = (rng.random(nx * ny * nz) < frac).astype(np.uint8)
+        fg[0] = fg[-1] = 1
+        assert np.array_equal(g.tags(fg), ol.tag(nx, ny, nz, fg, lab))
+    g.close()
