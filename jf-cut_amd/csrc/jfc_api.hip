@@ -582,6 +582,11 @@ int graph_work_plane(jfc_graph *g, int inst, int **plane, long long *n) {
   *n = g->inst_stored(inst);
   return JFC_OK;
 }
+// The instance's slice of the height plane, free between solves as well.
+int graph_work_plane2(jfc_graph *g, int inst, int **plane) {
+  *plane = g->h + g->inst[inst].node_off;
+  return JFC_OK;
+}
 }  // namespace jfc
 
 // ---- lifetime -------------------------------------------------------------------

@@ -5,8 +5,10 @@
 // Gaussian pairwise).
 //
 // Reference counterparts (src/QVisualizer/cl/GraphCut/):
-//   k_wm_seed_list   graphcut_count_cut / graphcut_scatter_cut   graphcut_count_block.cl:67-104
-//   k_wm_levels      graphcut_cut_histogram, _distribution       graphcut_histogram.cl:19-60
+//   k_wm_scan        graphcut_count_cut / graphcut_scatter_cut   graphcut_count_block.cl:67-104
+//                    + graphcut_cut_histogram, _distribution     graphcut_histogram.cl:19-60
+//   k_wm_lloyd       the whole k-means                           graphcut_kmeans.cl:21-159,
+//                                                                QGCWidget.cpp:2011-2102
 //   k_wm_assign      graphcut_kmeans                             graphcut_kmeans.cl:21-159
 //   k_wm_unary<lazy> graphcut_compute_excessflow_lazy / _bk      graphcut_compute_excessflow.cl:19-139
 //   k_wm_pairwise    graphcut_compute_capacity_lazy / _bk        graphcut_compute_capacity.cl:21-254
@@ -33,6 +35,7 @@
 #include "jfcut.h"
 #include "jfc_device.h"
 
+#include <algorithm>
 #include <climits>
 #include <cmath>
 #include <cstring>
@@ -49,6 +52,7 @@ hipStream_t graph_stream(jfc_graph *g);
 int graph_stage(jfc_graph *g, size_t bytes, void **p);
 int graph_scratch(jfc_graph *g, size_t bytes, void **p);
 int graph_work_plane(jfc_graph *g, int inst, int **plane, long long *n);
+int graph_work_plane2(jfc_graph *g, int inst, int **plane);
 }  // namespace jfc
 
 using namespace jfc;
@@ -80,10 +84,29 @@ __device__ __forceinline__ float dot4(const float a[4], const W4 &w) {
   return ((a[0] * w.v[0] + a[1] * w.v[1]) + a[2] * w.v[2]) + a[3] * w.v[3];
 }
 
-// OpenCL distance(c, p) = length(c - p)
-__device__ __forceinline__ float dist4(const float *c, const float p[4]) {
+// The square under OpenCL distance(c, p) = length(c - p).  Rounded square
+// roots keep the order of their arguments, so the nearest distance is the
+// root of the least square, and only near ties need the roots themselves.
+__device__ __forceinline__ float dist4_sq(const float *c, const float p[4]) {
   const float d0 = c[0] - p[0], d1 = c[1] - p[1], d2 = c[2] - p[2], d3 = c[3] - p[3];
-  return sqrtf(((d0 * d0 + d1 * d1) + d2 * d2) + d3 * d3);
+  return ((d0 * d0 + d1 * d1) + d2 * d2) + d3 * d3;
+}
+
+// The nearest of k centroids, first on ties of the rounded distances
+// (graphcut_kmeans.cl:37-47).  s < best (1 - 2^-20) makes the roots differ by
+// more than their rounding; s >= best makes them equal or larger.
+__device__ __forceinline__ int nearest4(const float *c, int k, const float p[4]) {
+  float best = dist4_sq(c, p);
+  int idx = 0;
+  for (int j = 1; j < k; ++j) {
+    const float s = dist4_sq(c + 4 * j, p);
+    if (s >= best) continue;
+    if (s < best * (1.0f - 0x1p-20f) || sqrtf(s) < sqrtf(best)) {
+      best = s;
+      idx = j;
+    }
+  }
+  return idx;
 }
 
 // histogram level of a seeded pixel: clamp(dot, 0, 1) * (size - 1) + 0.5,
@@ -102,55 +125,193 @@ __device__ __forceinline__ int unary_int(float v) {
   return (int)r;
 }
 
-__global__ void k_wm_seed_list(const unsigned char *seeds, long long n, int *list, int *count) {
-  for (long long base = (long long)blockIdx.x * blockDim.x; base < n;
-       base += (long long)gridDim.x * blockDim.x) {
-    const long long i = base + threadIdx.x;
-    wave_append(i < n && seeds[i] != 0, (int)i, list, count, nullptr, nullptr);
+// Scratch of one call.  Everything up to rep is copied back at the end.
+struct WmScratch {
+  int *ctl;          // [0,1] seeded pixels per side, [2] a side has more than kLloydSeeds,
+                     // [3,4] k-means iterations
+  unsigned *hist;    // [2][kLevels] seeded pixels per level
+  float *cent;       // [2][kMaxK * 4] the centroids of the unary, side 1 from k * 4 on
+  unsigned *rep;     // [2][kLevels] highest node index + 1 per seeded level
+  unsigned *acc;     // [kMaxK * 4][kLevels] byte counts of an assignment (k_wm_assign)
+  uchar4 *list[2];   // the seeded pixels
+};
+constexpr size_t kCtlBytes = 64, kHistBytes = 2 * kLevels * 4, kCentBytes = 2 * kMaxK * 4 * 4,
+                 kRepBytes = kHistBytes, kAccBytes = (size_t)kMaxK * 4 * kLevels * 4;
+constexpr size_t kBackBytes = kCtlBytes + kHistBytes + kCentBytes;
+
+// One pass over the seed bytes: per side the seeded pixels in a list, their
+// level histogram (graphcut_cut_histogram) and the highest node index + 1 per
+// level (graphcut_cut_distribution).  Four pixels per lane; a workgroup's
+// histograms meet in LDS.
+__global__ __launch_bounds__(256) void k_wm_scan(const uchar4 *img, const unsigned char *fg,
+                                                 const unsigned char *bg, long long n, W4 w,
+                                                 WmScratch S) {
+  __shared__ unsigned s_h[2][kLevels], s_r[2][kLevels];
+  __shared__ int s_any;
+  for (int i = threadIdx.x; i < 2 * kLevels; i += 256) (&s_h[0][0])[i] = (&s_r[0][0])[i] = 0;
+  if (threadIdx.x == 0) s_any = 0;
+  __syncthreads();
+  const bool al = (((size_t)fg | (size_t)bg) & 3) == 0;
+  const long long groups = (n + 3) / 4;
+  for (long long base = (long long)blockIdx.x * 256; base < groups;
+       base += (long long)gridDim.x * 256) {
+    const long long g = base + threadIdx.x, v0 = 4 * g;
+    unsigned m[2] = {0u, 0u};
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+      const unsigned char *p = side ? bg : fg;
+      if (g < groups) {
+        if (al && v0 + 4 <= n) {
+          m[side] = *(const unsigned *)(p + v0);
+        } else {
+          for (int j = 0; j < 4; ++j)
+            if (v0 + j < n) m[side] |= (unsigned)p[v0 + j] << (8 * j);
+        }
+      }
+    }
+    if (!__ballot((m[0] | m[1]) != 0)) continue;
+    s_any = 1;
+#pragma unroll
+    for (int side = 0; side < 2; ++side)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const bool on = ((m[side] >> (8 * j)) & 255u) != 0;
+        const unsigned long long b = __ballot(on);
+        if (!b) continue;
+        int at = 0;
+        if (lane_id() == 0) at = atomicAdd(&S.ctl[side], __popcll(b));
+        at = __builtin_amdgcn_readfirstlane(at);
+        if (!on) continue;
+        const uchar4 t = img[v0 + j];
+        S.list[side][at + __popcll(b & ((1ull << lane_id()) - 1ull))] = t;
+        const float f[4] = {unorm8(t.x), unorm8(t.y), unorm8(t.z), unorm8(t.w)};
+        const int lv = level_clamped(dot4(f, w));
+        atomicAdd(&s_h[side][lv], 1u);
+        atomicMax(&s_r[side][lv], (unsigned)(v0 + j) + 1u);
+      }
+  }
+  __syncthreads();
+  if (!s_any) return;
+  for (int i = threadIdx.x; i < 2 * kLevels; i += 256) {
+    const unsigned h = (&s_h[0][0])[i];
+    if (!h) continue;
+    atomicAdd(&S.hist[i], h);
+    atomicMax(&S.rep[i], (&s_r[0][0])[i]);
   }
 }
 
-// Per seeded pixel of one side: the level histogram (graphcut_cut_histogram)
-// and the highest node index + 1 per level (graphcut_cut_distribution).
-__global__ void k_wm_levels(const uchar4 *img, const int *list, const int *count, W4 w,
-                            unsigned *hist, unsigned *rep) {
-  const int n = *count;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const int v = list[i];
-    unsigned t[4];
-    texel(img, v, t);
-    float f[4];
-    for (int c = 0; c < 4; ++c) f[c] = unorm8(t[c]);
-    const int lv = level_clamped(dot4(f, w));
-    atomicAdd(&hist[lv], 1u);
-    atomicMax(&rep[lv], (unsigned)v + 1u);
+// The k-means of a side (blockIdx.x) with up to kLloydSeeds seeded pixels, one
+// workgroup of 1024 lanes: initial centroids from the seeded levels'
+// representatives, picked at (count - 1) * i / (k - 1) and scaled by weight /
+// 255 (QGCW:2011-2039), then Lloyd iterations (QGCW:2073-2102) until the
+// centroids move by less than 1 / 1024.  The centroids of the last assignment
+// are the ones the unary uses.  An assignment counts bytes per cluster and
+// channel; a mean is the exact sum of count * value, which float64 holds in
+// any order (a term is a multiple of the smallest value's last bit, and
+// 2^16 of them span under 53 bits), divided and rounded once.
+// A launch, two copies and a host wait per iteration took 60-65 us; here one
+// takes ~10 us at 5,000 seeds, which are 6 rounds of the workgroup.
+constexpr int kLloydSeeds = 65536;
+
+template <int KB>
+__global__ __launch_bounds__(1024) void k_wm_lloyd(const uchar4 *img, W4 w, W4 scale, int k,
+                                                   int iterations, WmScratch S) {
+  __shared__ unsigned s_acc[KB * 4][kLevels];
+  __shared__ float s_val[4][kLevels];  // weighted feature of a byte per channel
+  __shared__ float s_c[KB * 4], s_n[KB * 4];
+  __shared__ int s_lv[kLevels];        // seeded levels in order
+  __shared__ int s_levels, s_err;
+  const int side = blockIdx.x, tid = threadIdx.x;
+  const int n = S.ctl[side];
+  if (n == 0) return;
+  if (n > kLloydSeeds) {
+    if (tid == 0) S.ctl[2] = 1;
+    return;
   }
+  (&s_val[0][0])[tid] = unorm8(tid & 255) * w.v[tid >> 8];
+  if (tid < 64) {
+    int c = 0;
+#pragma unroll
+    for (int q = 0; q < kLevels / 64; ++q) {
+      const unsigned rp = S.rep[side * kLevels + 64 * q + tid];
+      const unsigned long long b = __ballot(rp != 0);
+      if (rp) s_lv[c + __popcll(b & ((1ull << tid) - 1ull))] = (int)(rp - 1u);
+      c += __popcll(b);
+    }
+    if (tid == 0) s_levels = c;
+  }
+  __syncthreads();
+  if (tid < k * 4) {
+    const unsigned dsize = (unsigned)s_levels - 1u;
+    const uchar4 t = img[s_lv[dsize * (unsigned)(tid >> 2) / (unsigned)(k - 1)]];
+    const int c = tid & 3;
+    s_n[tid] = (float)(c == 0 ? t.x : c == 1 ? t.y : c == 2 ? t.z : t.w) * scale.v[c];
+  }
+  int it = 0;
+  for (;;) {
+    for (int i = tid; i < k * 4 * kLevels; i += 1024) (&s_acc[0][0])[i] = 0;
+    __syncthreads();
+    if (tid < k * 4) s_c[tid] = s_n[tid];
+    if (tid == 0) s_err = 0;
+    __syncthreads();
+    const uchar4 *list = S.list[side];
+    for (int i = tid; i < n; i += 1024) {
+      const uchar4 t = list[i];
+      const float p[4] = {s_val[0][t.x], s_val[1][t.y], s_val[2][t.z], s_val[3][t.w]};
+      const int j = nearest4(s_c, k, p);
+      atomicAdd(&s_acc[j * 4][t.x], 1u);
+      atomicAdd(&s_acc[j * 4 + 1][t.y], 1u);
+      atomicAdd(&s_acc[j * 4 + 2][t.z], 1u);
+      atomicAdd(&s_acc[j * 4 + 3][t.w], 1u);
+    }
+    __syncthreads();
+    // one wave per cluster and channel, four byte values per lane
+    for (int r = tid >> 6; r < k * 4; r += 16) {
+      double sum = 0.0;
+      unsigned members = 0;
+#pragma unroll
+      for (int q = 0; q < kLevels / 64; ++q) {
+        const int b = 64 * q + (tid & 63);
+        const unsigned m = s_acc[r][b];
+        sum += (double)m * (double)s_val[r & 3][b];
+        members += m;
+      }
+      for (int o = 32; o > 0; o >>= 1) {
+        sum += __shfl_xor(sum, o);
+        members += __shfl_xor(members, o);
+      }
+      if ((tid & 63) == 0) s_n[r] = members ? (float)(sum / (double)members) : 0.0f;
+    }
+    __syncthreads();
+    ++it;
+    if (tid < k) {
+      // glm::length(centroid - previous)
+      float d[4];
+      for (int c = 0; c < 4; ++c) d[c] = s_n[tid * 4 + c] - s_c[tid * 4 + c];
+      const float len = sqrtf((d[0] * d[0] + d[1] * d[1]) + (d[2] * d[2] + d[3] * d[3]));
+      if (!(len < 1.0f / 1024)) s_err = 1;
+    }
+    __syncthreads();
+    if (!s_err || it >= iterations) break;
+  }
+  if (tid < k * 4) S.cent[side * k * 4 + tid] = s_c[tid];
+  if (tid == 0) S.ctl[3 + side] = it;
 }
 
-// One Lloyd assignment over the seeded pixels of a side: the nearest
-// centroid (first on ties, graphcut_kmeans.cl:37-47) and, per cluster and
-// channel, a count per byte value, from which the host forms exact sums.
-__global__ void k_wm_assign(const uchar4 *img, const int *list, const int *count, W4 w,
-                            const float *cent, int k, unsigned *acc) {
+// One Lloyd assignment over more seeded pixels of a side than k_wm_lloyd
+// takes: per cluster and channel, a count per byte value, from which the
+// host forms exact sums.
+__global__ void k_wm_assign(const uchar4 *list, int n, W4 w, const float *cent, int k,
+                            unsigned *acc) {
   __shared__ float s_c[kMaxK * 4];
   for (int i = threadIdx.x; i < k * 4; i += blockDim.x) s_c[i] = cent[i];
   __syncthreads();
-  const int n = *count;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const int v = list[i];
-    unsigned t[4];
-    texel(img, v, t);
+    const uchar4 u = list[i];
+    const unsigned t[4] = {u.x, u.y, u.z, u.w};
     float p[4];
     for (int c = 0; c < 4; ++c) p[c] = unorm8(t[c]) * w.v[c];
-    float best = 3.402823466e38f;
-    int idx = 0;
-    for (int j = 0; j < k; ++j) {
-      const float d = dist4(s_c + 4 * j, p);
-      if (d < best) {
-        best = d;
-        idx = j;
-      }
-    }
+    const int idx = nearest4(s_c, k, p);
     for (int c = 0; c < 4; ++c) atomicAdd(&acc[(idx * 4 + c) * kLevels + t[c]], 1u);
   }
 }
@@ -159,22 +320,32 @@ __global__ void k_wm_assign(const uchar4 *img, const int *list, const int *count
 // nearest centroid of each side (graphcut_compute_excessflow.cl:47-77,
 // 109-139); BK: negative log-likelihood from the seeded level histograms
 // (graphcut_compute_excessflow.cl:19-45, 79-107).  Seeds: +-cl_max_flow,
-// foreground first.
+// foreground first.  Nothing is written when a side has no seeds, or too many
+// for k_wm_lloyd (the host then runs the k-means and launches again).
 template <bool LAZY>
 __global__ __launch_bounds__(256) void k_wm_unary(
-    const uchar4 *img, const unsigned char *fg, const unsigned char *bg, long long n, W4 w,
-    const float *cent, int k, const unsigned *hist, unsigned sum_f, unsigned sum_b, int shift,
-    float lambda, int nx, int px, int *cs, int *ct) {
+    const uchar4 *img, const unsigned char *fg, const unsigned char *bg, int n, W4 w,
+    WmScratch S, int k, int shift, float lambda, int nx, int px, int *cs, int *ct) {
   __shared__ float s_c[2 * kMaxK * 4];
-  __shared__ unsigned s_h[2 * kLevels];
-  if (LAZY)
-    for (int i = threadIdx.x; i < 2 * k * 4; i += blockDim.x) s_c[i] = cent[i];
-  else
-    for (int i = threadIdx.x; i < 2 * kLevels; i += blockDim.x) s_h[i] = hist[i];
+  __shared__ float s_val[4][kLevels];
+  __shared__ unsigned s_h[2 * kLevels], s_sum[2];
+  if (S.ctl[0] == 0 || S.ctl[1] == 0 || S.ctl[2]) return;
+  if (threadIdx.x < 2) s_sum[threadIdx.x] = 0;
   __syncthreads();
+  if (LAZY) {
+    for (int i = threadIdx.x; i < 2 * k * 4; i += blockDim.x) s_c[i] = S.cent[i];
+    for (int c = 0; c < 4; ++c) s_val[c][threadIdx.x] = unorm8(threadIdx.x) * w.v[c];
+  } else {
+    for (int i = threadIdx.x; i < 2 * kLevels; i += blockDim.x) {
+      s_h[i] = S.hist[i];
+      if (s_h[i]) atomicAdd(&s_sum[i / kLevels], s_h[i]);
+    }
+  }
+  __syncthreads();
+  const unsigned sum_f = s_sum[0], sum_b = s_sum[1];
   const float gain = (float)(kMaxFlow >> shift) * lambda;
-  for (long long v = blockIdx.x * (long long)blockDim.x + threadIdx.x; v < n;
-       v += (long long)gridDim.x * blockDim.x) {
+  for (unsigned v = blockIdx.x * blockDim.x + threadIdx.x; v < (unsigned)n;
+       v += gridDim.x * blockDim.x) {
     int ef;
     if (fg[v]) {
       ef = kMaxFlow;
@@ -183,20 +354,22 @@ __global__ __launch_bounds__(256) void k_wm_unary(
     } else {
       unsigned t[4];
       texel(img, v, t);
-      float f[4];
-      for (int c = 0; c < 4; ++c) f[c] = unorm8(t[c]);
       float val;
       if (LAZY) {
         float p[4];
-        for (int c = 0; c < 4; ++c) p[c] = f[c] * w.v[c];
+        for (int c = 0; c < 4; ++c) p[c] = s_val[c][t[c]];
         float dx = 3.402823466e38f, dy = 3.402823466e38f;
         for (int j = 0; j < k; ++j) {
-          dx = fminf(dx, dist4(s_c + 4 * j, p));
-          dy = fminf(dy, dist4(s_c + 4 * (k + j), p));
+          dx = fminf(dx, dist4_sq(s_c + 4 * j, p));
+          dy = fminf(dy, dist4_sq(s_c + 4 * (k + j), p));
         }
+        dx = sqrtf(dx);
+        dy = sqrtf(dy);
         const float r = (dx + dy == 0.0f) ? 0.0f : (dy - dx) / (dx + dy);
         val = gain * r;
       } else {
+        float f[4];
+        for (int c = 0; c < 4; ++c) f[c] = unorm8(t[c]);
         int lv = (int)(dot4(f, w) * (float)(kLevels - 1) + 0.5f);
         lv = lv < 0 ? 0 : (lv > kLevels - 1 ? kLevels - 1 : lv);
         const float qf = (float)s_h[lv] / (float)sum_f;
@@ -207,7 +380,8 @@ __global__ __launch_bounds__(256) void k_wm_unary(
       ef = unary_int(val);
     }
     // the planes store row r at r * px
-    const long long sv = (v / nx) * px + v % nx;
+    const unsigned row = v / (unsigned)nx;
+    const long long sv = (long long)row * px + (v - row * (unsigned)nx);
     cs[sv] = ef > 0 ? ef : 0;
     ct[sv] = ef < 0 ? -ef : 0;
   }
@@ -244,7 +418,9 @@ __device__ __forceinline__ int wm_arc(const int a[4], const int b[4], float scal
 // and (-z, -y, -x) in 3D).
 template <bool LAZY, bool D3>
 __global__ __launch_bounds__(256) void k_wm_pairwise(InstDesc I, const uchar4 *img, W4 w,
-                                                     float scale, int *c0, long long stride) {
+                                                     float scale, const int *ctl, int *c0,
+                                                     long long stride) {
+  if (ctl[0] == 0 || ctl[1] == 0) return;
   const long long rows = (long long)I.ny * I.nz;
   for (long long row = blockIdx.x; row < rows; row += gridDim.x) {
     const int y = (int)(row % I.ny), z = (int)(row / I.ny);
@@ -283,6 +459,98 @@ W4 normalize_weight(const float in[4]) {
 }
 
 }  // namespace
+
+#define WM_RET(call)                                                                    \
+  do {                                                                                  \
+    hipError_t e_ = (call);                                                             \
+    if (e_ != hipSuccess)                                                               \
+      return model_fail(JFC_ERR_DEVICE, std::string(#call) + ": " + hipGetErrorString(e_)); \
+  } while (0)
+
+// The k-means of the sides with more seeds than k_wm_lloyd takes, an
+// assignment per launch and the update here; ctl and cent of `back` (the host
+// copy of the scratch) and of the scratch are completed, the unary's guard
+// lifted.
+static int lloyd_on_host(const uchar4 *img, const W4 &w, int k, int iterations,
+                         const WmScratch &S, unsigned char *back, hipStream_t st) {
+  int *ctl = (int *)back;
+  float *cent_used = (float *)(back + kCtlBytes + kHistBytes);
+  // weighted feature value of each byte per channel: unorm8(b) * w
+  float val[4][kLevels];
+  for (int c = 0; c < 4; ++c)
+    for (int b = 0; b < kLevels; ++b) val[c][b] = unorm8(b) * w.v[c];
+  for (int side = 0; side < 2; ++side) {
+    const int cnt = ctl[side];
+    if (cnt <= kLloydSeeds) continue;
+    // initial centroids: the representatives of the seeded levels, picked at
+    // (count - 1) * i / (k - 1) (QGCW:2011-2039), scaled by weight / 255
+    std::vector<unsigned> rep(kLevels);
+    WM_RET(hipMemcpyAsync(rep.data(), S.rep + side * kLevels, kLevels * sizeof(unsigned),
+                          hipMemcpyDeviceToHost, st));
+    WM_RET(hipStreamSynchronize(st));
+    std::vector<unsigned> dist;
+    for (int l = 0; l < kLevels; ++l)
+      if (rep[l]) dist.push_back(rep[l]);
+    const unsigned dsize = (unsigned)dist.size() - 1u;
+    float scale[4];
+    for (int c = 0; c < 4; ++c) scale[c] = w.v[c] / 255.0f;
+    std::vector<float> cent(k * 4), prev(k * 4);
+    std::vector<uchar4> picked(k);
+    for (int i = 0; i < k; ++i) {
+      const long long idx = (long long)dist[dsize * (unsigned)i / (unsigned)(k - 1)] - 1;
+      WM_RET(hipMemcpyAsync(&picked[i], img + idx, sizeof(uchar4), hipMemcpyDeviceToHost, st));
+    }
+    WM_RET(hipStreamSynchronize(st));
+    for (int i = 0; i < k; ++i) {
+      const uchar4 t = picked[i];
+      const unsigned tb[4] = {t.x, t.y, t.z, t.w};
+      for (int c = 0; c < 4; ++c) cent[i * 4 + c] = (float)tb[c] * scale[c];
+    }
+    // Lloyd iterations (QGCW:2073-2102): the centroids of the last
+    // assignment are the ones the unary uses
+    std::vector<unsigned> acc((size_t)k * 4 * kLevels);
+    float *d_cent = S.cent + side * k * 4;
+    int it = 0;
+    while (it < iterations) {
+      prev = cent;
+      WM_RET(hipMemcpyAsync(d_cent, prev.data(), k * 4 * sizeof(float), hipMemcpyHostToDevice, st));
+      launch_fill_i32((int *)S.acc, (long long)acc.size(), 0, st);
+      k_wm_assign<<<std::min(grid1(cnt), 1024), 256, 0, st>>>(S.list[side], cnt, w, d_cent, k, S.acc);
+      WM_RET(hipGetLastError());
+      WM_RET(hipMemcpyAsync(acc.data(), S.acc, acc.size() * sizeof(unsigned), hipMemcpyDeviceToHost, st));
+      WM_RET(hipStreamSynchronize(st));
+      ++it;
+      float err = 0.0f;
+      for (int i = 0; i < k; ++i) {
+        long long members = 0;
+        for (int b = 0; b < kLevels; ++b) members += acc[(i * 4) * kLevels + b];
+        for (int c = 0; c < 4; ++c) {
+          if (!members) {
+            cent[i * 4 + c] = 0.0f;
+            continue;
+          }
+          double sum = 0.0;
+          for (int b = 0; b < kLevels; ++b) {
+            const unsigned m = acc[(i * 4 + c) * kLevels + b];
+            if (m) sum += (double)m * (double)val[c][b];
+          }
+          cent[i * 4 + c] = (float)(sum / (double)members);
+        }
+        // glm::length(centroid - previous)
+        float d[4];
+        for (int c = 0; c < 4; ++c) d[c] = cent[i * 4 + c] - prev[i * 4 + c];
+        const float len = std::sqrt((d[0] * d[0] + d[1] * d[1]) + (d[2] * d[2] + d[3] * d[3]));
+        err = std::max(err, len);
+      }
+      if (err < 1.0f / 1024) break;
+    }
+    ctl[3 + side] = it;
+    for (int i = 0; i < k * 4; ++i) cent_used[side * k * 4 + i] = prev[i];
+  }
+  ctl[2] = 0;
+  WM_RET(hipMemcpyAsync(S.ctl, back, kBackBytes, hipMemcpyHostToDevice, st));
+  return JFC_OK;
+}
 
 extern "C" void jfc_default_widget_model_params(jfc_widget_model_params *p) {
   if (!p) return;
@@ -338,24 +606,19 @@ extern "C" int jfc_model_widget(jfc_graph *g, int inst, const uint8_t *rgba, con
   if (n >= (1LL << 31) - 1) return model_fail(JFC_ERR_INVALID, "instance too large for the model path");
 
   // Everything runs on the graph's stream.  Host inputs cross in one copy
-  // each through the graph's staging buffer; the small scratch (seed count,
-  // histograms, level representatives, k-means sums, centroids) is the
-  // graph's data-term block; the seed list borrows the instance's slice of
-  // the excess plane, which every solve rewrites from the inputs.
+  // each through the graph's staging buffer; the small scratch (WmScratch) is the
+  // graph's data-term block.
   const hipStream_t st = graph_stream(g);
   const W4 w = normalize_weight(prm->weight);
   const int k = prm->k;
   const uchar4 *img = reinterpret_cast<const uchar4 *>(rgba);
   const unsigned char *dfg = fg, *dbg = bg;
-  int *d_list = nullptr, *d_cnt = nullptr;
-  unsigned *d_hist = nullptr, *d_rep = nullptr, *d_acc = nullptr;
-  float *d_cent = nullptr;
-  long long list_cap = 0;
+  WmScratch S{};
   bool written = false;
   jfc_widget_model_stats st_local;
   jfc_widget_model_stats &ST = stats ? *stats : st_local;
-  std::vector<float> cent_used(2 * k * 4, 0.0f);
-  std::vector<unsigned> hist(2 * kLevels, 0);
+  unsigned char back[kBackBytes];
+  const int *ctl = (const int *)back;
   memset(&ST, 0, sizeof(ST));
 
   if (!on_device) {
@@ -370,147 +633,92 @@ extern "C" int jfc_model_widget(jfc_graph *g, int inst, const uint8_t *rgba, con
     dbg = sp + n * 5;
   }
   {
-    const size_t o_cnt = 0, o_hist = 256, o_rep = o_hist + 2 * kLevels * 4,
-                 o_acc = o_rep + kLevels * 4, o_cent = o_acc + (size_t)kMaxK * 4 * kLevels * 4,
-                 total = o_cent + 2 * kMaxK * 4 * 4;
     void *sc = nullptr;
-    if ((rc = graph_scratch(g, total, &sc))) return rc;
+    if ((rc = graph_scratch(g, kBackBytes + kRepBytes + kAccBytes, &sc))) return rc;
     unsigned char *b = (unsigned char *)sc;
-    d_cnt = (int *)(b + o_cnt);
-    d_hist = (unsigned *)(b + o_hist);
-    d_rep = (unsigned *)(b + o_rep);
-    d_acc = (unsigned *)(b + o_acc);
-    d_cent = (float *)(b + o_cent);
-    if ((rc = graph_work_plane(g, inst, &d_list, &list_cap))) return rc;
-  }
-  WM_HIP(hipMemsetAsync(d_hist, 0, 2 * kLevels * sizeof(unsigned), st));
-
-  for (int side = 0; side < 2; ++side) {
-    int cnt = 0;
-    WM_HIP(hipMemsetAsync(d_cnt, 0, sizeof(int), st));
-    k_wm_seed_list<<<grid1(n), 256, 0, st>>>(side ? dbg : dfg, n, d_list, d_cnt);
-    WM_HIP(hipGetLastError());
-    WM_HIP(hipMemcpyAsync(&cnt, d_cnt, sizeof(int), hipMemcpyDeviceToHost, st));
-    WM_HIP(hipStreamSynchronize(st));
-    ST.seeds[side] = cnt;
-    if (cnt == 0) {
-      // computeBFS / kmeans "no labels." (QGCW:2015-2016)
-      rc = model_fail(JFC_ERR_NO_SEEDS, side ? "no background seeds" : "no foreground seeds");
-      goto done;
-    }
-    WM_HIP(hipMemsetAsync(d_rep, 0, kLevels * sizeof(unsigned), st));
-    k_wm_levels<<<grid1(cnt), 256, 0, st>>>(img, d_list, d_cnt, w, d_hist + side * kLevels, d_rep);
-    WM_HIP(hipGetLastError());
-    if (!prm->lazy) continue;
-
-    // initial centroids: the representatives of the seeded levels, picked at
-    // (count - 1) * i / (k - 1) (QGCW:2011-2039), scaled by weight / 255
-    std::vector<unsigned> rep(kLevels);
-    WM_HIP(hipMemcpyAsync(rep.data(), d_rep, kLevels * sizeof(unsigned), hipMemcpyDeviceToHost, st));
-    WM_HIP(hipStreamSynchronize(st));
-    std::vector<unsigned> dist;
-    for (int l = 0; l < kLevels; ++l)
-      if (rep[l]) dist.push_back(rep[l]);
-    const unsigned dsize = (unsigned)dist.size() - 1u;
-    float scale[4];
-    for (int c = 0; c < 4; ++c) scale[c] = w.v[c] / 255.0f;
-    std::vector<float> cent(k * 4), prev(k * 4);
-    std::vector<uchar4> picked(k);
-    for (int i = 0; i < k; ++i) {
-      const long long idx = (long long)dist[dsize * (unsigned)i / (unsigned)(k - 1)] - 1;
-      WM_HIP(hipMemcpyAsync(&picked[i], img + idx, sizeof(uchar4), hipMemcpyDeviceToHost, st));
-    }
-    WM_HIP(hipStreamSynchronize(st));
-    for (int i = 0; i < k; ++i) {
-      const uchar4 t = picked[i];
-      const unsigned tb[4] = {t.x, t.y, t.z, t.w};
-      for (int c = 0; c < 4; ++c) cent[i * 4 + c] = (float)tb[c] * scale[c];
-    }
-    // weighted feature value of each byte per channel: unorm8(b) * w
-    float val[4][kLevels];
-    for (int c = 0; c < 4; ++c)
-      for (int b = 0; b < kLevels; ++b) val[c][b] = unorm8(b) * w.v[c];
-    // Lloyd iterations (QGCW:2073-2102): the centroids of the last
-    // assignment are the ones the unary uses
-    std::vector<unsigned> acc((size_t)k * 4 * kLevels);
-    int it = 0;
-    for (; it < prm->kmeans_iterations;) {
-      prev = cent;
-      WM_HIP(hipMemcpyAsync(d_cent, prev.data(), k * 4 * sizeof(float), hipMemcpyHostToDevice, st));
-      WM_HIP(hipMemsetAsync(d_acc, 0, acc.size() * sizeof(unsigned), st));
-      k_wm_assign<<<std::min(grid1(cnt), 1024), 256, 0, st>>>(img, d_list, d_cnt, w, d_cent, k, d_acc);
-      WM_HIP(hipGetLastError());
-      WM_HIP(hipMemcpyAsync(acc.data(), d_acc, acc.size() * sizeof(unsigned), hipMemcpyDeviceToHost, st));
-      WM_HIP(hipStreamSynchronize(st));
-      ++it;
-      float err = 0.0f;
-      for (int i = 0; i < k; ++i) {
-        long long members = 0;
-        for (int b = 0; b < kLevels; ++b) members += acc[(i * 4) * kLevels + b];
-        for (int c = 0; c < 4; ++c) {
-          if (!members) {
-            cent[i * 4 + c] = 0.0f;
-            continue;
-          }
-          double sum = 0.0;
-          for (int b = 0; b < kLevels; ++b) {
-            const unsigned m = acc[(i * 4 + c) * kLevels + b];
-            if (m) sum += (double)m * (double)val[c][b];
-          }
-          cent[i * 4 + c] = (float)(sum / (double)members);
-        }
-        // glm::length(centroid - previous)
-        float d[4];
-        for (int c = 0; c < 4; ++c) d[c] = cent[i * 4 + c] - prev[i * 4 + c];
-        const float len = std::sqrt((d[0] * d[0] + d[1] * d[1]) + (d[2] * d[2] + d[3] * d[3]));
-        err = std::max(err, len);
-      }
-      if (err < 1.0f / 1024) break;
-    }
-    ST.iterations[side] = it;
-    for (int i = 0; i < k * 4; ++i) {
-      cent_used[side * k * 4 + i] = prev[i];
-      ST.centroids[side][i / 4][i % 4] = prev[i];
-    }
+    S.ctl = (int *)b;
+    S.hist = (unsigned *)(b + kCtlBytes);
+    S.cent = (float *)(b + kCtlBytes + kHistBytes);
+    S.rep = (unsigned *)(b + kBackBytes);
+    S.acc = (unsigned *)(b + kBackBytes + kRepBytes);
+    // the seed lists borrow the instance's slices of the excess and height
+    // planes, which every solve rewrites before reading them
+    int *l0 = nullptr, *l1 = nullptr;
+    long long cap = 0;
+    if ((rc = graph_work_plane(g, inst, &l0, &cap)) || (rc = graph_work_plane2(g, inst, &l1)))
+      return rc;
+    S.list[0] = (uchar4 *)l0;
+    S.list[1] = (uchar4 *)l1;
   }
   {
-    WM_HIP(hipMemcpyAsync(hist.data(), d_hist, hist.size() * sizeof(unsigned), hipMemcpyDeviceToHost, st));
-    WM_HIP(hipStreamSynchronize(st));
-    for (int side = 0; side < 2; ++side)
-      for (int l = 0; l < kLevels; ++l) ST.hist_sum[side] += hist[side * kLevels + l];
-    const int shift = d3 ? 3 : 2;
-    written = true;
+    // everything is queued without a look at the counts: with a side without
+    // seeds the kernels write no plane
+    launch_fill_i32(S.ctl, (kBackBytes + kRepBytes) / 4, 0, st);
+    k_wm_scan<<<std::min(grid1((n + 3) / 4), 1024), 256, 0, st>>>(img, dfg, dbg, n, w, S);
     if (prm->lazy) {
-      WM_HIP(hipMemcpyAsync(d_cent, cent_used.data(), cent_used.size() * sizeof(float),
-                            hipMemcpyHostToDevice, st));
-      k_wm_unary<true><<<grid1(n), 256, 0, st>>>(img, dfg, dbg, n, w, d_cent, k, nullptr, 0, 0,
-                                                 shift, prm->lazy_terminal, I.nx, I.px,
-                                                 cs + I.node_off, ct + I.node_off);
-    } else {
-      k_wm_unary<false><<<grid1(n), 256, 0, st>>>(img, dfg, dbg, n, w, nullptr, 0, d_hist,
-                                                  ST.hist_sum[0], ST.hist_sum[1], shift,
-                                                  prm->bk_terminal, I.nx, I.px, cs + I.node_off,
-                                                  ct + I.node_off);
+      W4 scale;
+      for (int c = 0; c < 4; ++c) scale.v[c] = w.v[c] / 255.0f;
+      const int iters = prm->kmeans_iterations;
+      if (k <= 8) k_wm_lloyd<8><<<2, 1024, 0, st>>>(img, w, scale, k, iters, S);
+      else if (k <= 16) k_wm_lloyd<16><<<2, 1024, 0, st>>>(img, w, scale, k, iters, S);
+      else k_wm_lloyd<32><<<2, 1024, 0, st>>>(img, w, scale, k, iters, S);
     }
+    WM_HIP(hipGetLastError());
+    const int shift = d3 ? 3 : 2;
+    auto unary = [&]() {
+      if (prm->lazy)
+        k_wm_unary<true><<<grid1(n), 256, 0, st>>>(img, dfg, dbg, (int)n, w, S, k, shift,
+                                                   prm->lazy_terminal, I.nx, I.px,
+                                                   cs + I.node_off, ct + I.node_off);
+      else
+        k_wm_unary<false><<<grid1(n), 256, 0, st>>>(img, dfg, dbg, (int)n, w, S, 0, shift,
+                                                    prm->bk_terminal, I.nx, I.px,
+                                                    cs + I.node_off, ct + I.node_off);
+    };
+    unary();
     WM_HIP(hipGetLastError());
     const int grid = (int)std::min<long long>((long long)I.ny * I.nz, 65536);
     if (prm->lazy) {
       // lambda / SHRT_MAX (graphcut_compute_capacity.cl:82)
       const float scale = prm->lazy_neighbor / (float)SHRT_MAX;
-      if (d3) k_wm_pairwise<true, true><<<grid, 256, 0, st>>>(I, img, w, scale, c0, stride);
-      else k_wm_pairwise<true, false><<<grid, 256, 0, st>>>(I, img, w, scale, c0, stride);
+      if (d3) k_wm_pairwise<true, true><<<grid, 256, 0, st>>>(I, img, w, scale, S.ctl, c0, stride);
+      else k_wm_pairwise<true, false><<<grid, 256, 0, st>>>(I, img, w, scale, S.ctl, c0, stride);
     } else {
       // 1 / (SHRT_MAX * sigma) (graphcut_compute_capacity.cl:29)
       const float scale = 1.0f / ((float)SHRT_MAX * prm->bk_neighbor);
-      if (d3) k_wm_pairwise<false, true><<<grid, 256, 0, st>>>(I, img, w, scale, c0, stride);
-      else k_wm_pairwise<false, false><<<grid, 256, 0, st>>>(I, img, w, scale, c0, stride);
+      if (d3) k_wm_pairwise<false, true><<<grid, 256, 0, st>>>(I, img, w, scale, S.ctl, c0, stride);
+      else k_wm_pairwise<false, false><<<grid, 256, 0, st>>>(I, img, w, scale, S.ctl, c0, stride);
     }
+    written = true;
     WM_HIP(hipGetLastError());
+    WM_HIP(hipMemcpyAsync(back, S.ctl, kBackBytes, hipMemcpyDeviceToHost, st));
     WM_HIP(hipStreamSynchronize(st));
+    for (int side = 0; side < 2; ++side) {
+      ST.seeds[side] = ctl[side];
+      if (ctl[side] == 0) {
+        // computeBFS / kmeans "no labels." (QGCW:2015-2016); no plane was written
+        written = false;
+        rc = model_fail(JFC_ERR_NO_SEEDS, side ? "no background seeds" : "no foreground seeds");
+        goto done;
+      }
+    }
+    if (prm->lazy && ctl[2]) {
+      if ((rc = lloyd_on_host(img, w, k, prm->kmeans_iterations, S, back, st))) goto done;
+      unary();
+      WM_HIP(hipGetLastError());
+      WM_HIP(hipStreamSynchronize(st));
+    }
+    const unsigned *hist = (const unsigned *)(back + kCtlBytes);
+    const float *cent = (const float *)(back + kCtlBytes + kHistBytes);
+    for (int side = 0; side < 2; ++side) {
+      for (int l = 0; l < kLevels; ++l) ST.hist_sum[side] += hist[side * kLevels + l];
+      if (!prm->lazy) continue;
+      ST.iterations[side] = ctl[3 + side];
+      for (int i = 0; i < k * 4; ++i) ST.centroids[side][i / 4][i % 4] = cent[side * k * 4 + i];
+    }
     graph_mark_inputs(g, inst);
   }
 done:
   if (rc && written) graph_inputs_failed(g, inst);
-  (void)list_cap;
   return rc;
 }

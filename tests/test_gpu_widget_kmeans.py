@@ -1,0 +1,88 @@
+"""The widget model's seed scan and k-means (jfc_model_widget) against the
+oracle: every capacity, the iteration counts and the centroids, bit-exact, at
+the sizes where a path begins or ends -- one seed, k at its limits and at the
+edges of the kernel's cluster counts, pixels seeded on both sides, seed maps
+that do not start at a multiple of four bytes, and more seeds than one
+workgroup takes.  A side without seeds is refused and changes no plane."""
+import numpy as np
+import pytest
+
+from test_gpu_widget_model import check, random_case, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("k", [2, 8, 9, 16, 17, 32])
+def test_cluster_counts_gpu(gpu, k):
+    shape = (131, 67, 1)
+    say("case widget k", k)
+    rgba, fg, bg = random_case(shape, k)
+    check(gpu, shape, rgba, fg, bg, dict(lazy=True, k=k, weight=(0.3, 0.5, 0.2, 0.1)), solve=False)
+
+
+@pytest.mark.parametrize("lazy", [True, False])
+def test_seed_maps_gpu(gpu, lazy):
+    shape = (97, 45, 1)
+    rgba, fg, bg = random_case(shape, 3)
+    kw = dict(lazy=lazy, k=5, bk_terminal=0.7)
+    one_f, one_b = np.zeros_like(fg), np.zeros_like(bg)
+    one_f[-1], one_b[0] = 1, 255
+    say("case widget one seed a side", lazy)
+    check(gpu, shape, rgba, one_f, one_b, kw, solve=False)
+    both = fg | bg
+    say("case widget pixels seeded on both sides", lazy)
+    check(gpu, shape, rgba, both, both, kw, solve=False)
+
+
+@pytest.mark.parametrize("rows", [171, 172])  # 65,322 / 65,704 seeds a side
+def test_many_seeds_gpu(gpu, rows):
+    shape = (382, 400, 1)
+    say("case widget many seeds", rows)
+    rgba, fg, bg = random_case(shape, rows)
+    fg = fg.reshape(400, 382)
+    bg = bg.reshape(400, 382)
+    fg[:], bg[:] = 0, 0
+    fg[:rows] = 1
+    bg[400 - rows:] = 3
+    check(gpu, shape, rgba, fg.ravel(), bg.ravel(), dict(lazy=True, k=8, kmeans_iterations=6),
+          solve=False)
+
+
+def test_unaligned_seed_maps_gpu(gpu):
+    import torch
+    shape = (61, 33, 1)
+    n = shape[0] * shape[1]
+    rgba, fg, bg = random_case(shape, 7)
+    g = gpu.GridGraph([shape + (4,)])
+    g.model_widget(rgba, fg, bg, k=6)
+    want = g.terminal_caps() + (g.neighbor_caps(),)
+    for off in (1, 2, 3):
+        say("case widget unaligned", off)
+        pad = torch.zeros(2, n + 8, dtype=torch.uint8, device="cuda")
+        pad[0, off:off + n] = torch.from_numpy(fg).cuda()
+        pad[1, off + 1:off + 1 + n] = torch.from_numpy(bg).cuda()
+        h = gpu.GridGraph([shape + (4,)])
+        h.model_widget(torch.from_numpy(rgba).cuda(), pad[0, off:off + n],
+                       pad[1, off + 1:off + 1 + n], k=6)
+        for a, b in zip(want, h.terminal_caps() + (h.neighbor_caps(),)):
+            assert np.array_equal(a, b)
+        h.close()
+    g.close()
+
+
+@pytest.mark.parametrize("lazy", [True, False])
+def test_no_seeds_gpu(gpu, lazy):
+    shape = (40, 30, 1)
+    rgba, fg, bg = random_case(shape, 5)
+    g = gpu.GridGraph([shape + (4,)])
+    g.model_widget(rgba, fg, bg, lazy=lazy, k=3)
+    want = g.terminal_caps() + (g.neighbor_caps(),)
+    none = np.zeros_like(fg)
+    for f, b in ((none, bg), (fg, none), (none, none)):
+        say("case widget no seeds", lazy)
+        with pytest.raises(gpu.JFCError) as e:
+            g.model_widget(255 - rgba, f, b, lazy=lazy, k=3)
+        assert e.value.code == gpu.ERR_NO_SEEDS
+        for a, c in zip(want, g.terminal_caps() + (g.neighbor_caps(),)):
+            assert np.array_equal(a, c)
+    g.close()
