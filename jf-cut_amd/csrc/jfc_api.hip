@@ -189,6 +189,11 @@ struct jfc_graph {
     unsigned char *d_open = nullptr;      // floods: regions with packed arcs
     int tag = 1;           // of the last relabel
     int seq = 0;           // passes run, the number their posted words carry
+    int *d_marks = nullptr;  // words of a one-launch relabel
+    size_t mark_words() const { return (size_t)kRelabelLine * (2 * kRelabelSlots + n); }
+    // idle wait of a one-launch search before it leaves the rest to passes:
+    // far above the ~50 us of a visit, below what a caller would notice
+    long long wait_ticks = 2000000;  // 20 ms
   } rg;
   // One device block holds every word a solve reads back at its end (one
   // copy): the per-instance sums, the remaining deficits, the counters, the
@@ -473,6 +478,7 @@ struct jfc_graph {
       carve(rg.d_inst, rg.inst.size());
       carve(rg.d_tile_inst, n);
       carve(rg.d_any, 4);
+      carve(rg.d_marks, rg.mark_words());
       carve(rg.d_dirty[0], n);
       carve(rg.d_dirty[1], n);
       carve(rg.d_open, n);
@@ -1062,8 +1068,9 @@ struct Solver {
   // once and says so in its group's word.  The first groups are short, as
   // most searches of dense graphs settle within them; later ones grow, as
   // each check costs a gap of about 6 us between two passes.
+  // packed: the regions are packed, and every one is marked for the first pass.
   template <class Issue>
-  int region_passes(int slots, int *passes, Issue issue) {
+  int region_passes(int slots, int *passes, bool packed, Issue issue) {
     if (int rc = g->ensure_pin()) return rc;
     auto &rg = g->rg;
     int pass = 0;
@@ -1080,7 +1087,7 @@ struct Solver {
       issue(kind, c);
       ++pass;
     };
-    next(kPack, 0);
+    if (!packed) next(kPack, 0);
     int want[2] = {0, 0};
     auto issue_group = [&](int k) -> int {
       const int size = k < 2 ? 2 : k < 4 ? 4 : 8;
@@ -1130,7 +1137,7 @@ struct Solver {
     A.stop = stop;
     A.def = g->inst.size() == 1 ? g->d_total + kDefSlots : g->d_def;
     A.object = g->lab;
-    return region_passes(kFloodSlots, passes, [&](int kind, const PassCtl &c) {
+    return region_passes(kFloodSlots, passes, false, [&](int kind, const PassCtl &c) {
       A.c = c;
       launch_flood(d3, tag, T, P, R, A, kind, 2 * g->nwg, st);
     });
@@ -1142,12 +1149,14 @@ struct Solver {
   // is left, then every region again to write the heights.
   int global_relabel() {
     hipEvent_t a = tm.mark();
+    if (int rc = g->ensure_pin()) return rc;
     auto &rg = g->rg;
     rg.tag = 3 - rg.tag;
     {
       FillSet f;
       region_fills(f);
       f.add(g->d_flag, g->ntiles, 0, 1);  // kFinal sets the active tiles' flags
+      f.add(rg.d_marks, (long long)rg.mark_words(), 0, 4);
       launch_fill_multi(f, st);
     }
     const bool d3 = g->dim == 3;
@@ -1161,11 +1170,37 @@ struct Solver {
     A.pinst = g->d_inst;
     A.pone = g->inst[0];
     A.pdims = __builtin_ctz(tw) | __builtin_ctz(th) << 4 | __builtin_ctz(td) << 8;
-    if (int rc = region_passes(kRegionSlots, &s.relabel_passes, [&](int kind, const PassCtl &c) {
-          A.c = c;
-          launch_region(d3, T, P, rg.buf, A, kind, 2 * g->nwg, st);
-        }))
-      return rc;
+    A.sums = rg.d_marks;
+    A.state = A.sums + kRelabelLine * kRelabelSlots;
+    A.marks = A.state + kRelabelLine * kRelabelSlots;
+    A.wait_ticks = rg.wait_ticks;
+    A.c.post = g->d_ring + kStopRing;
+    A.c.visits = g->d_total + kRegionSlots;
+    int *const quit = g->ring + kStopRing;
+    *quit = 0;
+    bool passes = !launch_relabel(d3, T, P, rg.buf, A, st);
+    bool packed = false;
+    if (!passes) {
+      s.relabel_passes++;
+      JFC_HIP(hipEventRecord(g->cnt_ev[0], st));
+      JFC_HIP(hipEventSynchronize(g->cnt_ev[0]));
+      passes = packed = *(const volatile int *)quit != 0;
+    }
+    if (packed) {
+      FillSet f;
+      region_fills(f);
+      f.seg[0].v = 1;  // every region marked for the first pass
+      f.seg[2].v = 1;
+      launch_fill_multi(f, st);
+    }
+    if (passes)
+      if (int rc = region_passes(kRegionSlots, &s.relabel_passes, packed,
+                                 [&](int kind, const PassCtl &c) {
+                                   A.c = c;
+                                   A.sums = nullptr;
+                                   launch_region(d3, T, P, rg.buf, A, kind, 2 * g->nwg, st);
+                                 }))
+        return rc;
     launch_fill_u8(g->d_hmat, g->ntiles, 1, st);  // every height is stored now
     gr_ev.push_back({a, tm.mark()});
     s.global_relabels++;
@@ -1855,6 +1890,12 @@ extern "C" int jfc_backward_all(jfc_graph *g, float *d_cap_source, float *d_cap_
   if (b) JFC_HIP(hipMemcpyAsync(d_cap_sink, b, n * 4, hipMemcpyDeviceToHost, st));
   if (c) JFC_HIP(hipMemcpyAsync(d_neighbor, c, n * g->Kg * 4, hipMemcpyDeviceToHost, st));
   return sync_user(g);
+}
+
+extern "C" int jfc_debug_relabel_wait(jfc_graph *g, int64_t ticks) {
+  if (!g || ticks < 0) return fail(JFC_ERR_INVALID, "bad argument");
+  g->rg.wait_ticks = ticks;
+  return JFC_OK;
 }
 
 extern "C" int jfc_debug_sweep_counts(jfc_graph *g, int32_t *counts, int32_t n) {

@@ -162,7 +162,7 @@ void launch_tile_order(int shape, const Tiles &T, const unsigned char *seed,
                        int *order, int max_tile_dim, int *max_dist,
                        const TileLines &lines, int jump_flooding, hipStream_t st);
 
-// Sweep bookkeeping on the device.  state (8 ints): [0] active tiles of the
+// Sweep bookkeeping on the device.  state (kSweepState ints): [0] active tiles of the
 // running sweep, [1] sweep index, [2] stop word (0 sweep on, 1 no active
 // tile, 2 active set stalled, 3 sweep budget spent, 4 relabel budget
 // spent), [3] sweep index of the last
@@ -237,6 +237,7 @@ struct PassCtl {
   int seq;
   long long *visits;                  // 64 counters of kBorders visits
 };
+constexpr int kRelabelSlots = 64, kRelabelLine = 32;
 struct RegionPass {
   PassCtl c;
   int tag;                            // of this relabel, 1 or 2, alternating
@@ -244,6 +245,12 @@ struct RegionPass {
   const InstDesc *pinst;              // push tiling
   InstDesc pone;                      // its instance 0
   int pdims;                          // push tile dimensions, log2 (x | y << 4 | z << 8)
+  // launch_relabel (else null); all zeroed by the caller, words kRelabelLine
+  // ints apart
+  int *sums;             // kRelabelSlots pairs: marks served, marks made
+  int *state;            // kRelabelSlots
+  int *marks;            // per region: marks made so far
+  long long wait_ticks;  // idle wait before it gives up (100 MHz clock)
 };
 // Cut and tag floods on the same regions (jfc_flood.hip).
 struct FloodBuf {
@@ -265,6 +272,10 @@ struct FloodPass {
 int flood_out_words(bool d3);
 void launch_flood(bool d3, bool tag, const Tiles &T, const Planes &P, const FloodBuf &R,
                   const FloodPass &A, int pass, int nwg, hipStream_t st);
+// The whole relabel; A.c.post becomes 1 if it gave up waiting (every region is
+// packed, no height written).  false: the graph has too many regions for it.
+bool launch_relabel(bool d3, const Tiles &T, const Planes &P, const RegionBuf &R,
+                    const RegionPass &A, hipStream_t st);
 int region_border_words(bool d3);
 int region_state_planes();
 void region_dims(bool d3, int *tw, int *th, int *td);

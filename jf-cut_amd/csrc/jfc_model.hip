@@ -516,7 +516,7 @@ struct KmSums {
     unsigned mine = 0;
 #pragma unroll
     for (int k = 0; k < KB; ++k) {
-      if (k >= K) break;
+      if (k < K)
 #pragma unroll
       for (int c = 0; c <= C; ++c) {
         unsigned t = acc[k][c];

@@ -122,4 +122,43 @@ __device__ __forceinline__ RegionRef region_ref(const InstDesc &I, int t, int la
   return r;
 }
 
+// Step from a region to its neighbour b: 0 / 1 left / right, 2 / 3 low / high y,
+// 4 / 5 low / high z; 2D 4-7 the corners (-x,-y), (-x,+y), (+x,-y), (+x,+y).
+template <bool D3>
+__device__ __forceinline__ int neighbour_step(const RegionRef &r, int b) {
+  switch (b) {
+    case 0: return -1;
+    case 1: return 1;
+    case 2: return -r.sy;
+    case 3: return r.sy;
+    case 4: return D3 ? -r.sz : -1 - r.sy;
+    case 5: return D3 ? r.sz : -1 + r.sy;
+    case 6: return 1 - r.sy;
+    default: return 1 + r.sy;
+  }
+}
+
+// The neighbours a visit marks: bit b of the uniform set, whose region index
+// lane b holds.
+struct Marks {
+  unsigned set = 0;
+  int at = 0;
+  __device__ __forceinline__ void add(int b, bool on) { set |= on ? 1u << b : 0u; }
+  __device__ __forceinline__ bool on(int lane) const { return lane < 8 && ((set >> lane) & 1u); }
+};
+
+// Workgroups of a persistent launch that the device holds at once.
+int device_cus();
+template <auto Kernel, int Block = 256>
+int resident_grid_b(int want) {
+  static const int per_cu = [] {
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, Kernel, Block, 0) != hipSuccess || n < 1)
+      n = 1;
+    return n;
+  }();
+  const int cap = per_cu * device_cus();
+  return want < 1 ? 1 : want < cap ? want : cap;
+}
+
 }  // namespace jfc

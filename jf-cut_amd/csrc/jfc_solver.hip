@@ -14,7 +14,7 @@
 // reached through different arcs, so within a push-relabel launch every
 // residual plane entry has one writer and only excess and mask words need
 // atomics.
-#include "jfc_device.h"
+#include "jfc_rows.h"
 
 #include <algorithm>
 #include <atomic>
@@ -349,7 +349,7 @@ struct InstSums {
 // kernel (occupancy per CU, from its register and LDS use, times CUs).
 // Compute units of the current device, queried once per device (every
 // persistent launch sizes its grid with it).
-static int device_cus() {
+int device_cus() {
   static std::atomic<int> cache[16];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) dev = 0;
@@ -363,17 +363,6 @@ static int device_cus() {
     cus = 1;
   if (dev >= 0 && dev < 16) cache[dev].store(cus, std::memory_order_relaxed);
   return cus;
-}
-
-template <auto Kernel, int Block = 256>
-static int resident_grid_b(int want) {
-  static const int per_cu = [] {
-    int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, Kernel, Block, 0) != hipSuccess || n < 1)
-      n = 1;
-    return n;
-  }();
-  return std::max(1, std::min(want, per_cu * device_cus()));
 }
 
 template <auto Kernel>

@@ -74,3 +74,26 @@ def test_region_edges_tag_gpu(gpu, shape):
         fg[0] = fg[-1] = 1
         assert np.array_equal(g.tags(fg), ol.tag(nx, ny, nz, fg, lab))
     g.close()
+
+
+@pytest.mark.parametrize("conn,shape", [(8, (300, 217, 1)), (4, (2100, 1100, 1)), (6, (70, 41, 33)),
+                                        (6, (300, 190, 70))])
+def test_relabel_gives_up_waiting_gpu(gpu, conn, shape):
+    """A relabel whose waves give up waiting at once is finished by passes: one
+    launch for everything (up to 512 regions) and above."""
+    import ctypes
+    nx, ny, nz = shape
+    rng = np.random.default_rng(nx)
+    cs, ct, caps = random_grid(rng, nx, ny, nz, conn, term_max=20, seed_frac=0.001)
+    f, l, ok = ol.maxflow(nx, ny, nz, conn, cs, ct, caps)
+    g = gpu.GridGraph([(nx, ny, nz, conn)])
+    g.set_terminal_caps(cs, ct)
+    g.set_all_neighbor_caps(caps)
+    for ticks in (0, 1 << 22, 0):
+        say("case relabel wait", conn, shape, ticks)
+        assert gpu.lib().jfc_debug_relabel_wait(g._h, ctypes.c_int64(ticks)) == 0
+        st = g.solve(initial_relabel=1)
+        assert st.converged == 1 and st.global_relabels >= 1
+        assert g.flow() == f
+        assert np.array_equal(g.labels(), l)
+    g.close()
