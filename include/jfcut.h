@@ -90,7 +90,9 @@ typedef struct {
                              sweep stays within [r, 1/r] of the previous sweep's,
                              or two sweeps running repeat the two before them
                              (the active set has stopped changing, or trades
-                             places between two sets of tiles; 0 = off) */
+                             places between two sets of tiles; 0 = off), once
+                             the sweeps since the last relabel have run as
+                             long as that relabel took */
   int graph_sweeps;       /* 1 = replay each sweep's launches (compaction and
                              push per colour class) as one captured hipGraph
                              (default); 0 = launch them one by one.  profile = 1

@@ -167,7 +167,8 @@ void launch_tile_order(int shape, const Tiles &T, const unsigned char *seed,
 // tile, 2 active set stalled, 3 sweep budget spent, 4 relabel budget
 // spent), [3] sweep index of the last
 // relabel, [4..5] tile visits (int64) at the last relabel, [6] sweeps ended
-// (no-ops included) in the solve.
+// (no-ops included) in the solve, [8..9] the clock (int64) at the last stop or
+// resumption, [10..11] the time from the last stop to its resumption.
 struct SweepCtl {
   int *hist;             // active tiles per sweep
   int *state;
@@ -181,7 +182,7 @@ struct SweepCtl {
   int *ring;
   int ring_n;
 };
-constexpr int kSweepState = 8;
+constexpr int kSweepState = 12;
 void launch_sweep_end(const SweepCtl &c, hipStream_t st);
 void launch_sweep_resume(const SweepCtl &c, hipStream_t st);
 

@@ -925,8 +925,8 @@ __global__ __launch_bounds__(kCompactBlock) void k_compact(const int *src, int n
 // the count, so that the host can queue sweeps ahead of its checks:
 //   stop = 1: no tile was active (converged, or the certificate decides);
 //   stop = 2: the active set neither shrank nor grew by more than
-//             (1 - stall_ratio) over the last sweep since the last relabel
-//             (a global relabel is due, or the remaining excess is cut off
+//             (1 - stall_ratio) over the last sweep since the last relabel,
+//             whose time the sweeps since have made up for (a global relabel is due, or the remaining excess is cut off
 //             from every deficit);
 //   stop = 3: the sweep budget is spent;
 //   stop = 4: the tile visits since the last relabel exceed the budget (the
@@ -968,7 +968,17 @@ __global__ void k_sweep_end(SweepCtl c) {
       return (double)a >= c.stall_ratio * b && a * c.stall_ratio <= (double)b;
     };
     bool stalled = false;
-    if (c.stall_ratio > 0.0 && since >= 1 && i < c.cap) {
+    // A stall counts once the sweeps since the last relabel have run as long
+    // as that relabel took, its host wait included: a steady active set is
+    // often flow on its way, and a relabel costs many sweeps on large graphs
+    // and less than one on small ones.  Geometric means over seeds without
+    // this, at half, once, twice and four times the relabel's time:
+    // 3750x2500 strokes 78.7, 71.3, 68.3, 65.0, 67.3 ms; 2560x1440x50 video
+    // 60.5, 46.5, 39.9, 40.9, 38.0; 512^3 volume 27.0, 20.5, 19.7, 22.1, 26.7;
+    // 181x217x181 scan 2.94, 3.07, 3.00, 3.36, 3.88; 1023x767 2.59, 2.73, 2.33,
+    // 2.03, 2.05; 600x450 widget 1.90, 1.89, 1.78, 1.70, 1.56.
+    const bool paid = wall_clock64() - *(const long long *)(st + 8) >= *(const long long *)(st + 10);
+    if (c.stall_ratio > 0.0 && since >= 1 && paid && i < c.cap) {
       stalled = near(cnt, c.hist[i - 1]);
       if (!stalled && since >= 3)
         stalled = near(cnt, c.hist[i - 2]) && near(c.hist[i - 1], c.hist[i - 3]);
@@ -979,6 +989,7 @@ __global__ void k_sweep_end(SweepCtl c) {
     else if (budget) stop = 4;
   }
   st[2] = stop;
+  if (stop) *(long long *)(st + 8) = wall_clock64();
   post_stop(c, seq, stop);
 }
 
@@ -991,6 +1002,9 @@ __global__ void k_sweep_resume(SweepCtl c) {
   st[2] = 0;
   st[3] = st[1];
   *(long long *)(st + 4) = c.total[0];
+  const long long now = wall_clock64();
+  *(long long *)(st + 10) = now - *(const long long *)(st + 8);
+  *(long long *)(st + 8) = now;
 }
 
 void launch_sweep_resume(const SweepCtl &c, hipStream_t st) {
