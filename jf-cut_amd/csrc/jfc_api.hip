@@ -236,14 +236,13 @@ struct jfc_graph {
     long long total;  // tile visits so far (sweep checks)
     int recent[3];    // active tiles of the latest sweeps
     int flag;         // certificate word of a cut search
-    int bad;          // validation word of a setter
     long long red[RED_SLOTS];  // one instance's sums (energy)
   } *pin = nullptr;
   // Pinned copy of d_res (the solve's results).
   long long *pin_res = nullptr;
   // Stop words the sweeps post (k_sweep_end), then the words of two groups
-  // of relabel passes, in fine-grained pinned memory the device writes
-  // through to; d_ring is its device address.
+  // of relabel passes and of a setter's range check, in fine-grained pinned
+  // memory the device writes through to; d_ring is its device address.
   int *ring = nullptr, *d_ring = nullptr;
   hipEvent_t cnt_ev[2] = {nullptr, nullptr};
   hipEvent_t stop_ev[kStopRing] = {};
@@ -262,7 +261,7 @@ struct jfc_graph {
     if (hipHostMalloc((void **)&pin, sizeof(HostPin), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void **)&pin_res, res_words * sizeof(long long), hipHostMallocDefault) !=
             hipSuccess ||
-        hipHostMalloc((void **)&ring, (kStopRing + 2) * sizeof(int), hipHostMallocCoherent) !=
+        hipHostMalloc((void **)&ring, (kStopRing + 4) * sizeof(int), hipHostMallocCoherent) !=
             hipSuccess ||
         hipHostGetDevicePointer((void **)&d_ring, ring, 0) != hipSuccess) {
       (void)hipGetLastError();
@@ -838,28 +837,59 @@ static int get_rows(jfc_graph *g, const InstDesc &I, void *dst, const void *src,
   JFC_HIP(hipMemcpyAsync(dst, tmp, row * rows, hipMemcpyDeviceToHost, st));
   return JFC_OK;
 }
-static int put_plane(jfc_graph *g, const InstDesc &I, int *dst, const int32_t *src,
-                     int on_device) {
-  return put_rows(g, I, dst, src, sizeof(int32_t), on_device);
+// A kernel may read the bytes at p in place: within one allocation, on the
+// device that holds `own`.  Anything else is left to a copy, which takes it (another
+// device's memory) or refuses it.
+static bool readable_in_place(const void *p, size_t bytes, const void *own) {
+  hipPointerAttribute_t at{}, mine{};
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (hipPointerGetAttributes(&at, p) != hipSuccess || at.type != hipMemoryTypeDevice ||
+      hipPointerGetAttributes(&mine, own) != hipSuccess || at.device != mine.device ||
+      hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return (const char *)p + bytes <= (const char *)base + size;
 }
 
-// Range check of up to two planes of n stored values on the graph's stream;
-// waits for the stream.  Returns JFC_ERR_OVERFLOW naming the first plane
-// with a value outside [lo, hi].
-static int validate(jfc_graph *g, const int *p0, const int *p1, long long n, int lo, int hi,
-                    const char *what0, const char *what1) {
+// Capacity planes of the caller onto the stored ones with their range check,
+// on the graph's stream; waits for the stream.  Device arrays are read in
+// place; others cross in one copy each, to the stored plane itself where its
+// rows have no padding (signed values: to the instance's slice of the excess
+// plane, which every solve rewrites before reading it), else through the
+// staging buffer.  Returns JFC_ERR_OVERFLOW naming the first plane with a
+// value outside [lo, hi].
+static int put_caps(jfc_graph *g, int inst, const PutPlanes &planes, int on_device, bool excess,
+                    int dir, int lo, int hi, const char *const *what) {
   if (int rc = g->ensure_pin()) return rc;
-  hipStream_t st = g->ustream;
-  launch_fill_i32(g->d_flagword + 1, 2, 0, st);
-  launch_validate(p0, n, lo, hi, g->d_flagword + 1, st);
-  if (p1) launch_validate(p1, n, lo, hi, g->d_flagword + 2, st);
-  JFC_HIP(hipMemcpyAsync(&g->pin->bad, g->d_flagword + 1, sizeof(int), hipMemcpyDeviceToHost, st));
-  JFC_HIP(hipMemcpyAsync(&g->pin->flag, g->d_flagword + 2, sizeof(int), hipMemcpyDeviceToHost, st));
+  const InstDesc &I = g->inst[inst];
+  const size_t bytes = (size_t)I.nx * I.ny * I.nz * sizeof(int32_t);
+  volatile int *const bad = g->ring + kStopRing + 2;
+  int *const d_bad = g->d_ring + kStopRing + 2;
+  bad[0] = bad[1] = 0;
+  const bool direct = on_device && readable_in_place(planes.src[0], bytes, g->cs) &&
+                      (!planes.src[1] || readable_in_place(planes.src[1], bytes, g->cs));
+  if (direct) {
+    launch_put(I, planes, excess, dir, lo, hi, d_bad, g->ustream);
+  } else {
+    for (int k = 0; k < 2 && planes.src[k]; ++k) {
+      void *at = excess ? g->e + I.node_off : planes.dst[k];
+      if (I.px != I.nx)
+        if (int rc = stage_for(g, bytes, &at)) return rc;
+      JFC_HIP(hipMemcpyAsync(at, planes.src[k], bytes,
+                             on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice,
+                             g->ustream));
+      launch_put(I, {{(const int *)at, nullptr}, {planes.dst[k], planes.dst[1]}}, excess, dir, lo, hi,
+                 d_bad + k, g->ustream);
+    }
+  }
+  JFC_HIP(hipGetLastError());
   if (int rc = sync_user(g)) return rc;
-  const char *bad = g->pin->bad ? what0 : (p1 && g->pin->flag) ? what1 : nullptr;
-  if (bad)
-    return fail(JFC_ERR_OVERFLOW, std::string(bad) + " outside [" + std::to_string(lo) + ", " +
-                                      std::to_string(hi) + "]");
+  const int out = bad[0] ? 0 : bad[1] ? 1 : -1;
+  if (out >= 0)
+    return fail(JFC_ERR_OVERFLOW, std::string(what[out]) + " outside [" + std::to_string(lo) +
+                                      ", " + std::to_string(hi) + "]");
   return JFC_OK;
 }
 
@@ -885,10 +915,9 @@ extern "C" int jfc_set_terminal_caps(jfc_graph *g, int inst, const int32_t *cap_
   if (!cap_source || !cap_sink) return fail(JFC_ERR_INVALID, "null capacity pointer");
   const long long n = g->inst_stored(inst);
   const long long o = g->inst[inst].node_off;
-  if (!(rc = put_plane(g, g->inst[inst], g->cs + o, cap_source, on_device)) &&
-      !(rc = put_plane(g, g->inst[inst], g->ct + o, cap_sink, on_device)))
-    rc = validate(g, g->cs + o, g->ct + o, n, 0, JFC_MAX_TERMINAL_CAP, "source capacity",
-                  "sink capacity");
+  static const char *const what[2] = {"source capacity", "sink capacity"};
+  rc = put_caps(g, inst, {{cap_source, cap_sink}, {g->cs + o, g->ct + o}}, on_device, false, -1, 0,
+                JFC_MAX_TERMINAL_CAP, what);
   if (rc) {
     launch_fill_i32(g->cs + o, n, 0, g->ustream);
     launch_fill_i32(g->ct + o, n, 0, g->ustream);
@@ -908,16 +937,9 @@ extern "C" int jfc_set_excess(jfc_graph *g, int inst, const int32_t *ef, int on_
   if (!ef) return fail(JFC_ERR_INVALID, "null excess pointer");
   const long long n = g->inst_stored(inst);
   const long long o = g->inst[inst].node_off;
-  // staged in the instance's slice of the excess plane, which every solve
-  // rewrites from cs - ct before reading it
-  rc = put_plane(g, g->inst[inst], g->e + o, ef, on_device);
-  if (!rc)
-    rc = validate(g, g->e + o, nullptr, n, -JFC_MAX_TERMINAL_CAP, JFC_MAX_TERMINAL_CAP,
-                  "excess", nullptr);
-  if (!rc) {
-    launch_excess_split(g->e + o, g->cs + o, g->ct + o, n, g->ustream);
-    rc = sync_user(g);
-  }
+  static const char *const what[1] = {"excess"};
+  rc = put_caps(g, inst, {{ef, nullptr}, {g->cs + o, g->ct + o}}, on_device, true, -1,
+                -JFC_MAX_TERMINAL_CAP, JFC_MAX_TERMINAL_CAP, what);
   if (rc) {
     launch_fill_i32(g->cs + o, n, 0, g->ustream);
     launch_fill_i32(g->ct + o, n, 0, g->ustream);
@@ -940,8 +962,9 @@ extern "C" int jfc_set_neighbor_caps(jfc_graph *g, int inst, int arc, const int3
     return fail(JFC_ERR_INVALID, "arc index outside the instance's connectivity");
   const long long n = g->inst_stored(inst);
   int *dst = g->c0 + (long long)arc * g->Ntot + g->inst[inst].node_off;
-  rc = put_plane(g, g->inst[inst], dst, cap, on_device);
-  if (!rc) rc = validate(g, dst, nullptr, n, 0, JFC_MAX_NEIGHBOR_CAP, "neighbour capacity", nullptr);
+  static const char *const what[1] = {"neighbour capacity"};
+  rc = put_caps(g, inst, {{cap, nullptr}, {dst, nullptr}}, on_device, false, arc, 0,
+                JFC_MAX_NEIGHBOR_CAP, what);
   // on failure the plane is zeroed and the mask of the inputs is rebuilt
   // before the next solve, so no stale residual bit of the old arcs survives
   g->mask_dirty = true;
@@ -952,8 +975,6 @@ extern "C" int jfc_set_neighbor_caps(jfc_graph *g, int inst, int arc, const int3
     input_failed(g, inst, 2 << arc);
     return rc;
   }
-  launch_zero_border(g->shape, g->inst[inst], g->c0 + (long long)arc * g->Ntot, arc, g->ustream);
-  if ((rc = sync_user(g))) return rc;
   g->caps_set[inst] |= 2 << arc;
   g->caps_failed[inst] &= ~(2 << arc);
   return JFC_OK;

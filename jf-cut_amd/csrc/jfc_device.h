@@ -38,7 +38,7 @@ using S32x4x2 = Shape<32, 4, 2>;
 // Direction d -> offset.  2D: +x -x +y -y (+x+y) (-x-y) (-x+y) (+x-y);
 // 3D: +x -x +y -y +z -z.  The reverse of d is d^1.
 template <bool D3>
-__device__ __forceinline__ void dir_of(int d, int &dx, int &dy, int &dz) {
+__host__ __device__ __forceinline__ void dir_of(int d, int &dx, int &dy, int &dz) {
   if (D3) {
     dx = (d == 0) - (d == 1);
     dy = (d == 2) - (d == 3);

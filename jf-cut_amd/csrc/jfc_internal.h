@@ -140,15 +140,19 @@ void launch_fill_multi(const FillSet &f, hipStream_t st);
 void launch_fold(int shape, const Tiles &T, const Planes &P, long long *red,
                  unsigned char *active, unsigned char *defi, bool zero_h, unsigned *mask0,
                  int masks, hipStream_t st, bool cleared = false);
-void launch_validate(const int *p, long long n, int lo, int hi, int *bad,
-                     hipStream_t st);
-void launch_zero_border(int shape, const InstDesc &I, int *plane, int d,
-                        hipStream_t st);
+// Capacities in the caller's numbering (rows of nx) onto stored planes (rows of
+// px): src[1] may be null; excess: src[0] holds signed values, dst both
+// terminals.  dir: the arcs' direction (-1: none leaves the grid).  bad: two
+// host words, 1 where src[k] has a value outside [lo, hi].
+struct PutPlanes {
+  const int *src[2];
+  int *dst[2];
+};
+void launch_put(const InstDesc &I, const PutPlanes &p, bool excess, int dir, int lo, int hi,
+                int *bad, hipStream_t st);
 // fg / bg: rows of nx bytes (the caller's numbering); cs / ct: rows of px.
 void launch_seeds(int *cs, int *ct, const unsigned char *fg, const unsigned char *bg, int nx,
                   int px, long long rows, hipStream_t st);
-void launch_excess_split(const int *ef, int *cs, int *ct, long long n,
-                         hipStream_t st);
 
 // Jump-flooding tile distance + counting sort of tiles by distance.
 // Lines of the tile grids along each axis: prefix[a][i] = lines along axis a
