@@ -93,10 +93,9 @@ typedef struct {
                              places between two sets of tiles; 0 = off), once
                              the sweeps since the last relabel have run as
                              long as that relabel took */
-  int graph_sweeps;       /* 1 = replay each sweep's launches (compaction and
-                             push per colour class) as one captured hipGraph
-                             (default); 0 = launch them one by one.  profile = 1
-                             always launches them one by one. */
+  int graph_sweeps;       /* 0 or 1 (default); both launch a sweep's kernels one
+                             by one: a replayed hipGraph of them started later
+                             than they did.  Results do not depend on it. */
   int tile_order;         /* method of the tile distance field
                              (jfc_debug_tile_order): 0 = separable taxicab
                              distance transform (default), 1 = jump flooding
