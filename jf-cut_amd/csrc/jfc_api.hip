@@ -1264,7 +1264,7 @@ struct Solver {
                        g->d_hmat);
       }
       hipEvent_t a = o.profile ? tm.mark() : nullptr;
-      launch_push(g->shape, std::min(g->nwg, std::max(1, n)), T, P, q, g->d_flag, g->d_mat,
+      launch_push(g->shape, g->Kg, std::min(g->nwg, std::max(1, n)), T, P, q, g->d_flag, g->d_mat,
                   g->d_touched, g->d_hmat, o.max_local_iters, o.sparse_local_iters,
                   g->d_sweep_state, g->d_total + kIterSlots, st);
       if (o.profile) push_ev.push_back({a, tm.mark()});

@@ -215,7 +215,7 @@ void launch_compact(const int *src, int n, int reverse, unsigned char *flag,
 // words (cleared when a solve starts).
 // sweep_state: the solve's SweepCtl state ([1] = sweep index).
 constexpr int kSparseAfter = 8;  // sweeps before the sparse cap applies
-void launch_push(int shape, int nwg, const Tiles &T, const Planes &P,
+void launch_push(int shape, int kmax, int nwg, const Tiles &T, const Planes &P,
                  const Queue &q, unsigned char *flag, unsigned char *mat,
                  unsigned char *touched, unsigned char *hmat,
                  int max_iters, int sparse_iters, const int *sweep_state,

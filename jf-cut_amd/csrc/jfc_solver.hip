@@ -1262,18 +1262,23 @@ __device__ __forceinline__ int inward_dir(int p) {
 // step).
 // ONE: a one-instance graph, whose descriptor every visit reads from the
 // kernel arguments instead of loading it behind the tile index.
-template <class S, bool ONE>
-// 7 waves per SIMD: with one ring cell per lane the visit fits 69 VGPRs
-// without spills (the 15000x10000 8-connected cut: 4.67 ms at 5 waves, 4.54
-// at 6, 4.48 at 7, 4.54 at 8, where it spills).  Two ring cells per lane
-// (32x4x2, slim flush) fit 96: 5 waves.
-__global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
+template <class S, bool ONE, int KK>
+// KK: directions of the arrays (4 in a 2D graph without 8-connected
+// instances).  A visit is bound by its chain of LDS round trips and, with
+// several tiles on a CU, by VALU issue: heights and residuals kept in
+// registers through an iteration and 4 directions instead of 8 took a
+// 600x450 widget cut from 1.08 to 0.87 ms and a 181x217x181 scan from 2.5 to
+// 2.1; with 8 directions 3750x2500 strokes from 46 to 42.
+// 7 waves per SIMD fit without spills but for 8 directions, where they cost
+// more than the wave gives (15000x10000: 4.00 ms at 7, 3.92 at 6).  Two ring
+// cells per lane (32x4x2, slim flush) fit 96 VGPRs: 5 waves.
+__global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : KK == 8 ? 6 : 7) void k_push(
     Tiles T, Planes P, Queue q, unsigned char *flag, unsigned char *mat, unsigned char *touched,
     unsigned char *hmat, int max_iters, int sparse_iters,
     const int *sweep_state, long long *iter_total) {
   __shared__ int s_h[S::PADN];
   __shared__ int s_e[S::PADN];
-  __shared__ int s_c[S::KMAX][S::PADN];
+  __shared__ int s_c[KK][S::PADN];
   // Two ring cells per lane (3D 32x4x2): the flush finds its cells again
   // from the lane index and their mask words in LDS, and takes flow back on
   // a cell's one inward plane, so no ring state is held in registers
@@ -1297,7 +1302,7 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
     const int t = ent & kEntryTile;
     const TileRef r = ONE ? tile_ref_of<S>(T.one, t) : tile_ref<S>(T, t);
     const InstDesc &I = r.I;
-    const int K = I.K;
+    const int K = ONE || KK < 8 ? KK : I.K;  // (a compile-time count but in mixed batches)
     const int gx = r.ox + L.lx, gy = r.oy + L.ly, gz = r.oz + L.lz;
     const bool valid = gx < I.nx && gy < I.ny && gz < I.nz;
     // A valid label never exceeds the distance to a deficit node, which is
@@ -1318,9 +1323,9 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
     // used; lanes off the grid, planes d >= K and dead halo cells read a
     // valid dummy address and discard the value.
     const long long gv = valid ? node_index(I, gx, gy, gz) : 0;
-    long long ca[S::KMAX];
+    long long ca[KK];
 #pragma unroll
-    for (int d = 0; d < S::KMAX; ++d) ca[d] = (valid && d < K) ? d * st + gv : 0;
+    for (int d = 0; d < KK; ++d) ca[d] = (valid && d < K) ? d * st + gv : 0;
     // halo: the ring cells (sides and corners in 2D, faces in 3D), split
     // evenly over the four waves so that each wave loads, clears and flushes
     // the same number of cells; the workgroup barrier after the flush then
@@ -1354,20 +1359,20 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
     const int hw0 = P.h[gv];
     int e0 = P.e[gv], h0 = h_stored ? hw0 : 0;
     unsigned rm = 0;
-    int c0r[S::KMAX];
+    int c0r[KK];
     if (!fresh_tile) {
 #pragma unroll
-      for (int d = 0; d < S::KMAX; ++d) c0r[d] = P.cap[ca[d]];
+      for (int d = 0; d < KK; ++d) c0r[d] = P.cap[ca[d]];
     } else if (clean) {
 #pragma unroll
-      for (int d = 0; d < S::KMAX; ++d) c0r[d] = P.c0[ca[d]];
+      for (int d = 0; d < KK; ++d) c0r[d] = P.c0[ca[d]];
 #pragma unroll
-      for (int d = 0; d < S::KMAX; ++d)
+      for (int d = 0; d < KK; ++d)
         if (d < K) rm |= (1u << (8 + d)) | ((unsigned)(c0r[d] > 0) << d);
     } else {
       rm = P.rmask[gv];
 #pragma unroll
-      for (int d = 0; d < S::KMAX; ++d) c0r[d] = ((rm >> (8 + d)) & 1u ? P.c0 : P.cap)[ca[d]];
+      for (int d = 0; d < KK; ++d) c0r[d] = ((rm >> (8 + d)) & 1u ? P.c0 : P.cap)[ca[d]];
     }
     if (!valid) {
       e0 = 0;
@@ -1375,13 +1380,13 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
       rm = 0;
     }
 #pragma unroll
-    for (int d = 0; d < S::KMAX; ++d)
+    for (int d = 0; d < KK; ++d)
       if (!(valid && d < K)) c0r[d] = 0;
 
     s_e[L.me] = e0;
     s_h[L.me] = h0;
 #pragma unroll
-    for (int d = 0; d < S::KMAX; ++d) s_c[d][L.me] = c0r[d];
+    for (int d = 0; d < KK; ++d) s_c[d][L.me] = c0r[d];
 #pragma unroll
     for (int c = 0; c < kRingPerLane<S>; ++c) {
       if (!hc[c].halo) continue;
@@ -1390,75 +1395,68 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
       s_e[p] = 0;
       if constexpr (kSlim) s_hm[p] = hm[c];
 #pragma unroll
-      for (int d = 0; d < S::KMAX; ++d) s_c[d][p] = 0;
+      for (int d = 0; d < KK; ++d) s_c[d][p] = 0;
     }
     __syncthreads();
     // the next entry loads while the tile iterates
     if (tid == 0) Qc.prefetch();
 
-    int it = 0, any;
+    // The iterations.  A node's height is written by its own lane alone and
+    // stays in a register, as do its residuals from the relabel to the push.
+    // Every LDS word a phase needs is read before any is used, so a phase
+    // waits on LDS once instead of once per direction.
+    int it = 0, any, e = e0, h = h0;
     do {
       // relabel (monotone; neighbours may be read before or after their own
-      // relabel in this iteration, which keeps the labelling valid).  Every
-      // LDS word a phase needs is read before any is used, so a phase waits
-      // on LDS once instead of once per direction.
-      if (valid) {
-        const int e = s_e[L.me];
-        const int h = s_h[L.me];
-        if (e > 0 && h < HINF) {
-          int cv[S::KMAX], hv[S::KMAX];
+      // relabel in this iteration, which keeps the labelling valid)
+      const bool live = valid && e > 0 && h < HINF;
+      int cv[KK], hv[KK];
+      if (live) {
 #pragma unroll
-          for (int d = 0; d < S::KMAX; ++d) {
-            cv[d] = s_c[d][L.me];
-            hv[d] = s_h[L.me + lds_off<S>(d)];
-          }
-          int m = HINF;
-#pragma unroll
-          for (int d = 0; d < S::KMAX; ++d)
-            if (d < K && cv[d] > 0) m = min(m, hv[d] + 1);
-          if (m >= hcap) m = HINF;
-          if (m > h) s_h[L.me] = m;
+        for (int d = 0; d < KK; ++d) {
+          cv[d] = s_c[d][L.me];
+          hv[d] = s_h[L.me + lds_off<S>(d)];
         }
+        // planes d >= K hold 0, so their arcs drop out like saturated ones
+        int m = HINF;
+#pragma unroll
+        for (int d = 0; d < KK; d += 2)
+          m = min(m, min(cv[d] > 0 ? hv[d] : HINF, cv[d + 1] > 0 ? hv[d + 1] : HINF));
+        m = m + 1 < hcap ? m + 1 : HINF;
+        if (m > h) s_h[L.me] = h = m;
       }
       __syncthreads();
       // push.  The reverse residual s_c[d^1][nb] is written only by this
       // lane during the phase (its owner nb cannot push back along an arc
-      // this lane pushes on: heights are frozen), so it is read up front too.
+      // this lane pushes on: heights are frozen).
       int pushed = 0;
-      if (valid) {
-        const int e = s_e[L.me];
-        const int h = s_h[L.me];
-        if (e > 0 && h < HINF) {
-          int cv[S::KMAX], hv[S::KMAX], rv[S::KMAX];
+      if (live && h < HINF) {
 #pragma unroll
-          for (int d = 0; d < S::KMAX; ++d) {
+        for (int d = 0; d < KK; ++d) hv[d] = s_h[L.me + lds_off<S>(d)];
+        int rem = e;
+        int f[KK];
+#pragma unroll
+        for (int d = 0; d < KK; ++d) f[d] = hv[d] == h - 1 ? cv[d] : 0;
+#pragma unroll
+        for (int d = 0; d < KK; ++d) {
+          f[d] = min(rem, f[d]);
+          rem -= f[d];
+        }
+#pragma unroll
+        for (int d = 0; d < KK; ++d)
+          if (f[d] > 0) {
             const int nb = L.me + lds_off<S>(d);
-            cv[d] = s_c[d][L.me];
-            hv[d] = s_h[nb];
-            rv[d] = s_c[d ^ 1][nb];
+            s_c[d][L.me] = cv[d] - f[d];
+            atomicAdd(&s_c[d ^ 1][nb], f[d]);
+            atomicAdd(&s_e[nb], f[d]);
           }
-          int rem = e;
-#pragma unroll
-          for (int d = 0; d < S::KMAX; ++d) {
-            if (d < K && rem > 0) {
-              const int nb = L.me + lds_off<S>(d);
-              const int c = cv[d];
-              if (c > 0 && h == hv[d] + 1) {
-                const int f = min(rem, c);
-                s_c[d][L.me] = c - f;
-                s_c[d ^ 1][nb] = rv[d] + f;
-                atomicAdd(&s_e[nb], f);
-                rem -= f;
-              }
-            }
-          }
-          if (rem != e) {
-            atomicAdd(&s_e[L.me], rem - e);
-            pushed = 1;
-          }
+        if (rem != e) {
+          atomicAdd(&s_e[L.me], rem - e);
+          pushed = 1;
         }
       }
       any = block_any(pushed, s_w, par);
+      e = s_e[L.me];
     } while (any && ++it < cap_iters);
     my_iters += it + (any ? 0 : 1);
     if (tid == 0) Qc.publish();
@@ -1469,7 +1467,7 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
     // to, loaded before the interior write-back so that its stores cover the
     // load latency.
     int fl[kRingPerLane<S>];
-    int dc[kRingPerLane<S>][kSlim ? 1 : S::KMAX], cv[kRingPerLane<S>][kSlim ? 1 : S::KMAX];
+    int dc[kRingPerLane<S>][kSlim ? 1 : KK], cv[kRingPerLane<S>][kSlim ? 1 : KK];
     unsigned fr[kRingPerLane<S>], fp[kRingPerLane<S>];
     if constexpr (kSlim) {
       // the ring cells found again (an opaque copy of the lane index keeps
@@ -1490,7 +1488,7 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
       fr[c] = fp[c] = 0;
       if constexpr (!kSlim) {
 #pragma unroll
-        for (int d = 0; d < S::KMAX; ++d) dc[c][d] = cv[c][d] = 0;
+        for (int d = 0; d < KK; ++d) dc[c][d] = cv[c][d] = 0;
       } else {
         dc[c][0] = cv[c][0] = 0;
       }
@@ -1509,7 +1507,7 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
         continue;
       } else {
 #pragma unroll
-      for (int d = 0; d < S::KMAX; ++d) {
+      for (int d = 0; d < KK; ++d) {
         dc[c][d] = d < K ? s_c[d][p] : 0;
         if (dc[c][d] != 0) {
           if ((hm[c] >> (8 + d)) & 1u) fr[c] |= 1u << d;
@@ -1519,7 +1517,7 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
       if (fr[c]) {
         const long long g = hc[c].g;
 #pragma unroll
-        for (int d = 0; d < S::KMAX; ++d) cv[c][d] = P.c0[((fr[c] >> d) & 1u) ? d * st + g : 0];
+        for (int d = 0; d < KK; ++d) cv[c][d] = P.c0[((fr[c] >> d) & 1u) ? d * st + g : 0];
       }
       }
     }
@@ -1527,14 +1525,14 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
     // ---- write back what changed (stores only)
     int act = 0;
     if (valid) {
-      const int e1 = s_e[L.me], h1 = s_h[L.me];
+      const int e1 = e, h1 = h;
       if (e1 != e0) P.e[gv] = e1;
       if (h1 != h0 || !h_stored) P.h[gv] = h1;
       // fresh planes are written whether or not they changed; the mask word
       // of a written tile holds residual bits only (exact, no fresh bits)
       unsigned m0 = 0, m1 = 0;
 #pragma unroll
-      for (int d = 0; d < S::KMAX; ++d)
+      for (int d = 0; d < KK; ++d)
         if (d < K) {
           const int c1 = s_c[d][L.me];
           if (c1 != c0r[d] || ((rm >> (8 + d)) & 1u)) P.cap[d * st + gv] = c1;
@@ -1571,7 +1569,7 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
         else if (dc[c][0] != 0) atomicAdd(&P.cap[a], dc[c][0]);
       } else {
 #pragma unroll
-        for (int d = 0; d < S::KMAX; ++d) {
+        for (int d = 0; d < KK; ++d) {
           if ((fr[c] >> d) & 1u) P.cap[d * st + g] = cv[c][d] + dc[c][d];
           else if (dc[c][d] != 0) atomicAdd(&P.cap[d * st + g], dc[c][d]);
         }
@@ -1590,20 +1588,26 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : 7) void k_push(
     atomicAdd((unsigned long long *)&iter_total[blockIdx.x & 63], (unsigned long long)my_iters);
 }
 
-void launch_push(int shape, int nwg, const Tiles &T, const Planes &P,
+// kmax: the most directions of any instance (a 2D graph of 4-connected
+// instances iterates over 4: half the LDS reads of 8).
+void launch_push(int shape, int kmax, int nwg, const Tiles &T, const Planes &P,
                  const Queue &q, unsigned char *flag, unsigned char *mat,
                  unsigned char *touched, unsigned char *hmat,
                  int max_iters, int sparse_iters, const int *sweep_state,
                  long long *iter_total, hipStream_t st) {
-  if (T.ninst == 1) {
-    JFC_DISPATCH(shape, (k_push<S, true><<<resident_grid<&k_push<S, true>>(nwg), 256, 0, st>>>(
-                            T, P, q, flag, mat, touched, hmat, max_iters, sparse_iters,
-                            sweep_state, iter_total)));
-  } else {
-    JFC_DISPATCH(shape, (k_push<S, false><<<resident_grid<&k_push<S, false>>(nwg), 256, 0, st>>>(
-                            T, P, q, flag, mat, touched, hmat, max_iters, sparse_iters,
-                            sweep_state, iter_total)));
-  }
+  const auto go = [&](auto *kernel, int grid) {
+    kernel<<<grid, 256, 0, st>>>(T, P, q, flag, mat, touched, hmat, max_iters, sparse_iters,
+                                 sweep_state, iter_total);
+  };
+#define JFC_PUSH(ONE, KK) go(&k_push<S, ONE, KK>, resident_grid<&k_push<S, ONE, KK>>(nwg))
+  JFC_DISPATCH(shape, {
+    constexpr int k0 = S::D3 ? 6 : 4;
+    if (T.ninst == 1 && kmax <= k0) JFC_PUSH(true, k0);
+    else if (T.ninst == 1) JFC_PUSH(true, S::KMAX);
+    else if (kmax <= k0) JFC_PUSH(false, k0);
+    else JFC_PUSH(false, S::KMAX);
+  });
+#undef JFC_PUSH
 }
 
 }  // namespace jfc
