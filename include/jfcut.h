@@ -112,9 +112,10 @@ typedef struct {
   int sparse_local_iters; /* cap on LDS discharge iterations per visit in a
                              push launch whose active-tile list is no longer
                              than its grid (each workgroup visits at most one
-                             tile), from the solve's 8th sweep on: 0 (default)
+                             tile); the cap starts at max_local_iters and
+                             doubles every sweep up to this: 0 (default)
                              = the cap jfc_autotune chose for the graph's size
-                             class, else 32; negative = max_local_iters (the
+                             class, else 16; negative = max_local_iters (the
                              reference loops each visit until no push,
                              graphcut_push_relabel.cl:77-182) */
   int stall_certify;      /* when the active set stalls (stall_ratio): 1 = run

@@ -99,11 +99,14 @@ struct Tuned {
 };
 
 // Default cap on the local iterations of a launch whose list fits its grid,
-// from the solve's kSparseAfter-th sweep on (the reference fixtures: 4.6 ->
-// 2.2-3.0 ms against a cap of 2; from the first sweep on, larger caps slowed
-// graphs whose few active tiles iterate without effect, the 512x512
-// 4-connected cut 0.48 -> 0.71 ms at 64).
-constexpr int kSparseIters = 32;
+// reached by doubling the dense cap once a sweep.  A launch lasts as long as
+// its longest visit, which flow that goes nowhere keeps at the cap: over four
+// inputs each, 12 / 16 / 24 / 32 iterations took 47 / 39 / 40 / 42 ms for
+// 3750x2500 strokes and 3.08 / 3.25 / 3.20 / 3.5 ms for a 181x217x181 scan.
+// At 16 from the eighth sweep on, from the first, and doubling: a 640x480
+// grid 1.25 / 0.83 / 0.95 ms, a 600x450 widget cut 1.43 / 1.20 / 1.03, a
+// 512x512 cut, done after four sweeps, 0.63 / 0.69 / 0.64.
+constexpr int kSparseIters = 16;
 std::mutex g_tune_mu;
 std::map<std::string, Tuned> g_tune;
 

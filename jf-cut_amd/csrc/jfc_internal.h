@@ -209,12 +209,11 @@ void launch_compact(const int *src, int n, int reverse, unsigned char *flag,
 // this solve (by a push visit, which then writes all of them, or by a global
 // relabel); heights of a tile with hmat 0 read as 0, the labelling a solve
 // starts from.  max_iters caps the local iterations of a visit, sparse_iters
-// those of a launch whose list fits its grid once kSparseAfter sweeps ran.  iter_total: 64 int64 counters
-// of local iterations (or null).
+// those of a launch whose list fits its grid, max_iters << sweep until then.
+// iter_total: 64 int64 counters of local iterations (or null).
 // touched: per tile, 1 once a flush wrote into the tile's planes or mask
 // words (cleared when a solve starts).
 // sweep_state: the solve's SweepCtl state ([1] = sweep index).
-constexpr int kSparseAfter = 8;  // sweeps before the sparse cap applies
 void launch_push(int shape, int kmax, int nwg, const Tiles &T, const Planes &P,
                  const Queue &q, unsigned char *flag, unsigned char *mat,
                  unsigned char *touched, unsigned char *hmat,

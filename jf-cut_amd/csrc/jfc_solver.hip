@@ -1255,11 +1255,10 @@ __device__ __forceinline__ int inward_dir(int p) {
 // only excess needs LDS atomics.  Flow pushed into halo cells accumulates in
 // their LDS slots and is flushed to HBM once per visit.  The loop ends when a
 // whole iteration pushes nothing (graphcut_push_relabel.cl:77-182) or after
-// max_iters iterations -- sparse_iters when the launch's list is no longer
-// than its grid and the solve has run kSparseAfter sweeps (every workgroup
-// holds at most one tile, so a visit that keeps iterating delays no other
-// tile, and the flow crosses the tile in one visit instead of one sweep per
-// step).
+// max_iters iterations -- up to sparse_iters when the launch's list is no
+// longer than its grid (every workgroup holds at most one tile, so a visit
+// that keeps iterating delays no other tile, and the flow crosses the tile in
+// one visit instead of one sweep per step).
 // ONE: a one-instance graph, whose descriptor every visit reads from the
 // kernel arguments instead of loading it behind the tile index.
 template <class S, bool ONE, int KK>
@@ -1291,10 +1290,12 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : KK == 8 ? 6 : 7) voi
   __shared__ int s_w[8];
   int par = 0;
   VisitCursor Qc(q, s_next);
-  // the sparse cap from the solve's kSparseAfter-th sweep on: a solve that
-  // ends within a few sweeps has nothing to gain from long visits
-  const int cap_iters =
-      Qc.count <= (int)gridDim.x && sweep_state[1] >= kSparseAfter ? sparse_iters : max_iters;
+  // a sparse launch's cap doubles with every sweep up to sparse_iters: a solve
+  // that ends within a few sweeps has nothing to gain from long visits
+  const int sweep = min(sweep_state[1], 30);
+  const int cap_iters = Qc.count > (int)gridDim.x           ? max_iters
+                        : (sparse_iters >> sweep) < max_iters ? sparse_iters
+                                                              : max_iters << sweep;
   const long long st = P.stride;
   long long my_iters = 0;
   while (Qc.idx >= 0) {
