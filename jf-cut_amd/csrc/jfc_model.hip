@@ -426,17 +426,18 @@ __device__ __forceinline__ void near_d2(const double (*X)[C], const double *n2, 
 
 // The rounded mean of each non-empty cluster, else the old centre, into s_new
 // (which may be `old`), by a whole workgroup; returns whether any moved.
-__device__ bool km_means(const unsigned long long *s_sum, const long long *old, int K, int C,
-                         long long *s_new) {
+// total(k, c): cluster k's sum of channel c, for c = C its seeds.
+template <class F>
+__device__ bool km_means(F total, const long long *old, int K, int C, long long *s_new) {
   const int j = threadIdx.x;
   int changed = 0;
   if (j < K * C) {
     const int k = j / C, c = j % C;
-    const long long nk = (long long)s_sum[k * (C + 1) + C];
+    const long long nk = total(k, C);
     long long nc = old[j];
     if (nk) {
       // floor(a / nk) for 0 <= a < 2^53: the float64 quotient is off by one at most
-      const long long a = (long long)s_sum[k * (C + 1) + c] * (1 << KM_FRAC) + nk / 2;
+      const long long a = total(k, c) * (1 << KM_FRAC) + nk / 2;
       long long v = (long long)((double)a / (double)nk);
       const long long r = a - v * nk;
       v += r < 0 ? -1 : r >= nk ? 1 : 0;
@@ -462,7 +463,8 @@ __device__ bool km_update(const long long *part, int nb, const long long *old, i
     if (v) atomicAdd(&s_sum[i % E], v);
   }
   __syncthreads();
-  return km_means(s_sum, old, K, C, s_new);
+  return km_means([&](int k, int c) { return (long long)s_sum[k * (C + 1) + c]; }, old, K, C,
+                  s_new);
 }
 
 // The final centres of a side: stored with their table, and the done flag
@@ -605,39 +607,166 @@ __global__ __launch_bounds__(256) void k_km_iter(Scratch s, int Kf, int Kb, int 
            threadIdx.x] = (long long)s_sum[threadIdx.x];
 }
 
-// The whole k-means of a side with up to kLoopSeeds seeds, one workgroup of
-// 1024 lanes per side (blockIdx.x): the initial centres, then Lloyd
-// iterations from seeds held in LDS until no centre moves or `iters`
-// are done.  A few thousand seeds are one or a few rounds of a workgroup, less
-// than the launches between iterations cost, and the loop ends with the
-// iteration that converges.
+// ---- the k-means in one launch ----
+//
+// A side with up to kLoopSeeds seeds takes one workgroup of 1024 lanes
+// (blockIdx.x): the initial centres, then Lloyd iterations from seeds held in
+// registers until no centre moves or `iters` are done.  Few seeds are a few
+// rounds of a workgroup, less than the launches between iterations cost, and
+// the loop ends with the iteration that converges.  It is bound by the VALU
+// work per seed, so the sums are a matrix product -- (clusters x seeds, one-hot)
+// times (seeds x bytes of their features) on the matrix cores, exact in
+// int32 -- and 8-bit features find their centre in 24-bit integers: 5 centres,
+// 4,800 RGB seeds took 193 us for 32 iterations with float64 distances
+// and a register sum per cluster, and take 122.
 constexpr int kLoopSeeds = 8192;
+constexpr int kLoopRounds = kLoopSeeds / 1024;
+typedef int v4i __attribute__((ext_vector_type(4)));
 
-template <int BPC, int C, int KB>
+// The centres in the order a round names them ("row"), for the assignment of
+// 8-bit features x: |X - c|^2 - |X|^2 = 512 (floor(|c|^2 / 512) - x.c) +
+// |c|^2 mod 512 with X = 2^8 x, so a minimum, ties to the lowest index, is that of
+// floor(|c|^2 / 512) - x.c, ties to the lowest (|c|^2 mod 512, index).  Rows
+// are the centres sorted by the latter; v[0] = 16 floor(|c|^2 / 512) + row and
+// v[1 + c] = -16 c_c give 16 times the former plus the row, below 2^30.
+struct NearRow {
+  int v[4];
+};
+
+template <int C>
+__device__ __forceinline__ void put_rows(NearRow *s_row, int *s_cluster, const long long *c, int K) {
+  const int k = threadIdx.x;
+  if (k >= K) return;
+  const auto sq = [&](int j) {
+    long long t = 0;
+    for (int i = 0; i < C; ++i) t += c[j * C + i] * c[j * C + i];
+    return t;
+  };
+  const long long mine = sq(k);
+  int row = 0;
+  for (int j = 0; j < K; ++j) {
+    const int r = (int)(sq(j) & 511), m = (int)(mine & 511);
+    row += r < m || (r == m && j < k);
+  }
+  s_cluster[row] = k;
+  s_row[k].v[0] = (int)(mine >> 9) * 16 + row;
+  for (int i = 0; i < 3; ++i) s_row[k].v[1 + i] = i < C ? -16 * (int)c[k * C + i] : 0;
+}
+
+// Byte j of a seed's row of the sums' right operand: the feature's bytes less
+// 128, then 1; zero from there on.
+template <int BPC, int C>
+__device__ __forceinline__ unsigned seed_byte(unsigned packed, int j) {
+  constexpr int B = BPC == 2 ? 2 : C;
+  return j < B ? ((packed >> (8 * j)) & 255u) ^ 128u : j == B ? 1u : 0u;
+}
+
+template <int BPC, int C>
 __global__ __launch_bounds__(1024) void k_km_loop(Scratch s, int nkeys, int Kf, int Kb, int iters) {
-  __shared__ unsigned s_list[kLoopSeeds];
+  constexpr int B = BPC == 2 ? 2 : C;  // bytes of a feature
+  __shared__ __attribute__((aligned(16))) unsigned s_list[1024];
+  __shared__ __attribute__((aligned(16))) unsigned char s_best[16][kLoopRounds][64];
   __shared__ long long s_c[KMAX_CLUSTERS * 3];
   __shared__ double s_q[KMAX_CLUSTERS * 4];
-  __shared__ unsigned long long s_sum[KMAX_CLUSTERS * 4];
+  __shared__ NearRow s_row[KMAX_CLUSTERS];
+  __shared__ int s_cluster[KMAX_CLUSTERS];
+  __shared__ int s_sum[KMAX_CLUSTERS * 4];  // per cluster: its bytes' sums less 128 each, its seeds
   const int side = blockIdx.x, K = side ? Kb : Kf, tid = threadIdx.x;
-  const int n = (int)min((long long)s.ctl[side], s.cap);
+  const int wave = tid >> 6, lane = tid & 63, j = lane & 15, kb = lane >> 4;
+  const int n = min((int)min((long long)s.ctl[side], s.cap), kLoopSeeds);
   if (!km_init<1024>(s, side, C, nkeys, K, s_c)) return;
-  // each lane reads back only the entries it wrote
-  for (int i = tid; i < n; i += 1024) s_list[i] = (unsigned)s.list[side ? s.cap - 1 - i : i];
+  const int rounds = (n + 1023) / 1024;
+  unsigned mine[kLoopRounds];  // this lane's seeds
+  v4i feat[kLoopRounds];       // byte j of 16 seeds of the wave's round
+#pragma unroll
+  for (int g = 0; g < kLoopRounds; ++g) {
+    mine[g] = 0;
+    feat[g] = v4i{0, 0, 0, 0};
+    if (g >= rounds) continue;
+    const int i = g * 1024 + tid;
+    mine[g] = i < n ? (unsigned)s.list[side ? s.cap - 1 - i : i] : 0u;
+    s_list[tid] = mine[g];
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int q = wave * 64 + kb * 16 + e;
+      const unsigned b = g * 1024 + q < n ? seed_byte<BPC, C>(s_list[q], j) : 0u;
+      feat[g][e / 4] |= (int)(b << (8 * (e % 4)));
+    }
+    __syncthreads();
+  }
+  if (BPC == 2 && tid < KMAX_CLUSTERS) s_cluster[tid] = tid;
   bool moved = true;
   int it = 0;
   while (moved && it < iters) {
     ++it;
-    put_table(s_q, s_c, K, C);
+    if constexpr (BPC == 1) put_rows<C>(s_row, s_cluster, s_c, K);
+    else put_table(s_q, s_c, K, C);
     if (tid < KMAX_CLUSTERS * 4) s_sum[tid] = 0;
     __syncthreads();
-    KmSums<C, KB> sums;
-    sums.clear();
-#pragma unroll 1
-    for (int i = tid; i < n; i += 1024) sums.template add<BPC>(s_list[i], s_q, K);
-    sums.flush(s_sum, K);
+    // the assignment (graphcut_kmeans.cl:21-89): nearest centroid, lowest
+    // index on ties, as a row of the one-hot operand
+    if constexpr (BPC == 1) {
+      int key[kLoopRounds];
+#pragma unroll
+      for (int g = 0; g < kLoopRounds; ++g) key[g] = 0x7fffffff;
+      for (int k = 0; k < K; ++k) {
+        const NearRow r = s_row[k];
+#pragma unroll
+        for (int g = 0; g < kLoopRounds; ++g) {
+          if (g >= rounds) break;
+          int e = r.v[0];
+#pragma unroll
+          for (int c = 0; c < C; ++c) e += __mul24((int)((mine[g] >> (8 * c)) & 255u), r.v[1 + c]);
+          key[g] = min(key[g], e);
+        }
+      }
+#pragma unroll
+      for (int g = 0; g < kLoopRounds; ++g)
+        if (g < rounds) s_best[wave][g][lane] = (unsigned char)(key[g] & 15);
+    } else {
+#pragma unroll
+      for (int g = 0; g < kLoopRounds; ++g) {
+        if (g >= rounds) break;
+        const int x[1] = {(int)mine[g]};
+        double X[1], n2;
+        scaled_feature<1>(x, X, &n2);
+        int best;
+        near_part<1>(X, s_q, K, &best);
+        s_best[wave][g][lane] = (unsigned char)best;
+      }
+    }
+    // the wave reads back what its own lanes wrote
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    v4i acc{0, 0, 0, 0};
+#pragma unroll
+    for (int g = 0; g < kLoopRounds; ++g) {
+      if (g >= rounds) break;
+      const v4i b = *(const v4i *)&s_best[wave][g][kb * 16];
+      v4i hot;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        // bytes equal to j: rows are below 16, so no byte carries
+        const unsigned t = ((unsigned)b[w] ^ (unsigned)(j * 0x01010101)) + 0x7f7f7f7fu;
+        hot[w] = (int)((~t >> 7) & 0x01010101u);
+      }
+      acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(hot, feat[g], acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (kb * 4 + r < K && j <= B) atomicAdd(&s_sum[s_cluster[kb * 4 + r] * 4 + j], acc[r]);
     __syncthreads();
-    moved = km_means(s_sum, s_c, K, C, s_c);
+    moved = km_means(
+        [&](int k, int c) {
+          const int *v = s_sum + k * 4;
+          const long long nk = v[B];
+          if (c == C) return nk;
+          if (BPC == 2) return v[0] + 128 * nk + 256 * (v[1] + 128 * nk);
+          return v[c] + 128 * nk;
+        },
+        s_c, K, C, s_c);
   }
   km_finish(s, side, s_c, K, C, !moved, it);
 }
@@ -1300,9 +1429,7 @@ int run_model(const InstDesc &I, const void *img, const unsigned char *seeds,
   const long long most = std::max(ctl[0], ctl[1]);
   const int Kf = prm->k_fg, Kb = prm->k_bg, kmax = std::max(Kf, Kb);
   if (most <= kLoopSeeds && iters > 0) {
-    if (kmax <= 4) k_km_loop<BPC, C, 4><<<2, 1024, 0, st>>>(s, nkeys, Kf, Kb, iters);
-    else if (kmax <= 8) k_km_loop<BPC, C, 8><<<2, 1024, 0, st>>>(s, nkeys, Kf, Kb, iters);
-    else k_km_loop<BPC, C, 16><<<2, 1024, 0, st>>>(s, nkeys, Kf, Kb, iters);
+    k_km_loop<BPC, C><<<2, 1024, 0, st>>>(s, nkeys, Kf, Kb, iters);
   } else {
     k_km_init<<<2, 256, 0, st>>>(s, C, nkeys, Kf, Kb);
     // up to KM_GRID workgroups per side, about 4 seeds per lane
