@@ -1151,9 +1151,14 @@ struct Solver {
   // Exact relabel (graphcut_init_global_relabel + graphcut_global_relabel,
   // graphcut_global_relabel.cl:19-124) on the graph's regions
   // (jfc_region.hip): every region once, then the marked ones until no mark
-  // is left, then every region again to write the heights.
-  int global_relabel() {
+  // is left, then every region again to write the heights.  Where one launch
+  // takes every pass, nothing waits for it here: should its waves have given
+  // up waiting, the sweeps queued behind it do nothing and post stop word 5,
+  // and finish_relabel() does it by passes.  resume: sweeping goes on after a
+  // stop.
+  int global_relabel(bool resume) {
     hipEvent_t a = tm.mark();
+    relabel_start = a;
     if (int rc = g->ensure_pin()) return rc;
     auto &rg = g->rg;
     rg.tag = 3 - rg.tag;
@@ -1164,9 +1169,35 @@ struct Solver {
       f.add(rg.d_marks, (long long)rg.mark_words(), 0, 4);
       launch_fill_multi(f, st);
     }
-    const bool d3 = g->dim == 3;
-    const Tiles T = g->region_tiles();
-    const Planes P = g->planes();
+    RegionPass A = relabel_pass();
+    if (launch_relabel(g->dim == 3, g->region_tiles(), g->planes(), rg.buf, A, st)) {
+      s.relabel_passes++;
+      relabelled(A.quit, resume);
+    } else {
+      if (int rc = relabel_passes(A, false)) return rc;
+      relabelled(nullptr, resume);
+    }
+    return JFC_OK;
+  }
+
+  // The relabel whose waves gave up waiting, by passes over its packed regions.
+  int finish_relabel() {
+    FillSet f;
+    region_fills(f);
+    f.seg[0].v = 1;  // every region marked for the first pass
+    f.seg[2].v = 1;
+    launch_fill_multi(f, st);
+    if (int rc = relabel_passes(relabel_pass(), true)) return rc;
+    gr_ev.pop_back();
+    s.global_relabels--;
+    relabelled(nullptr, true);
+    return JFC_OK;
+  }
+
+  hipEvent_t relabel_start = nullptr;
+
+  RegionPass relabel_pass() const {
+    auto &rg = g->rg;
     int tw, th, td;
     shape_dims(g->shape, &tw, &th, &td);
     RegionPass A{};
@@ -1179,37 +1210,26 @@ struct Solver {
     A.state = A.sums + kRelabelLine * kRelabelSlots;
     A.marks = A.state + kRelabelLine * kRelabelSlots;
     A.wait_ticks = rg.wait_ticks;
-    A.c.post = g->d_ring + kStopRing;
+    A.quit = A.state + 1;
     A.c.visits = g->d_total + kRegionSlots;
-    int *const quit = g->ring + kStopRing;
-    *quit = 0;
-    bool passes = !launch_relabel(d3, T, P, rg.buf, A, st);
-    bool packed = false;
-    if (!passes) {
-      s.relabel_passes++;
-      JFC_HIP(hipEventRecord(g->cnt_ev[0], st));
-      JFC_HIP(hipEventSynchronize(g->cnt_ev[0]));
-      passes = packed = *(const volatile int *)quit != 0;
-    }
-    if (packed) {
-      FillSet f;
-      region_fills(f);
-      f.seg[0].v = 1;  // every region marked for the first pass
-      f.seg[2].v = 1;
-      launch_fill_multi(f, st);
-    }
-    if (passes)
-      if (int rc = region_passes(kRegionSlots, &s.relabel_passes, packed,
-                                 [&](int kind, const PassCtl &c) {
-                                   A.c = c;
-                                   A.sums = nullptr;
-                                   launch_region(d3, T, P, rg.buf, A, kind, 2 * g->nwg, st);
-                                 }))
-        return rc;
-    launch_fill_u8(g->d_hmat, g->ntiles, 1, st);  // every height is stored now
-    gr_ev.push_back({a, tm.mark()});
+    return A;
+  }
+
+  int relabel_passes(RegionPass A, bool packed) {
+    A.sums = nullptr;
+    const Tiles T = g->region_tiles();
+    const Planes P = g->planes();
+    return region_passes(kRegionSlots, &s.relabel_passes, packed, [&](int kind, const PassCtl &c) {
+      A.c = c;
+      launch_region(g->dim == 3, T, P, g->rg.buf, A, kind, 2 * g->nwg, st);
+    });
+  }
+
+  // after a relabel: every height is stored now, sweeping resumes
+  void relabelled(const int *quit, bool resume) {
+    launch_relabel_end(sweep_ctl(), g->d_hmat, g->ntiles, quit, resume, st);
+    gr_ev.push_back({relabel_start, tm.mark()});
     s.global_relabels++;
-    return JFC_OK;
   }
 
   int cuts = 0;  // canonical-cut searches run
@@ -1353,7 +1373,7 @@ struct Solver {
     std::vector<long long> red((size_t)nI * RED_SLOTS);
     int rc;
     if (o.initial_relabel) {
-      if ((rc = global_relabel())) return rc;
+      if ((rc = global_relabel(false))) return rc;
     }  // else the zero heights (a valid labelling) and the fold's flags
     // Sweeps go out up to `ahead` beyond the last one whose stop word the
     // host has read.  The device decides after every sweep whether to go on
@@ -1413,8 +1433,11 @@ struct Solver {
         }
       }
       if (stopw == 2 || stopw == 4) {
-        if ((rc = global_relabel())) return rc;
-        launch_sweep_resume(sweep_ctl(), st);
+        if ((rc = global_relabel(true))) return rc;
+        continue;
+      }
+      if (stopw == 5) {  // the last relabel is not done
+        if ((rc = finish_relabel())) return rc;
         continue;
       }
       // no active tile: the canonical cut doubles as the certificate
@@ -1427,8 +1450,7 @@ struct Solver {
       // an augmenting path survived: relabel exactly and continue
       s.certificate_failures++;
       if (++cert_rounds > 16) return fail(JFC_ERR_STATE, "certificate kept failing");
-      if ((rc = global_relabel())) return rc;
-      launch_sweep_resume(sweep_ctl(), st);
+      if ((rc = global_relabel(true))) return rc;
     }
     if (!done) {
       // labels of the current preflow are still useful to callers

@@ -169,7 +169,7 @@ void launch_tile_order(int shape, const Tiles &T, const unsigned char *seed,
 // Sweep bookkeeping on the device.  state (kSweepState ints): [0] active tiles of the
 // running sweep, [1] sweep index, [2] stop word (0 sweep on, 1 no active
 // tile, 2 active set stalled, 3 sweep budget spent, 4 relabel budget
-// spent), [3] sweep index of the last
+// spent, 5 the last relabel is unfinished), [3] sweep index of the last
 // relabel, [4..5] tile visits (int64) at the last relabel, [6] sweeps ended
 // (no-ops included) in the solve, [8..9] the clock (int64) at the last stop or
 // resumption, [10..11] the time from the last stop to its resumption.
@@ -188,7 +188,8 @@ struct SweepCtl {
 };
 constexpr int kSweepState = 12;
 void launch_sweep_end(const SweepCtl &c, hipStream_t st);
-void launch_sweep_resume(const SweepCtl &c, hipStream_t st);
+void launch_relabel_end(const SweepCtl &c, unsigned char *hmat, int n, const int *quit, bool resume,
+                        hipStream_t st);
 
 // Queue list entries: tile index, plus, when compacted with `mat`, kEntryMat
 // if mat[t] is set, else kEntryClean if touched[t] is clear (no visit and no
@@ -254,6 +255,7 @@ struct RegionPass {
   int *sums;             // kRelabelSlots pairs: marks served, marks made
   int *state;            // kRelabelSlots
   int *marks;            // per region: marks made so far
+  int *quit;             // set when it gave up waiting
   long long wait_ticks;  // idle wait before it gives up (100 MHz clock)
 };
 // Cut and tag floods on the same regions (jfc_flood.hip).
@@ -276,7 +278,7 @@ struct FloodPass {
 int flood_out_words(bool d3);
 void launch_flood(bool d3, bool tag, const Tiles &T, const Planes &P, const FloodBuf &R,
                   const FloodPass &A, int pass, int nwg, hipStream_t st);
-// The whole relabel; A.c.post becomes 1 if it gave up waiting (every region is
+// The whole relabel; *A.quit becomes 1 if it gave up waiting (every region is
 // packed, no height written).  false: the graph has too many regions for it.
 bool launch_relabel(bool d3, const Tiles &T, const Planes &P, const RegionBuf &R,
                     const RegionPass &A, hipStream_t st);

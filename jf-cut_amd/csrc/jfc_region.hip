@@ -764,7 +764,7 @@ __global__ __launch_bounds__(64 * W) void k_settle(Tiles T, Planes P, RegionBuf 
       if (tick - since >= A.wait_ticks) {
         tell(kQuit);
         if (lane == 0)
-          __hip_atomic_store(A.c.post, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+          __hip_atomic_store(A.quit, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         break;
       }
       __builtin_amdgcn_s_sleep(8);

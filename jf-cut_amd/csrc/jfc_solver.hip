@@ -1001,20 +1001,34 @@ __global__ void k_sweep_end(SweepCtl c) {
 
 void launch_sweep_end(const SweepCtl &c, hipStream_t st) { k_sweep_end<<<1, 1, 0, st>>>(c); }
 
-// After a global relabel: sweeping resumes, and the relabel's sweep index
-// and visit total are the base of the next stall and budget tests.
-__global__ void k_sweep_resume(SweepCtl c) {
+// After a global relabel: every height is stored (hmat); with resume, sweeping
+// goes on, and the relabel's sweep index and visit total are the base of the
+// next stall and budget tests.  *quit (or null): the relabel's waves gave up
+// waiting, so sweeping stops until the host has finished it.
+__global__ void k_relabel_end(SweepCtl c, unsigned char *hmat, int n, const int *quit, int resume) {
   int *st = c.state;
-  st[2] = 0;
-  st[3] = st[1];
-  *(long long *)(st + 4) = c.total[0];
-  const long long now = wall_clock64();
-  *(long long *)(st + 10) = now - *(const long long *)(st + 8);
-  *(long long *)(st + 8) = now;
+  const bool unfinished = quit && *quit;
+  const int tid = blockIdx.x * blockDim.x + threadIdx.x;
+  if (tid == 0) {
+    const long long now = wall_clock64();
+    if (unfinished) {
+      st[2] = 5;
+      if (!resume) *(long long *)(st + 8) = now;
+    } else if (resume) {
+      st[2] = 0;
+      st[3] = st[1];
+      *(long long *)(st + 4) = c.total[0];
+      *(long long *)(st + 10) = now - *(const long long *)(st + 8);
+      *(long long *)(st + 8) = now;
+    }
+  }
+  if (unfinished) return;
+  for (int i = tid; i < n; i += gridDim.x * blockDim.x) hmat[i] = 1;
 }
 
-void launch_sweep_resume(const SweepCtl &c, hipStream_t st) {
-  k_sweep_resume<<<1, 1, 0, st>>>(c);
+void launch_relabel_end(const SweepCtl &c, unsigned char *hmat, int n, const int *quit, bool resume,
+                        hipStream_t st) {
+  k_relabel_end<<<grid_for(n, 256, 1024), 256, 0, st>>>(c, hmat, n, quit, resume);
 }
 
 void launch_compact(const int *src, int n, int reverse, unsigned char *flag,
