@@ -131,6 +131,7 @@ constexpr size_t kResFixed = kTotals + (kSweepState + 4) / 2;
 
 // Sweeps whose stop words can be in flight at once (pinned words and events).
 constexpr int kStopRing = 8;
+constexpr int kQuitWord = kStopRing + 4;
 
 // algorithmic HBM bytes per node of one push-relabel visit: read and write
 // e, h and K residual planes (int32)
@@ -193,7 +194,7 @@ struct jfc_graph {
     int tag = 1;           // of the last relabel
     int seq = 0;           // passes run, the number their posted words carry
     int *d_marks = nullptr;  // words of a one-launch relabel
-    size_t mark_words() const { return (size_t)kRelabelLine * (2 * kRelabelSlots + n); }
+    size_t mark_words() const { return (size_t)kSettleLine * (2 * kSettleSlots + n); }
     // idle wait of a one-launch search before it leaves the rest to passes:
     // far above the ~50 us of a visit, below what a caller would notice
     long long wait_ticks = 2000000;  // 20 ms
@@ -244,8 +245,8 @@ struct jfc_graph {
   // Pinned copy of d_res (the solve's results).
   long long *pin_res = nullptr;
   // Stop words the sweeps post (k_sweep_end), then the words of two groups
-  // of relabel passes and of a setter's range check, in fine-grained pinned
-  // memory the device writes through to; d_ring is its device address.
+  // of search passes, of a setter's range check, and of a flood that gave up
+  // waiting, in fine-grained pinned memory the device writes through to; d_ring is its device address.
   int *ring = nullptr, *d_ring = nullptr;
   hipEvent_t cnt_ev[2] = {nullptr, nullptr};
   hipEvent_t stop_ev[kStopRing] = {};
@@ -264,7 +265,7 @@ struct jfc_graph {
     if (hipHostMalloc((void **)&pin, sizeof(HostPin), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void **)&pin_res, res_words * sizeof(long long), hipHostMallocDefault) !=
             hipSuccess ||
-        hipHostMalloc((void **)&ring, (kStopRing + 4) * sizeof(int), hipHostMallocCoherent) !=
+        hipHostMalloc((void **)&ring, (kStopRing + 5) * sizeof(int), hipHostMallocCoherent) !=
             hipSuccess ||
         hipHostGetDevicePointer((void **)&d_ring, ring, 0) != hipSuccess) {
       (void)hipGetLastError();
@@ -1125,26 +1126,73 @@ struct Solver {
     f.add(g->rg.d_any, 4, 0, 4);
   }
 
+  // Every region marked for the first of the passes that finish a search.
+  void mark_all_regions() {
+    FillSet f;
+    region_fills(f);
+    f.seg[0].v = 1;
+    f.seg[2].v = 1;
+    launch_fill_multi(f, st);
+  }
+
   // A cut or tag flood over the regions (jfc_flood.hip).  fills: zeroing of the
-  // caller's, done in the same launch.
+  // caller's, done in the same launch.  Where one launch takes every pass the
+  // stream has to be waited for and finish_flood() asked afterwards.
   int flood(bool tag, bool stop, FillSet fills, int *passes) {
     auto &rg = g->rg;
     const bool d3 = g->dim == 3;
     region_fills(fills);
     fills.add(rg.d_out, 2LL * rg.n * flood_out_words(d3), 0, 4);
+    fills.add(rg.d_marks, (long long)rg.mark_words(), 0, 4);
+    if (int rc = g->ensure_pin()) return rc;
+    g->ring[kQuitWord] = 0;
     launch_fill_multi(fills, st);
-    const Tiles T = g->region_tiles();
+    FloodPass A = flood_pass(stop);
     Planes P = g->planes();
     if (tag) P.lab = g->tag;
-    const FloodBuf R{rg.buf.packed, rg.d_out, rg.d_open, rg.buf.planes};
+    if (launch_flood_all(d3, tag, g->region_tiles(), P, flood_buf(), A, st)) {
+      ++*passes;
+      return JFC_OK;
+    }
+    return flood_passes(tag, A, passes, false);
+  }
+
+  // After a wait for the flood: one that gave up waiting is finished by passes
+  // over its packed regions (true in *again), to be waited for once more.
+  int finish_flood(bool tag, bool stop, int *passes, bool *again) {
+    *again = *(const volatile int *)(g->ring + kQuitWord) != 0;
+    if (!*again) return JFC_OK;
+    g->ring[kQuitWord] = 0;
+    mark_all_regions();
+    return flood_passes(tag, flood_pass(stop), passes, true);
+  }
+
+  FloodBuf flood_buf() const {
+    auto &rg = g->rg;
+    return FloodBuf{rg.buf.packed, rg.d_out, rg.d_open, rg.buf.planes};
+  }
+
+  FloodPass flood_pass(bool stop) const {
     FloodPass A{};
+    A.w = settle_words();
+    A.w.quit_host = g->d_ring + kQuitWord;
+    A.c.visits = g->d_total + kFloodSlots;
     A.cert = g->d_flagword;
     A.stop = stop;
     A.def = g->inst.size() == 1 ? g->d_total + kDefSlots : g->d_def;
     A.object = g->lab;
-    return region_passes(kFloodSlots, passes, false, [&](int kind, const PassCtl &c) {
+    return A;
+  }
+
+  int flood_passes(bool tag, FloodPass A, int *passes, bool packed) {
+    A.w.sums = nullptr;
+    const Tiles T = g->region_tiles();
+    const FloodBuf R = flood_buf();
+    Planes P = g->planes();
+    if (tag) P.lab = g->tag;
+    return region_passes(kFloodSlots, passes, packed, [&](int kind, const PassCtl &c) {
       A.c = c;
-      launch_flood(d3, tag, T, P, R, A, kind, 2 * g->nwg, st);
+      launch_flood(g->dim == 3, tag, T, P, R, A, kind, 2 * g->nwg, st);
     });
   }
 
@@ -1172,7 +1220,7 @@ struct Solver {
     RegionPass A = relabel_pass();
     if (launch_relabel(g->dim == 3, g->region_tiles(), g->planes(), rg.buf, A, st)) {
       s.relabel_passes++;
-      relabelled(A.quit, resume);
+      relabelled(A.w.quit, resume);
     } else {
       if (int rc = relabel_passes(A, false)) return rc;
       relabelled(nullptr, resume);
@@ -1182,11 +1230,7 @@ struct Solver {
 
   // The relabel whose waves gave up waiting, by passes over its packed regions.
   int finish_relabel() {
-    FillSet f;
-    region_fills(f);
-    f.seg[0].v = 1;  // every region marked for the first pass
-    f.seg[2].v = 1;
-    launch_fill_multi(f, st);
+    mark_all_regions();
     if (int rc = relabel_passes(relabel_pass(), true)) return rc;
     gr_ev.pop_back();
     s.global_relabels--;
@@ -1195,6 +1239,17 @@ struct Solver {
   }
 
   hipEvent_t relabel_start = nullptr;
+
+  SettleWords settle_words() const {
+    SettleWords w;
+    w.sums = g->rg.d_marks;
+    w.state = w.sums + kSettleLine * kSettleSlots;
+    w.marks = w.state + kSettleLine * kSettleSlots;
+    w.quit = w.state + 1;
+    w.quit_host = nullptr;
+    w.wait_ticks = g->rg.wait_ticks;
+    return w;
+  }
 
   RegionPass relabel_pass() const {
     auto &rg = g->rg;
@@ -1206,17 +1261,13 @@ struct Solver {
     A.pinst = g->d_inst;
     A.pone = g->inst[0];
     A.pdims = __builtin_ctz(tw) | __builtin_ctz(th) << 4 | __builtin_ctz(td) << 8;
-    A.sums = rg.d_marks;
-    A.state = A.sums + kRelabelLine * kRelabelSlots;
-    A.marks = A.state + kRelabelLine * kRelabelSlots;
-    A.wait_ticks = rg.wait_ticks;
-    A.quit = A.state + 1;
+    A.w = settle_words();
     A.c.visits = g->d_total + kRegionSlots;
     return A;
   }
 
   int relabel_passes(RegionPass A, bool packed) {
-    A.sums = nullptr;
+    A.w.sums = nullptr;
     const Tiles T = g->region_tiles();
     const Planes P = g->planes();
     return region_passes(kRegionSlots, &s.relabel_passes, packed, [&](int kind, const PassCtl &c) {
@@ -1248,12 +1299,15 @@ struct Solver {
     f.add(g->d_def, 2LL * (long long)g->inst.size(), 0, 4);
     f.add(g->d_total + kDefSlots, 2 * 64, 0, 4);
     if (int rc = flood(false, stop, f, &s.cut_passes)) return rc;
-    last_cut_end = tm.mark();
+    for (bool again = true; again;) {
+      last_cut_end = tm.mark();
+      JFC_HIP(hipMemcpyAsync(g->pin_res, g->d_res, g->res_words * sizeof(long long),
+                             hipMemcpyDeviceToHost, st));
+      JFC_HIP(hipEventRecord(g->cnt_ev[0], st));
+      JFC_HIP(hipEventSynchronize(g->cnt_ev[0]));
+      if (int rc = finish_flood(false, stop, &s.cut_passes, &again)) return rc;
+    }
     cut_ev.push_back({a, last_cut_end});
-    JFC_HIP(hipMemcpyAsync(g->pin_res, g->d_res, g->res_words * sizeof(long long),
-                           hipMemcpyDeviceToHost, st));
-    JFC_HIP(hipEventRecord(g->cnt_ev[0], st));
-    JFC_HIP(hipEventSynchronize(g->cnt_ev[0]));
     *found = *((const int *)g->pin_res + ((const int *)g->d_flagword - (const int *)g->d_res));
     return JFC_OK;
   }
@@ -1617,8 +1671,12 @@ extern "C" int jfc_get_tags(jfc_graph *g, int inst, const uint8_t *fg, uint8_t *
   S.tm.st = g->ustream;
   int passes = 0;
   if ((rc = S.flood(true, false, FillSet{}, &passes))) return rc;
-  if ((rc = get_rows(g, g->inst[inst], tags, g->tag + o, 1, on_device))) return rc;
-  return sync_user(g);
+  for (bool again = true; again;) {
+    if ((rc = get_rows(g, g->inst[inst], tags, g->tag + o, 1, on_device))) return rc;
+    if ((rc = sync_user(g))) return rc;
+    if ((rc = S.finish_flood(true, false, &passes, &again))) return rc;
+  }
+  return JFC_OK;
 }
 
 extern "C" int jfc_get_energy(jfc_graph *g, int inst, int64_t *energy) {

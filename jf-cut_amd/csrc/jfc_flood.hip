@@ -19,6 +19,8 @@
 //             deficit) packed; regions holding one are flooded;
 //   kBorders  the regions sent new labels: flooded from them;
 //   kFinal    every region, once no region is sent any: the labels written.
+// One launch takes every pass of graphs of up to 512 regions, and the passes
+// between the first and the last of the others (k_flood_all).
 // A region's arcs are packed when a label first reaches it, so regions off
 // the source side read their excess and nothing else.  Once *cert is set the
 // labels of a search that only proves the cut (FloodPass::stop) are not
@@ -59,7 +61,7 @@ __device__ __forceinline__ void send(u64 *p, u64 v) {
 // and its labels, 64 / W rows each; the flood is the first wave's alone.
 template <bool D3, bool TAG, int PASS, bool ONE, int W>
 __device__ __forceinline__ void flood_visit(const Tiles &T, const Planes &P, const FloodBuf &R,
-                                            const FloodPass &A, int t, bool &marked) {
+                                            const FloodPass &A, int t, Marks &marks) {
   constexpr int KM = D3 ? 6 : TAG ? 4 : 8;
   const int lane = threadIdx.x & 63;
   const int wv0 = W > 1 ? 64 / W * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;  // first row
@@ -269,17 +271,14 @@ __device__ __forceinline__ void flood_visit(const Tiles &T, const Planes &P, con
     if (!__ballot(F != 0)) break;
   }
   ps[64] = S;
-  if (!TAG && __ballot((S & D) != 0) && lane == 0) *A.cert = 1;
+  if (!TAG && __ballot((S & D) != 0)) {
+    marks.found = true;
+    if (lane == 0) *A.cert = 1;
+  }
 
   // ---- what the region sends, and the marks of the neighbours sent more
   u64 lw = __ballot((S & M[1] & 1) != 0), rw = __ballot((S & M[0]) >> 63 != 0);
-  bool any = false;
-  auto mark = [&](bool have, bool changed, int nb) {
-    if (have && changed) {
-      any = true;
-      if (lane == 0) A.c.dirty_out[t + nb] = 1;
-    }
-  };
+  marks.at = t + neighbour_step<D3>(r, lane);
   if constexpr (D3) {
     const u64 vy = S & ey & ~owny, vz = S & ez & ~ownz;
     const u64 vx = (lane == 0 ? lw : lane == 1 ? rw : 0) & ~own;
@@ -288,12 +287,12 @@ __device__ __forceinline__ void flood_visit(const Tiles &T, const Planes &P, con
     if (vz) send(R.out + o0 + iz, ownz | vz);
     const u64 cx = __ballot(vx != 0), cy = __ballot(vy != 0), cz = __ballot(vz != 0);
     constexpr u64 low_y = 0x0101010101010101ull;
-    mark(r.hasl, cx & 1, -1);
-    mark(r.hasr, cx & 2, 1);
-    mark(r.hasd, cy & low_y, -r.sy);
-    mark(r.hasu, cy & ~low_y, r.sy);
-    mark(r.hasf, cz & 0xffull, -r.sz);
-    mark(r.hasb, cz & ~0xffull, r.sz);
+    marks.add(0, r.hasl && (cx & 1));
+    marks.add(1, r.hasr && (cx & 2));
+    marks.add(2, r.hasd && (cy & low_y));
+    marks.add(3, r.hasu && (cy & ~low_y));
+    marks.add(4, r.hasf && (cz & 0xffull));
+    marks.add(5, r.hasb && (cz & ~0xffull));
   } else {
     u64 bw = S & M[2], tw = S & M[3], corners = 0;
     if constexpr (!TAG) {
@@ -314,16 +313,15 @@ __device__ __forceinline__ void flood_visit(const Tiles &T, const Planes &P, con
     if (v) send(R.out + o0 + lane, own | v);
     const u64 ch = __ballot(v != 0);
     const u64 cc = row_word(v, 4);
-    mark(r.hasl, ch & 1, -1);
-    mark(r.hasr, ch & 2, 1);
-    mark(r.hasd, ch & 4, -r.sy);
-    mark(r.hasu, ch & 8, r.sy);
-    mark(r.hasl && r.hasd, cc & 1, -1 - r.sy);
-    mark(r.hasl && r.hasu, cc & 2, -1 + r.sy);
-    mark(r.hasr && r.hasd, cc & 4, 1 - r.sy);
-    mark(r.hasr && r.hasu, cc & 8, 1 + r.sy);
+    marks.add(0, r.hasl && (ch & 1));
+    marks.add(1, r.hasr && (ch & 2));
+    marks.add(2, r.hasd && (ch & 4));
+    marks.add(3, r.hasu && (ch & 8));
+    marks.add(4, r.hasl && r.hasd && (cc & 1));
+    marks.add(5, r.hasl && r.hasu && (cc & 2));
+    marks.add(6, r.hasr && r.hasd && (cc & 4));
+    marks.add(7, r.hasr && r.hasu && (cc & 8));
   }
-  marked |= any;
 }
 
 template <bool D3, bool TAG, int PASS, bool ONE, int W>
@@ -331,6 +329,10 @@ __global__ __launch_bounds__(64 * W) void k_flood(Tiles T, Planes P, FloodBuf R,
   const int lane = threadIdx.x & 63;
   bool marked = false;
   const bool found = !TAG && PASS != kPack && A.stop && *A.cert;
+  auto mark = [&](const Marks &marks) {
+    if (marks.on(lane)) A.c.dirty_out[marks.at] = 1;
+    marked |= marks.set != 0;
+  };
   if (PASS == kBorders) {
     // some region was marked for this pass; the host learns it from here
     const bool work = *A.c.any_in && !found;
@@ -353,15 +355,60 @@ __global__ __launch_bounds__(64 * W) void k_flood(Tiles T, Planes P, FloodBuf R,
       while (m) {
         const int i = __builtin_ctzll(m);
         m &= m - 1;
-        flood_visit<D3, TAG, PASS, ONE, 1>(T, P, R, A, base + i * G, marked);
+        Marks marks;
+        flood_visit<D3, TAG, PASS, ONE, 1>(T, P, R, A, base + i * G, marks);
+        mark(marks);
       }
     }
     if (visits && lane == 0) atomicAdd((u64 *)&A.c.visits[blockIdx.x & 63], (u64)visits);
   } else {
-    if (found) return;
-    flood_visit<D3, TAG, PASS, ONE, W>(T, P, R, A, blockIdx.x, marked);
+    if (found || (PASS == kFinal && A.w.sums && shared_word(A.w.state) != kDone)) return;
+    Marks marks;
+    flood_visit<D3, TAG, PASS, ONE, W>(T, P, R, A, blockIdx.x, marks);
+    if (PASS == kPack && A.w.sums) {
+      if (threadIdx.x < 64) publish(A.w, marks, 0, lane);
+      return;
+    }
+    mark(marks);
   }
   if (PASS != kFinal && marked && lane == 0) *A.c.any_out = 1;
+}
+
+// The passes between kPack and kFinal in one launch (settle); W = 4 (one region
+// per workgroup): kPack and kFinal too.  A search that only proves the cut ends
+// for every wave with the first labelled deficit.  Launches, gaps and the
+// host's checks of the passes cost small graphs more than the visits: solves of
+// 512x512 0.57 -> 0.54 ms, 600x450 with tags 1.08 -> 1.01, 96x80 0.69 -> 0.64,
+// 181x217x181 with tags 2.64 -> 2.53; 15000x10000 4.43 -> 4.40.
+template <bool D3, bool TAG, bool ONE, int W>
+__global__ __launch_bounds__(64 * W) void k_flood_all(Tiles T, Planes P, FloodBuf R, FloodPass A) {
+  __shared__ int s_done;
+  constexpr bool kAll = W > 1;
+  const int lane = threadIdx.x & 63;
+  if (!kAll && !TAG && A.stop && *A.cert) return;  // found while packing
+  bool done = false, found = false;
+  if (kAll) {
+    Marks marks;
+    flood_visit<D3, TAG, kPack, ONE, W>(T, P, R, A, blockIdx.x, marks);
+    if (threadIdx.x < 64) {
+      publish(A.w, marks, 1, lane);
+      found = !TAG && A.stop && marks.found;
+      if (found) tell(A.w, kStop, lane);
+    }
+  }
+  if (threadIdx.x < 64 && !found)
+    done = settle(A.w, T.ntiles, kAll, A.c.visits, [&](int t, int served) {
+      Marks marks;
+      flood_visit<D3, TAG, kBorders, ONE, 1>(T, P, R, A, t, marks);
+      publish(A.w, marks, served, lane);
+      return !TAG && A.stop && marks.found;
+    });
+  if constexpr (!kAll) return;
+  if (threadIdx.x == 0) s_done = done;
+  __syncthreads();
+  if (!s_done) return;
+  Marks marks;
+  flood_visit<D3, TAG, kFinal, ONE, W>(T, P, R, A, blockIdx.x, marks);
 }
 
 template <bool D3, bool TAG, bool ONE>
@@ -378,6 +425,30 @@ void launch(const Tiles &T, const Planes &P, const FloodBuf &R, const FloodPass 
     if (shared) k_flood<D3, TAG, kFinal, ONE, 4><<<n, 256, 0, st>>>(T, P, R, A);
     else k_flood<D3, TAG, kFinal, ONE, 1><<<n, 64, 0, st>>>(T, P, R, A);
   }
+}
+
+// A workgroup of k_flood_all looks after at most 64 regions (W = 4: after one).
+template <bool D3, bool TAG, bool ONE>
+bool launch_all(const Tiles &T, const Planes &P, const FloodBuf &R, const FloodPass &A,
+                hipStream_t st) {
+  const int n = T.ntiles;
+  if (n <= kSharedRegions && resident_grid_b<&k_flood_all<D3, TAG, ONE, 4>, 256>(n) == n) {
+    k_flood_all<D3, TAG, ONE, 4><<<n, 256, 0, st>>>(T, P, R, A);
+    return true;
+  }
+  const int grid = resident_grid_b<&k_flood_all<D3, TAG, ONE, 1>, 64>(n);
+  if (64LL * grid < n) return false;
+  launch<D3, TAG, ONE>(T, P, R, A, kPack, 0, st);
+  k_flood_all<D3, TAG, ONE, 1><<<grid, 64, 0, st>>>(T, P, R, A);
+  launch<D3, TAG, ONE>(T, P, R, A, kFinal, 0, st);
+  return true;
+}
+
+template <bool D3, bool TAG>
+bool launch_all(const Tiles &T, const Planes &P, const FloodBuf &R, const FloodPass &A,
+                hipStream_t st) {
+  return T.ninst == 1 ? launch_all<D3, TAG, true>(T, P, R, A, st)
+                      : launch_all<D3, TAG, false>(T, P, R, A, st);
 }
 
 template <bool D3, bool TAG>
@@ -400,6 +471,12 @@ void launch_flood(bool d3, bool tag, const Tiles &T, const Planes &P, const Floo
     if (tag) launch<false, true>(T, P, R, A, pass, nwg, st);
     else launch<false, false>(T, P, R, A, pass, nwg, st);
   }
+}
+
+bool launch_flood_all(bool d3, bool tag, const Tiles &T, const Planes &P, const FloodBuf &R,
+                      const FloodPass &A, hipStream_t st) {
+  if (d3) return tag ? launch_all<true, true>(T, P, R, A, st) : launch_all<true, false>(T, P, R, A, st);
+  return tag ? launch_all<false, true>(T, P, R, A, st) : launch_all<false, false>(T, P, R, A, st);
 }
 
 }  // namespace jfc

@@ -242,7 +242,17 @@ struct PassCtl {
   int seq;
   long long *visits;                  // 64 counters of kBorders visits
 };
-constexpr int kRelabelSlots = 64, kRelabelLine = 32;
+// A search in one launch (settle): the words its waves share, zeroed by the
+// caller, kSettleLine ints apart.
+constexpr int kSettleSlots = 64, kSettleLine = 32;
+struct SettleWords {
+  int *sums = nullptr;   // kSettleSlots pairs: marks served, marks made
+  int *state;            // kSettleSlots
+  int *marks;            // per region: marks made so far
+  int *quit;             // set when it gave up waiting
+  int *quit_host;        // (or null) pinned word set then, too
+  long long wait_ticks;  // idle wait before it gives up (100 MHz clock)
+};
 struct RegionPass {
   PassCtl c;
   int tag;                            // of this relabel, 1 or 2, alternating
@@ -250,13 +260,7 @@ struct RegionPass {
   const InstDesc *pinst;              // push tiling
   InstDesc pone;                      // its instance 0
   int pdims;                          // push tile dimensions, log2 (x | y << 4 | z << 8)
-  // launch_relabel (else null); all zeroed by the caller, words kRelabelLine
-  // ints apart
-  int *sums;             // kRelabelSlots pairs: marks served, marks made
-  int *state;            // kRelabelSlots
-  int *marks;            // per region: marks made so far
-  int *quit;             // set when it gave up waiting
-  long long wait_ticks;  // idle wait before it gives up (100 MHz clock)
+  SettleWords w;                      // launch_relabel (else w.sums null)
 };
 // Cut and tag floods on the same regions (jfc_flood.hip).
 struct FloodBuf {
@@ -268,6 +272,7 @@ struct FloodBuf {
 };
 struct FloodPass {
   PassCtl c;
+  SettleWords w;         // launch_flood_all (else w.sums null)
   int *cert;             // cut: set when a labelled node has a deficit
   bool stop;             // cut: end the search once *cert is set
   long long *def;        // cut: remaining deficit, per instance, or (one
@@ -276,9 +281,13 @@ struct FloodPass {
                                 // foreground seeds on entry, the tags at the end
 };
 int flood_out_words(bool d3);
+// The whole flood; *A.w.quit becomes 1 if it gave up waiting (every region is
+// packed, no label written).  false: the graph has too many regions for it.
+bool launch_flood_all(bool d3, bool tag, const Tiles &T, const Planes &P, const FloodBuf &R,
+                      const FloodPass &A, hipStream_t st);
 void launch_flood(bool d3, bool tag, const Tiles &T, const Planes &P, const FloodBuf &R,
                   const FloodPass &A, int pass, int nwg, hipStream_t st);
-// The whole relabel; *A.quit becomes 1 if it gave up waiting (every region is
+// The whole relabel; *A.w.quit becomes 1 if it gave up waiting (every region is
 // packed, no height written).  false: the graph has too many regions for it.
 bool launch_relabel(bool d3, const Tiles &T, const Planes &P, const RegionBuf &R,
                     const RegionPass &A, hipStream_t st);

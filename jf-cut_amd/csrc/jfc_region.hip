@@ -589,30 +589,7 @@ __device__ __forceinline__ void region_visit(const Tiles &T, const Planes &P,
   }
 }
 
-constexpr int kSlots = kRelabelSlots, kLine = kRelabelLine;
-static_assert(kSlots == 64, "a lane per slot");
-enum { kGo = 0, kDone = 1, kQuit = 2 };
-
-// Counts the marks of a visit that served `served` marks, then makes them
-// (k_settle).
-__device__ __forceinline__ void publish(const RegionPass &A, const Marks &marks, int served,
-                                        int lane) {
-  if (lane == 0)
-    (void)__hip_atomic_fetch_add((u64 *)(A.sums + kLine * (blockIdx.x & (kSlots - 1))),
-                                 (u64)__popc(marks.set) << 32 | (unsigned)served,
-                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (marks.set) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (marks.on(lane))
-      (void)__hip_atomic_fetch_add(A.marks + kLine * (long long)marks.at, 1, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-  }
-}
-__device__ __forceinline__ int shared_word(const int *p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// One pass.  With A.sums, kPack and kFinal are the first and last step around
+// One pass.  With A.w.sums, kPack and kFinal are the first and last step around
 // k_settle: kPack counts its marks for it, kFinal runs if it finished.
 template <bool D3, int PASS, bool ONE, int W>
 __global__ __launch_bounds__(64 * W) void k_region(Tiles T, Planes P, RegionBuf R, RegionPass A) {
@@ -622,14 +599,14 @@ __global__ __launch_bounds__(64 * W) void k_region(Tiles T, Planes P, RegionBuf 
   auto visit = [&](int t, auto w) {
     Marks marks;
     region_visit<D3, PASS, ONE, decltype(w)::value>(T, P, R, A, t, inj, marks);
-    if (PASS == kPack && A.sums) {
-      if (threadIdx.x < 64) publish(A, marks, 0, lane);
+    if (PASS == kPack && A.w.sums) {
+      if (threadIdx.x < 64) publish(A.w, marks, 0, lane);
       return;
     }
     if (marks.on(lane)) A.c.dirty_out[marks.at] = 1;
     marked |= marks.set != 0;
   };
-  if (PASS == kFinal && A.sums && shared_word(A.state) != kDone) return;
+  if (PASS == kFinal && A.w.sums && shared_word(A.w.state) != kDone) return;
   if (PASS == kBorders) {
     // some region was marked for this pass; the host learns it from here
     const int work = *A.c.any_in;
@@ -669,46 +646,17 @@ __global__ __launch_bounds__(64 * W) void k_region(Tiles T, Planes P, RegionBuf 
   if (PASS != kFinal && marked && threadIdx.x == 0) *A.c.any_out = 1;
 }
 
-// The passes between kPack and kFinal in one launch.  A wave owns the regions
-// t = blockIdx.x + i gridDim.x and visits those its neighbours mark until no
-// mark is left anywhere.  W = 4 (one region per workgroup): kPack and kFinal
-// too, whose rows the workgroup's other waves share.
-//
-// Marks are counts: a wave that changed a border adds 1 to the neighbour's
-// count, the owner remembers the count it has served.  Each wave's marks made
-// (high half) and marks served (low half) are summed in one of kSlots words; a
-// visit adds the marks it is about to make, with those it served, before it
-// makes them.   The first
-// workgroup, when idle, reads every word for the marks served and then again
-// for the marks made: equal sums mean that nothing was left to do between the
-// two readings, and nothing will be (a mark is only made while one is being
-// served).  It then tells the others through kSlots words of their own.  Every
-// polled word has a cache line to itself: one word for all took 1.9 ms for a
-// relabel of the 3750x2500 cut, its polling waves holding back the visits.
-// The border words and the sums are written through at device scope and have
-// arrived (s_waitcnt) before a mark is made, and the owner reads them at device
-// scope after it has seen the mark; a region's planes are touched by its owner
-// only.
-//
-// Every workgroup is resident on an idle device (the launcher caps the grid),
-// but other kernels may hold their places back, so the wait is bounded: a wave
-// idle for A.wait_ticks tells the others to quit and posts it to the host, which
-// then finishes with passes over every region.
-//
-// A pass costs its slowest visit, its launch and, every few passes, the host's
-// check; here a front moves on as soon as one region is searched.
+// The passes between kPack and kFinal in one launch (settle).  W = 4 (one
+// region per workgroup): kPack and kFinal too, whose rows the workgroup's other
+// waves share.  A pass costs its slowest visit, its launch and, every few
+// passes, the host's check; here a front moves on as soon as one region is
+// searched.
 template <bool D3, bool ONE, int W>
 __global__ __launch_bounds__(64 * W) void k_settle(Tiles T, Planes P, RegionBuf R, RegionPass A) {
   __shared__ __attribute__((aligned(8))) unsigned inj[kBlock * kWinPitch];
   __shared__ int s_done;
   constexpr bool kAll = W > 1;
   const int lane = threadIdx.x & 63;
-  const int slot = blockIdx.x & (kSlots - 1);
-  const int G = gridDim.x;
-  // the state every workgroup waits for: kGo, kDone or kQuit, a word per slot
-  auto tell = [&](int what) {
-    __hip_atomic_store(A.state + kLine * lane, what, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
   if (threadIdx.x < 64) {
     for (int l = 0; l < kBlock; ++l) *(u64 *)&inj[l * kWinPitch + 2 * lane] = 0;
     lds_order();
@@ -717,60 +665,16 @@ __global__ __launch_bounds__(64 * W) void k_settle(Tiles T, Planes P, RegionBuf 
     Marks marks;
     region_visit<D3, kPack, ONE, W>(T, P, R, A, blockIdx.x, inj, marks);
     // served: the packing, which counts as a mark made before the launch
-    if (threadIdx.x < 64) publish(A, marks, 1, lane);
+    if (threadIdx.x < 64) publish(A.w, marks, 1, lane);
   }
   bool done = false;
-  if (threadIdx.x < 64) {
-    const int mine = blockIdx.x + lane * G;  // the lane's region of up to 64
-    const bool own = mine < T.ntiles;
-    int seen = 0, visits = 0, turn = 0;
-    long long since = 0;
-    for (;;) {
-      const int now = own ? shared_word(A.marks + kLine * (long long)mine) : 0;
-      const int state = shared_word(A.state + kLine * slot);
-      u64 m = __ballot(now != seen);
-      if (m) {
-        since = 0;
-        // one region per poll, in turn: marks made meanwhile for the others are
-        // served by one visit each
-        const u64 ahead = m & (~0ull << turn);
-        const int i = __builtin_ctzll(ahead ? ahead : m);
-        turn = (i + 1) & 63;
-        const int served = __builtin_amdgcn_readlane(now - seen, i);
-        if (lane == i) seen = now;
-        Marks marks;
-        region_visit<D3, kBorders, ONE, 1>(T, P, R, A, blockIdx.x + i * G, inj, marks);
-        publish(A, marks, served, lane);
-        ++visits;
-        continue;
-      }
-      done = state == kDone;
-      if (state != kGo) break;
-      if (blockIdx.x == 0) {
-        auto sum = [&](int half) {
-          int v = shared_word(A.sums + kLine * lane + half);
-          for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-          return v;
-        };
-        const int served = sum(0);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        if (sum(1) + (kAll ? T.ntiles : 0) == served) {
-          tell(kDone);
-          continue;
-        }
-      }
-      const long long tick = wall_clock64();
-      if (since == 0) since = tick;
-      if (tick - since >= A.wait_ticks) {
-        tell(kQuit);
-        if (lane == 0)
-          __hip_atomic_store(A.quit, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        break;
-      }
-      __builtin_amdgcn_s_sleep(8);
-    }
-    if (visits && lane == 0) atomicAdd((u64 *)&A.c.visits[blockIdx.x & 63], (u64)visits);
-  }
+  if (threadIdx.x < 64)
+    done = settle(A.w, T.ntiles, kAll, A.c.visits, [&](int t, int served) {
+      Marks marks;
+      region_visit<D3, kBorders, ONE, 1>(T, P, R, A, t, inj, marks);
+      publish(A.w, marks, served, lane);
+      return false;
+    });
   if constexpr (!kAll) return;
   if (threadIdx.x == 0) s_done = done;
   __syncthreads();

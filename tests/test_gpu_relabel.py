@@ -97,3 +97,25 @@ def test_relabel_gives_up_waiting_gpu(gpu, conn, shape):
         assert g.flow() == f
         assert np.array_equal(g.labels(), l)
     g.close()
+
+
+@pytest.mark.parametrize("conn,shape", [(8, (300, 217, 1)), (4, (2100, 1100, 1)), (6, (70, 41, 33)),
+                                        (6, (300, 190, 70))])
+def test_tag_gives_up_waiting_gpu(gpu, conn, shape):
+    """A tag flood whose waves give up waiting at once is finished by passes:
+    one launch for everything (up to 512 regions) and above."""
+    import ctypes
+    nx, ny, nz = shape
+    rng = np.random.default_rng(ny)
+    cs, ct, caps = random_grid(rng, nx, ny, nz, conn, term_max=20, seed_frac=0.001)
+    g, st = solve_grid(gpu, nx, ny, nz, conn, cs, ct, caps)
+    assert st.converged == 1
+    lab = g.labels()
+    fg = (rng.random(nx * ny * nz) < 0.001).astype(np.uint8)
+    fg[0] = 1
+    want = ol.tag(nx, ny, nz, fg, lab)
+    for ticks in (0, 1 << 22, 0):
+        say("case tag wait", conn, shape, ticks)
+        assert gpu.lib().jfc_debug_relabel_wait(g._h, ctypes.c_int64(ticks)) == 0
+        assert np.array_equal(g.tags(fg), want)
+    g.close()
