@@ -344,6 +344,16 @@ struct jfc_graph {
                  inst.empty() ? InstDesc{} : inst[0]};
   }
   Planes planes() const { return Planes{e, h, cap, c0, cs, ct, lab, Ntot, rmask}; }
+  int max_nx() const {
+    int m = 1;
+    for (const InstDesc &I : inst) m = std::max(m, I.nx);
+    return m;
+  }
+  int first_row(int i) const {
+    int r = 0;
+    for (int k = 0; k < i; ++k) r += inst[k].ny * inst[k].nz;
+    return r;
+  }
   long long inst_nodes(int i) const {
     return (long long)inst[i].nx * inst[i].ny * inst[i].nz;
   }
@@ -1916,7 +1926,7 @@ extern "C" int jfc_backward_all(jfc_graph *g, float *d_cap_source, float *d_cap_
   const long long n = g->Nuser;
   hipStream_t st = g->ustream;
   if (on_device) {
-    launch_backward_all(g->shape, g->tiles(), g->planes(), d_cap_source, d_cap_sink,
+    launch_backward_all(g->shape, g->tiles(), g->planes(), g->max_nx(), d_cap_source, d_cap_sink,
                         d_neighbor, n, st);
     return sync_user(g);
   }
@@ -1928,7 +1938,7 @@ extern "C" int jfc_backward_all(jfc_graph *g, float *d_cap_source, float *d_cap_
   float *c = d_neighbor ? (float *)tmp + 2 * n : nullptr;
   // planes beyond an instance's connectivity keep the caller's values
   if (c) JFC_HIP(hipMemcpyAsync(c, d_neighbor, n * g->Kg * 4, hipMemcpyHostToDevice, st));
-  launch_backward_all(g->shape, g->tiles(), g->planes(), a, b, c, n, st);
+  launch_backward_all(g->shape, g->tiles(), g->planes(), g->max_nx(), a, b, c, n, st);
   if (a) JFC_HIP(hipMemcpyAsync(d_cap_source, a, n * 4, hipMemcpyDeviceToHost, st));
   if (b) JFC_HIP(hipMemcpyAsync(d_cap_sink, b, n * 4, hipMemcpyDeviceToHost, st));
   if (c) JFC_HIP(hipMemcpyAsync(d_neighbor, c, n * g->Kg * 4, hipMemcpyDeviceToHost, st));
@@ -1957,8 +1967,8 @@ extern "C" int jfc_backward(jfc_graph *g, int inst, float *d_cap_source, float *
   const long long n = g->inst_nodes(inst);
   hipStream_t st = g->ustream;
   if (on_device) {
-    launch_backward(g->shape, g->tiles(), g->planes(), I, d_cap_source, d_cap_sink,
-                    d_neighbor, st);
+    launch_backward(g->shape, g->tiles(), g->planes(), I, g->first_row(inst), d_cap_source,
+                    d_cap_sink, d_neighbor, st);
     return sync_user(g);
   }
   void *tmp = nullptr;
@@ -1966,7 +1976,7 @@ extern "C" int jfc_backward(jfc_graph *g, int inst, float *d_cap_source, float *
   float *a = d_cap_source ? (float *)tmp : nullptr;
   float *b = d_cap_sink ? (float *)tmp + n : nullptr;
   float *c = d_neighbor ? (float *)tmp + 2 * n : nullptr;
-  launch_backward(g->shape, g->tiles(), g->planes(), I, a, b, c, st);
+  launch_backward(g->shape, g->tiles(), g->planes(), I, g->first_row(inst), a, b, c, st);
   if (a) JFC_HIP(hipMemcpyAsync(d_cap_source, a, n * 4, hipMemcpyDeviceToHost, st));
   if (b) JFC_HIP(hipMemcpyAsync(d_cap_sink, b, n * 4, hipMemcpyDeviceToHost, st));
   if (c) JFC_HIP(hipMemcpyAsync(d_neighbor, c, n * I.K * 4, hipMemcpyDeviceToHost, st));

@@ -35,6 +35,14 @@ using S32x4x2 = Shape<32, 4, 2>;
     default: break;                                         \
   }
 
+#define JFC_DISPATCH_2D(shape, BODY)                        \
+  switch (shape) {                                          \
+    case SH_32x8: { using S = S32x8; BODY; } break;         \
+    case SH_64x4: { using S = S64x4; BODY; } break;         \
+    case SH_16x16: { using S = S16x16; BODY; } break;       \
+    default: break;                                         \
+  }
+
 // Direction d -> offset.  2D: +x -x +y -y (+x+y) (-x-y) (-x+y) (+x-y);
 // 3D: +x -x +y -y +z -z.  The reverse of d is d^1.
 template <bool D3>

@@ -299,10 +299,10 @@ void launch_region(bool d3, const Tiles &T, const Planes &P, const RegionBuf &R,
 // energy: one int64 per instance, zeroed by the caller.
 void launch_energy(int shape, const Tiles &T, const Planes &P, long long *energy,
                    hipStream_t st);
-void launch_backward(int shape, const Tiles &T, const Planes &P,
-                     const InstDesc &I, float *dcs, float *dct, float *dnb,
-                     hipStream_t st);
-void launch_backward_all(int shape, const Tiles &T, const Planes &P, float *dcs,
+// row0: the instance's first row.  max_nx: the longest row of the graph.
+void launch_backward(int shape, const Tiles &T, const Planes &P, const InstDesc &I, int row0,
+                     float *dcs, float *dct, float *dnb, hipStream_t st);
+void launch_backward_all(int shape, const Tiles &T, const Planes &P, int max_nx, float *dcs,
                          float *dct, float *dnb, long long user_total, hipStream_t st);
 
 }  // namespace jfc

@@ -471,6 +471,87 @@ __global__ __launch_bounds__(256) void k_fold(Tiles T, Planes P, long long *red,
   sums.flush(dst, stride, buf);
 }
 
+// The fold of a 2D graph of several instances with new masks: a wave takes a
+// tile at a time, 4 nodes per lane, so that every lane has work whatever the
+// instances' row lengths are, and consecutive waves take neighbouring tiles.
+// Bound by its reads and writes.  Row by row, each step a search for the
+// instance and half of the lanes idle on rows of 400, 256 uneven images (171,000
+// tiles) took 708 us; this takes 444.
+constexpr int kFoldTiles = 8;  // tiles per wave
+
+template <class S, int MASKS>
+__global__ __launch_bounds__(256) void k_fold_tiles(Tiles T, Planes P, long long *red,
+                                                    unsigned char *active, unsigned char *defi,
+                                                    int zero_h, unsigned *mask0) {
+  const int lane = threadIdx.x & 63;
+  const int lx = lane % (S::TW / 4) * 4, ly = lane / (S::TW / 4);
+  const int t0 = blockIdx.x * (4 * kFoldTiles) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  long long sum[3] = {0, 0, 0};
+  int cur = -1;
+  auto flush = [&]() {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      for (int o = 32; o > 0; o >>= 1) sum[k] += __shfl_xor(sum[k], o);
+      const int slot = k == 0 ? RED_CONST : k == 1 ? RED_DEF0 : RED_SUP0;
+      if (lane == 0 && sum[k])
+        atomicAdd((unsigned long long *)&red[(long long)cur * RED_SLOTS + slot],
+                  (unsigned long long)sum[k]);
+      sum[k] = 0;
+    }
+  };
+  for (int i = 0; i < kFoldTiles; ++i) {
+    const int t = t0 + 4 * i;
+    if (t >= T.ntiles) break;
+    const int inst = T.tile_inst[t];
+    if (inst != cur) {
+      if (cur >= 0) flush();
+      cur = inst;
+    }
+    const TileRef r = tile_ref_of<S>(T.inst[inst], t);
+    const int K = r.I.K, y = r.oy + ly;
+    // rows start at multiples of 32 nodes, so a lane's 4 nodes are aligned and
+    // its loads past the row's end stay in its padding
+    const int n = y < r.I.ny ? min(4, r.I.nx - (r.ox + lx)) : 0;
+    const bool in = n > 0;
+    const long long v = in ? node_index(r.I, r.ox + lx, y, 0) : 0;
+    const int4 a = *(const int4 *)(P.cs + v), b = *(const int4 *)(P.ct + v);
+    int4 c[S::KMAX];
+#pragma unroll
+    for (int d = 0; d < S::KMAX; ++d)
+      c[d] = d < K ? *(const int4 *)(P.c0 + d * P.stride + v) : make_int4(0, 0, 0, 0);
+    int4 m = make_int4(0, 0, 0, 0);
+#pragma unroll
+    for (int d = 0; d < S::KMAX; ++d) {
+      const int fresh = d < K ? 1 << (8 + d) : 0;
+      m.x |= (c[d].x > 0 ? 1 << d : 0) | fresh; m.y |= (c[d].y > 0 ? 1 << d : 0) | fresh;
+      m.z |= (c[d].z > 0 ? 1 << d : 0) | fresh; m.w |= (c[d].w > 0 ? 1 << d : 0) | fresh;
+    }
+    bool excess = false, deficit = false;
+    if (in) {
+      int4 e;
+      e.x = a.x - b.x; e.y = a.y - b.y; e.z = a.z - b.z; e.w = a.w - b.w;
+      store4(P.e, v, n, e);
+      if (zero_h) store4(P.h, v, n, make_int4(0, 0, 0, 0));
+      store4((int *)P.rmask, v, n, m);
+      if (MASKS == 2) store4((int *)mask0, v, n, m);
+      for (int j = 0; j < n; ++j) {
+        const int s = comp(a, j), u = comp(b, j);
+        sum[0] += min(s, u);
+        sum[1] += max(u - s, 0);
+        sum[2] += max(s - u, 0);
+        excess |= s > u;
+        deficit |= s < u;
+      }
+    }
+    const bool any_excess = __ballot(excess) != 0, any_deficit = __ballot(deficit) != 0;
+    if (lane == 0) {
+      if (active && any_excess) active[t] = 1;
+      if (defi && any_deficit) defi[t] = 1;
+    }
+  }
+  if (cur >= 0) flush();
+}
+
 void launch_fold(int shape, const Tiles &T, const Planes &P, long long *red,
                  unsigned char *active, unsigned char *defi, bool zero_h, unsigned *mask0,
                  int masks, hipStream_t st, bool cleared) {
@@ -480,7 +561,13 @@ void launch_fold(int shape, const Tiles &T, const Planes &P, long long *red,
   }
   const int z = zero_h ? 1 : 0;
   const int n = (T.nrows + T.row_step - 1) / T.row_step;
-  if (masks == 3) {
+  if (masks >= 2 && T.ninst > 1 && !shape_is_3d(shape)) {
+    const int grid = (T.ntiles + 4 * kFoldTiles - 1) / (4 * kFoldTiles);
+    const auto go = [&](auto *kernel) {
+      kernel<<<grid, 256, 0, st>>>(T, P, red, active, defi, z, mask0);
+    };
+    JFC_DISPATCH_2D(shape, go(masks == 3 ? &k_fold_tiles<S, 3> : &k_fold_tiles<S, 2>));
+  } else if (masks == 3) {
     JFC_DISPATCH(shape, (k_fold<S, 3><<<row_grid<&k_fold<S, 3>>(n), 256, 0, st>>>(
                             T, P, red, active, defi, z, mask0)));
   } else if (masks == 2) {
@@ -548,54 +635,129 @@ void launch_energy(int shape, const Tiles &T, const Planes &P, long long *energy
 
 // Subgradient of the cut energy for instance `inst` (outputs in the
 // instance's own node numbering).
-template <class S>
-__global__ __launch_bounds__(256) void k_backward(Tiles T, Planes P, int t_begin,
-                                                  int t_count, float *dcs,
-                                                  float *dct, float *dnb,
-                                                  long long user_total) {
-  const Lane<S> L(threadIdx.x);
-  for (int t = t_begin + blockIdx.x; t < t_begin + t_count; t += gridDim.x) {
-    const TileRef r = tile_ref<S>(T, t);
-    const InstDesc &I = r.I;
-    const int gx = r.ox + L.lx, gy = r.oy + L.ly, gz = r.oz + L.lz;
-    if (!(gx < I.nx && gy < I.ny && gz < I.nz)) continue;
-    const long long v = node_index(I, gx, gy, gz);
+// Bound by its writes, a float per node and output plane.  A wave takes chunks of
+// 256 nodes of consecutive rows, 4 nodes per lane: the callers' rows have no
+// padding, so what a wave writes to a plane is one run that shares only its end
+// lines with the next (rows of 32-node tiles, of which every line was shared,
+// took 807 us for 256 uneven images; this takes 446), and a lane reads the
+// labels around its nodes as words.
+struct alignas(4) Float4 {
+  float v[4];
+};
+
+template <bool D3>
+__global__ __launch_bounds__(256) void k_backward(Tiles T, Planes P, int row0, int nrows,
+                                                  int rows_per_wave, float *dcs, float *dct,
+                                                  float *dnb, long long user_total) {
+  constexpr int KMAX = D3 ? 6 : 8;
+  const int lane = threadIdx.x & 63;
+  const int wave = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int row = row0 + wave * rows_per_wave;
+  const int end = min(row0 + nrows, row + rows_per_wave);
+  if (row >= end) return;
+  int inst = 0;
+  for (int hi = T.ninst - 1; inst < hi;) {
+    const int mid = (inst + hi + 1) >> 1;
+    if (T.row_off[mid] <= row) inst = mid;
+    else hi = mid - 1;
+  }
+  InstDesc I = T.inst[inst];
+  int last = T.row_off[inst + 1], rr = row - T.row_off[inst];
+  int y = rr % I.ny, z = rr / I.ny;
+  for (; row < end; ++row) {
+    if (row == last) {
+      I = T.inst[++inst];
+      last = T.row_off[inst + 1];
+      rr = y = z = 0;
+    }
     // outputs in the callers' numbering: one instance (user_total = 0) its
     // own, with plane stride = its node count; all instances the graph's
     // concatenation, with plane stride = all their nodes
-    const long long own = gx + (long long)I.nx * (gy + (long long)I.ny * gz);
-    const long long lv = user_total ? I.user_off + own : own;
     const long long n = user_total ? user_total : (long long)I.nx * I.ny * I.nz;
-    const bool s = P.lab[v] != 0;
-    if (dcs) dcs[lv] = s ? 0.f : 1.f;
-    if (dct) dct[lv] = s ? 1.f : 0.f;
-    if (dnb) {
+    const long long out0 = (user_total ? I.user_off : 0) + (long long)rr * I.nx;
+    const long long base = I.node_off + (long long)rr * I.px, slice = (long long)I.px * I.ny;
+    for (int x = (blockIdx.y * 64 + lane) * 4; x < I.nx; x += gridDim.y * 256) {
+      // bit i of the labels around the 4 nodes: column x - 1 + i of a row, set
+      // off the grid
+      auto nonzero = [](unsigned w) {
+        w |= w >> 4;
+        w |= w >> 2;
+        w |= w >> 1;
+        return ((w & 0x01010101u) * 0x01020408u) >> 24;
+      };
+      auto around = [&](bool have, long long step, bool wide) {
+        if (!have) return 63u;
+        const unsigned char *p = P.lab + base + step + x;
+        const int left = I.nx - x;  // columns x ... of the row
+        unsigned m = nonzero(*(const unsigned *)p) << 1;
+        if (wide && x > 0) m |= p[-1] ? 1u : 0u;
+        else m |= 1u;
+        if (wide && left > 4) m |= p[4] ? 32u : 0u;
+        else m |= 32u;
+        if (left < 4) m |= 63u << (left + 1) & 63u;
+        return m;
+      };
+      const unsigned own = around(true, 0, true);
+      const unsigned s = own >> 1 & 15u;
+      const int cnt = min(4, I.nx - x);
+      auto put = [&](float *plane, unsigned bits) {
+        float *q = plane + out0 + x;
+        if (cnt == 4) {
+          Float4 f;
 #pragma unroll
-      for (int d = 0; d < S::KMAX; ++d) {
+          for (int i = 0; i < 4; ++i) f.v[i] = (bits >> i) & 1u ? 1.f : 0.f;
+          *(Float4 *)q = f;
+        } else {
+          for (int i = 0; i < cnt; ++i) q[i] = (bits >> i) & 1u ? 1.f : 0.f;
+        }
+      };
+      if (dcs) put(dcs, ~s);
+      if (dct) put(dct, s);
+      if (!dnb) continue;
+      const bool diag = !D3 && I.K > 4;
+      const unsigned up = around(y + 1 < I.ny, I.px, diag), dn = around(y > 0, -I.px, diag);
+      unsigned front = 0, back = 0;
+      if constexpr (D3) {
+        back = around(z + 1 < I.nz, slice, false);
+        front = around(z > 0, -slice, false);
+      }
+#pragma unroll
+      for (int d = 0; d < KMAX; ++d) {
         if (d >= I.K) break;
         int dx, dy, dz;
-        dir_of<S::D3>(d, dx, dy, dz);
-        const int X = gx + dx, Y = gy + dy, Z = gz + dz;
-        float g = 0.f;
-        if (s && X >= 0 && X < I.nx && Y >= 0 && Y < I.ny && Z >= 0 && Z < I.nz)
-          g = P.lab[node_index(I, X, Y, Z)] ? 0.f : 1.f;
-        dnb[d * n + lv] = g;
+        dir_of<D3>(d, dx, dy, dz);
+        const unsigned m = dz > 0 ? back : dz < 0 ? front : dy > 0 ? up : dy < 0 ? dn : own;
+        put(dnb + d * n, s & ~(m >> (1 + dx)));
       }
+    }
+    ++rr;
+    if (++y == I.ny) {
+      y = 0;
+      ++z;
     }
   }
 }
 
-void launch_backward(int shape, const Tiles &T, const Planes &P,
-                     const InstDesc &I, float *dcs, float *dct, float *dnb,
-                     hipStream_t st) {
-  JFC_DISPATCH(shape, (k_backward<S><<<tile_grid(I.ntiles), 256, 0, st>>>(
-                          T, P, I.tile_off, I.ntiles, dcs, dct, dnb, 0)));
+// Rows [row0, row0 + nrows) of the graph; nx: the longest of them.
+static void backward_rows(int shape, const Tiles &T, const Planes &P, int row0, int nrows, int nx,
+                          float *dcs, float *dct, float *dnb, long long user_total,
+                          hipStream_t st) {
+  const int chunks = std::min((nx + 255) / 256, 64);
+  const int per_wave = (int)std::max(1LL, (long long)nrows * chunks / 16384);
+  const dim3 grid((nrows + 4 * per_wave - 1) / (4 * per_wave), chunks);
+  if (shape_is_3d(shape))
+    k_backward<true><<<grid, 256, 0, st>>>(T, P, row0, nrows, per_wave, dcs, dct, dnb, user_total);
+  else
+    k_backward<false><<<grid, 256, 0, st>>>(T, P, row0, nrows, per_wave, dcs, dct, dnb, user_total);
 }
 
-void launch_backward_all(int shape, const Tiles &T, const Planes &P, float *dcs,
+void launch_backward(int shape, const Tiles &T, const Planes &P, const InstDesc &I, int row0,
+                     float *dcs, float *dct, float *dnb, hipStream_t st) {
+  backward_rows(shape, T, P, row0, I.ny * I.nz, I.nx, dcs, dct, dnb, 0, st);
+}
+void launch_backward_all(int shape, const Tiles &T, const Planes &P, int max_nx, float *dcs,
                          float *dct, float *dnb, long long user_total, hipStream_t st) {
-  JFC_DISPATCH(shape, (k_backward<S><<<tile_grid(T.ntiles), 256, 0, st>>>(
-                          T, P, 0, T.ntiles, dcs, dct, dnb, user_total)));
+  backward_rows(shape, T, P, 0, T.nrows, max_nx, dcs, dct, dnb, user_total, st);
 }
 
 // ---- jump flooding over the tile grid + counting sort --------------------------
