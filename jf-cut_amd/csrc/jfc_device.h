@@ -131,41 +131,6 @@ __device__ __forceinline__ void pad_coords(int p, int &x, int &y, int &z,
   interior = nout == 0;
 }
 
-// Halo cell needed by a connectivity: face cells always, 2D corners only for
-// 8-connectivity, 3D edges/corners never.
-template <class S>
-__device__ __forceinline__ bool halo_needed(int nout, int K) {
-  if (nout == 1) return true;
-  return !S::D3 && nout == 2 && K == 8;
-}
-
-// Padded cell p of a tile as seen by one lane: halo (not interior), and
-// live = a halo cell the connectivity needs that lies inside the instance,
-// with its node index (0 otherwise, a valid dummy address for loads).
-struct HaloCell {
-  bool halo, live;
-  long long g;
-};
-
-template <class S>
-__device__ __forceinline__ HaloCell halo_cell(const InstDesc &I, int ox, int oy, int oz,
-                                              int p, int K) {
-  HaloCell c{false, false, 0};
-  if (p >= S::PADN) return c;
-  int x, y, z, nout;
-  bool inter;
-  pad_coords<S>(p, x, y, z, inter, nout);
-  if (inter) return c;
-  c.halo = true;
-  if (!halo_needed<S>(nout, K)) return c;
-  const int X = ox + x, Y = oy + y, Z = oz + z;
-  if (X >= 0 && X < I.nx && Y >= 0 && Y < I.ny && Z >= 0 && Z < I.nz) {
-    c.live = true;
-    c.g = node_index(I, X, Y, Z);
-  }
-  return c;
-}
-
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
 
 // Append `t` (if pred) to a list with one atomic per wave.

@@ -1408,16 +1408,46 @@ constexpr int kRingQ = (Ring<S>::N + 3) / 4;
 template <class S>
 constexpr int kRingPerLane = (kRingQ<S> + 63) / 64;
 
-// A 3D ring cell (a face cell of the padded tile) has one arc into the tile
-// (6-connected arcs cross faces only): its direction from the cell, which is
-// also the one plane of the cell that flow out of the tile changes.
-template <class S>
-__device__ __forceinline__ int inward_dir(int p) {
-  int x, y, z, nout;
-  bool inter;
-  pad_coords<S>(p, x, y, z, inter, nout);
-  return x < 0 ? 0 : x >= S::TW ? 1 : y < 0 ? 2 : y >= S::TH ? 3 : z < 0 ? 4 : 5;
-}
+// A ring cell by its place: the padded cell, its coordinates in the tile and
+// the arcs it has into the tile, which are the planes of the cell that flow
+// out of the tile changes -- one across a face, three from a side of an
+// 8-connected tile (a corner has one of the three).
+template <class S, int KK>
+struct RingCell {
+  static constexpr int ARCS = !S::D3 && KK == 8 ? 3 : 1;
+  int p, xyz;  // padded cell; x, y, z (a byte each), side, corner
+  __device__ __forceinline__ explicit RingCell(int k) {
+    p = Ring<S>::pos(k);
+    int x, y, z, nout;
+    bool inter;
+    pad_coords<S>(p, x, y, z, inter, nout);
+    const int side = x < 0 ? 0 : x >= S::TW ? 1 : y < 0 ? 2 : y >= S::TH ? 3 : z < 0 ? 4 : 5;
+    xyz = (x & 255) | (y & 255) << 8 | (z & 255) << 16 | side << 24 | (nout > 1 ? 1 << 30 : 0);
+  }
+  // The cell as a value of its own: what a phase of the visit derives from it is
+  // computed there, instead of being kept in registers from the launch's start.
+  __device__ __forceinline__ RingCell again() const {
+    RingCell q = *this;
+    asm volatile("" : "+v"(q.p), "+v"(q.xyz));
+    return q;
+  }
+  __device__ __forceinline__ int x() const { return __builtin_amdgcn_sbfe(xyz, 0, 8); }
+  __device__ __forceinline__ int y() const { return __builtin_amdgcn_sbfe(xyz, 8, 8); }
+  __device__ __forceinline__ int z() const { return S::D3 ? __builtin_amdgcn_sbfe(xyz, 16, 8) : 0; }
+  // 0 / 1 left / right side, 2 / 3 low / high y, 4 / 5 low / high z
+  __device__ __forceinline__ int side() const { return xyz >> 24 & 7; }
+  // direction of arc i
+  __device__ __forceinline__ int arc(int i) const {
+    const int q = side();
+    return i == 0 ? q : i == 1 ? 4 + (q & 1) : 0x7667 >> 4 * q & 15;
+  }
+  // the tile it lies in, relative to this one
+  __device__ __forceinline__ int tile_step(const InstDesc &I) const {
+    const int x_ = x(), y_ = y(), z_ = z();
+    return (x_ >= S::TW) - (x_ < 0) +
+           I.tx * ((y_ >= S::TH) - (y_ < 0) + (S::D3 ? I.ty * ((z_ >= S::TD) - (z_ < 0)) : 0));
+  }
+};
 
 // ---- block-wise push-relabel -------------------------------------------------------
 //
@@ -1444,22 +1474,21 @@ template <class S, bool ONE, int KK>
 // registers through an iteration and 4 directions instead of 8 took a
 // 600x450 widget cut from 1.08 to 0.87 ms and a 181x217x181 scan from 2.5 to
 // 2.1; with 8 directions 3750x2500 strokes from 46 to 42.
-// 7 waves per SIMD fit without spills but for 8 directions, where they cost
-// more than the wave gives (15000x10000: 4.00 ms at 7, 3.92 at 6).  Two ring
-// cells per lane (32x4x2, slim flush) fit 96 VGPRs: 5 waves.
-__global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : KK == 8 ? 6 : 7) void k_push(
+// Dense launches visit 121 tiles a microsecond at any shape and K (15000x10000,
+// 256 images, the 2560x1440x50 video), with 20 KB moved per visit at 2.3 TB/s,
+// the VALU busy 38% of the time; 6, 7 or 8 waves per SIMD and plain stores
+// instead of half of the atomics change it by 1%: bound by the scattered 64-byte
+// requests of borders.  What a visit derives per plane and per ring cell it
+// derives in its phase, from one lane offset and two words a cell: 77 VGPRs
+// for 8 directions (24 spilled otherwise, 4.77 ms against 4.40), and 4000x3000
+// 1.349 -> 1.322 ms, the video's launches 1.36 -> 1.28.
+__global__ __launch_bounds__(256, kRingPerLane<S> > 1 || KK == 8 ? 6 : 7) void k_push(
     Tiles T, Planes P, Queue q, unsigned char *flag, unsigned char *mat, unsigned char *touched,
     unsigned char *hmat, int max_iters, int sparse_iters,
     const int *sweep_state, long long *iter_total) {
   __shared__ int s_h[S::PADN];
   __shared__ int s_e[S::PADN];
   __shared__ int s_c[KK][S::PADN];
-  // Two ring cells per lane (3D 32x4x2): the flush finds its cells again
-  // from the lane index and their mask words in LDS, and takes flow back on
-  // a cell's one inward plane, so no ring state is held in registers
-  // through the local iterations (4 waves per SIMD otherwise).
-  constexpr bool kSlim = S::D3 && kRingPerLane<S> > 1;
-  __shared__ unsigned s_hm[kSlim ? S::PADN : 1];
   const int tid = threadIdx.x;
   const Lane<S> L(tid);
   __shared__ int s_next[3];
@@ -1472,15 +1501,33 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : KK == 8 ? 6 : 7) voi
   const int cap_iters = Qc.count > (int)gridDim.x           ? max_iters
                         : (sparse_iters >> sweep) < max_iters ? sparse_iters
                                                               : max_iters << sweep;
-  const long long st = P.stride;
   long long my_iters = 0;
+  // a wave's lanes cover RW rows of one slice of the tile from row wy, slice wz
+  constexpr int RW = 64 / S::TW, RPL = kRingPerLane<S>;
+  using Cell = RingCell<S, KK>;
+  // Four colour classes (2D graphs with 8-connected instances): no two tiles of
+  // a class touch one node, so a ring cell's excess and mask word are stored
+  // plainly.  With two classes a node at the corner of its tile is in the ring
+  // of two tiles of the other class.
+  constexpr bool kAlone = !S::D3 && KK == 8;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int wy = wave * RW % S::TH, wz = wave * RW / S::TH;
+  // the ring, split evenly over the four waves so that each wave loads, clears
+  // and flushes the same number of cells; the workgroup barrier after the flush
+  // then waits for no straggling wave
+  const int k0 = wave * kRingQ<S> + lane;
+  const Cell cell0(min(k0, Ring<S>::N - 1)), cell1(min(k0 + 64, Ring<S>::N - 1));
+  auto ring_cell = [&](int c) { return (c ? cell1 : cell0).again(); };
+  auto has_cell = [&](int c) {
+    return c * 64 + lane < kRingQ<S> && wave * kRingQ<S> + c * 64 + lane < Ring<S>::N;
+  };
   while (Qc.idx >= 0) {
     const int ent = Qc.ent;
     const int t = ent & kEntryTile;
     const TileRef r = ONE ? tile_ref_of<S>(T.one, t) : tile_ref<S>(T, t);
     const InstDesc &I = r.I;
     const int K = ONE || KK < 8 ? KK : I.K;  // (a compile-time count but in mixed batches)
-    const int gx = r.ox + L.lx, gy = r.oy + L.ly, gz = r.oz + L.lz;
+    const int gx = r.ox + L.lx, gy = r.oy + L.ly, gz = r.oz + wz;
     const bool valid = gx < I.nx && gy < I.ny && gz < I.nz;
     // A valid label never exceeds the distance to a deficit node, which is
     // below the node count; a label that reaches it proves the node cut off
@@ -1498,58 +1545,64 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : KK == 8 ? 6 : 7) voi
 
     // ---- loads: every global load of the visit is issued before any is
     // used; lanes off the grid, planes d >= K and dead halo cells read a
-    // valid dummy address and discard the value.
-    const long long gv = valid ? node_index(I, gx, gy, gz) : 0;
-    long long ca[KK];
+    // valid dummy address and discard the value.  Addresses are a uniform
+    // base per plane and one lane offset for all planes.
+    const bool wave_in = r.oy + wy < I.ny && gz < I.nz;
+    const long long wb = wave_in ? node_index(I, r.ox, r.oy + wy, gz) : I.node_off;
+    const long long off = valid ? L.lx + (long long)I.px * (lane / S::TW) : 0;
+    // (the stride as a value of the phase, so that its multiples are not kept)
+    auto phase_stride = [&]() {
+      long long v = P.stride;
+      asm volatile("" : "+s"(v));
+      return v;
+    };
+    long long st = phase_stride();
+    auto plane = [&](int d) { return (d < K ? d * st : 0) + wb; };
+    // the node of a live ring cell, relative to the tile's first
+    const long long tb = node_index(I, r.ox, r.oy, r.oz);
+    auto ring_node = [&](const Cell &q) {
+      return q.x() + (long long)I.px * (q.y() + (S::D3 ? I.ny * q.z() : 0));
+    };
+    bool live[RPL];
+    int hh[RPL], he[RPL];
+    unsigned hm[RPL];
 #pragma unroll
-    for (int d = 0; d < KK; ++d) ca[d] = (valid && d < K) ? d * st + gv : 0;
-    // halo: the ring cells (sides and corners in 2D, faces in 3D), split
-    // evenly over the four waves so that each wave loads, clears and flushes
-    // the same number of cells; the workgroup barrier after the flush then
-    // waits for no straggling wave
-    HaloCell hc[kRingPerLane<S>];
-    int hp[kRingPerLane<S>];
-    int hh[kRingPerLane<S>];
-    unsigned hm[kRingPerLane<S>];
-#pragma unroll
-    for (int c = 0; c < kRingPerLane<S>; ++c) {
-      const int j = c * 64 + (tid & 63);
-      const int k = (tid >> 6) * kRingQ<S> + j;
-      hp[c] = j < kRingQ<S> && k < Ring<S>::N ? Ring<S>::pos(k) : S::PADN;
-      hc[c] = halo_cell<S>(I, r.ox, r.oy, r.oz, hp[c], K);
+    for (int c = 0; c < RPL; ++c) {
+      const Cell q = ring_cell(c);
+      live[c] = has_cell(c) && (unsigned)(r.ox + q.x()) < (unsigned)I.nx &&
+                (unsigned)(r.oy + q.y()) < (unsigned)I.ny &&
+                (!S::D3 || (unsigned)(r.oz + q.z()) < (unsigned)I.nz) &&
+                (S::D3 || K > 4 || !(q.xyz >> 30));
+      const long long g = tb + (live[c] ? ring_node(q) : 0);
       // a neighbour tile without stored heights in this solve reads as 0
-      int ht = t;
-      if (hc[c].live) {
-        int x, y, z, nout;
-        bool inter;
-        pad_coords<S>(hp[c], x, y, z, inter, nout);
-        ht = tile_of<S>(I, r.ox + x, r.oy + y, r.oz + z);
-      }
-      const int hw = P.h[hc[c].g];
-      hh[c] = hmat[ht] ? hw : 0;
-      hm[c] = P.rmask[hc[c].g];
+      const int hw = P.h[g];
+      hh[c] = hmat[live[c] ? t + q.tile_step(I) : t] ? hw : 0;
+      hm[c] = P.rmask[g];
+      he[c] = kAlone ? P.e[g] : 0;
     }
     // heights not yet stored in this solve read as 0 (the start labelling);
     // the visit then stores all of them.  The compaction read hmat[t] into
     // the entry, so no load stands between the entry and the plane loads.
     const bool h_stored = (ent & kEntryHeights) != 0;
-    const int hw0 = P.h[gv];
-    int e0 = P.e[gv], h0 = h_stored ? hw0 : 0;
+    const int hw0 = (P.h + wb)[off];
+    int e0 = (P.e + wb)[off], h0 = h_stored ? hw0 : 0;
     unsigned rm = 0;
     int c0r[KK];
     if (!fresh_tile) {
 #pragma unroll
-      for (int d = 0; d < KK; ++d) c0r[d] = P.cap[ca[d]];
+      for (int d = 0; d < KK; ++d) c0r[d] = (P.cap + plane(d))[off];
     } else if (clean) {
 #pragma unroll
-      for (int d = 0; d < KK; ++d) c0r[d] = P.c0[ca[d]];
+      for (int d = 0; d < KK; ++d) c0r[d] = (P.c0 + plane(d))[off];
+      rm = ((1u << K) - 1) << 8;
 #pragma unroll
       for (int d = 0; d < KK; ++d)
-        if (d < K) rm |= (1u << (8 + d)) | ((unsigned)(c0r[d] > 0) << d);
+        if (d < K) rm |= min((unsigned)c0r[d], 1u) << d;
     } else {
-      rm = P.rmask[gv];
+      rm = (P.rmask + wb)[off];
 #pragma unroll
-      for (int d = 0; d < KK; ++d) c0r[d] = ((rm >> (8 + d)) & 1u ? P.c0 : P.cap)[ca[d]];
+      for (int d = 0; d < KK; ++d)
+        c0r[d] = (((rm >> (8 + d)) & 1u ? P.c0 : P.cap) + plane(d))[off];
     }
     if (!valid) {
       e0 = 0;
@@ -1565,14 +1618,13 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : KK == 8 ? 6 : 7) voi
 #pragma unroll
     for (int d = 0; d < KK; ++d) s_c[d][L.me] = c0r[d];
 #pragma unroll
-    for (int c = 0; c < kRingPerLane<S>; ++c) {
-      if (!hc[c].halo) continue;
-      const int p = hp[c];
-      s_h[p] = hc[c].live ? hh[c] : HINF;
-      s_e[p] = 0;
-      if constexpr (kSlim) s_hm[p] = hm[c];
+    for (int c = 0; c < RPL; ++c) {
+      if (!has_cell(c)) continue;
+      const Cell q = ring_cell(c);
+      s_h[q.p] = live[c] ? hh[c] : HINF;
+      s_e[q.p] = 0;
 #pragma unroll
-      for (int d = 0; d < KK; ++d) s_c[d][p] = 0;
+      for (int i = 0; i < Cell::ARCS; ++i) s_c[q.arc(i)][q.p] = 0;
     }
     __syncthreads();
     // the next entry loads while the tile iterates
@@ -1643,59 +1695,20 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : KK == 8 ? 6 : 7) voi
     // plane that is still fresh (its value lives in c0) the c0 value they add
     // to, loaded before the interior write-back so that its stores cover the
     // load latency.
-    int fl[kRingPerLane<S>];
-    int dc[kRingPerLane<S>][kSlim ? 1 : KK], cv[kRingPerLane<S>][kSlim ? 1 : KK];
-    unsigned fr[kRingPerLane<S>], fp[kRingPerLane<S>];
-    if constexpr (kSlim) {
-      // the ring cells found again (an opaque copy of the lane index keeps
-      // the compiler from holding the load phase's values instead)
-      int tid2 = tid;
-      asm volatile("" : "+v"(tid2));
+    int fl[RPL], dc[RPL][Cell::ARCS], cf[RPL][Cell::ARCS];
+    st = phase_stride();
 #pragma unroll
-      for (int c = 0; c < kRingPerLane<S>; ++c) {
-        const int j = c * 64 + (tid2 & 63);
-        const int k = (tid2 >> 6) * kRingQ<S> + j;
-        hp[c] = j < kRingQ<S> && k < Ring<S>::N ? Ring<S>::pos(k) : S::PADN;
-        hc[c] = halo_cell<S>(I, r.ox, r.oy, r.oz, hp[c], K);
-      }
-    }
+    for (int c = 0; c < RPL; ++c) {
+      const Cell q = ring_cell(c);
+      fl[c] = live[c] ? s_e[q.p] : 0;
 #pragma unroll
-    for (int c = 0; c < kRingPerLane<S>; ++c) {
-      fl[c] = 0;
-      fr[c] = fp[c] = 0;
-      if constexpr (!kSlim) {
+      for (int i = 0; i < Cell::ARCS; ++i) dc[c][i] = cf[c][i] = 0;
+      if (fl[c] == 0) continue;
 #pragma unroll
-        for (int d = 0; d < KK; ++d) dc[c][d] = cv[c][d] = 0;
-      } else {
-        dc[c][0] = cv[c][0] = 0;
-      }
-      if (!hc[c].live) continue;
-      const int p = hp[c];
-      fl[c] = s_e[p];
-      if constexpr (kSlim) {
-        const int d = inward_dir<S>(p);
-        const unsigned m = s_hm[p];
-        dc[c][0] = s_c[d][p];
-        if (dc[c][0] != 0) {
-          if ((m >> (8 + d)) & 1u) fr[c] = 1u << d;
-          if (!((m >> d) & 1u)) fp[c] = 1u << d;
-        }
-        if (fr[c]) cv[c][0] = P.c0[d * st + hc[c].g];
-        continue;
-      } else {
-#pragma unroll
-      for (int d = 0; d < KK; ++d) {
-        dc[c][d] = d < K ? s_c[d][p] : 0;
-        if (dc[c][d] != 0) {
-          if ((hm[c] >> (8 + d)) & 1u) fr[c] |= 1u << d;
-          if (!((hm[c] >> d) & 1u)) fp[c] |= 1u << d;
-        }
-      }
-      if (fr[c]) {
-        const long long g = hc[c].g;
-#pragma unroll
-        for (int d = 0; d < KK; ++d) cv[c][d] = P.c0[((fr[c] >> d) & 1u) ? d * st + g : 0];
-      }
+      for (int i = 0; i < Cell::ARCS; ++i) {
+        const int d = q.arc(i);
+        dc[c][i] = s_c[d][q.p];
+        if (dc[c][i] != 0 && ((hm[c] >> (8 + d)) & 1u)) cf[c][i] = P.c0[d * st + tb + ring_node(q)];
       }
     }
 
@@ -1703,8 +1716,8 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : KK == 8 ? 6 : 7) voi
     int act = 0;
     if (valid) {
       const int e1 = e, h1 = h;
-      if (e1 != e0) P.e[gv] = e1;
-      if (h1 != h0 || !h_stored) P.h[gv] = h1;
+      if (e1 != e0) (P.e + wb)[off] = e1;
+      if (h1 != h0 || !h_stored) (P.h + wb)[off] = h1;
       // fresh planes are written whether or not they changed; the mask word
       // of a written tile holds residual bits only (exact, no fresh bits)
       unsigned m0 = 0, m1 = 0;
@@ -1712,11 +1725,11 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : KK == 8 ? 6 : 7) voi
       for (int d = 0; d < KK; ++d)
         if (d < K) {
           const int c1 = s_c[d][L.me];
-          if (c1 != c0r[d] || ((rm >> (8 + d)) & 1u)) P.cap[d * st + gv] = c1;
-          m0 |= (unsigned)(c0r[d] > 0) << d;
-          m1 |= (unsigned)(c1 > 0) << d;
+          if (clean || c1 != c0r[d] || ((rm >> (8 + d)) & 1u)) (P.cap + plane(d))[off] = c1;
+          m0 |= min((unsigned)c0r[d], 1u) << d;
+          m1 |= min((unsigned)c1, 1u) << d;
         }
-      if (m1 != (fresh_tile ? rm : m0)) P.rmask[gv] = m1;
+      if (m1 != (fresh_tile ? rm : m0)) (P.rmask + wb)[off] = m1;
       act = e1 > 0 && h1 < HINF;
     }
     // ---- flush flow that crossed into the halo: excess and the reverse
@@ -1727,32 +1740,35 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 ? 5 : KK == 8 ? 6 : 7) voi
     // hence atomics.  A plane that is still fresh is written as c0 + dc; the
     // others take a fire-and-forget atomic add.
 #pragma unroll
-    for (int c = 0; c < kRingPerLane<S>; ++c) {
-      if (!hc[c].live) continue;
-      const int p = hp[c];
-      const long long g = hc[c].g;
-      if (fl[c] != 0) {
-        // flow entered g, so some plane of g changes below: g's tile is no
-        // longer clean
-        atomicAdd(&P.e[g], fl[c]);
-        const int ht = tile_of<S>(I, r.ox + (p % S::PW) - 1, r.oy + (p / S::PW) % S::PH - 1,
-                                  S::D3 ? r.oz + p / (S::PW * S::PH) - 1 : 0);
-        flag[ht] = 1;
-        touched[ht] = 1;
-      }
-      if constexpr (kSlim) {
-        const long long a = inward_dir<S>(p) * st + g;
-        if (fr[c]) P.cap[a] = cv[c][0] + dc[c][0];
-        else if (dc[c][0] != 0) atomicAdd(&P.cap[a], dc[c][0]);
-      } else {
+    for (int c = 0; c < RPL; ++c) {
+      if (fl[c] == 0) continue;
+      const Cell q = ring_cell(c);
+      const long long g = tb + ring_node(q);
+      // flow entered g, so some plane of g changes below: g's tile is no
+      // longer clean
+      if (kAlone) P.e[g] = he[c] + fl[c];
+      else atomicAdd(&P.e[g], fl[c]);
+      const int ht = t + q.tile_step(I);
+      flag[ht] = 1;
+      touched[ht] = 1;
+      unsigned flip = 0;
 #pragma unroll
-        for (int d = 0; d < KK; ++d) {
-          if ((fr[c] >> d) & 1u) P.cap[d * st + g] = cv[c][d] + dc[c][d];
-          else if (dc[c][d] != 0) atomicAdd(&P.cap[d * st + g], dc[c][d]);
+      for (int i = 0; i < Cell::ARCS; ++i) {
+        const int d = q.arc(i);
+        if (dc[c][i] == 0) continue;
+        if ((hm[c] >> (8 + d)) & 1u) {
+          P.cap[d * st + g] = cf[c][i] + dc[c][i];
+          flip |= 256u << d;
+        } else {
+          atomicAdd(&P.cap[d * st + g], dc[c][i]);
         }
+        if (!((hm[c] >> d) & 1u)) flip |= 1u << d;
       }
-      const unsigned flip = fp[c] | (fr[c] << 8);
-      if (flip) atomicXor(&P.rmask[g], flip);
+      if (kAlone) {
+        if (flip) P.rmask[g] = hm[c] ^ flip;
+      } else if (flip) {
+        atomicXor(&P.rmask[g], flip);
+      }
     }
     act = block_any(act, s_w, par);
     if (act && tid == 0) flag[t] = 1;
