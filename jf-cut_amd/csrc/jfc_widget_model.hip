@@ -109,6 +109,54 @@ __device__ __forceinline__ int nearest4(const float *c, int k, const float p[4])
   return idx;
 }
 
+// nearest4 for up to KB centroids held in registers (c), whose copy in memory
+// is m.  The squares are compared without branches; a centroid whose square is
+// alone within 2^-18 of the least has the least rounded distance, and anything
+// else (near ties, squares next to or at zero, values that are not finite) is
+// nearest4's.
+template <int KB>
+__device__ __forceinline__ int nearest4_of(const float (&c)[4 * KB], const float *m, int k,
+                                           const float p[4]) {
+  float s[KB];
+  s[0] = dist4_sq(c, p);
+  float least = s[0];
+#pragma unroll
+  for (int j = 1; j < KB; ++j) {
+    if (j >= k) break;
+    s[j] = dist4_sq(c + 4 * j, p);
+    least = fminf(least, s[j]);
+  }
+  const float near = least * (1.0f + 0x1p-18f);
+  int idx = 0, within = 0;
+#pragma unroll
+  for (int j = 0; j < KB; ++j) {
+    if (j >= k) break;
+    const bool in = s[j] <= near;
+    idx = in ? j : idx;
+    within += in;
+  }
+  if (within != 1 || !(least >= 1e-30f) || !(s[0] == s[0])) return nearest4(m, k, p);
+  return idx;
+}
+
+// the wave's sum of v, in lane 63
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_update_dpp(0u, (unsigned)b, CTRL, ROWS, 0xf, ROWS == 0xf);
+  const unsigned hi =
+      __builtin_amdgcn_update_dpp(0u, (unsigned)(b >> 32), CTRL, ROWS, 0xf, ROWS == 0xf);
+  return v + __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+__device__ __forceinline__ double wave_sum(double v) {
+  v = dpp_add<0x111, 0xf>(v);  // row_shr:1
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast:15
+  return dpp_add<0x143, 0xc>(v);  // row_bcast:31
+}
+
 // histogram level of a seeded pixel: clamp(dot, 0, 1) * (size - 1) + 0.5,
 // truncated (graphcut_histogram.cl:33-35)
 __device__ __forceinline__ int level_clamped(float data) {
@@ -134,9 +182,12 @@ struct WmScratch {
   unsigned *rep;     // [2][kLevels] highest node index + 1 per seeded level
   unsigned *acc;     // [kMaxK * 4][kLevels] byte counts of an assignment (k_wm_assign)
   uchar4 *list[2];   // the seeded pixels
+  unsigned char *owner;  // [2][kLloydSeeds] their clusters (k_wm_lloyd)
 };
+constexpr int kLloydSeeds = 65536;
 constexpr size_t kCtlBytes = 64, kHistBytes = 2 * kLevels * 4, kCentBytes = 2 * kMaxK * 4 * 4,
-                 kRepBytes = kHistBytes, kAccBytes = (size_t)kMaxK * 4 * kLevels * 4;
+                 kRepBytes = kHistBytes, kAccBytes = (size_t)kMaxK * 4 * kLevels * 4,
+                 kOwnerBytes = 2 * kLloydSeeds;
 constexpr size_t kBackBytes = kCtlBytes + kHistBytes + kCentBytes;
 
 // One pass over the seed bytes: per side the seeded pixels in a list, their
@@ -209,18 +260,21 @@ __global__ __launch_bounds__(256) void k_wm_scan(const uchar4 *img, const unsign
 // channel; a mean is the exact sum of count * value, which float64 holds in
 // any order (a term is a multiple of the smallest value's last bit, and
 // 2^16 of them span under 53 bits), divided and rounded once.
-// A launch, two copies and a host wait per iteration took 60-65 us; here one
-// takes ~10 us at 5,000 seeds, which are 6 rounds of the workgroup.
-constexpr int kLloydSeeds = 65536;
-
+// Bound by the vector and LDS instructions of one compute unit, an iteration a
+// chain of them: the k-means of a 600x450 image, 8 clusters, takes 140 us; with
+// every pixel counted anew in each iteration (an opaque image counts one alpha
+// value: 64 lanes on one LDS word), a branch per centroid and sums over lane
+// shifts it took 208.  The counts are kept from iteration to iteration, only
+// the pixels that change cluster touch them, and up to 8 centroids stay in
+// scalar registers.
 template <int KB>
 __global__ __launch_bounds__(1024) void k_wm_lloyd(const uchar4 *img, W4 w, W4 scale, int k,
                                                    int iterations, WmScratch S) {
   __shared__ unsigned s_acc[KB * 4][kLevels];
   __shared__ float s_val[4][kLevels];  // weighted feature of a byte per channel
-  __shared__ float s_c[KB * 4], s_n[KB * 4];
+  __shared__ float s_cent[2][KB * 4];  // the centroids, and those of the next iteration
   __shared__ int s_lv[kLevels];        // seeded levels in order
-  __shared__ int s_levels, s_err;
+  __shared__ int s_levels;
   const int side = blockIdx.x, tid = threadIdx.x;
   const int n = S.ctl[side];
   if (n == 0) return;
@@ -245,56 +299,82 @@ __global__ __launch_bounds__(1024) void k_wm_lloyd(const uchar4 *img, W4 w, W4 s
     const unsigned dsize = (unsigned)s_levels - 1u;
     const uchar4 t = img[s_lv[dsize * (unsigned)(tid >> 2) / (unsigned)(k - 1)]];
     const int c = tid & 3;
-    s_n[tid] = (float)(c == 0 ? t.x : c == 1 ? t.y : c == 2 ? t.z : t.w) * scale.v[c];
+    s_cent[0][tid] = (float)(c == 0 ? t.x : c == 1 ? t.y : c == 2 ? t.z : t.w) * scale.v[c];
   }
-  int it = 0;
-  for (;;) {
-    for (int i = tid; i < k * 4 * kLevels; i += 1024) (&s_acc[0][0])[i] = 0;
-    __syncthreads();
-    if (tid < k * 4) s_c[tid] = s_n[tid];
-    if (tid == 0) s_err = 0;
-    __syncthreads();
-    const uchar4 *list = S.list[side];
+  for (int i = tid; i < k * 4 * kLevels; i += 1024) (&s_acc[0][0])[i] = 0;
+  __syncthreads();
+  const uchar4 *list = S.list[side];
+  unsigned char *owner = S.owner + side * kLloydSeeds;
+  constexpr int kNone = 255;
+  int it = 0, cur = 0;
+  for (;; cur ^= 1) {
+    const float *m = s_cent[cur];
+    constexpr bool kRegs = KB <= 8;  // (more centroids don't fit the scalar registers)
+    float c[kRegs ? 4 * KB : 1];
+    if constexpr (kRegs) {
+#pragma unroll
+      for (int q = 0; q < 4 * KB; ++q)
+        c[q] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(m[q])));
+    }
+    uchar4 t = make_uchar4(0, 0, 0, 0);
+    int old = kNone;
+    if (tid < n) {
+      t = list[tid];
+      if (it) old = owner[tid];
+    }
     for (int i = tid; i < n; i += 1024) {
-      const uchar4 t = list[i];
-      const float p[4] = {s_val[0][t.x], s_val[1][t.y], s_val[2][t.z], s_val[3][t.w]};
-      const int j = nearest4(s_c, k, p);
-      atomicAdd(&s_acc[j * 4][t.x], 1u);
-      atomicAdd(&s_acc[j * 4 + 1][t.y], 1u);
-      atomicAdd(&s_acc[j * 4 + 2][t.z], 1u);
-      atomicAdd(&s_acc[j * 4 + 3][t.w], 1u);
+      const uchar4 now = t;
+      const int was = old;
+      if (i + 1024 < n) {  // the next pixel loads meanwhile
+        t = list[i + 1024];
+        if (it) old = owner[i + 1024];
+      }
+      const float p[4] = {s_val[0][now.x], s_val[1][now.y], s_val[2][now.z], s_val[3][now.w]};
+      int j;
+      if constexpr (kRegs) j = nearest4_of<KB>(c, m, k, p);
+      else j = nearest4(m, k, p);
+      if (j == was) continue;
+      owner[i] = (unsigned char)j;
+      const int v[4] = {now.x, now.y, now.z, now.w};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) atomicAdd(&s_acc[j * 4 + q][v[q]], 1u);
+      if (was != kNone) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) atomicSub(&s_acc[was * 4 + q][v[q]], 1u);
+      }
     }
     __syncthreads();
     // one wave per cluster and channel, four byte values per lane
+    float *next = s_cent[cur ^ 1];
     for (int r = tid >> 6; r < k * 4; r += 16) {
       double sum = 0.0;
       unsigned members = 0;
 #pragma unroll
       for (int q = 0; q < kLevels / 64; ++q) {
         const int b = 64 * q + (tid & 63);
-        const unsigned m = s_acc[r][b];
-        sum += (double)m * (double)s_val[r & 3][b];
-        members += m;
+        const unsigned count = s_acc[r][b];
+        sum += (double)count * (double)s_val[r & 3][b];
+        members += count;
       }
-      for (int o = 32; o > 0; o >>= 1) {
-        sum += __shfl_xor(sum, o);
-        members += __shfl_xor(members, o);
-      }
-      if ((tid & 63) == 0) s_n[r] = members ? (float)(sum / (double)members) : 0.0f;
+      sum = wave_sum(sum);
+      const double all = wave_sum((double)members);
+      if ((tid & 63) == 63) next[r] = all > 0.0 ? (float)(sum / all) : 0.0f;
     }
     __syncthreads();
     ++it;
-    if (tid < k) {
+    // every wave for itself, from the same words
+    bool moved = false;
+    if ((tid & 63) < k) {
       // glm::length(centroid - previous)
+      const int at = (tid & 63) * 4;
       float d[4];
-      for (int c = 0; c < 4; ++c) d[c] = s_n[tid * 4 + c] - s_c[tid * 4 + c];
+      for (int q = 0; q < 4; ++q) d[q] = next[at + q] - m[at + q];
       const float len = sqrtf((d[0] * d[0] + d[1] * d[1]) + (d[2] * d[2] + d[3] * d[3]));
-      if (!(len < 1.0f / 1024)) s_err = 1;
+      moved = !(len < 1.0f / 1024);
     }
-    __syncthreads();
-    if (!s_err || it >= iterations) break;
+    if (!__ballot(moved) || it >= iterations) break;
   }
-  if (tid < k * 4) S.cent[side * k * 4 + tid] = s_c[tid];
+  if (tid < k * 4) S.cent[side * k * 4 + tid] = s_cent[cur][tid];
   if (tid == 0) S.ctl[3 + side] = it;
 }
 
@@ -634,13 +714,14 @@ extern "C" int jfc_model_widget(jfc_graph *g, int inst, const uint8_t *rgba, con
   }
   {
     void *sc = nullptr;
-    if ((rc = graph_scratch(g, kBackBytes + kRepBytes + kAccBytes, &sc))) return rc;
+    if ((rc = graph_scratch(g, kBackBytes + kRepBytes + kAccBytes + kOwnerBytes, &sc))) return rc;
     unsigned char *b = (unsigned char *)sc;
     S.ctl = (int *)b;
     S.hist = (unsigned *)(b + kCtlBytes);
     S.cent = (float *)(b + kCtlBytes + kHistBytes);
     S.rep = (unsigned *)(b + kBackBytes);
     S.acc = (unsigned *)(b + kBackBytes + kRepBytes);
+    S.owner = b + kBackBytes + kRepBytes + kAccBytes;
     // the seed lists borrow the instance's slices of the excess and height
     // planes, which every solve rewrites before reading them
     int *l0 = nullptr, *l1 = nullptr;

@@ -86,3 +86,16 @@ def test_no_seeds_gpu(gpu, lazy):
         for a, c in zip(want, g.terminal_caps() + (g.neighbor_caps(),)):
             assert np.array_equal(a, c)
     g.close()
+
+
+@pytest.mark.parametrize("levels", [2, 3, 9])
+@pytest.mark.parametrize("k", [8, 12])
+def test_ties_gpu(gpu, k, levels):
+    """Few grey levels: centroids that coincide, pixels on their centroid or
+    halfway between two, clusters that empty."""
+    shape = (67, 45, 1)
+    say("case widget ties", levels, "clusters", k)
+    rgba, fg, bg = random_case(shape, levels)
+    rgba[:, :3] = (rgba[:, :1] % levels) * (255 // (levels - 1))
+    rgba[:, 3] = 255
+    check(gpu, shape, rgba, fg, bg, dict(lazy=True, k=k), solve=False)
