@@ -17,6 +17,7 @@
 #include "jfc_internal.h"
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -24,6 +25,7 @@
 #include <mutex>
 #include <numeric>
 #include <string>
+#include <thread>
 #include <type_traits>
 #include <vector>
 
@@ -249,15 +251,9 @@ struct jfc_graph {
   // waiting, in fine-grained pinned memory the device writes through to; d_ring is its device address.
   int *ring = nullptr, *d_ring = nullptr;
   hipEvent_t cnt_ev[2] = {nullptr, nullptr};
-  hipEvent_t stop_ev[kStopRing] = {};
   int ensure_pin() {
     if (pin) return JFC_OK;
     for (hipEvent_t &ev : cnt_ev)
-      if (!ev && hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
-        ev = nullptr;
-        return fail(JFC_ERR_DEVICE, "event creation failed");
-      }
-    for (hipEvent_t &ev : stop_ev)
       if (!ev && hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
         ev = nullptr;
         return fail(JFC_ERR_DEVICE, "event creation failed");
@@ -317,10 +313,6 @@ struct jfc_graph {
     priv_stream = nullptr;
     release_aux();
     for (hipEvent_t &ev : cnt_ev) {
-      if (ev) (void)hipEventDestroy(ev);
-      ev = nullptr;
-    }
-    for (hipEvent_t &ev : stop_ev) {
       if (ev) (void)hipEventDestroy(ev);
       ev = nullptr;
     }
@@ -1360,6 +1352,45 @@ struct Solver {
     launch_sweep_end(sweep_ctl(), st);
   }
 
+  // Waits for the stop word of sweep `seq` of the solve, which its end kernel
+  // writes through to the ring.  An event per sweep to wait for put 5.5 us
+  // between the sweeps (600x450 widget, a sweep of 22-40 us); the word itself
+  // costs nothing there.  The stream is looked at once a millisecond, for an
+  // error or an end without the word.
+  int await_stop(int seq, int *stopw) {
+    const volatile int *at = g->ring + seq % kStopRing;
+    auto here = [&]() {
+      const int w = *at;
+      *stopw = w & 7;
+      return (w >> 3) == seq;
+    };
+    auto looked = std::chrono::steady_clock::now();
+    const auto begin = looked;
+    for (;;) {
+      for (int spin = 0; spin < 64; ++spin) {
+        if (here()) return JFC_OK;
+        __builtin_ia32_pause();
+      }
+      const auto now = std::chrono::steady_clock::now();
+      if (now - begin > std::chrono::microseconds(100)) std::this_thread::yield();
+      if (now - looked < std::chrono::milliseconds(1)) continue;
+      looked = now;
+      JFC_HIP(hipGetLastError());
+      const hipError_t e = hipStreamQuery(st);
+      if (e == hipErrorNotReady) {
+        (void)hipGetLastError();  // no error of the caller's
+        continue;
+      }
+      JFC_HIP(e);
+      // every kernel has completed, so the word is in the ring; re-read a few
+      // times before giving up on it
+      for (int spin = 0; spin < (1 << 20); ++spin)
+        if (here()) return JFC_OK;
+      return fail(JFC_ERR_DEVICE, "sweep " + std::to_string(seq) +
+                                      ": its stop word did not reach the host");
+    }
+  }
+
   // One Fast-Cut sweep (QGCWidget::relabelPushFast, QGCW:2156-2205): every
   // active tile in one list, Jacobi relabel, line pushes, active flags.
   void issue_fast_sweep() {
@@ -1463,21 +1494,9 @@ struct Solver {
             issue_sweep();
             s.push_launches += g->ncolors;
           }
-          JFC_HIP(hipEventRecord(g->stop_ev[sent % kStopRing], st));
           ++sent;
         }
-        const int k = known % kStopRing;
-        JFC_HIP(hipEventSynchronize(g->stop_ev[k]));
-        // the sweep's end kernel has completed, so its word is in the ring
-        // (written through to host memory); re-read a few times before
-        // giving up on a word that does not carry the expected number
-        const volatile int *ring = g->ring;
-        int w = ring[k];
-        for (int spin = 0; (w >> 3) != known && spin < (1 << 20); ++spin) w = ring[k];
-        if ((w >> 3) != known)
-          return fail(JFC_ERR_DEVICE, "sweep " + std::to_string(known) +
-                                          ": its stop word did not reach the host");
-        stopw = w & 7;
+        if ((rc = await_stop(known, &stopw))) return rc;
         ++known;
         if (stopw) break;
       }
