@@ -465,8 +465,8 @@ def main():
         st = g.solve(**topt)
         log(f"warmup {i}: {st.ms_total:.2f} ms, sweeps {st.sweeps}, flow {st.flow}")
 
-    # headline: fresh inputs, the solve as a caller runs it (sweeps after the
-    # first replay a captured graph, no timing events between launches)
+    # headline: fresh inputs, the solve as a caller runs it (no timing events
+    # between launches)
     ms_per_step, stats = timed_steps(g, args.steps, fresh=True, **topt)
     for i, st in enumerate(stats):
         log(f"step {i}: {st.ms_total:.2f} ms device, sweeps {st.sweeps}, "

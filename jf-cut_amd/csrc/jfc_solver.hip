@@ -1208,7 +1208,7 @@ void launch_compact(const int *src, int n, int reverse, unsigned char *flag,
 // lists, down to 1 for short ones).  Each workgroup's first run is static
 // (group b takes run first(b) < G, G = grid size), so short or empty lists
 // cost no atomics.  Later runs are claimed dynamically, which balances tiles
-// of very different cost (a relabel visit iterates to its tile's fixpoint).
+// of very different cost.
 // Workgroups are dispatched to the 8 XCDs round-robin (b % 8), so with 8
 // heads, head x serves the workgroups of XCD x: runs >= G form groups of 8
 // consecutive runs, group q belongs to head q % nheads, and a head hands out
@@ -1217,14 +1217,13 @@ void launch_compact(const int *src, int n, int reverse, unsigned char *flag,
 // different cache lines.  Every run
 // belongs to one head and every head has workgroups, so the list is always
 // drained.  When the static first runs already cover the list (G * chunk >=
-// count, the short lists of late sweeps and relabel passes) no claim is
+// count, the short lists of late sweeps) no claim is
 // issued at all: thousands of workgroups claiming on 8 addresses would
 // serialise there.  Slot s of `ctr` holds the list count at [QSLOT*s] and
 // head h at [QSLOT*s + QWORD*(1+h)]; the consumer of slot s zeroes the other
 // slot's words for the next producer.
 //
-// VisitCursor walks a queue that way for the tile-visit kernels (push, relax,
-// cut flood).  A workgroup learns its next list entry while it discharges
+// VisitCursor walks a queue that way for the push kernel.  A workgroup learns its next list entry while it discharges
 // the current tile, so that a visit starts with neither a global load nor a
 // barrier of its own: thread 0 works out the next position during the local
 // iterations (the rest of the current run, else the run its claim obtained,
