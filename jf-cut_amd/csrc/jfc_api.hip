@@ -1375,10 +1375,10 @@ struct Solver {
       if (now - begin > std::chrono::microseconds(100)) std::this_thread::yield();
       if (now - looked < std::chrono::milliseconds(1)) continue;
       looked = now;
-      JFC_HIP(hipGetLastError());
       const hipError_t e = hipStreamQuery(st);
       if (e == hipErrorNotReady) {
-        (void)hipGetLastError();  // no error of the caller's
+        // no error for the caller to find; one that was there stays
+        if (hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError();
         continue;
       }
       JFC_HIP(e);
