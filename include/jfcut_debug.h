@@ -44,8 +44,9 @@ int jfc_debug_tile_flags(jfc_graph *g, int which, uint8_t *flags);
  * at most n counts. */
 int jfc_debug_sweep_counts(jfc_graph *g, int32_t *counts, int32_t n);
 
-/* Idle wait, in ticks of the device's 100 MHz clock, after which a wavefront
- * of a one-launch relabel leaves the rest to separate passes (0: at once). */
+/* Time without progress, in ticks of the device's 100 MHz clock, after which a
+ * one-launch search (relabel, cut, tags) leaves the rest to separate passes
+ * (0: as soon as a wavefront is idle). */
 int jfc_debug_relabel_wait(jfc_graph *g, int64_t ticks);
 
 #ifdef __cplusplus

@@ -197,8 +197,8 @@ struct jfc_graph {
     int seq = 0;           // passes run, the number their posted words carry
     int *d_marks = nullptr;  // words of a one-launch relabel
     size_t mark_words() const { return (size_t)kSettleLine * (2 * kSettleSlots + n); }
-    // idle wait of a one-launch search before it leaves the rest to passes:
-    // far above the ~50 us of a visit, below what a caller would notice
+    // time without progress after which a one-launch search leaves the rest to
+    // passes: far above the ~50 us of a visit
     long long wait_ticks = 2000000;  // 20 ms
   } rg;
   // One device block holds every word a solve reads back at its end (one

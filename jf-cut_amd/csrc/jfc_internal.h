@@ -251,7 +251,7 @@ struct SettleWords {
   int *marks;            // per region: marks made so far
   int *quit;             // set when it gave up waiting
   int *quit_host;        // (or null) pinned word set then, too
-  long long wait_ticks;  // idle wait before it gives up (100 MHz clock)
+  long long wait_ticks;  // time without progress before it gives up (100 MHz clock)
 };
 struct RegionPass {
   PassCtl c;

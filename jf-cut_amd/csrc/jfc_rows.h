@@ -169,11 +169,15 @@ struct Marks {
 // planes are touched by its owner only.
 //
 // Every workgroup is resident on an idle device (the launcher caps the grid),
-// but other kernels may hold their places back, so the wait is bounded: a wave
-// idle for wait_ticks tells the others to quit and sets *quit, and the search is
+// but other kernels may hold their places back, so the wait is bounded.  What is
+// bounded is the time without progress, not a wave's own idleness (a front may
+// be far away for as long as the search takes): a wave idle for wait_ticks looks
+// at the marks made and served, and where they have not moved for another
+// wait_ticks it tells the others to quit and sets *quit, and the search is
 // finished with passes over every region.
 constexpr int kSlots = kSettleSlots, kLine = kSettleLine;
 static_assert(kSlots == 64, "a lane per slot");
+constexpr int kServed = 0, kMade = 1;  // the words of a slot's line of sums
 enum { kGo = 0, kDone = 1, kQuit = 2, kStop = 3 };
 
 // Counts the marks of a visit that served `served` marks, then makes them.
@@ -212,7 +216,13 @@ __device__ __forceinline__ bool settle(const SettleWords &A, int n, bool all, lo
   const bool own = mine < n;
   bool done = false;
   int seen = 0, visits = 0, turn = 0;
-  long long since = 0;
+  long long since = 0;  // idle, and without progress as far as known, since then
+  int progress = 0;     // the sums at the last look
+  auto sum = [&](int word) {
+    int v = shared_word(A.sums + kLine * lane + word);
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    return v;
+  };
   for (;;) {
     const int now = own ? shared_word(A.marks + kLine * (long long)mine) : 0;
     const int state = shared_word(A.state + kLine * slot);
@@ -236,21 +246,25 @@ __device__ __forceinline__ bool settle(const SettleWords &A, int n, bool all, lo
     }
     done = state == kDone;
     if (state != kGo) break;
+    const long long tick = wall_clock64();
+    if (since == 0) since = tick;
+    int now_at = progress;
     if (blockIdx.x == 0) {
-      auto sum = [&](int half) {
-        int v = shared_word(A.sums + kLine * lane + half);
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-        return v;
-      };
-      const int served = sum(0);
+      const int served = sum(kServed);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      if (sum(1) + (all ? n : 0) == served) {
+      const int made = sum(kMade);
+      if (made + (all ? n : 0) == served) {
         tell(A, kDone, lane);
         continue;
       }
+      now_at = served + made;
+    } else if (A.wait_ticks > 0 && tick - since >= A.wait_ticks) {
+      now_at = sum(kServed) + sum(kMade);
     }
-    const long long tick = wall_clock64();
-    if (since == 0) since = tick;
+    if (now_at != progress) {
+      progress = now_at;
+      since = tick;
+    }
     if (tick - since >= A.wait_ticks) {
       tell(A, kQuit, lane);
       if (lane == 0) {
