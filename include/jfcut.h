@@ -31,7 +31,9 @@
  *     jfc_solve, which may also return JFC_NOT_CONVERGED (1).  The message of
  *     the last error of the calling thread is returned by jfc_last_error().
  *   - A graph may be used by one host thread at a time; distinct graphs are
- *     independent.  Streams: every call of a graph issues its device work on
+ *     independent (solved at the same time they share the device: a search that
+ *     is kept from some of its workgroups for 0.2 ms goes on with a launch per
+ *     pass, and so do the solve's later ones).  Streams: every call of a graph issues its device work on
  *     the graph's stream (jfc_set_stream; NULL = the legacy default stream),
  *     ordered after the work the caller queued there before the call, and
  *     returns after that work completed (it waits for that stream only, not

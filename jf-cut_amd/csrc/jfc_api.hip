@@ -1137,6 +1137,10 @@ struct Solver {
     launch_fill_multi(f, st);
   }
 
+  // A search of this solve gave up waiting: something else holds places on the
+  // device, and the searches left go by passes.
+  bool by_passes = false;
+
   // A cut or tag flood over the regions (jfc_flood.hip).  fills: zeroing of the
   // caller's, done in the same launch.  Where one launch takes every pass the
   // stream has to be waited for and finish_flood() asked afterwards.
@@ -1152,7 +1156,7 @@ struct Solver {
     FloodPass A = flood_pass(stop);
     Planes P = g->planes();
     if (tag) P.lab = g->tag;
-    if (launch_flood_all(d3, tag, g->region_tiles(), P, flood_buf(), A, st)) {
+    if (!by_passes && launch_flood_all(d3, tag, g->region_tiles(), P, flood_buf(), A, st)) {
       ++*passes;
       return JFC_OK;
     }
@@ -1164,6 +1168,7 @@ struct Solver {
   int finish_flood(bool tag, bool stop, int *passes, bool *again) {
     *again = *(const volatile int *)(g->ring + kQuitWord) != 0;
     if (!*again) return JFC_OK;
+    by_passes = true;
     g->ring[kQuitWord] = 0;
     mark_all_regions();
     return flood_passes(tag, flood_pass(stop), passes, true);
@@ -1220,7 +1225,7 @@ struct Solver {
       launch_fill_multi(f, st);
     }
     RegionPass A = relabel_pass();
-    if (launch_relabel(g->dim == 3, g->region_tiles(), g->planes(), rg.buf, A, st)) {
+    if (!by_passes && launch_relabel(g->dim == 3, g->region_tiles(), g->planes(), rg.buf, A, st)) {
       s.relabel_passes++;
       relabelled(A.w.quit, resume);
     } else {
@@ -1232,6 +1237,7 @@ struct Solver {
 
   // The relabel whose waves gave up waiting, by passes over its packed regions.
   int finish_relabel() {
+    by_passes = true;
     mark_all_regions();
     if (int rc = relabel_passes(relabel_pass(), true)) return rc;
     gr_ev.pop_back();

@@ -246,7 +246,7 @@ struct PassCtl {
 // caller, kSettleLine ints apart.
 constexpr int kSettleSlots = 64, kSettleLine = 32;
 struct SettleWords {
-  int *sums = nullptr;   // kSettleSlots pairs: marks served, marks made
+  int *sums = nullptr;   // kSettleSlots times: marks served, marks made, workgroups begun
   int *state;            // kSettleSlots
   int *marks;            // per region: marks made so far
   int *quit;             // set when it gave up waiting

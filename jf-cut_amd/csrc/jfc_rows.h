@@ -168,16 +168,23 @@ struct Marks {
 // owner reads them at device scope after it has seen the mark; a region's
 // planes are touched by its owner only.
 //
-// Every workgroup is resident on an idle device (the launcher caps the grid),
-// but other kernels may hold their places back, so the wait is bounded.  What is
-// bounded is the time without progress, not a wave's own idleness (a front may
-// be far away for as long as the search takes): a wave idle for wait_ticks looks
-// at the marks made and served, and where they have not moved for another
-// wait_ticks it tells the others to quit and sets *quit, and the search is
-// finished with passes over every region.
+// The launcher caps the grid at what the device holds, but other kernels (a search
+// of another graph, say) may hold places back, so every wait is bounded.  What is
+// bounded is the time without progress, not a wave's own idleness: the marks
+// made and served and the workgroups begun are looked at before a wave gives up.
+//   - Once every workgroup has begun, nothing can hold the search up;
+//     wait_ticks without progress is a way out only.
+//   - Until then the marks of a workgroup without a place stay unserved, and two
+//     searches that hold each other's places would wait for each other, so the
+//     first workgroup gives up after kPlaceTicks without progress.
+// It tells the others to quit and sets *quit, and the search is finished with
+// passes over every region.  Three threads that solve 128^3 volumes of their own:
+// 57 ms a solve where waves without a place were waited for 20 ms, 31 now (41 with a
+// launch per pass); 256x192x176: 138 and 83 (109).
 constexpr int kSlots = kSettleSlots, kLine = kSettleLine;
 static_assert(kSlots == 64, "a lane per slot");
-constexpr int kServed = 0, kMade = 1;  // the words of a slot's line of sums
+constexpr int kServed = 0, kMade = 1, kBegun = 2;  // the words of a slot's line of sums
+constexpr long long kPlaceTicks = 20000;           // 200 us: a visit takes 10 to 50
 enum { kGo = 0, kDone = 1, kQuit = 2, kStop = 3 };
 
 // Counts the marks of a visit that served `served` marks, then makes them.
@@ -218,11 +225,15 @@ __device__ __forceinline__ bool settle(const SettleWords &A, int n, bool all, lo
   int seen = 0, visits = 0, turn = 0;
   long long since = 0;  // idle, and without progress as far as known, since then
   int progress = 0;     // the sums at the last look
+  bool placed = false;  // (first workgroup) every workgroup has begun
   auto sum = [&](int word) {
     int v = shared_word(A.sums + kLine * lane + word);
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
     return v;
   };
+  if (lane == 0)
+    (void)__hip_atomic_fetch_add(A.sums + kLine * slot + kBegun, 1, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
   for (;;) {
     const int now = own ? shared_word(A.marks + kLine * (long long)mine) : 0;
     const int state = shared_word(A.state + kLine * slot);
@@ -248,8 +259,11 @@ __device__ __forceinline__ bool settle(const SettleWords &A, int n, bool all, lo
     if (state != kGo) break;
     const long long tick = wall_clock64();
     if (since == 0) since = tick;
+    long long limit = A.wait_ticks;
     int now_at = progress;
     if (blockIdx.x == 0) {
+      const int begun = placed ? G : sum(kBegun);
+      placed = begun == G;
       const int served = sum(kServed);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       const int made = sum(kMade);
@@ -257,15 +271,16 @@ __device__ __forceinline__ bool settle(const SettleWords &A, int n, bool all, lo
         tell(A, kDone, lane);
         continue;
       }
-      now_at = served + made;
-    } else if (A.wait_ticks > 0 && tick - since >= A.wait_ticks) {
-      now_at = sum(kServed) + sum(kMade);
+      now_at = begun + served + made;
+      if (!placed) limit = min(limit, kPlaceTicks);
+    } else if (limit > 0 && tick - since >= limit) {
+      now_at = sum(kBegun) + sum(kServed) + sum(kMade);
     }
     if (now_at != progress) {
       progress = now_at;
       since = tick;
     }
-    if (tick - since >= A.wait_ticks) {
+    if (tick - since >= limit) {
       tell(A, kQuit, lane);
       if (lane == 0) {
         __hip_atomic_store(A.quit, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

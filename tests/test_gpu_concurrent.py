@@ -1,12 +1,16 @@
-"""One-launch searches (relabel, cut and tag floods) and what ends them: searches
-longer than the time a wave waits.  Flows and labels against the oracle,
-bit-exact."""
+"""One-launch searches (relabel, cut and tag floods) beside other work: graphs
+solved from several threads on streams of their own, whose searches hold each
+other's places on the device, and searches longer than the time a wave waits.
+Flows and labels against the oracle, bit-exact."""
 import ctypes
+import threading
+import time
 
 import numpy as np
 import pytest
 
 import oracle_lib as ol
+from conftest import random_grid
 from test_gpu_parity import say, serpentine
 
 pytestmark = pytest.mark.gpu
@@ -19,6 +23,47 @@ def make(gpu, shape, cs, ct, caps, ticks=None):
     if ticks is not None:
         assert gpu.lib().jfc_debug_relabel_wait(g._h, ctypes.c_int64(ticks)) == 0
     return g
+
+
+@pytest.mark.parametrize("shape", [(96, 96, 96, 6), (1400, 1400, 1, 4)])
+def test_graphs_solved_at_the_same_time_gpu(gpu, shape):
+    """Three graphs from three threads.  A search that another one keeps from its
+    places does not wait for them until the bound, here 2 seconds."""
+    import torch
+    work = []
+    for seed in range(3):
+        rng = np.random.default_rng(seed)
+        cs, ct, caps = random_grid(rng, *shape, term_max=3, seed_frac=0.0005)
+        g = make(gpu, shape, cs, ct, caps, ticks=200_000_000)
+        s = torch.cuda.Stream()
+        g.set_stream(s.cuda_stream)
+        g.solve(initial_relabel=1)
+        work.append((g, s, g.flow(), g.labels(), ol.maxflow(*shape, cs, ct, caps)))
+    for g, s, f, l, want in work:
+        assert f == want[0] and np.array_equal(l, want[1])
+    slow, wrong = [], []
+
+    def solve(g, f, l):
+        for i in range(6):
+            t = time.perf_counter()
+            st = g.solve(initial_relabel=1)
+            slow.append(time.perf_counter() - t)
+            fg = np.zeros(l.size, np.uint8)
+            fg[::31] = 1
+            g.tags(fg)
+            if not (st.converged == 1 and g.flow() == f and np.array_equal(g.labels(), l)):
+                wrong.append(i)
+
+    say("case graphs at the same time", shape)
+    threads = [threading.Thread(target=solve, args=(g, f, l)) for g, s, f, l, _ in work]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+    assert max(slow) < 2.0, slow
+    for g, *_ in work:
+        g.close()
 
 
 @pytest.mark.parametrize("shape", [(64, 4001, 1), (70, 31, 9)])
