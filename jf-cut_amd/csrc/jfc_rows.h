@@ -225,7 +225,7 @@ __device__ __forceinline__ bool settle(const SettleWords &A, int n, bool all, lo
   int seen = 0, visits = 0, turn = 0;
   long long since = 0;  // idle, and without progress as far as known, since then
   int progress = 0;     // the sums at the last look
-  bool placed = false;  // (first workgroup) every workgroup has begun
+  int begun = 0;        // (first workgroup) the workgroups begun, at the last look
   auto sum = [&](int word) {
     int v = shared_word(A.sums + kLine * lane + word);
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
@@ -262,8 +262,6 @@ __device__ __forceinline__ bool settle(const SettleWords &A, int n, bool all, lo
     long long limit = A.wait_ticks;
     int now_at = progress;
     if (blockIdx.x == 0) {
-      const int begun = placed ? G : sum(kBegun);
-      placed = begun == G;
       const int served = sum(kServed);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       const int made = sum(kMade);
@@ -271,8 +269,12 @@ __device__ __forceinline__ bool settle(const SettleWords &A, int n, bool all, lo
         tell(A, kDone, lane);
         continue;
       }
-      now_at = begun + served + made;
-      if (!placed) limit = min(limit, kPlaceTicks);
+      if (begun < G) {
+        limit = min(limit, kPlaceTicks);
+        if (tick - since >= limit) begun = sum(kBegun);
+        if (begun == G) limit = A.wait_ticks;
+      }
+      now_at = served + made + begun;
     } else if (limit > 0 && tick - since >= limit) {
       now_at = sum(kBegun) + sum(kServed) + sum(kMade);
     }
