@@ -93,8 +93,8 @@ typedef struct {
                              or two sweeps running repeat the two before them
                              (the active set has stopped changing, or trades
                              places between two sets of tiles; 0 = off), once
-                             the sweeps since the last relabel have run as
-                             long as that relabel took */
+                             the sweeps since the last relabel have cost as
+                             much as that relabel, by the work of both */
   int graph_sweeps;       /* 0 or 1 (default); both launch a sweep's kernels one
                              by one: a replayed hipGraph of them started later
                              than they did.  Results do not depend on it. */
@@ -239,7 +239,10 @@ int jfc_inputs_written(jfc_graph *g, int inst);
 /* ---- solve (QGCW:2364-2558 slotCutClicked) --------------------------------- */
 
 /* Run every instance to the max-flow certificate or opt->max_sweeps.
- * opt and stats may be NULL.  Returns JFC_OK, JFC_NOT_CONVERGED or an error. */
+ * opt and stats may be NULL.  Returns JFC_OK, JFC_NOT_CONVERGED or an error.
+ * Flows and labels of JFC_OK are the same in every run; those of
+ * JFC_NOT_CONVERGED are the preflow's at the last sweep, which the order of the
+ * wavefronts inside a tile visit can change from run to run. */
 int jfc_solve(jfc_graph *g, const jfc_options *opt, jfc_stats *stats);
 
 /* ---- outputs --------------------------------------------------------------- */

@@ -109,6 +109,24 @@ struct Tuned {
 // grid 1.25 / 0.83 / 0.95 ms, a 600x450 widget cut 1.43 / 1.20 / 1.03, a
 // 512x512 cut, done after four sweeps, 0.63 / 0.69 / 0.64.
 constexpr int kSparseIters = 16;
+
+// Cost of a relabel in ns: its launches, the passes over every region, a chain of
+// visits as long as its longest distance, and the cut search that was tried
+// before it (stall_certify).  Fitted so that stalls relabel about as often as
+// they best do, at 0.7 to 1.2 of what relabels take; this and measured, in us:
+// 3750x2500 strokes 750 and 960, 1500x1100 random 510 and 450, 1023x767 105 and
+// 150, 4000x3000 60 and 90; 100^3 random 220 and 300, 181x217x181 scan 210 and
+// 340, 256x192x176 random 360 and 520, 512^3 volume 1180 and 1560,
+// 2560x1440x50 video with its cut search 4250 and 3560.
+struct RelabelCost {
+  long long launch, region, level, certify;
+};
+constexpr RelabelCost kCost2D{15000, 16, 500, 20}, kCost3D{15000, 26, 1600, 20};
+// And of a sweep: its push launches, each as long as its longest visit (22 us
+// with 8 directions, else 15 to 20), and its tile visits, by the length of a
+// tile's rows.
+constexpr long long kPushNs = 18000, kPushNs8 = 22000, kVisitNs2D = 7, kVisitNs8x8x4 = 11,
+                    kVisitNs32x4x2 = 5;
 std::mutex g_tune_mu;
 std::map<std::string, Tuned> g_tune;
 
@@ -196,6 +214,7 @@ struct jfc_graph {
     int tag = 1;           // of the last relabel
     int seq = 0;           // passes run, the number their posted words carry
     int *d_marks = nullptr;  // words of a one-launch relabel
+    int *d_far = nullptr;    // largest distances of the last relabel
     size_t mark_words() const { return (size_t)kSettleLine * (2 * kSettleSlots + n); }
     // time without progress after which a one-launch search leaves the rest to
     // passes: far above the ~50 us of a visit
@@ -464,6 +483,7 @@ struct jfc_graph {
       carve(rg.d_inst, rg.inst.size());
       carve(rg.d_tile_inst, n);
       carve(rg.d_any, 4);
+      carve(rg.d_far, kFarSlots * kFarLine);
       carve(rg.d_marks, rg.mark_words());
       carve(rg.d_dirty[0], n);
       carve(rg.d_dirty[1], n);
@@ -1061,6 +1081,13 @@ struct Solver {
     c.budget = o.relabel_work > 0 ? (long long)std::floor(o.relabel_work * g->ntiles) : 0;
     c.ring = g->d_ring;
     c.ring_n = kStopRing;
+    c.sweep_ns = (g->Kg == 8 ? kPushNs8 : kPushNs) *
+                 (o.method == JFC_METHOD_FASTCUT ? 2 + 2 * g->dim : g->ncolors);
+    c.visit_ns = g->dim == 2 ? kVisitNs2D : g->shape == SH_8x8x4 ? kVisitNs8x8x4 : kVisitNs32x4x2;
+    const RelabelCost &cost = g->dim == 3 ? kCost3D : kCost2D;
+    c.relabel_ns = cost.launch + (cost.region + (o.stall_certify > 0 ? cost.certify : 0)) * g->rg.n;
+    c.level_ns = cost.level;
+    c.far = g->rg.d_far;
     return c;
   }
 
@@ -1212,8 +1239,8 @@ struct Solver {
   // and finish_relabel() does it by passes.  resume: sweeping goes on after a
   // stop.
   int global_relabel(bool resume) {
-    hipEvent_t a = tm.mark();
-    relabel_start = a;
+    relabel_start = tm.mark();
+    first_relabel = !resume;
     if (int rc = g->ensure_pin()) return rc;
     auto &rg = g->rg;
     rg.tag = 3 - rg.tag;
@@ -1221,6 +1248,7 @@ struct Solver {
       FillSet f;
       region_fills(f);
       f.add(g->d_flag, g->ntiles, 0, 1);  // kFinal sets the active tiles' flags
+      f.add(rg.d_far, kFarSlots * kFarLine, 0, 4);
       f.add(rg.d_marks, (long long)rg.mark_words(), 0, 4);
       launch_fill_multi(f, st);
     }
@@ -1247,6 +1275,7 @@ struct Solver {
   }
 
   hipEvent_t relabel_start = nullptr;
+  bool first_relabel = false;  // the last relabel came before the first sweep
 
   SettleWords settle_words() const {
     SettleWords w;
@@ -1271,6 +1300,7 @@ struct Solver {
     A.pdims = __builtin_ctz(tw) | __builtin_ctz(th) << 4 | __builtin_ctz(td) << 8;
     A.w = settle_words();
     A.c.visits = g->d_total + kRegionSlots;
+    A.far = rg.d_far;
     return A;
   }
 
@@ -1286,7 +1316,7 @@ struct Solver {
 
   // after a relabel: every height is stored now, sweeping resumes
   void relabelled(const int *quit, bool resume) {
-    launch_relabel_end(sweep_ctl(), g->d_hmat, g->ntiles, quit, resume, st);
+    launch_relabel_end(sweep_ctl(), g->d_hmat, g->ntiles, quit, resume, !first_relabel, st);
     gr_ev.push_back({relabel_start, tm.mark()});
     s.global_relabels++;
   }

@@ -171,8 +171,8 @@ void launch_tile_order(int shape, const Tiles &T, const unsigned char *seed,
 // tile, 2 active set stalled, 3 sweep budget spent, 4 relabel budget
 // spent, 5 the last relabel is unfinished), [3] sweep index of the last
 // relabel, [4..5] tile visits (int64) at the last relabel, [6] sweeps ended
-// (no-ops included) in the solve, [8..9] the clock (int64) at the last stop or
-// resumption, [10..11] the time from the last stop to its resumption.
+// (no-ops included) in the solve, [8..9] the sweeps' cost (int64, ns) since the
+// last relabel, [10..11] that relabel's.
 struct SweepCtl {
   int *hist;             // active tiles per sweep
   int *state;
@@ -185,11 +185,17 @@ struct SweepCtl {
   // s % ring_n (null: no posting).
   int *ring;
   int ring_n;
+  long long sweep_ns;    // cost of a sweep's launches
+  long long visit_ns;    // and of each of its tile visits
+  long long relabel_ns;  // cost of a relabel of no depth
+  long long level_ns;    // and of each level of its longest distance
+  const int *far;        // largest distances of the last relabel: kFarSlots, kFarLine apart
 };
+constexpr int kFarSlots = 64, kFarLine = 16;
 constexpr int kSweepState = 12;
 void launch_sweep_end(const SweepCtl &c, hipStream_t st);
 void launch_relabel_end(const SweepCtl &c, unsigned char *hmat, int n, const int *quit, bool resume,
-                        hipStream_t st);
+                        bool charge, hipStream_t st);
 
 // Queue list entries: tile index, plus, when compacted with `mat`, kEntryMat
 // if mat[t] is set, else kEntryClean if touched[t] is clear (no visit and no
@@ -260,6 +266,7 @@ struct RegionPass {
   const InstDesc *pinst;              // push tiling
   InstDesc pone;                      // its instance 0
   int pdims;                          // push tile dimensions, log2 (x | y << 4 | z << 8)
+  int *far;                           // kFarSlots, zeroed by the caller: largest distances
   SettleWords w;                      // launch_relabel (else w.sums null)
 };
 // Cut and tag floods on the same regions (jfc_flood.hip).

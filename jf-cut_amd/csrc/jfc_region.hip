@@ -193,6 +193,20 @@ __device__ __forceinline__ void region_visit(const Tiles &T, const Planes &P,
     for (int x = 0; x < 64; x += 1 << lw)
       if ((act >> x) & seg) A.active[row + ((ox + x) >> lw)] = 1;
   };
+  // the largest distance among `found`: the highest count bit that any of them
+  // has, then the next among those that have it
+  auto note_farthest = [&](u64 found, int top) {
+    if (!__ballot(found != 0)) return;
+    int d = 0;
+#pragma unroll
+    for (int j = kCntBits - 1; j >= 0; --j) {
+      if ((1 << j) >= top) continue;
+      const u64 t = found & cnt[j];
+      if (__ballot(t != 0)) d |= 1 << j, found = t;
+    }
+    int *at = A.far + kFarLine * (t & (kFarSlots - 1));
+    if (lane == 0 && *at < ebase + d) atomicMax(at, ebase + d);
+  };
   // 2D visits load their state with everything else; a 3D visit's borders are
   // as large as its planes, and half of them end before the search, so it
   // loads its state after they are compared
@@ -201,9 +215,9 @@ __device__ __forceinline__ void region_visit(const Tiles &T, const Planes &P,
   if (PASS == kFinal && ebase != kNoBase) {
     load_state();
     const u64 high = cnt[8] | cnt[9] | cnt[10] | cnt[11], mid = cnt[4] | cnt[5] | cnt[6] | cnt[7];
-    write_heights(vis & valid, valid & ~vis,
-                  __ballot(high != 0) ? kCntMax : __ballot(mid != 0) ? 256 : 16, wv0, wv0 + 64 / W);
-    if (wv0 == 0) write_active(ps[64]);
+    const int top = __ballot(high != 0) ? kCntMax : __ballot(mid != 0) ? 256 : 16;
+    write_heights(vis & valid, valid & ~vis, top, wv0, wv0 + 64 / W);
+    if (wv0 == 0) write_active(ps[64]), note_farthest(vis & valid, top);
     return;
   }
   if (PASS == kFinal && wv0 > 0) return;
@@ -472,6 +486,7 @@ __device__ __forceinline__ void region_visit(const Tiles &T, const Planes &P,
     const u64 found = vis & ~vis0;
     if (PASS == kFinal) {
       write_heights(found, last ? valid & ~vis : 0, top, 0, 64);
+      note_farthest(found, kCntMax);
     } else {
       int *bw = R.border + b0;
       const bool all = PASS == kPack && !wrote;

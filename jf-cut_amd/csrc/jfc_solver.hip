@@ -1093,9 +1093,9 @@ __global__ __launch_bounds__(kCompactBlock) void k_compact(const int *src, int n
 // the count, so that the host can queue sweeps ahead of its checks:
 //   stop = 1: no tile was active (converged, or the certificate decides);
 //   stop = 2: the active set neither shrank nor grew by more than
-//             (1 - stall_ratio) over the last sweep since the last relabel,
-//             whose time the sweeps since have made up for (a global relabel is due, or the remaining excess is cut off
-//             from every deficit);
+//             (1 - stall_ratio) over the last sweep since the last relabel, whose
+//             cost the sweeps since have reached (a global relabel is due, or the
+//             remaining excess is cut off from every deficit);
 //   stop = 3: the sweep budget is spent;
 //   stop = 4: the tile visits since the last relabel exceed the budget (the
 //             work of relabel_work visits per tile): a relabel is due.
@@ -1122,6 +1122,7 @@ __global__ void k_sweep_end(SweepCtl c) {
   if (i < c.cap) c.hist[i] = cnt;
   st[0] = 0;
   st[1] = i + 1;
+  *(long long *)(st + 8) += c.sweep_ns + c.visit_ns * cnt;
   int stop = 0;
   if (cnt == 0) {
     stop = 1;
@@ -1136,16 +1137,20 @@ __global__ void k_sweep_end(SweepCtl c) {
       return (double)a >= c.stall_ratio * b && a * c.stall_ratio <= (double)b;
     };
     bool stalled = false;
-    // A stall counts once the sweeps since the last relabel have run as long
-    // as that relabel took, its host wait included: a steady active set is
-    // often flow on its way, and a relabel costs many sweeps on large graphs
-    // and less than one on small ones.  Geometric means over seeds without
-    // this, at half, once, twice and four times the relabel's time:
-    // 3750x2500 strokes 78.7, 71.3, 68.3, 65.0, 67.3 ms; 2560x1440x50 video
+    // A stall counts once the sweeps since the last relabel have cost as much as
+    // that relabel: a steady active set is often flow on its way, and a relabel
+    // costs many sweeps on large graphs and less than one on small ones.  Costs
+    // are those of the work (SweepCtl), not times: a host that looks late, or a
+    // device that others use, changes nothing.  By the clock, geometric means
+    // over seeds without this, at half, once, twice and four times the relabel's
+    // time: 3750x2500 strokes 78.7, 71.3, 68.3, 65.0, 67.3 ms; 2560x1440x50 video
     // 60.5, 46.5, 39.9, 40.9, 38.0; 512^3 volume 27.0, 20.5, 19.7, 22.1, 26.7;
     // 181x217x181 scan 2.94, 3.07, 3.00, 3.36, 3.88; 1023x767 2.59, 2.73, 2.33,
-    // 2.03, 2.05; 600x450 widget 1.90, 1.89, 1.78, 1.70, 1.56.
-    const bool paid = wall_clock64() - *(const long long *)(st + 8) >= *(const long long *)(st + 10);
+    // 2.03, 2.05; 600x450 widget 1.90, 1.89, 1.78, 1.70, 1.56: once is a compromise.
+    // Over other seeds, once by the clock and by cost: strokes 51.1 and 51.3, video
+    // 8.87 and 8.92, volume 11.2 and 11.2, scan 1.71 and 1.70, 1023x767 0.95 and
+    // 0.98, widget 0.53 and 0.53.
+    const bool paid = *(const long long *)(st + 8) >= *(const long long *)(st + 10);
     if (c.stall_ratio > 0.0 && since >= 1 && paid && i < c.cap) {
       stalled = near(cnt, c.hist[i - 1]);
       if (!stalled && since >= 3)
@@ -1157,7 +1162,6 @@ __global__ void k_sweep_end(SweepCtl c) {
     else if (budget) stop = 4;
   }
   st[2] = stop;
-  if (stop) *(long long *)(st + 8) = wall_clock64();
   post_stop(c, seq, stop);
 }
 
@@ -1165,23 +1169,25 @@ void launch_sweep_end(const SweepCtl &c, hipStream_t st) { k_sweep_end<<<1, 1, 0
 
 // After a global relabel: every height is stored (hmat); with resume, sweeping
 // goes on, and the relabel's sweep index and visit total are the base of the
-// next stall and budget tests.  *quit (or null): the relabel's waves gave up
-// waiting, so sweeping stops until the host has finished it.
-__global__ void k_relabel_end(SweepCtl c, unsigned char *hmat, int n, const int *quit, int resume) {
+// next stall and budget tests, its cost what the sweeps have to reach (charge; the
+// relabel before the first sweep costs nothing here).  *quit (or null): the
+// relabel's waves gave up waiting, so sweeping stops until the host has finished it.
+__global__ void k_relabel_end(SweepCtl c, unsigned char *hmat, int n, const int *quit, int resume,
+                              int charge) {
   int *st = c.state;
   const bool unfinished = quit && *quit;
   const int tid = blockIdx.x * blockDim.x + threadIdx.x;
-  if (tid == 0) {
-    const long long now = wall_clock64();
-    if (unfinished) {
-      st[2] = 5;
-      if (!resume) *(long long *)(st + 8) = now;
-    } else if (resume) {
-      st[2] = 0;
-      st[3] = st[1];
-      *(long long *)(st + 4) = c.total[0];
-      *(long long *)(st + 10) = now - *(const long long *)(st + 8);
-      *(long long *)(st + 8) = now;
+  if (tid < kFarSlots && (unfinished || resume)) {
+    int far = unfinished ? 0 : c.far[kFarLine * tid];
+    for (int o = 32; o > 0; o >>= 1) far = max(far, __shfl_xor(far, o));
+    if (tid == 0) {
+      st[2] = unfinished ? 5 : 0;
+      if (!unfinished) {
+        st[3] = st[1];
+        *(long long *)(st + 4) = c.total[0];
+        *(long long *)(st + 8) = 0;
+        *(long long *)(st + 10) = charge ? c.relabel_ns + c.level_ns * far : 0;
+      }
     }
   }
   if (unfinished) return;
@@ -1189,8 +1195,8 @@ __global__ void k_relabel_end(SweepCtl c, unsigned char *hmat, int n, const int 
 }
 
 void launch_relabel_end(const SweepCtl &c, unsigned char *hmat, int n, const int *quit, bool resume,
-                        hipStream_t st) {
-  k_relabel_end<<<grid_for(n, 256, 1024), 256, 0, st>>>(c, hmat, n, quit, resume);
+                        bool charge, hipStream_t st) {
+  k_relabel_end<<<grid_for(n, 256, 1024), 256, 0, st>>>(c, hmat, n, quit, resume, charge);
 }
 
 void launch_compact(const int *src, int n, int reverse, unsigned char *flag,

@@ -84,3 +84,36 @@ def test_search_longer_than_the_wait_gpu(gpu, shape):
     assert np.array_equal(g.labels(), l)
     assert st.relabel_passes == st.global_relabels
     g.close()
+
+
+def test_sweeps_do_not_depend_on_the_clock_gpu(gpu):
+    """When a stall relabels is decided by work, not by time: relabels that take
+    longer (a launch per pass) change no solve.  The graph's rows are chains of
+    their own, each in one wave of its tiles, so its sweeps are the same in every
+    run; a steady front moves along each."""
+    nx, ny = 4000, 64
+    rng = np.random.default_rng(5)
+    caps = np.zeros((4, ny, nx), np.int32)
+    caps[0, :, :-1] = rng.integers(40, 60, (ny, nx - 1))
+    caps[1, :, 1:] = rng.integers(0, 60, (ny, nx - 1))
+    cs, ct = np.zeros((2, ny, nx), np.int32)
+    cs[:, 0] = rng.integers(20, 60, ny)
+    ct[:, -1] = rng.integers(20, 60, ny)
+    cs, ct, caps = cs.ravel(), ct.ravel(), caps.reshape(4, -1)
+    f, l, ok = ol.maxflow(nx, ny, 1, 4, cs, ct, caps)
+    g = make(gpu, (nx, ny, 1, 4), cs, ct, caps)
+    seen, stopped = set(), set()
+    for ticks in (2_000_000, 0, 2_000_000, 0):
+        say("case sweeps and the clock", ticks)
+        assert gpu.lib().jfc_debug_relabel_wait(g._h, ctypes.c_int64(ticks)) == 0
+        st = g.solve(tile_shape="32x8")
+        assert st.converged == 1 and g.flow() == f
+        assert np.array_equal(g.labels(), l)
+        seen.add((st.sweeps, st.global_relabels))
+        for first in (0, 1):
+            st = g.solve(tile_shape="32x8", max_sweeps=100, initial_relabel=first)
+            assert st.converged == 0
+            stopped.add((first, st.sweeps, st.global_relabels, g.flow(), g.labels().tobytes()))
+    assert len(seen) == 1 and min(seen)[1] >= 3, seen
+    assert len(stopped) == 2
+    g.close()
