@@ -353,7 +353,7 @@ __global__ __launch_bounds__(1024) void k_wm_lloyd(const uchar4 *img, W4 w, W4 s
       for (int q = 0; q < kLevels / 64; ++q) {
         const int b = 64 * q + (tid & 63);
         const unsigned count = s_acc[r][b];
-        sum += (double)count * (double)s_val[r & 3][b];
+        sum += count ? (double)count * (double)s_val[r & 3][b] : 0.0;  // (a value may be infinite)
         members += count;
       }
       sum = wave_sum(sum);
@@ -370,7 +370,7 @@ __global__ __launch_bounds__(1024) void k_wm_lloyd(const uchar4 *img, W4 w, W4 s
       float d[4];
       for (int q = 0; q < 4; ++q) d[q] = next[at + q] - m[at + q];
       const float len = sqrtf((d[0] * d[0] + d[1] * d[1]) + (d[2] * d[2] + d[3] * d[3]));
-      moved = !(len < 1.0f / 1024);
+      moved = len >= 1.0f / 1024;  // (a centroid that is not a number does not count)
     }
     if (!__ballot(moved) || it >= iterations) break;
   }

@@ -99,3 +99,24 @@ def test_ties_gpu(gpu, k, levels):
     rgba[:, :3] = (rgba[:, :1] % levels) * (255 // (levels - 1))
     rgba[:, 3] = 255
     check(gpu, shape, rgba, fg, bg, dict(lazy=True, k=k), solve=False)
+
+
+def test_weights_without_a_norm_gpu(gpu):
+    """Weights whose squares underflow normalise to infinity, and a 0 beside them
+    to no number.  A movement that is no number does not count, so one such
+    weight ends the k-means with its first assignment; with four, the clusters
+    but the first empty, and a byte that no member has adds nothing to a mean."""
+    shape = (67, 45, 1)
+    rgba, fg, bg = random_case(shape, 4)
+    rgba = np.maximum(rgba, 1)
+    g = gpu.GridGraph([shape + (4,)])
+    for n, its in ((1, 1), (4, 2)):
+        say("case widget weights without a norm", n)
+        st = g.model_widget(rgba, fg, bg, lazy=True, k=5, weight=[1e-30] * n + [0.0] * (4 - n))
+        assert list(st.iterations) == [its, its]
+        cent = np.ctypeslib.as_array(st.centroids)[:, :5]
+        if n == 1:
+            assert np.isposinf(cent[..., 0]).all() and np.isnan(cent[..., 1:]).all()
+        else:
+            assert np.isposinf(cent[:, 0]).all() and (cent[:, 1:] == 0).all()
+    g.close()
