@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <cstdint>
 #include <string>
+#include <vector>
 
 namespace jfc {
 
@@ -112,7 +113,8 @@ void set_last_error(const std::string &msg);
 // ---- launchers (all asynchronous on `st`) --------------------------------
 void launch_fill_i32(int *p, long long n, int v, hipStream_t st);
 void launch_fill_u8(unsigned char *p, long long n, unsigned char v, hipStream_t st);
-// Up to 8 fills in one launch (bytes = 1 or 4 per element).
+// Fills in one launch, up to kMax of them, else in several (bytes = 1 or 4 per
+// element).
 struct FillSeg {
   void *p;
   long long n;
@@ -120,11 +122,10 @@ struct FillSeg {
   int bytes;
 };
 struct FillSet {
-  static constexpr int kMax = 12;
-  FillSeg seg[kMax];
-  int n = 0;
+  static constexpr int kMax = 8;
+  std::vector<FillSeg> seg;
   void add(void *p, long long count, int v, int bytes) {
-    if (count > 0 && n < kMax) seg[n++] = FillSeg{p, count, v, bytes};
+    if (count > 0) seg.push_back(FillSeg{p, count, v, bytes});
   }
 };
 void launch_fill_multi(const FillSet &f, hipStream_t st);

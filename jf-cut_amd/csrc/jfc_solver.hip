@@ -59,8 +59,11 @@ void launch_fill_u8(unsigned char *p, long long n, unsigned char v, hipStream_t 
 }
 
 // Several fills in one launch: blockIdx.y picks the segment.
-__global__ void k_fill_multi(FillSet f) {
-  if ((int)blockIdx.y >= f.n) return;
+struct FillArgs {
+  FillSeg seg[FillSet::kMax];
+};
+
+__global__ void k_fill_multi(FillArgs f) {
   const FillSeg s = f.seg[blockIdx.y];
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < s.n;
        i += (long long)gridDim.x * blockDim.x) {
@@ -70,10 +73,16 @@ __global__ void k_fill_multi(FillSet f) {
 }
 
 void launch_fill_multi(const FillSet &f, hipStream_t st) {
-  if (f.n <= 0) return;
-  long long most = 1;
-  for (int k = 0; k < f.n; ++k) most = std::max(most, f.seg[k].n);
-  k_fill_multi<<<dim3(grid_for(most, 256, 1024), f.n), 256, 0, st>>>(f);
+  for (size_t k0 = 0; k0 < f.seg.size(); k0 += FillSet::kMax) {
+    const int n = (int)std::min<size_t>(FillSet::kMax, f.seg.size() - k0);
+    FillArgs a{};
+    long long most = 1;
+    for (int k = 0; k < n; ++k) {
+      a.seg[k] = f.seg[k0 + k];
+      most = std::max(most, a.seg[k].n);
+    }
+    k_fill_multi<<<dim3(grid_for(most, 256, 1024), n), 256, 0, st>>>(a);
+  }
 }
 
 // Hard seeds from the caller's unpadded seed bytes (row r of nx bytes) onto
