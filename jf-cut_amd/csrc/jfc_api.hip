@@ -183,6 +183,7 @@ struct jfc_graph {
   int ntiles = 0, ncolors = 2, max_tile_dim = 1, nbins = 2;
   std::vector<int> color_off;
   // device planes
+  int *node_block = nullptr;  // cs, ct, e, h, mask0 and rmask
   int *cs = nullptr, *ct = nullptr, *c0 = nullptr, *cap = nullptr;
   int *e = nullptr, *h = nullptr;
   unsigned char *lab = nullptr;
@@ -316,7 +317,10 @@ struct jfc_graph {
     release_tiles();
     dfree(rg.block);
     rg = Regions{};
-    dfree(cs); dfree(ct); dfree(c0); dfree(cap); dfree(e); dfree(h); dfree(lab); dfree(tag);
+    dfree(node_block);
+    cs = ct = e = h = nullptr;
+    mask0 = rmask = nullptr;
+    dfree(c0); dfree(cap); dfree(lab); dfree(tag);
     dfree(d_ctr); dfree(d_res); dfree(d_sweep); dfree(d_energy); dfree(d_row_off);
     d_red = d_total = d_def = nullptr;
     d_sweep_state = d_flagword = nullptr;
@@ -341,7 +345,6 @@ struct jfc_graph {
     pin = nullptr;
     pin_res = nullptr;
     ring = d_ring = nullptr;
-    dfree(mask0); dfree(rmask);
     for (hipEvent_t ev : ev_pool) (void)hipEventDestroy(ev);
     ev_pool.clear();
   }
@@ -404,7 +407,8 @@ struct jfc_graph {
     // so no node is in one tile of the class and in the halo of another it
     // pushes across.  2D 4C and 3D 6C: checkerboard; 2D 8C: 2x2 pattern.
     ncolors = (dim == 2 && !all4) ? 4 : 2;
-    std::vector<int> tile_inst(ntiles);
+    const bool one = inst.size() == 1;  // (its tiles' instance is 0)
+    std::vector<int> tile_inst(one ? 0 : ntiles);
     std::vector<std::vector<int>> cls(ncolors);
     for (size_t i = 0; i < inst.size(); ++i) {
       const InstDesc &I = inst[i];
@@ -412,7 +416,7 @@ struct jfc_graph {
         for (int y = 0; y < I.ty; ++y)
           for (int x = 0; x < I.tx; ++x) {
             const int t = I.tile_off + x + I.tx * (y + I.ty * z);
-            tile_inst[t] = (int)i;
+            if (!one) tile_inst[t] = (int)i;
             const int c = ncolors == 4 ? ((x & 1) | ((y & 1) << 1)) : ((x + y + z) & 1);
             cls[c].push_back(t);
           }
@@ -437,7 +441,8 @@ struct jfc_graph {
         (rc = dalloc(&d_touched, ntiles, "tile states")))
       return rc;
     JFC_HIP(hipMemcpy(d_inst, inst.data(), inst.size() * sizeof(InstDesc), hipMemcpyHostToDevice));
-    JFC_HIP(hipMemcpy(d_tile_inst, tile_inst.data(), ntiles * sizeof(int), hipMemcpyHostToDevice));
+    if (one) launch_fill_i32(d_tile_inst, ntiles, 0, 0);  // (done before the copy behind it)
+    else JFC_HIP(hipMemcpy(d_tile_inst, tile_inst.data(), ntiles * sizeof(int), hipMemcpyHostToDevice));
     JFC_HIP(hipMemcpy(d_color_tiles, flat.data(), ntiles * sizeof(int), hipMemcpyHostToDevice));
     return JFC_OK;
   }
@@ -461,11 +466,6 @@ struct jfc_graph {
     }
     rg.n = (int)off;
     rg.buf.planes = Kg + region_state_planes();
-    std::vector<int> tile_inst(rg.n);
-    for (size_t i = 0; i < rg.inst.size(); ++i) {
-      const InstDesc &I = rg.inst[i];
-      std::fill(tile_inst.begin() + I.tile_off, tile_inst.begin() + I.tile_off + I.ntiles, (int)i);
-    }
     const size_t border = (size_t)rg.n * region_border_words(d3);
     // one allocation, carved in 256-byte steps (the first walk sizes it)
     const size_t n = rg.n;
@@ -496,6 +496,15 @@ struct jfc_graph {
     launch_fill_i32(rg.buf.border, (long long)border, 0, 0);
     JFC_HIP(hipMemcpy(rg.d_inst, rg.inst.data(), rg.inst.size() * sizeof(InstDesc),
                       hipMemcpyHostToDevice));
+    if (rg.inst.size() == 1) {
+      launch_fill_i32(rg.d_tile_inst, rg.n, 0, 0);
+      return JFC_OK;
+    }
+    std::vector<int> tile_inst(rg.n);
+    for (size_t i = 0; i < rg.inst.size(); ++i) {
+      const InstDesc &I = rg.inst[i];
+      std::fill(tile_inst.begin() + I.tile_off, tile_inst.begin() + I.tile_off + I.ntiles, (int)i);
+    }
     JFC_HIP(hipMemcpy(rg.d_tile_inst, tile_inst.data(), rg.n * sizeof(int),
                       hipMemcpyHostToDevice));
     return JFC_OK;
@@ -668,20 +677,27 @@ static int create_impl(jfc_graph **out, int count, const int32_t *shapes) {
   g->flows.assign(count, 0);
   int rc;
   const size_t N = (size_t)off;
-  if ((rc = dalloc(&g->cs, N, "source capacities")) ||
-      (rc = dalloc(&g->ct, N, "sink capacities")) ||
+  // the planes of one word per node in one block: an allocation of megabytes
+  // takes 20 to 30 us, and freeing it more
+  if ((rc = dalloc(&g->node_block, 6 * N, "node planes")) ||
       (rc = dalloc(&g->c0, N * g->Kg, "neighbour capacities")) ||
       (rc = dalloc(&g->cap, N * g->Kg, "residual capacities")) ||
-      (rc = dalloc(&g->e, N, "excess")) || (rc = dalloc(&g->h, N, "heights")) ||
       (rc = dalloc(&g->lab, N, "labels")) || (rc = dalloc(&g->d_ctr, 2 * QSLOT, "queues")) ||
-      (rc = dalloc(&g->mask0, N, "residual masks")) ||
-      (rc = dalloc(&g->rmask, N, "residual masks")) ||
       (rc = dalloc(&g->d_res, kResFixed + (size_t)count * (RED_SLOTS + 1), "results")) ||
       (rc = dalloc(&g->d_energy, (size_t)count, "reductions")) ||
       (rc = dalloc(&g->d_row_off, (size_t)count + 1, "row table"))) {
     delete g;
     return rc;
   }
+  // (rows are padded to 32 nodes, so every plane starts at a multiple of 128 bytes)
+  int *const plane[6] = {g->node_block,         g->node_block + N,     g->node_block + 2 * N,
+                         g->node_block + 3 * N, g->node_block + 4 * N, g->node_block + 5 * N};
+  g->cs = plane[0];
+  g->ct = plane[1];
+  g->e = plane[2];
+  g->h = plane[3];
+  g->mask0 = (unsigned *)plane[4];
+  g->rmask = (unsigned *)plane[5];
   g->res_words = kResFixed + (size_t)count * (RED_SLOTS + 1);
   g->d_red = g->d_res;
   g->d_def = g->d_red + (size_t)count * RED_SLOTS;
@@ -705,14 +721,9 @@ static int create_impl(jfc_graph **out, int count, const int32_t *shapes) {
     }
   }
   // everything zero, so the pad nodes of the rows stay isolated and empty
-  launch_fill_i32(g->cs, off, 0, 0);
-  launch_fill_i32(g->ct, off, 0, 0);
+  launch_fill_i32(g->node_block, 6 * off, 0, 0);
   launch_fill_i32(g->c0, off * g->Kg, 0, 0);
   launch_fill_i32(g->cap, off * g->Kg, 0, 0);
-  launch_fill_i32(g->e, off, 0, 0);
-  launch_fill_i32(g->h, off, 0, 0);
-  launch_fill_i32((int *)g->mask0, off, 0, 0);
-  launch_fill_i32((int *)g->rmask, off, 0, 0);
   launch_fill_u8(g->lab, off, 0, 0);
   int dev = 0;
   hipDeviceProp_t prop;
