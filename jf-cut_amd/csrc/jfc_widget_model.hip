@@ -269,7 +269,7 @@ __global__ __launch_bounds__(256) void k_wm_scan(const uchar4 *img, const unsign
 // scalar registers.
 template <int KB>
 __global__ __launch_bounds__(1024) void k_wm_lloyd(const uchar4 *img, W4 w, W4 scale, int k,
-                                                   int iterations, WmScratch S) {
+                                                   int iterations, int limit, WmScratch S) {
   __shared__ unsigned s_acc[KB * 4][kLevels];
   __shared__ float s_val[4][kLevels];  // weighted feature of a byte per channel
   __shared__ float s_cent[2][KB * 4];  // the centroids, and those of the next iteration
@@ -278,7 +278,7 @@ __global__ __launch_bounds__(1024) void k_wm_lloyd(const uchar4 *img, W4 w, W4 s
   const int side = blockIdx.x, tid = threadIdx.x;
   const int n = S.ctl[side];
   if (n == 0) return;
-  if (n > kLloydSeeds) {
+  if (n > limit) {
     if (tid == 0) S.ctl[2] = 1;
     return;
   }
@@ -353,7 +353,7 @@ __global__ __launch_bounds__(1024) void k_wm_lloyd(const uchar4 *img, W4 w, W4 s
       for (int q = 0; q < kLevels / 64; ++q) {
         const int b = 64 * q + (tid & 63);
         const unsigned count = s_acc[r][b];
-        sum += count ? (double)count * (double)s_val[r & 3][b] : 0.0;  // (a value may be infinite)
+        sum += (double)count * (double)s_val[r & 3][b];
         members += count;
       }
       sum = wave_sum(sum);
@@ -370,7 +370,7 @@ __global__ __launch_bounds__(1024) void k_wm_lloyd(const uchar4 *img, W4 w, W4 s
       float d[4];
       for (int q = 0; q < 4; ++q) d[q] = next[at + q] - m[at + q];
       const float len = sqrtf((d[0] * d[0] + d[1] * d[1]) + (d[2] * d[2] + d[3] * d[3]));
-      moved = len >= 1.0f / 1024;  // (a centroid that is not a number does not count)
+      moved = !(len < 1.0f / 1024);
     }
     if (!__ballot(moved) || it >= iterations) break;
   }
@@ -551,7 +551,7 @@ W4 normalize_weight(const float in[4]) {
 // assignment per launch and the update here; ctl and cent of `back` (the host
 // copy of the scratch) and of the scratch are completed, the unary's guard
 // lifted.
-static int lloyd_on_host(const uchar4 *img, const W4 &w, int k, int iterations,
+static int lloyd_on_host(const uchar4 *img, const W4 &w, int k, int iterations, int limit,
                          const WmScratch &S, unsigned char *back, hipStream_t st) {
   int *ctl = (int *)back;
   float *cent_used = (float *)(back + kCtlBytes + kHistBytes);
@@ -561,7 +561,7 @@ static int lloyd_on_host(const uchar4 *img, const W4 &w, int k, int iterations,
     for (int b = 0; b < kLevels; ++b) val[c][b] = unorm8(b) * w.v[c];
   for (int side = 0; side < 2; ++side) {
     const int cnt = ctl[side];
-    if (cnt <= kLloydSeeds) continue;
+    if (cnt <= limit) continue;
     // initial centroids: the representatives of the seeded levels, picked at
     // (count - 1) * i / (k - 1) (QGCW:2011-2039), scaled by weight / 255
     std::vector<unsigned> rep(kLevels);
@@ -694,6 +694,11 @@ extern "C" int jfc_model_widget(jfc_graph *g, int inst, const uint8_t *rgba, con
   const uchar4 *img = reinterpret_cast<const uchar4 *>(rgba);
   const unsigned char *dfg = fg, *dbg = bg;
   WmScratch S{};
+  // Seeds a side that k_wm_lloyd takes: none where a weight has no finite norm,
+  // whose sums and movements (infinite, or no number) are the host's.
+  int limit = kLloydSeeds;
+  for (int c = 0; c < 4; ++c)
+    if (!std::isfinite(w.v[c])) limit = 0;
   bool written = false;
   jfc_widget_model_stats st_local;
   jfc_widget_model_stats &ST = stats ? *stats : st_local;
@@ -740,9 +745,9 @@ extern "C" int jfc_model_widget(jfc_graph *g, int inst, const uint8_t *rgba, con
       W4 scale;
       for (int c = 0; c < 4; ++c) scale.v[c] = w.v[c] / 255.0f;
       const int iters = prm->kmeans_iterations;
-      if (k <= 8) k_wm_lloyd<8><<<2, 1024, 0, st>>>(img, w, scale, k, iters, S);
-      else if (k <= 16) k_wm_lloyd<16><<<2, 1024, 0, st>>>(img, w, scale, k, iters, S);
-      else k_wm_lloyd<32><<<2, 1024, 0, st>>>(img, w, scale, k, iters, S);
+      if (k <= 8) k_wm_lloyd<8><<<2, 1024, 0, st>>>(img, w, scale, k, iters, limit, S);
+      else if (k <= 16) k_wm_lloyd<16><<<2, 1024, 0, st>>>(img, w, scale, k, iters, limit, S);
+      else k_wm_lloyd<32><<<2, 1024, 0, st>>>(img, w, scale, k, iters, limit, S);
     }
     WM_HIP(hipGetLastError());
     const int shift = d3 ? 3 : 2;
@@ -784,7 +789,7 @@ extern "C" int jfc_model_widget(jfc_graph *g, int inst, const uint8_t *rgba, con
       }
     }
     if (prm->lazy && ctl[2]) {
-      if ((rc = lloyd_on_host(img, w, k, prm->kmeans_iterations, S, back, st))) goto done;
+      if ((rc = lloyd_on_host(img, w, k, prm->kmeans_iterations, limit, S, back, st))) goto done;
       unary();
       WM_HIP(hipGetLastError());
       WM_HIP(hipStreamSynchronize(st));
