@@ -386,6 +386,7 @@ __global__ __launch_bounds__(64 * W) void k_flood_all(Tiles T, Planes P, FloodBu
   constexpr bool kAll = W > 1;
   const int lane = threadIdx.x & 63;
   if (!kAll && !TAG && A.stop && *A.cert) return;  // found while packing
+  begin(A.w);
   bool done = false, found = false;
   if (kAll) {
     Marks marks;

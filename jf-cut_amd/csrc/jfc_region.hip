@@ -204,8 +204,7 @@ __device__ __forceinline__ void region_visit(const Tiles &T, const Planes &P,
       const u64 t = found & cnt[j];
       if (__ballot(t != 0)) d |= 1 << j, found = t;
     }
-    int *at = A.far + kFarLine * (t & (kFarSlots - 1));
-    if (lane == 0 && *at < ebase + d) atomicMax(at, ebase + d);
+    if (lane == 0) atomicMax(A.far + kFarLine * (t & (kFarSlots - 1)), ebase + d);
   };
   // 2D visits load their state with everything else; a 3D visit's borders are
   // as large as its planes, and half of them end before the search, so it
@@ -672,6 +671,7 @@ __global__ __launch_bounds__(64 * W) void k_settle(Tiles T, Planes P, RegionBuf 
   __shared__ int s_done;
   constexpr bool kAll = W > 1;
   const int lane = threadIdx.x & 63;
+  begin(A.w);
   if (threadIdx.x < 64) {
     for (int l = 0; l < kBlock; ++l) *(u64 *)&inj[l * kWinPitch + 2 * lane] = 0;
     lds_order();

@@ -187,6 +187,12 @@ constexpr int kServed = 0, kMade = 1, kBegun = 2;  // the words of a slot's line
 constexpr long long kPlaceTicks = 20000;           // 200 us: a visit takes 10 to 50
 enum { kGo = 0, kDone = 1, kQuit = 2, kStop = 3 };
 
+// Counts a workgroup that has begun, at its start.
+__device__ __forceinline__ void begin(const SettleWords &A) {
+  if (threadIdx.x == 0)
+    (void)__hip_atomic_fetch_add(A.sums + kLine * (blockIdx.x & (kSlots - 1)) + kBegun, 1,
+                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 // Counts the marks of a visit that served `served` marks, then makes them.
 __device__ __forceinline__ void publish(const SettleWords &A, const Marks &marks, int served,
                                         int lane) {
@@ -231,9 +237,6 @@ __device__ __forceinline__ bool settle(const SettleWords &A, int n, bool all, lo
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
     return v;
   };
-  if (lane == 0)
-    (void)__hip_atomic_fetch_add(A.sums + kLine * slot + kBegun, 1, __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_AGENT);
   for (;;) {
     const int now = own ? shared_word(A.marks + kLine * (long long)mine) : 0;
     const int state = shared_word(A.state + kLine * slot);

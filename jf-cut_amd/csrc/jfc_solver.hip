@@ -1119,26 +1119,33 @@ __device__ __forceinline__ void post_stop(const SweepCtl &c, int seq, int stop) 
 }
 
 __global__ void k_sweep_end(SweepCtl c) {
+  // every word is loaded before any is stored: one lane's chain of round trips
+  // is what the kernel takes
   int *st = c.state;
-  const int seq = st[6];
+  const int seq = st[6], stopped = st[2], i = st[1], cnt = st[0], last = st[3];
+  const long long visits = c.total[0], from = *(const long long *)(st + 4);
+  const long long work = *(const long long *)(st + 8) + c.sweep_ns + c.visit_ns * cnt;
+  const long long cost = *(const long long *)(st + 10);
+  const int since = i - last;  // sweeps since the last relabel, before this one
+  const bool filed = c.stall_ratio > 0.0 && i < c.cap;
+  const int one = filed && since >= 1 ? c.hist[i - 1] : 0;
+  const int two = filed && since >= 3 ? c.hist[i - 2] : 0;
+  const int three = filed && since >= 3 ? c.hist[i - 3] : 0;
   st[6] = seq + 1;
-  if (st[2]) {
-    post_stop(c, seq, st[2]);
+  if (stopped) {
+    post_stop(c, seq, stopped);
     return;
   }
-  const int i = st[1];
-  const int cnt = st[0];
   if (i < c.cap) c.hist[i] = cnt;
   st[0] = 0;
   st[1] = i + 1;
-  *(long long *)(st + 8) += c.sweep_ns + c.visit_ns * cnt;
+  *(long long *)(st + 8) = work;
   int stop = 0;
   if (cnt == 0) {
     stop = 1;
   } else if (i + 1 >= c.max_sweeps) {
     stop = 3;
   } else {
-    const int since = i - st[3];  // sweeps since the last relabel, before this one
     // stalled: the active count repeats that of the sweep before, or two
     // sweeps running repeat the two before them (excess trading places
     // between two sets of tiles, sweep after sweep)
@@ -1159,14 +1166,11 @@ __global__ void k_sweep_end(SweepCtl c) {
     // Over other seeds, once by the clock and by cost: strokes 51.1 and 51.3, video
     // 8.87 and 8.92, volume 11.2 and 11.2, scan 1.71 and 1.70, 1023x767 0.95 and
     // 0.98, widget 0.53 and 0.53.
-    const bool paid = *(const long long *)(st + 8) >= *(const long long *)(st + 10);
-    if (c.stall_ratio > 0.0 && since >= 1 && paid && i < c.cap) {
-      stalled = near(cnt, c.hist[i - 1]);
-      if (!stalled && since >= 3)
-        stalled = near(cnt, c.hist[i - 2]) && near(c.hist[i - 1], c.hist[i - 3]);
+    if (filed && since >= 1 && work >= cost) {
+      stalled = near(cnt, one);
+      if (!stalled && since >= 3) stalled = near(cnt, two) && near(one, three);
     }
-    const long long done = c.total[0] - *(const long long *)(st + 4);
-    const bool budget = c.budget > 0 && (double)done > (double)c.budget;
+    const bool budget = c.budget > 0 && (double)(visits - from) > (double)c.budget;
     if (stalled) stop = 2;
     else if (budget) stop = 4;
   }
@@ -1184,16 +1188,18 @@ void launch_sweep_end(const SweepCtl &c, hipStream_t st) { k_sweep_end<<<1, 1, 0
 __global__ void k_relabel_end(SweepCtl c, unsigned char *hmat, int n, const int *quit, int resume,
                               int charge) {
   int *st = c.state;
-  const bool unfinished = quit && *quit;
   const int tid = blockIdx.x * blockDim.x + threadIdx.x;
+  int far = tid < kFarSlots ? c.far[kFarLine * tid] : 0;
+  const long long total = c.total[0];
+  const int sweep = st[1];
+  const bool unfinished = quit && *quit;
   if (tid < kFarSlots && (unfinished || resume)) {
-    int far = unfinished ? 0 : c.far[kFarLine * tid];
     for (int o = 32; o > 0; o >>= 1) far = max(far, __shfl_xor(far, o));
     if (tid == 0) {
       st[2] = unfinished ? 5 : 0;
       if (!unfinished) {
-        st[3] = st[1];
-        *(long long *)(st + 4) = c.total[0];
+        st[3] = sweep;
+        *(long long *)(st + 4) = total;
         *(long long *)(st + 8) = 0;
         *(long long *)(st + 10) = charge ? c.relabel_ns + c.level_ns * far : 0;
       }
