@@ -49,6 +49,10 @@ int jfc_debug_sweep_counts(jfc_graph *g, int32_t *counts, int32_t n);
  * (0: as soon as a wavefront is idle). */
 int jfc_debug_relabel_wait(jfc_graph *g, int64_t ticks);
 
+/* on: the graph's searches go by a launch per pass, as those of graphs with more
+ * regions than a one-launch search can look after do. */
+int jfc_debug_search_passes(jfc_graph *g, int on);
+
 #ifdef __cplusplus
 }
 #endif

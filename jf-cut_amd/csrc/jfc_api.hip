@@ -220,6 +220,7 @@ struct jfc_graph {
     // time without progress after which a one-launch search leaves the rest to
     // passes: far above the ~50 us of a visit
     long long wait_ticks = 2000000;  // 20 ms
+    bool by_passes = false;  // every search takes a launch per pass
   } rg;
   // One device block holds every word a solve reads back at its end (one
   // copy): the per-instance sums, the remaining deficits, the counters, the
@@ -1175,8 +1176,8 @@ struct Solver {
     launch_fill_multi(f, st);
   }
 
-  // A search of this solve gave up waiting: something else holds places on the
-  // device, and the searches left go by passes.
+  // The searches go by passes: one gave up waiting, as something else holds places
+  // on the device, or the graph has it so.
   bool by_passes = false;
 
   // A cut or tag flood over the regions (jfc_flood.hip).  fills: zeroing of the
@@ -1645,6 +1646,7 @@ extern "C" int jfc_solve(jfc_graph *g, const jfc_options *opt, jfc_stats *stats)
   if (!g) return fail(JFC_ERR_INVALID, "null graph");
   Solver S{};
   S.g = g;
+  S.by_passes = g->rg.by_passes;
   if (opt) S.o = *opt;
   else jfc_default_options(&S.o);
   if (S.o.max_sweeps <= 0) S.o.max_sweeps = 1 << 20;
@@ -1741,6 +1743,7 @@ extern "C" int jfc_get_tags(jfc_graph *g, int inst, const uint8_t *fg, uint8_t *
   if ((rc = put_rows(g, g->inst[inst], g->tag + o, fg, 1, on_device))) return rc;
   Solver S{};
   S.g = g;
+  S.by_passes = g->rg.by_passes;
   jfc_default_options(&S.o);
   S.st = g->ustream;
   S.tm.pool = &g->ev_pool;
@@ -2014,6 +2017,12 @@ extern "C" int jfc_backward_all(jfc_graph *g, float *d_cap_source, float *d_cap_
 extern "C" int jfc_debug_relabel_wait(jfc_graph *g, int64_t ticks) {
   if (!g || ticks < 0) return fail(JFC_ERR_INVALID, "bad argument");
   g->rg.wait_ticks = ticks;
+  return JFC_OK;
+}
+
+extern "C" int jfc_debug_search_passes(jfc_graph *g, int on) {
+  if (!g) return fail(JFC_ERR_INVALID, "null graph");
+  g->rg.by_passes = on != 0;
   return JFC_OK;
 }
 
