@@ -142,13 +142,15 @@ typedef struct {
   int converged;            /* 1 if every instance reached the certificate */
   int sweeps;               /* push-relabel sweeps run */
   int global_relabels;      /* exact global relabels run */
-  int relabel_passes;       /* region passes inside the global relabels */
-  int cut_passes;           /* tile passes of the canonical-cut search */
+  int relabel_passes;       /* region passes inside the global relabels (a relabel
+                               that takes them in one launch counts 1) */
+  int cut_passes;           /* region passes of the canonical-cut searches (one that
+                               takes them in one launch counts 1) */
   int certificate_failures; /* cut searches that still found an augmenting path */
   int64_t push_tiles;       /* tile visits of the push-relabel kernel */
   int64_t push_launches;    /* push-relabel kernel launches */
   int64_t relabel_tiles;    /* region visits of the relabel kernel */
-  int64_t cut_tiles;        /* tile visits of the cut kernel */
+  int64_t cut_tiles;        /* region visits of the cut kernel */
   int64_t push_bytes;       /* algorithmic HBM bytes of the push-relabel visits */
   double ms_total;          /* device time of the solve (HIP events) */
   double ms_push;           /* summed push-relabel launch time (profile = 1) */

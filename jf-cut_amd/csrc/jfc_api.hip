@@ -257,19 +257,13 @@ struct jfc_graph {
   // setters, the data term, the outputs and the backward issue their work
   // on it and wait for that stream alone.  NULL: the legacy default stream.
   hipStream_t ustream = nullptr;
-  // Pinned host words the solve's decisions read (asynchronous copies, then
-  // a wait on an event instead of a staged pageable copy).
-  struct HostPin {
-    long long total;  // tile visits so far (sweep checks)
-    int recent[3];    // active tiles of the latest sweeps
-    int flag;         // certificate word of a cut search
-    long long red[RED_SLOTS];  // one instance's sums (energy)
-  } *pin = nullptr;
+  long long *pin = nullptr;  // pinned word for jfc_get_energy's sum
   // Pinned copy of d_res (the solve's results).
   long long *pin_res = nullptr;
-  // Stop words the sweeps post (k_sweep_end), then the words of two groups
-  // of search passes, of a setter's range check, and of a flood that gave up
-  // waiting, in fine-grained pinned memory the device writes through to; d_ring is its device address.
+  // Stop words the sweeps post (k_sweep_end), then the words of two groups of
+  // search passes, of a setter's range check, and of a flood that gave up
+  // waiting, in fine-grained pinned memory the device writes through to; d_ring
+  // is its device address.
   int *ring = nullptr, *d_ring = nullptr;
   hipEvent_t cnt_ev[2] = {nullptr, nullptr};
   int ensure_pin() {
@@ -279,7 +273,7 @@ struct jfc_graph {
         ev = nullptr;
         return fail(JFC_ERR_DEVICE, "event creation failed");
       }
-    if (hipHostMalloc((void **)&pin, sizeof(HostPin), hipHostMallocDefault) != hipSuccess ||
+    if (hipHostMalloc((void **)&pin, sizeof(long long), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void **)&pin_res, res_words * sizeof(long long), hipHostMallocDefault) !=
             hipSuccess ||
         hipHostMalloc((void **)&ring, (kStopRing + 5) * sizeof(int), hipHostMallocCoherent) !=
@@ -1386,7 +1380,7 @@ struct Solver {
         q.total = g->d_total;
         q.stop = g->d_sweep_state + 2;
       } else {
-        launch_compact(g->d_color_tiles + g->color_off[c], n, 0, g->d_flag, g->d_mat,
+        launch_compact(g->d_color_tiles + g->color_off[c], n, g->d_flag, g->d_mat,
                        g->d_touched, q, g->d_sweep_state, g->d_total, g->d_sweep_state + 2, st,
                        g->d_hmat);
       }
@@ -1443,7 +1437,7 @@ struct Solver {
   // active tile in one list, Jacobi relabel, line pushes, active flags.
   void issue_fast_sweep() {
     Queue q = queue_from_list();
-    launch_compact(g->d_color_tiles, g->ntiles, 0, g->d_flag, nullptr, nullptr, q,
+    launch_compact(g->d_color_tiles, g->ntiles, g->d_flag, nullptr, nullptr, q,
                    g->d_sweep_state, g->d_total, g->d_sweep_state + 2, st);
     hipEvent_t a = o.profile ? tm.mark() : nullptr;
     launch_fc_sweep(g->shape, std::min(g->nwg, g->ntiles), g->tiles(), g->planes(), q,
@@ -1767,10 +1761,10 @@ extern "C" int jfc_get_energy(jfc_graph *g, int inst, int64_t *energy) {
   const int nI = (int)g->inst.size();
   launch_fill_i32((int *)g->d_energy, 2LL * nI, 0, g->ustream);
   launch_energy(g->shape, g->tiles(), g->planes(), g->d_energy, g->ustream);
-  JFC_HIP(hipMemcpyAsync(&g->pin->red[0], g->d_energy + inst, sizeof(long long),
+  JFC_HIP(hipMemcpyAsync(g->pin, g->d_energy + inst, sizeof(long long),
                          hipMemcpyDeviceToHost, g->ustream));
   if ((rc = sync_user(g))) return rc;
-  *energy = g->pin->red[0];
+  *energy = *g->pin;
   return JFC_OK;
 }
 

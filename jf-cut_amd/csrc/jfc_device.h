@@ -99,11 +99,6 @@ __device__ __forceinline__ long long node_index(const InstDesc &I, int x, int y,
   return I.node_off + x + (long long)I.px * (y + (long long)I.ny * z);
 }
 
-template <class S>
-__device__ __forceinline__ int tile_of(const InstDesc &I, int x, int y, int z) {
-  return I.tile_off + x / S::TW + I.tx * (y / S::TH + I.ty * (z / S::TD));
-}
-
 // Lane layout inside the tile.
 template <class S>
 struct Lane {
@@ -132,27 +127,5 @@ __device__ __forceinline__ void pad_coords(int p, int &x, int &y, int &z,
 }
 
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
-
-// Append `t` (if pred) to a list with one atomic per wave.
-__device__ __forceinline__ void wave_append(bool pred, int t, int *list,
-                                            int *count, int *sweep_cnt,
-                                            long long *total) {
-  const unsigned long long m = __ballot(pred);
-  const int n = __popcll(m);
-  if (n == 0) return;
-  const int lane = lane_id();
-  const int leader = __ffsll((long long)m) - 1;
-  int base = 0;
-  if (lane == leader) {
-    base = atomicAdd(count, n);
-    if (sweep_cnt) atomicAdd(sweep_cnt, n);
-    if (total) atomicAdd((unsigned long long *)total, (unsigned long long)n);
-  }
-  base = __shfl(base, leader);
-  if (pred) {
-    const unsigned long long below = m & ((1ull << lane) - 1ull);
-    list[base + __popcll(below)] = t;
-  }
-}
 
 }  // namespace jfc

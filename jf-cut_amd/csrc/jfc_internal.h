@@ -208,7 +208,7 @@ constexpr int kEntryClean = 1 << 29;
 constexpr int kEntryHeights = 1 << 28;
 constexpr int kEntryTile = kEntryHeights - 1;
 // stop (or null): a nonzero word makes the compaction a no-op.
-void launch_compact(const int *src, int n, int reverse, unsigned char *flag,
+void launch_compact(const int *src, int n, unsigned char *flag,
                     const unsigned char *mat, const unsigned char *touched, const Queue &q,
                     int *sweep_cnt, long long *total, const int *stop, hipStream_t st,
                     const unsigned char *hmat = nullptr);
