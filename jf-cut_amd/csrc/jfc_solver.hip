@@ -643,14 +643,19 @@ void launch_energy(int shape, const Tiles &T, const Planes &P, long long *energy
 // Subgradient of the cut energy for instance `inst` (outputs in the
 // instance's own node numbering).
 // Bound by its writes, a float per node and output plane.  A wave takes chunks of
-// 256 nodes of consecutive rows, 4 nodes per lane: the callers' rows have no
-// padding, so what a wave writes to a plane is one run that shares only its end
-// lines with the next (rows of 32-node tiles, of which every line was shared,
-// took 807 us for 256 uneven images; this takes 446), and a lane reads the
-// labels around its nodes as words.
+// 256 nodes of consecutive rows, 4 nodes per lane, or as many whole rows of up to
+// 128 nodes at once as its lanes hold: the callers' rows have no padding, so what
+// a wave writes to a plane is one run that shares only its end lines with the
+// next (rows of 32-node tiles, of which every line was shared, took 807 us for
+// 256 uneven images; this takes 446), and a lane reads the labels around its
+// nodes as words.  With a row at a time whatever its length, and a binary search
+// for its instance, a call over 1x2000000 took 996 us, over 8x256x256 49 and over
+// 2000 grids of 16x16 42; they take 44,
+// 23 and 25.
 struct alignas(4) Float4 {
   float v[4];
 };
+constexpr int kShortRow = 32;  // groups of 4 nodes in a row that is taken with others
 
 template <bool D3>
 __global__ __launch_bounds__(256) void k_backward(Tiles T, Planes P, int row0, int nrows,
@@ -662,96 +667,116 @@ __global__ __launch_bounds__(256) void k_backward(Tiles T, Planes P, int row0, i
   int row = row0 + wave * rows_per_wave;
   const int end = min(row0 + nrows, row + rows_per_wave);
   if (row >= end) return;
+  // the row's instance: the last that begins at or before it, a lane per candidate
   int inst = 0;
-  for (int hi = T.ninst - 1; inst < hi;) {
-    const int mid = (inst + hi + 1) >> 1;
-    if (T.row_off[mid] <= row) inst = mid;
-    else hi = mid - 1;
+  for (int n = T.ninst; n > 1;) {
+    const int step = (n + 63) / 64, mine = lane * step;
+    const bool begun = mine < n && T.row_off[inst + mine] <= row;
+    const int k = __popcll(__ballot(begun)) - 1;
+    inst += k * step;
+    n = min(step, n - k * step);
   }
   InstDesc I = T.inst[inst];
-  int last = T.row_off[inst + 1], rr = row - T.row_off[inst];
-  int y = rr % I.ny, z = rr / I.ny;
-  for (; row < end; ++row) {
-    if (row == last) {
-      I = T.inst[++inst];
-      last = T.row_off[inst + 1];
-      rr = y = z = 0;
-    }
+  int first = T.row_off[inst], last = T.row_off[inst + 1];
+  // the 4 nodes from column x of row rr (y, z) of the instance
+  auto group = [&](int rr, int y, int z, int x) {
     // outputs in the callers' numbering: one instance (user_total = 0) its
     // own, with plane stride = its node count; all instances the graph's
     // concatenation, with plane stride = all their nodes
     const long long n = user_total ? user_total : (long long)I.nx * I.ny * I.nz;
     const long long out0 = (user_total ? I.user_off : 0) + (long long)rr * I.nx;
     const long long base = I.node_off + (long long)rr * I.px, slice = (long long)I.px * I.ny;
-    for (int x = (blockIdx.y * 64 + lane) * 4; x < I.nx; x += gridDim.y * 256) {
-      // bit i of the labels around the 4 nodes: column x - 1 + i of a row, set
-      // off the grid
-      auto nonzero = [](unsigned w) {
-        w |= w >> 4;
-        w |= w >> 2;
-        w |= w >> 1;
-        return ((w & 0x01010101u) * 0x01020408u) >> 24;
-      };
-      auto around = [&](bool have, long long step, bool wide) {
-        if (!have) return 63u;
-        const unsigned char *p = P.lab + base + step + x;
-        const int left = I.nx - x;  // columns x ... of the row
-        unsigned m = nonzero(*(const unsigned *)p) << 1;
-        if (wide && x > 0) m |= p[-1] ? 1u : 0u;
-        else m |= 1u;
-        if (wide && left > 4) m |= p[4] ? 32u : 0u;
-        else m |= 32u;
-        if (left < 4) m |= 63u << (left + 1) & 63u;
-        return m;
-      };
-      const unsigned own = around(true, 0, true);
-      const unsigned s = own >> 1 & 15u;
-      const int cnt = min(4, I.nx - x);
-      auto put = [&](float *plane, unsigned bits) {
-        float *q = plane + out0 + x;
-        if (cnt == 4) {
-          Float4 f;
+    // bit i of the labels around the 4 nodes: column x - 1 + i of a row, set
+    // off the grid
+    auto nonzero = [](unsigned w) {
+      w |= w >> 4;
+      w |= w >> 2;
+      w |= w >> 1;
+      return ((w & 0x01010101u) * 0x01020408u) >> 24;
+    };
+    auto around = [&](bool have, long long step, bool wide) {
+      if (!have) return 63u;
+      const unsigned char *p = P.lab + base + step + x;
+      const int left = I.nx - x;  // columns x ... of the row
+      unsigned m = nonzero(*(const unsigned *)p) << 1;
+      if (wide && x > 0) m |= p[-1] ? 1u : 0u;
+      else m |= 1u;
+      if (wide && left > 4) m |= p[4] ? 32u : 0u;
+      else m |= 32u;
+      if (left < 4) m |= 63u << (left + 1) & 63u;
+      return m;
+    };
+    const unsigned own = around(true, 0, true);
+    const unsigned s = own >> 1 & 15u;
+    const int cnt = min(4, I.nx - x);
+    auto put = [&](float *plane, unsigned bits) {
+      float *q = plane + out0 + x;
+      if (cnt == 4) {
+        Float4 f;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) f.v[i] = (bits >> i) & 1u ? 1.f : 0.f;
-          *(Float4 *)q = f;
-        } else {
-          for (int i = 0; i < cnt; ++i) q[i] = (bits >> i) & 1u ? 1.f : 0.f;
-        }
-      };
-      if (dcs) put(dcs, ~s);
-      if (dct) put(dct, s);
-      if (!dnb) continue;
-      const bool diag = !D3 && I.K > 4;
-      const unsigned up = around(y + 1 < I.ny, I.px, diag), dn = around(y > 0, -I.px, diag);
-      unsigned front = 0, back = 0;
-      if constexpr (D3) {
-        back = around(z + 1 < I.nz, slice, false);
-        front = around(z > 0, -slice, false);
+        for (int i = 0; i < 4; ++i) f.v[i] = (bits >> i) & 1u ? 1.f : 0.f;
+        *(Float4 *)q = f;
+      } else {
+        for (int i = 0; i < cnt; ++i) q[i] = (bits >> i) & 1u ? 1.f : 0.f;
       }
-#pragma unroll
-      for (int d = 0; d < KMAX; ++d) {
-        if (d >= I.K) break;
-        int dx, dy, dz;
-        dir_of<D3>(d, dx, dy, dz);
-        const unsigned m = dz > 0 ? back : dz < 0 ? front : dy > 0 ? up : dy < 0 ? dn : own;
-        put(dnb + d * n, s & ~(m >> (1 + dx)));
-      }
+    };
+    if (dcs) put(dcs, ~s);
+    if (dct) put(dct, s);
+    if (!dnb) return;
+    const bool diag = !D3 && I.K > 4;
+    const unsigned up = around(y + 1 < I.ny, I.px, diag), dn = around(y > 0, -I.px, diag);
+    unsigned front = 0, back = 0;
+    if constexpr (D3) {
+      back = around(z + 1 < I.nz, slice, false);
+      front = around(z > 0, -slice, false);
     }
-    ++rr;
-    if (++y == I.ny) {
-      y = 0;
-      ++z;
+#pragma unroll
+    for (int d = 0; d < KMAX; ++d) {
+      if (d >= I.K) break;
+      int dx, dy, dz;
+      dir_of<D3>(d, dx, dy, dz);
+      const unsigned m = dz > 0 ? back : dz < 0 ? front : dy > 0 ? up : dy < 0 ? dn : own;
+      put(dnb + d * n, s & ~(m >> (1 + dx)));
+    }
+  };
+  while (row < end) {
+    if (row == last) {
+      I = T.inst[++inst];
+      first = last;
+      last = T.row_off[inst + 1];
+    }
+    const int stop = min(end, last), ng = (I.nx + 3) / 4;
+    if (ng <= kShortRow) {
+      const int r = lane / ng, rows = 64 / ng;
+      if (blockIdx.y == 0 && r < rows)
+        for (int mine = row + r; mine < stop; mine += rows) {
+          const int rr = mine - first;
+          group(rr, rr % I.ny, rr / I.ny, 4 * (lane - r * ng));
+        }
+      row = stop;
+    } else {
+      int rr = row - first, y = rr % I.ny, z = rr / I.ny;
+      for (; row < stop; ++row, ++rr) {
+        for (int x = (blockIdx.y * 64 + lane) * 4; x < I.nx; x += gridDim.y * 256)
+          group(rr, y, z, x);
+        if (++y == I.ny) {
+          y = 0;
+          ++z;
+        }
+      }
     }
   }
 }
 
-// Rows [row0, row0 + nrows) of the graph; nx: the longest of them.
+// Rows [row0, row0 + nrows) of the graph; nx: the longest of them.  About 16,000
+// waves: of few rows each its own chunks, of many short ones several each.
 static void backward_rows(int shape, const Tiles &T, const Planes &P, int row0, int nrows, int nx,
                           float *dcs, float *dct, float *dnb, long long user_total,
                           hipStream_t st) {
-  const int chunks = std::min((nx + 255) / 256, 64);
-  const int per_wave = (int)std::max(1LL, (long long)nrows * chunks / 16384);
-  const dim3 grid((nrows + 4 * per_wave - 1) / (4 * per_wave), chunks);
+  const int chunks = std::min((nx + 255) / 256, std::max(64, 16384 / nrows));
+  const int ng = (nx + 3) / 4, together = ng <= kShortRow ? 64 / ng : 1;
+  const int per_wave = (int)std::max<long long>(together, (long long)nrows * chunks / 16384);
+  const dim3 grid((nrows + 4LL * per_wave - 1) / (4LL * per_wave), chunks);
   if (shape_is_3d(shape))
     k_backward<true><<<grid, 256, 0, st>>>(T, P, row0, nrows, per_wave, dcs, dct, dnb, user_total);
   else

@@ -75,3 +75,39 @@ def test_batch_gradients_gpu(gpu, batch, relabel):
         assert np.array_equal(v[2].cpu().numpy().reshape(conn, n), c)
         assert all(float(q[0]) == -1 and float(q[-1]) == -1 for q in t)
     g.close()
+
+
+@pytest.mark.parametrize("batch", [
+    [(1, 40000, 1, 8)], [(3, 9000, 1, 4)], [(124, 70, 1, 8)], [(128, 67, 1, 4)], [(129, 40, 1, 8)],
+    [(5, 40, 90, 6)], [(126, 9, 7, 6)], [(20000, 1, 1, 8)],
+    [(16, 16, 1, 8)] * 30 + [(1, 3, 1, 4)] * 9, [(128, 5, 1, 8), (129, 5, 1, 4), (2, 60, 1, 8)] * 3,
+], ids=lambda b: f"{len(b)}x{b[0][0]}-{b[0][3]}c")
+def test_short_rows_gradients_gpu(gpu, batch):
+    """Rows that a wave takes several of at once: lengths up to and past the 128
+    nodes where it does, many rows per wave, instances that begin inside a wave's
+    rows, and one row that many waves share."""
+    rng = np.random.default_rng(len(batch) + batch[0][0])
+    g = gpu.GridGraph(batch)
+    labs = []
+    for i, (nx, ny, nz, conn) in enumerate(batch):
+        cs, ct, caps = random_grid(rng, nx, ny, nz, conn)
+        cs[0] += 1
+        labs.append(ol.maxflow(nx, ny, nz, conn, cs, ct, caps)[1])
+        g.set_terminal_caps(cs, ct, inst=i)
+        g.set_all_neighbor_caps(caps, inst=i)
+    print("case short rows", batch[0], len(batch), flush=True)
+    assert g.solve().converged == 1
+    dcs, dct, dnb = g.backward_all()
+    at = 0
+    for i, shape in enumerate(batch):
+        n, conn, lab = labs[i].size, shape[3], labs[i]
+        ref = gradients(lab, shape, gpu.DIRS_3D if conn == 6 else gpu.DIRS_2D)
+        assert np.array_equal(dcs[at:at + n], (lab == 0).astype(np.float32))
+        assert np.array_equal(dct[at:at + n], (lab == 1).astype(np.float32))
+        assert np.array_equal(dnb[:conn, at:at + n], ref)
+        at += n
+        a, b, c = g.backward(i)
+        assert np.array_equal(a, (lab == 0).astype(np.float32))
+        assert np.array_equal(b, (lab == 1).astype(np.float32))
+        assert np.array_equal(c, ref)
+    g.close()
