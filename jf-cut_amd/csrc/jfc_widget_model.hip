@@ -175,7 +175,7 @@ __device__ __forceinline__ int unary_int(float v) {
 
 // Scratch of one call.  Everything up to rep is copied back at the end.
 struct WmScratch {
-  int *ctl;          // [0,1] seeded pixels per side, [2] a side has more than kLloydSeeds,
+  int *ctl;          // [0,1] seeded pixels per side, [2] a side has more than k_wm_lloyd takes,
                      // [3,4] k-means iterations
   unsigned *hist;    // [2][kLevels] seeded pixels per level
   float *cent;       // [2][kMaxK * 4] the centroids of the unary, side 1 from k * 4 on
@@ -185,6 +185,12 @@ struct WmScratch {
   unsigned char *owner;  // [2][kLloydSeeds] their clusters (k_wm_lloyd)
 };
 constexpr int kLloydSeeds = 65536;
+// ... and seeds times clusters: one compute unit a side takes the time of their
+// product, the host's iterations (an assignment over the whole device, a wait, the
+// update) little more for more of either.  32 clusters: 6.0 ms on the device and 6.6
+// by the host for 40,000 seeds, 7.1 and 7.2 for 48,000, 9.4 and 8.0 for 65,000; 24
+// clusters, 65,000: 7.1 and 8.4.
+constexpr int kLloydWork = 49152 * 32;
 constexpr size_t kCtlBytes = 64, kHistBytes = 2 * kLevels * 4, kCentBytes = 2 * kMaxK * 4 * 4,
                  kRepBytes = kHistBytes, kAccBytes = (size_t)kMaxK * 4 * kLevels * 4,
                  kOwnerBytes = 2 * kLloydSeeds;
@@ -251,7 +257,7 @@ __global__ __launch_bounds__(256) void k_wm_scan(const uchar4 *img, const unsign
   }
 }
 
-// The k-means of a side (blockIdx.x) with up to kLloydSeeds seeded pixels, one
+// The k-means of a side (blockIdx.x) with up to `limit` seeded pixels, one
 // workgroup of 1024 lanes: initial centroids from the seeded levels'
 // representatives, picked at (count - 1) * i / (k - 1) and scaled by weight /
 // 255 (QGCW:2011-2039), then Lloyd iterations (QGCW:2073-2102) until the
@@ -696,7 +702,7 @@ extern "C" int jfc_model_widget(jfc_graph *g, int inst, const uint8_t *rgba, con
   WmScratch S{};
   // Seeds a side that k_wm_lloyd takes: none where a weight has no finite norm,
   // whose sums and movements (infinite, or no number) are the host's.
-  int limit = kLloydSeeds;
+  int limit = std::min(kLloydSeeds, kLloydWork / k);
   for (int c = 0; c < 4; ++c)
     if (!std::isfinite(w.v[c])) limit = 0;
   bool written = false;

@@ -120,3 +120,17 @@ def test_weights_without_a_norm_gpu(gpu):
         else:
             assert np.isposinf(cent[:, 0]).all() and (cent[:, 1:] == 0).all()
     g.close()
+
+
+@pytest.mark.parametrize("rows", [128, 129])  # 48,896 / 49,278 seeds a side
+def test_many_seeds_and_clusters_gpu(gpu, rows):
+    """32 clusters: the k-means is the device's up to 49,152 seeds a side, the
+    host's above."""
+    shape = (382, 400, 1)
+    say("case widget many seeds and clusters", rows)
+    rgba, fg, bg = random_case(shape, rows)
+    fg, bg = np.zeros((400, 382), np.uint8), np.zeros((400, 382), np.uint8)
+    fg[:rows] = 1
+    bg[400 - rows:] = 1
+    check(gpu, shape, rgba, fg.ravel(), bg.ravel(), dict(lazy=True, k=32, kmeans_iterations=4),
+          solve=False)
