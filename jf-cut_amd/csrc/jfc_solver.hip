@@ -1272,7 +1272,9 @@ __global__ __launch_bounds__(256, kRingPerLane<S> > 1 || KK == 8 ? 6 : 7) void k
   // a sparse launch's cap doubles with every sweep up to sparse_iters: a solve
   // that ends within a few sweeps has nothing to gain from long visits
   const int sweep = min(sweep_state[1], 30);
-  const int cap_iters = Qc.count > (int)gridDim.x           ? max_iters
+  // (a direct list is of at most a few thousand tiles and counts those that are not
+  // active, too: never dense)
+  const int cap_iters = Qc.count > (int)gridDim.x && !q.pick ? max_iters
                         : (sparse_iters >> sweep) < max_iters ? sparse_iters
                                                               : max_iters << sweep;
   long long my_iters = 0;

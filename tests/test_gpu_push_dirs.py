@@ -38,3 +38,22 @@ def test_push_directions_gpu(gpu, conns, tile):
                 assert g.flow(inst=k) == f
                 assert np.array_equal(g.labels(inst=k), l)
         g.close()
+
+
+@pytest.mark.parametrize("conn,shape", [(8, (1500, 1100)), (6, (96, 96, 110))])
+def test_cap_of_sparse_launches_past_the_grid_gpu(gpu, conn, shape):
+    """Colour classes of more tiles than workgroups of a push launch that takes
+    its tiles from the flags: its visits go up to the cap of sparse launches, as
+    those of smaller classes do."""
+    nx, ny, nz = shape + (1,) * (3 - len(shape))
+    rng = np.random.default_rng(0)
+    cs, ct, caps = random_grid(rng, nx, ny, nz, conn, term_max=3, seed_frac=0.001)
+    g = gpu.GridGraph([(nx, ny, nz, conn)])
+    g.set_terminal_caps(cs, ct)
+    g.set_all_neighbor_caps(caps)
+    print("case cap of sparse launches", shape, conn, flush=True)
+    for cap in (2, 16):
+        st = g.solve(max_local_iters=2, sparse_local_iters=cap, initial_relabel=1, max_sweeps=8)
+        per_visit = st.local_iters / st.push_tiles
+        assert per_visit <= 2 if cap == 2 else per_visit > 3, (cap, per_visit)
+    g.close()
