@@ -122,11 +122,12 @@ struct RelabelCost {
   long long launch, region, level, certify;
 };
 constexpr RelabelCost kCost2D{15000, 16, 500, 20}, kCost3D{15000, 26, 1600, 20};
-// And of a sweep: its push launches, each as long as its longest visit (22 us
-// with 8 directions, else 15 to 20), and its tile visits, by the length of a
-// tile's rows.
-constexpr long long kPushNs = 18000, kPushNs8 = 22000, kVisitNs2D = 7, kVisitNs8x8x4 = 11,
-                    kVisitNs32x4x2 = 5;
+// And of a sweep: its push launches, each as long as its longest visit (8 us at
+// 2 iterations and 22 at 16 with 8 directions, else 6 and 18), and its tile
+// visits, by the length of a tile's rows.
+constexpr long long kPushNs = 5000, kIterNs8 = 1060, kIterNs = 810, kVisitNs2D = 7,
+                    kVisitNs8x8x4 = 11, kVisitNs32x4x2 = 5;
+constexpr int kCostIters = 64;  // visits of higher caps end before them
 std::mutex g_tune_mu;
 std::map<std::string, Tuned> g_tune;
 
@@ -1087,7 +1088,8 @@ struct Solver {
     c.budget = o.relabel_work > 0 ? (long long)std::floor(o.relabel_work * g->ntiles) : 0;
     c.ring = g->d_ring;
     c.ring_n = kStopRing;
-    c.sweep_ns = (g->Kg == 8 ? kPushNs8 : kPushNs) *
+    const int cap = std::min(std::max(o.max_local_iters, o.sparse_local_iters), kCostIters);
+    c.sweep_ns = (kPushNs + cap * (g->Kg == 8 ? kIterNs8 : kIterNs)) *
                  (o.method == JFC_METHOD_FASTCUT ? 2 + 2 * g->dim : g->ncolors);
     c.visit_ns = g->dim == 2 ? kVisitNs2D : g->shape == SH_8x8x4 ? kVisitNs8x8x4 : kVisitNs32x4x2;
     const RelabelCost &cost = g->dim == 3 ? kCost3D : kCost2D;
