@@ -76,7 +76,8 @@ typedef struct {
                              spent); sweeps queued past that point do nothing */
   double relabel_work;    /* run an exact global relabel once the tiles visited
                              since the last one exceed this many times the tile
-                             count (0 = only at start and on certificate failure) */
+                             count, or the sweeps since have cost 16 times as much
+                             as it (0 = only at start and on certificate failure) */
   int max_local_iters;    /* cap on LDS discharge iterations per tile visit
                              (0 = the cap jfc_autotune chose for the graph's
                              size class, else 2) */
