@@ -35,17 +35,16 @@
 // others are searched again from there.  A visit where none improves ends
 // before its search.  No height word is touched before kFinal.
 //
-// What bounds it, and what it measured (against 32x8 and 8x8x4 tiles relaxed
-// node by node in LDS, one launch for the list and one for the visits per
-// pass).  Long searches are a chain of visits, a pass after the other: on the
-// 3750x2500 8-connected cut from strokes alone a relabel takes ~65 passes of
-// ~26 us instead of ~300 of ~30 us, 27 ms of relabels instead of 116-154 in a
-// solve.  A level costs ~50 vector instructions for 4096 nodes; written as one
-// loop with every counting plane per level it cost 85, and such a pass 44
-// us.  Passes over every region are bound by memory and packing: on the
-// 512^3 volume kPack takes 425 us (8 bytes per node read: 226 us at the rate
-// of a large copy), kFinal 156 us (134 us).  There a relabel goes from 1.8 to
-// 1.5 ms, on the 2560x1440x50 video volume from 2.9-3.0 to 2.5-2.7 ms.
+// What bounds it, and what it measured.  Long searches are a chain of visits: on
+// the 3750x2500 8-connected cut from strokes alone a relabel of 55-73 passes takes
+// 1.05 ms in one launch (settle) and 1.6 with a launch per pass; tiles of 32x8
+// relaxed node by node in LDS took ~300 passes, 9 ms.  A level costs ~50 vector
+// instructions for 4096 nodes; written as one loop with every counting plane
+// per level it cost 85.  The first and last step over every region are bound by
+// memory and packing: on the 512^3 volume kPack takes 425 us (8 bytes per node
+// read: 226 us at the rate of a large copy), kFinal 156 us (134 us).  A relabel
+// there takes 1.65 ms in one launch, 1.78 by passes (1.8 on 8x8x4 tiles), of the
+// 2560x1440x50 video volume 1.8-2.0 and 2.5-3.0 (2.9-3.0).
 #include "jfc_rows.h"
 
 #include <algorithm>

@@ -178,9 +178,10 @@ struct Marks {
 //     searches that hold each other's places would wait for each other, so the
 //     first workgroup gives up after kPlaceTicks without progress.
 // It tells the others to quit and sets *quit, and the search is finished with
-// passes over every region.  Three threads that solve 128^3 volumes of their own:
-// 57 ms a solve where waves without a place were waited for 20 ms, 31 now (41 with a
-// launch per pass); 256x192x176: 138 and 83 (109).
+// passes over every region, as the solve's later searches are (a launch per pass
+// takes 1.1 to 1.6 times as long).  Three threads that solve 128^3 volumes of
+// their own: 57 ms a solve where workgroups without a place were waited for 20
+// ms, 31 now; 256x192x176: 138 and 83.
 constexpr int kSlots = kSettleSlots, kLine = kSettleLine;
 static_assert(kSlots == 64, "a lane per slot");
 constexpr int kServed = 0, kMade = 1, kBegun = 2;  // the words of a slot's line of sums
